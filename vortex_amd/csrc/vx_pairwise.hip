@@ -9,11 +9,13 @@
 // targets spaced one block apart so that target loads and stores coalesce.
 #include <algorithm>
 #include <cfloat>
+#include <cmath>
 #include <mutex>
 #include <string>
 
 
 #include "vx_internal.h"
+#include "vx_math.h"
 #include "vx_prim.h"
 
 namespace vx {
@@ -29,7 +31,7 @@ struct Arith;
 template <>
 struct Arith<double> {
     static constexpr double kFar = 1e30;  // padding sources: squared distance stays finite
-    __device__ static __forceinline__ double div(double a, double b) { return a / b; }
+    __device__ static __forceinline__ double div(double a, double b) { return div_pos(a, b); }
     __device__ static __forceinline__ double med3(double a, double b, double c) {
         return fmax(fmin(a, b), fmin(fmax(a, b), c));
     }
@@ -50,22 +52,120 @@ struct Arith<float> {
 
 constexpr int kTile = 256;
 
+// ---- work split of the direct kernels ---------------------------------------
+// A direct launch is cut over targets (kTile * TPT per work-group) and over
+// runs of `len` sources, whose partials a second kernel adds in run order.
+// One run per work-group would leave most of the chip idle below 64 k
+// vortices (10 work-groups at 2.5 k), so the runs are made short enough for
+// kDirectWork blocks of kTile targets in all.  The split depends on the
+// counts alone, not on TPT or on a launch's bound, so every launch shape,
+// stream step and graph replay adds in the same order.
+//
+// 60001 vortices, FP32: Biot-Savart 2.66 -> 1.02 ms, diffusion 2.66 -> 1.29 ms
+// against one work-group per kTile targets over all sources; 20011 in FP64:
+// 1.76 -> 0.30 and 3.43 -> 0.47 ms.  With kDirectWork = 1024, 2048 and 8192
+// the first pair takes 1.30 and 1.59, 1.09 and 1.40, 1.01 and 1.27 ms; the
+// partials grow with it (48 B per target and run), so 4096.
+//
+// FP32 sums are taken over tiles of kTile sources and added in FP64, so up to
+// kOrdered sources a run is one tile and the result is that of one pass over
+// the sources in order, bit for bit; a run is several tiles above.  FP64 sums
+// up to kOrdered sources go to the ordered kernels below for the same reason:
+// a run of many steps multiplies a rounding by 1e6 in 25 steps, so long runs
+// at these counts keep the order.
+constexpr int64_t kDirectWork = 4096;
+constexpr int64_t kOrdered = 16384;
+
+struct DirectSplit {
+    int32_t len, runs;
+};
+
 template <typename T>
-__device__ __forceinline__ void stage_tile(Src4<T> *ls, const T *__restrict__ sx, const T *__restrict__ sy,
-                                           const T *__restrict__ sg, int64_t base, int64_t n_src) {
-    const int64_t j = base + threadIdx.x;
-    Src4<T> s;
-    if (j < n_src) {
-        s.x = sx[j];
-        s.y = sy[j];
-        s.g = sg[j];
-    } else {
-        s.x = Arith<T>::kFar;
-        s.y = Arith<T>::kFar;
-        s.g = T(0);
-    }
-    s.pad = T(0);
-    ls[threadIdx.x] = s;
+__host__ __device__ __forceinline__ DirectSplit direct_split(int64_t n_tgt, int64_t n_src) {
+    constexpr uint32_t unit = sizeof(T) == 4 ? kTile : kTile / 4;
+    const uint32_t tb = (uint32_t)((n_tgt + kTile - 1) / kTile), units = (uint32_t)((n_src + unit - 1) / unit);
+    if (units == 0 || tb == 0) return DirectSplit{(int32_t)unit, 1};
+    uint32_t want = ((uint32_t)kDirectWork + tb - 1) / tb;
+    if (want > units || n_src <= kOrdered) want = units;
+    const uint32_t per = (units + want - 1) / want;
+    return DirectSplit{(int32_t)(per * unit), (int32_t)((units + per - 1) / per)};
+}
+
+// Blocks of kTile * tpt targets times runs: exact for host counts, else a
+// bound over all smaller counts (kernels leave surplus blocks at once).  The
+// runs of n sources number at most max(kDirectWork / tb + 1, kOrdered units).
+template <typename T>
+static int64_t direct_runs_max(int64_t n_tgt, int64_t n_src) {
+    constexpr int64_t unit = sizeof(T) == 4 ? kTile : kTile / 4;
+    const int64_t units = (n_src + unit - 1) / unit, tb = (n_tgt + kTile - 1) / kTile;
+    return std::max<int64_t>(std::min(units, kOrdered / unit), std::min(units, kDirectWork / std::max<int64_t>(tb, 1) + 1));
+}
+
+template <typename T>
+static int64_t direct_blocks(Cnt n_tgt, Cnt n_src, int tpt) {
+    const int64_t w = kTile * tpt, tb = (n_tgt.ub + w - 1) / w;
+    if (!n_tgt.dev && !n_src.dev) return tb * direct_split<T>(n_tgt.ub, n_src.ub).runs;
+    return tb * direct_runs_max<T>(n_tgt.ub, n_src.ub) + kDirectWork / tpt;
+}
+
+// Doubles of partials for q values per target and run.
+template <typename T>
+static size_t direct_partials(Cnt n_tgt, Cnt n_src, int q) {
+    const int64_t t = n_tgt.ub > 0 ? n_tgt.ub : 1;
+    if (!n_tgt.dev && !n_src.dev) return (size_t)(q * t * direct_split<T>(n_tgt.ub, n_src.ub).runs);
+    return (size_t)(q * (t * direct_runs_max<T>(t, n_src.ub) + kTile * kDirectWork));
+}
+
+// The four smallest values seen so far, m0 <= m1 <= m2 <= m3.
+template <typename T>
+__device__ __forceinline__ void keep4(T &m0, T &m1, T &m2, T &m3, T r) {
+    using A = Arith<T>;
+    m3 = A::med3(m2, m3, r);
+    m2 = A::med3(m1, m2, r);
+    m1 = A::med3(m0, m1, r);
+    m0 = A::min_(m0, r);
+}
+
+__device__ __forceinline__ void order2(double &a, double &b) {
+    const double lo = fmin(a, b), hi = fmax(a, b);
+    a = lo;
+    b = hi;
+}
+
+// Four values at a time: they are sorted (5 exchanges), the pairwise minima
+// with the kept ones in reverse are the four smallest of the eight, a bitonic
+// run that 4 exchanges sort.  FP64 has no med3: 5.5 min/max a value against 13.
+__device__ __forceinline__ void keep4x4(double &m0, double &m1, double &m2, double &m3, double a, double b, double c,
+                                        double d) {
+    order2(a, b);
+    order2(c, d);
+    order2(a, c);
+    order2(b, d);
+    order2(b, c);
+    m0 = fmin(m0, d);
+    m1 = fmin(m1, c);
+    m2 = fmin(m2, b);
+    m3 = fmin(m3, a);
+    order2(m0, m2);
+    order2(m1, m3);
+    order2(m0, m1);
+    order2(m2, m3);
+}
+// Two values at a time, the same way (6 min/max a value).
+__device__ __forceinline__ void keep4x2(double &m0, double &m1, double &m2, double &m3, double a, double b) {
+    order2(a, b);
+    m2 = fmin(m2, b);
+    m3 = fmin(m3, a);
+    order2(m0, m2);
+    order2(m1, m3);
+    order2(m0, m1);
+    order2(m2, m3);
+}
+__device__ __forceinline__ void keep4x4(float &m0, float &m1, float &m2, float &m3, float a, float b, float c, float d) {
+    keep4(m0, m1, m2, m3, a);
+    keep4(m0, m1, m2, m3, b);
+    keep4(m0, m1, m2, m3, c);
+    keep4(m0, m1, m2, m3, d);
 }
 
 // ---- A6: src/kernel.cu:875-983 -------------------------------------------
@@ -74,45 +174,69 @@ __device__ __forceinline__ void stage_tile(Src4<T> *ls, const T *__restrict__ sx
 // The self pair contributes exactly 0 to the sums (dx = dy = 0); for d the
 // four smallest r^2 including the self 0 are kept and the smallest one is
 // dropped, which equals the three smallest over j != i.
+//
+// Bound by VALU issue.  The sources are wave-uniform, so they come through
+// scalar loads straight from the arrays: no LDS staging, no barriers, and the
+// pair arithmetic takes them as scalar operands.  Partials per run s and
+// target: part[(6 s + q) n_tgt + i], q = su, sv, then the four smallest r^2.
 template <typename T, int TPT>
-__global__ __launch_bounds__(kTile) void k_biot_savart(
-    const T *__restrict__ sx, const T *__restrict__ sy, const T *__restrict__ sg, Cnt cn_src,
-    Cnt cn_tgt, T eps2, double vinf_x, double vinf_y, double *__restrict__ u,
-    double *__restrict__ v, double *__restrict__ d) {
-    __shared__ Src4<T> ls[kTile];
+__global__ __launch_bounds__(kTile) void k_biot_savart(const T *__restrict__ sx, const T *__restrict__ sy,
+                                                       const T *__restrict__ sg, Cnt cn_src, Cnt cn_tgt, T eps2,
+                                                       double *__restrict__ part) {
     using A = Arith<T>;
-    const int64_t n_src = cn_src.get(), n_tgt = cn_tgt.get();
-    const int64_t t0 = (int64_t)blockIdx.x * (kTile * TPT) + threadIdx.x;
+    const int32_t n_src = (int32_t)cn_src.get(), n_tgt = (int32_t)cn_tgt.get();
+    if (sizeof(T) == 8 && n_src <= kOrdered) return;  // the ordered kernel's
+    const DirectSplit sp = direct_split<T>(n_tgt, n_src);
+    const uint32_t tb = ((uint32_t)n_tgt + kTile * TPT - 1) / (kTile * TPT);
+    if (tb == 0) return;
+    const uint32_t s = blockIdx.x / tb, t = blockIdx.x - s * tb;
+    if (s >= (uint32_t)sp.runs) return;
+    const int32_t lo = (int32_t)s * sp.len, hi = min(n_src, lo + sp.len);
+    const int32_t t0 = (int32_t)(t * (kTile * TPT) + threadIdx.x);
     T ax[TPT], ay[TPT], m0[TPT], m1[TPT], m2[TPT], m3[TPT], su[TPT], sv[TPT];
     double au[TPT], av[TPT];
 #pragma unroll
     for (int k = 0; k < TPT; ++k) {
-        const int64_t i = t0 + (int64_t)k * kTile;
-        ax[k] = i < n_tgt ? sx[i] : T(0);
-        ay[k] = i < n_tgt ? sy[i] : T(0);
+        const int32_t i = t0 + k * kTile;
+        ax[k] = i < n_tgt ? far_clamp(sx[i]) : T(0);
+        ay[k] = i < n_tgt ? far_clamp(sy[i]) : T(0);
         m0[k] = m1[k] = m2[k] = m3[k] = T(1e5);
         su[k] = sv[k] = T(0);
         au[k] = av[k] = 0.0;
     }
-    for (int64_t base = 0; base < n_src; base += kTile) {
-        __syncthreads();
-        stage_tile<T>(ls, sx, sy, sg, base, n_src);
-        __syncthreads();
-#pragma unroll 4
-        for (int jj = 0; jj < kTile; ++jj) {
-            const Src4<T> s = ls[jj];
+    auto pair = [&](int k, T x, T y, T g) {
+        const T dx = ax[k] - x, dy = ay[k] - y;
+        const T r2 = dx * dx + dy * dy;
+        const T w = A::div(g, A::max_(r2, eps2));
+        sv[k] += w * dx;
+        su[k] -= w * dy;
+        return r2;
+    };
+    for (int32_t base = lo; base < hi; base += kTile) {
+        const int32_t end = min(hi, base + kTile);
+        int32_t j = base;
+        for (; j + 4 <= end; j += 4) {
+            T x[4], y[4], g[4];
+#pragma unroll
+            for (int q = 0; q < 4; ++q) {
+                x[q] = far_clamp(sx[j + q]);
+                y[q] = far_clamp(sy[j + q]);
+                g[q] = sg[j + q];
+            }
 #pragma unroll
             for (int k = 0; k < TPT; ++k) {
-                const T dx = ax[k] - s.x;
-                const T dy = ay[k] - s.y;
-                const T r2 = dx * dx + dy * dy;
-                m3[k] = A::med3(m2[k], m3[k], r2);
-                m2[k] = A::med3(m1[k], m2[k], r2);
-                m1[k] = A::med3(m0[k], m1[k], r2);
-                m0[k] = A::min_(m0[k], r2);
-                const T w = A::div(s.g, A::max_(r2, eps2));
-                sv[k] += w * dx;
-                su[k] -= w * dy;
+                T r2[4];
+#pragma unroll
+                for (int q = 0; q < 4; ++q) r2[q] = pair(k, x[q], y[q], g[q]);
+                keep4x4(m0[k], m1[k], m2[k], m3[k], r2[0], r2[1], r2[2], r2[3]);
+            }
+        }
+        for (; j < end; ++j) {
+            const T x = far_clamp(sx[j]), y = far_clamp(sy[j]), g = sg[j];
+#pragma unroll
+            for (int k = 0; k < TPT; ++k) {
+                const T r2 = pair(k, x, y, g);
+                keep4(m0[k], m1[k], m2[k], m3[k], r2);
             }
         }
         if constexpr (sizeof(T) == 4) {
@@ -124,79 +248,126 @@ __global__ __launch_bounds__(kTile) void k_biot_savart(
             }
         }
     }
+    double *o = part + (int64_t)s * 6 * n_tgt;
 #pragma unroll
     for (int k = 0; k < TPT; ++k) {
-        const int64_t i = t0 + (int64_t)k * kTile;
+        const int32_t i = t0 + k * kTile;
         if (i >= n_tgt) continue;
-        if constexpr (sizeof(T) == 8) {
-            au[k] = (double)su[k];
-            av[k] = (double)sv[k];
-        }
-        u[i] = au[k] / (2 * kPi) + vinf_x;
-        v[i] = av[k] / (2 * kPi) + vinf_y;
-        if (d) d[i] = (sqrt((double)m1[k]) + sqrt((double)m2[k]) + sqrt((double)m3[k])) / 3;
+        const double q[6] = {sizeof(T) == 8 ? (double)su[k] : au[k], sizeof(T) == 8 ? (double)sv[k] : av[k],
+                             (double)m0[k], (double)m1[k], (double)m2[k], (double)m3[k]};
+#pragma unroll
+        for (int e = 0; e < 6; ++e) o[(int64_t)e * n_tgt + i] = q[e];
     }
+}
+
+// Adds the runs' partials in run order: 64 targets per work-group, kSumRuns
+// runs at a time read by the four waves, added by the first.
+constexpr int kSumRuns = 16;
+
+template <typename T>
+__global__ __launch_bounds__(256) void k_bs_sum(const double *__restrict__ part, Cnt cn_src, Cnt cn_tgt,
+                                                double vinf_x, double vinf_y, double *__restrict__ u,
+                                                double *__restrict__ v, double *__restrict__ d) {
+    __shared__ double ls[kSumRuns][2][64];
+    __shared__ double lm[3][4][64];
+    const int32_t n_src = (int32_t)cn_src.get(), n_tgt = (int32_t)cn_tgt.get();
+    if ((int32_t)blockIdx.x * 64 >= n_tgt || (sizeof(T) == 8 && n_src <= kOrdered)) return;
+    const int32_t runs = direct_split<T>(n_tgt, n_src).runs;
+    const int lane = threadIdx.x & 63, wv = threadIdx.x >> 6;
+    const int32_t i = (int32_t)blockIdx.x * 64 + lane, ic = min(i, n_tgt - 1);
+    double a = 0.0, b = 0.0, m0 = 1e5, m1 = 1e5, m2 = 1e5, m3 = 1e5;
+    for (int32_t s0 = 0; s0 < runs; s0 += kSumRuns) {
+#pragma unroll
+        for (int q = 0; q < kSumRuns / 4; ++q) {
+            const int32_t s = s0 + wv * (kSumRuns / 4) + q;
+            if (s >= runs) break;
+            const double *o = part + (int64_t)s * 6 * n_tgt + ic;
+            ls[s - s0][0][lane] = o[0];
+            ls[s - s0][1][lane] = o[(int64_t)n_tgt];
+            const double q0 = o[(int64_t)2 * n_tgt], q1 = o[(int64_t)3 * n_tgt], q2 = o[(int64_t)4 * n_tgt],
+                         q3 = o[(int64_t)5 * n_tgt];
+            keep4x4(m0, m1, m2, m3, q0, q1, q2, q3);
+        }
+        __syncthreads();
+        if (wv == 0) {
+            const int32_t c = min(kSumRuns, runs - s0);
+            for (int32_t q = 0; q < c; ++q) {
+                a += ls[q][0][lane];
+                b += ls[q][1][lane];
+            }
+        }
+        __syncthreads();
+    }
+    if (wv) {
+        const double q[4] = {m0, m1, m2, m3};
+        for (int e = 0; e < 4; ++e) lm[wv - 1][e][lane] = q[e];
+    }
+    __syncthreads();
+    if (wv || i >= n_tgt) return;
+    for (int w = 0; w < 3; ++w) keep4x4(m0, m1, m2, m3, lm[w][0][lane], lm[w][1][lane], lm[w][2][lane], lm[w][3][lane]);
+    u[i] = a / (2 * kPi) + vinf_x;
+    v[i] = b / (2 * kPi) + vinf_y;
+    d[i] = (sqrt(m1) + sqrt(m2) + sqrt(m3)) / 3;
 }
 
 // ---- A7: src/kernel.cu:985-1029 -------------------------------------------
 // Over j with r_ij > 0.001 ve_size: I2 += -g_j (r_i - r_j)/r e^{-r/d_i},
 // I1 += g_j e^{-r/d_i}; if |I1| > 1e-5: V_i += -nu I2 / (I1 d_i).
+// thr2 is the largest r^2 that the test leaves out.  Sources and partials as
+// in k_biot_savart: part[(3 s + q) n_tgt + i], q = x and y of the weighted
+// separations, then I1.
 template <typename T, int TPT>
-__global__ __launch_bounds__(kTile) void k_diffusion(
-    const T *__restrict__ sx, const T *__restrict__ sy, const T *__restrict__ sg, Cnt cn_src,
-    Cnt cn_tgt, const double *__restrict__ dd, double nu, double thr,
-    double *__restrict__ u, double *__restrict__ v) {
-    __shared__ Src4<T> ls[kTile];
-    const int64_t n_src = cn_src.get(), n_tgt = cn_tgt.get();
-    const int64_t t0 = (int64_t)blockIdx.x * (kTile * TPT) + threadIdx.x;
+__global__ __launch_bounds__(kTile) void k_diffusion(const T *__restrict__ sx, const T *__restrict__ sy,
+                                                     const T *__restrict__ sg, Cnt cn_src, Cnt cn_tgt,
+                                                     const double *__restrict__ dd, T thr2,
+                                                     double *__restrict__ part) {
+    const int32_t n_src = (int32_t)cn_src.get(), n_tgt = (int32_t)cn_tgt.get();
+    if (sizeof(T) == 8 && n_src <= kOrdered) return;  // the ordered kernel's
+    const DirectSplit sp = direct_split<T>(n_tgt, n_src);
+    const uint32_t tb = ((uint32_t)n_tgt + kTile * TPT - 1) / (kTile * TPT);
+    if (tb == 0) return;
+    const uint32_t s = blockIdx.x / tb, t = blockIdx.x - s * tb;
+    if (s >= (uint32_t)sp.runs) return;
+    const int32_t lo = (int32_t)s * sp.len, hi = min(n_src, lo + sp.len);
+    const int32_t t0 = (int32_t)(t * (kTile * TPT) + threadIdx.x);
     T ax[TPT], ay[TPT], kd[TPT], s2x[TPT], s2y[TPT], s1[TPT];
     double a2x[TPT], a2y[TPT], a1[TPT];
 #pragma unroll
     for (int k = 0; k < TPT; ++k) {
-        const int64_t i = t0 + (int64_t)k * kTile;
-        ax[k] = i < n_tgt ? sx[i] : T(0);
-        ay[k] = i < n_tgt ? sy[i] : T(0);
+        const int32_t i = t0 + k * kTile;
+        ax[k] = i < n_tgt ? far_clamp(sx[i]) : T(0);
+        ay[k] = i < n_tgt ? far_clamp(sy[i]) : T(0);
         const double di = i < n_tgt ? dd[i] : 1.0;
-        if constexpr (sizeof(T) == 4)
-            kd[k] = (T)(-1.4426950408889634 / di);  // exp(-r/d) = exp2(r * kd)
-        else
-            kd[k] = (T)(1.0 / di);
+        kd[k] = (T)(-1.4426950408889634 / di);  // exp(-r/d) = exp2(r * kd)
         s2x[k] = s2y[k] = s1[k] = T(0);
         a2x[k] = a2y[k] = a1[k] = 0.0;
     }
-    const T thr2 = (T)(thr * thr);
-    for (int64_t base = 0; base < n_src; base += kTile) {
-        __syncthreads();
-        stage_tile<T>(ls, sx, sy, sg, base, n_src);
-        __syncthreads();
+    for (int32_t base = lo; base < hi; base += kTile) {
+        const int32_t end = min(hi, base + kTile);
 #pragma unroll 4
-        for (int jj = 0; jj < kTile; ++jj) {
-            const Src4<T> s = ls[jj];
+        for (int32_t j = base; j < end; ++j) {
+            const T x = far_clamp(sx[j]), y = far_clamp(sy[j]), g = sg[j];
 #pragma unroll
             for (int k = 0; k < TPT; ++k) {
-                const T dx = ax[k] - s.x;
-                const T dy = ay[k] - s.y;
+                const T dx = ax[k] - x, dy = ay[k] - y;
                 const T r2 = dx * dx + dy * dy;
+                T e, rs;
                 if constexpr (sizeof(T) == 4) {
                     const T r2c = r2 > thr2 ? r2 : T(1e30f);
-                    const T rs = __builtin_amdgcn_rsqf(r2c);
-                    const T dist = r2c * rs;
-                    const T e = __builtin_amdgcn_exp2f(dist * kd[k]);
-                    const T ge = s.g * e;
-                    const T w = ge * rs;
-                    s2x[k] += w * dx;
-                    s2y[k] += w * dy;
-                    s1[k] += ge;
+                    rs = __builtin_amdgcn_rsqf(r2c);
+                    e = __builtin_amdgcn_exp2f((r2c * rs) * kd[k]);
                 } else {
-                    const T dist = sqrt(r2);
-                    if (dist > (T)thr) {
-                        const T w = s.g / dist;
-                        const T e = exp(-dist * kd[k]);
-                        s2x[k] += w * dx * e;
-                        s2y[k] += w * dy * e;
-                        s1[k] += s.g * e;
-                    }
+                    // left out: a distance of 1e150, whose exponential is zero
+                    const double r2c = r2 > thr2 ? r2 : __hiloint2double(0x7e37e43c, __double2loint(r2));
+                    double dist;
+                    rsqrt_sqrt_pos(r2c, rs, dist);
+                    e = exp2_neg(dist * kd[k]);
                 }
+                const T ge = g * e;
+                const T w = ge * rs;
+                s2x[k] += w * dx;
+                s2y[k] += w * dy;
+                s1[k] += ge;
             }
         }
         if constexpr (sizeof(T) == 4) {
@@ -209,22 +380,304 @@ __global__ __launch_bounds__(kTile) void k_diffusion(
             }
         }
     }
+    double *o = part + (int64_t)s * 3 * n_tgt;
 #pragma unroll
     for (int k = 0; k < TPT; ++k) {
-        const int64_t i = t0 + (int64_t)k * kTile;
+        const int32_t i = t0 + k * kTile;
         if (i >= n_tgt) continue;
-        if constexpr (sizeof(T) == 8) {
-            a2x[k] = s2x[k];
-            a2y[k] = s2y[k];
-            a1[k] = s1[k];
-        }
-        // I2 = -sum w (r_i - r_j) e, so -nu I2/(I1 d) = nu a2/(I1 d)
-        if (fabs(a1[k]) > 1e-5) {
-            const double di = dd[i];
-            u[i] += nu * a2x[k] / (a1[k] * di);
-            v[i] += nu * a2y[k] / (a1[k] * di);
-        }
+        o[i] = sizeof(T) == 8 ? (double)s2x[k] : a2x[k];
+        o[(int64_t)n_tgt + i] = sizeof(T) == 8 ? (double)s2y[k] : a2y[k];
+        o[(int64_t)2 * n_tgt + i] = sizeof(T) == 8 ? (double)s1[k] : a1[k];
     }
+}
+
+// I2 = -sum w (r_i - r_j) e, so -nu I2/(I1 d) = nu a2/(I1 d)
+__device__ __forceinline__ void diff_add(int32_t i, double a2x, double a2y, double a1, const double *__restrict__ dd,
+                                         double nu, double *__restrict__ u, double *__restrict__ v) {
+    if (fabs(a1) > 1e-5) {
+        const double di = dd[i];
+        u[i] += nu * a2x / (a1 * di);
+        v[i] += nu * a2y / (a1 * di);
+    }
+}
+
+// Adds the runs' partials as k_bs_sum does.
+template <typename T>
+__global__ __launch_bounds__(256) void k_diff_sum(const double *__restrict__ part, Cnt cn_src, Cnt cn_tgt,
+                                                  const double *__restrict__ dd, double nu, double *__restrict__ u,
+                                                  double *__restrict__ v) {
+    __shared__ double ls[kSumRuns][3][64];
+    const int32_t n_src = (int32_t)cn_src.get(), n_tgt = (int32_t)cn_tgt.get();
+    if ((int32_t)blockIdx.x * 64 >= n_tgt || (sizeof(T) == 8 && n_src <= kOrdered)) return;
+    const int32_t runs = direct_split<T>(n_tgt, n_src).runs;
+    const int lane = threadIdx.x & 63, wv = threadIdx.x >> 6;
+    const int32_t i = (int32_t)blockIdx.x * 64 + lane, ic = min(i, n_tgt - 1);
+    double a2x = 0.0, a2y = 0.0, a1 = 0.0;
+    for (int32_t s0 = 0; s0 < runs; s0 += kSumRuns) {
+#pragma unroll
+        for (int q = 0; q < kSumRuns / 4; ++q) {
+            const int32_t s = s0 + wv * (kSumRuns / 4) + q;
+            if (s >= runs) break;
+            const double *o = part + (int64_t)s * 3 * n_tgt + ic;
+            for (int e = 0; e < 3; ++e) ls[s - s0][e][lane] = o[(int64_t)e * n_tgt];
+        }
+        __syncthreads();
+        if (wv == 0) {
+            const int32_t c = min(kSumRuns, runs - s0);
+            for (int32_t q = 0; q < c; ++q) {
+                a2x += ls[q][0][lane];
+                a2y += ls[q][1][lane];
+                a1 += ls[q][2][lane];
+            }
+        }
+        __syncthreads();
+    }
+    if (wv || i >= n_tgt) return;
+    diff_add(i, a2x, a2y, a1, dd, nu, u, v);
+}
+
+// ---- ordered FP64 sums --------------------------------------------------------
+// The same sums with one accumulation chain per target over the sources in
+// order, for the counts at which the chip is far from full with one lane per
+// target.  The pair terms do not depend on the order, only their addition
+// does: in a work-group of 16 waves, 15 evaluate terms of TG targets, SL =
+// 64 / TG sources per wave and pass, into LDS, and one adds the tile before
+// in order, the components of a target on lanes of their own.  The term
+// arithmetic is correctly rounded as the plain expressions are, so the
+// results are those of the plain loop bit for bit.  Bound by the adding
+// wave's reads and adds (about 10 ns a source while there is a CU for each
+// work-group).  2500 vortices: Biot-Savart 243 -> 26 us, diffusion 475 -> 34
+// us against one lane per target over all sources.  Above kOrdered the split
+// sums are faster: at 17000 0.26 and 0.40 ms against 0.62 and 1.05 ms.
+constexpr int kOrdWaves = 15;
+constexpr int kAhead = 6;  // pairs of terms per batch: the LDS latency of one is covered by the adds of another
+
+// Sources of a tile, staged three tiles deep (the tile being evaluated, the
+// one being added and the next).  A vector load that fetches one or two
+// addresses for a wave still costs the load unit a full wave's turns.
+template <int TILE>
+struct OrdSrc {
+    double c[3][3][TILE];  // x, y, g
+    __device__ __forceinline__ void put(int b, int e, double3 s) {
+        c[b][0][e] = s.x;
+        c[b][1][e] = s.y;
+        c[b][2][e] = s.z;
+    }
+};
+__device__ __forceinline__ double3 ord_src(const double *__restrict__ sx, const double *__restrict__ sy,
+                                           const double *__restrict__ sg, int32_t j, int32_t n) {
+    j = min(j, n - 1);  // past the end: the last source, its terms replaced by zeros
+    return double3{sx[j], sy[j], sg[j]};
+}
+
+template <int TG, int Q>
+__global__ __launch_bounds__(1024) void k_biot_savart_ordered(const double *__restrict__ sx,
+                                                              const double *__restrict__ sy,
+                                                              const double *__restrict__ sg, Cnt cn_src, Cnt cn_tgt,
+                                                              double eps2, double vinf_x, double vinf_y,
+                                                              double *__restrict__ u, double *__restrict__ v,
+                                                              double *__restrict__ d) {
+    constexpr int SL = 64 / TG, TILE = kOrdWaves * SL * Q;
+    constexpr int kTerms = 2 * TILE * TG, kSmall = 4 * kOrdWaves * 64;
+    // terms [2][TILE / 2][TG][2] (a lane reads two sources' at once); at the
+    // end the nearest lists
+    __shared__ __align__(16) double lw[kTerms > kSmall ? kTerms : kSmall];
+    __shared__ __align__(16) OrdSrc<TILE> src;
+    const int32_t n_src = (int32_t)cn_src.get(), n_tgt = (int32_t)cn_tgt.get();
+    if ((int32_t)blockIdx.x * TG >= n_tgt || n_src > kOrdered) return;
+    const int lane = threadIdx.x & 63, wv = threadIdx.x >> 6;
+    const int t = lane & (TG - 1), slot = lane / TG;
+    const int32_t i = (int32_t)blockIdx.x * TG + t, ic = min(i, n_tgt - 1);
+    const double ax = sx[ic], ay = sy[ic];
+    double m0 = 1e5, m1 = 1e5, m2 = 1e5, m3 = 1e5;
+    // the chain of lane (t, slot): sv of dx for even slots, su of -dy for odd
+    const bool xr = !(slot & 1);
+    const double c1 = xr ? -1.0 : 1.0, c0 = xr ? ax : -ay;
+    double acc = 0.0;
+    const int32_t tiles = (n_src + TILE - 1) / TILE;
+    const bool stager = threadIdx.x < TILE;
+    if (stager && tiles) src.put(0, threadIdx.x, ord_src(sx, sy, sg, threadIdx.x, n_src));
+    __syncthreads();
+    int b0 = 0, b1 = 1, b2 = 2;  // source buffers of tiles k, k + 1 and k - 1
+    for (int32_t k = 0; k <= tiles; ++k) {
+        double3 next;
+        if (stager && k + 1 < tiles) next = ord_src(sx, sy, sg, (k + 1) * TILE + (int32_t)threadIdx.x, n_src);
+        if (wv < kOrdWaves) {
+            if (k < tiles) {
+                double *w_ = lw + (k & 1) * (TILE * TG);
+                double r2[Q];
+#pragma unroll
+                for (int q = 0; q < Q; ++q) {
+                    const int jj = (q * kOrdWaves + wv) * SL + slot;
+                    const double dx = ax - src.c[b0][0][jj], dy = ay - src.c[b0][1][jj], g = src.c[b0][2][jj];
+                    r2[q] = fma(dx, dx, dy * dy);
+                    const double a = fmax(r2[q], eps2);
+                    double w = div_pos_exact(g, a);
+                    if (__builtin_expect(__any(!(a < 1e300)), 0)) {
+                        asm volatile("; rare: kept out of the main path");
+                        w = g / a;
+                    }
+                    const bool in = k * TILE + jj < n_src;
+                    w_[(jj >> 1) * (2 * TG) + 2 * t + (jj & 1)] = in ? w : 0.0;
+                    r2[q] = in ? r2[q] : 1e5;
+                }
+                if constexpr (Q == 4)
+                    keep4x4(m0, m1, m2, m3, r2[0], r2[1], r2[2], r2[3]);
+                else
+                    keep4x2(m0, m1, m2, m3, r2[0], r2[1]);
+            }
+        } else if (k > 0 && lane < 2 * TG) {
+            __builtin_amdgcn_s_setprio(3);
+            const double2 *w_ = (const double2 *)(lw + ((k - 1) & 1) * (TILE * TG)) + t;
+            const double2 *s_ = (const double2 *)src.c[b2][xr ? 0 : 1];
+            // two batches of kAhead pairs in turn: one is added while the next is read
+            double2 w[2][kAhead], p[2][kAhead];
+#pragma unroll
+            for (int e = 0; e < kAhead; ++e) {
+                w[0][e] = w_[e * TG];
+                p[0][e] = s_[e];
+            }
+#pragma unroll
+            for (int h = 0; h < TILE / 2 / kAhead; ++h) {
+                if (h + 1 < TILE / 2 / kAhead) {
+#pragma unroll
+                    for (int e = 0; e < kAhead; ++e) {
+                        w[(h + 1) & 1][e] = w_[((h + 1) * kAhead + e) * TG];
+                        p[(h + 1) & 1][e] = s_[(h + 1) * kAhead + e];
+                    }
+                }
+#pragma unroll
+                for (int e = 0; e < kAhead; ++e) {
+                    acc = fma(w[h & 1][e].x, fma(p[h & 1][e].x, c1, c0), acc);
+                    acc = fma(w[h & 1][e].y, fma(p[h & 1][e].y, c1, c0), acc);
+                }
+            }
+            __builtin_amdgcn_s_setprio(0);
+        }
+        if (stager && k + 1 < tiles) src.put(b1, threadIdx.x, next);
+        __syncthreads();
+        const int r = b2;
+        b2 = b0;
+        b0 = b1;
+        b1 = r;
+    }
+    // the producers' nearest lists, merged by the adding wave
+    if (wv < kOrdWaves) {
+        const double q[4] = {m0, m1, m2, m3};
+        for (int e = 0; e < 4; ++e) lw[(wv * 4 + e) * 64 + lane] = q[e];
+    }
+    __syncthreads();
+    if (wv < kOrdWaves) return;
+    for (int w = 0; w < kOrdWaves; ++w) {
+        const double *q = lw + w * 256 + lane;
+        keep4x4(m0, m1, m2, m3, q[0], q[64], q[128], q[192]);
+    }
+#pragma unroll
+    for (int o = TG; o < 64; o <<= 1) {
+        const double q0 = __shfl_xor(m0, o, 64), q1 = __shfl_xor(m1, o, 64), q2 = __shfl_xor(m2, o, 64),
+                     q3 = __shfl_xor(m3, o, 64);
+        keep4x4(m0, m1, m2, m3, q0, q1, q2, q3);
+    }
+    if (i >= n_tgt || slot > 1) return;
+    if (xr) {
+        v[i] = acc / (2 * kPi) + vinf_y;
+        d[i] = (sqrt(m1) + sqrt(m2) + sqrt(m3)) / 3;
+    } else {
+        u[i] = acc / (2 * kPi) + vinf_x;
+    }
+}
+
+// The diffusion's three chains: x and y terms (w dx) e, (w dy) e with w = g /
+// r on lanes of their own, and I1's g e beside both.  A pair within the
+// threshold, or past the end, has e = 0.
+template <int TG, int Q>
+__global__ __launch_bounds__(1024) void k_diffusion_ordered(const double *__restrict__ sx,
+                                                            const double *__restrict__ sy,
+                                                            const double *__restrict__ sg, Cnt cn_src, Cnt cn_tgt,
+                                                            const double *__restrict__ dd, double nu, double thr,
+                                                            double *__restrict__ u, double *__restrict__ v) {
+    constexpr int SL = 64 / TG, TILE = kOrdWaves * SL * Q;
+    __shared__ __align__(16) double2 lt[2][3][TILE / 2][TG];  // w dx, w dy, e of two sources
+    __shared__ __align__(16) OrdSrc<TILE> src;
+    const int32_t n_src = (int32_t)cn_src.get(), n_tgt = (int32_t)cn_tgt.get();
+    if ((int32_t)blockIdx.x * TG >= n_tgt || n_src > kOrdered) return;
+    const int lane = threadIdx.x & 63, wv = threadIdx.x >> 6;
+    const int t = lane & (TG - 1), slot = lane / TG;
+    const int32_t i = (int32_t)blockIdx.x * TG + t, ic = min(i, n_tgt - 1);
+    const double ax = sx[ic], ay = sy[ic], kd = 1.0 / dd[ic];
+    double acc = 0.0, acc1 = 0.0;
+    const int32_t tiles = (n_src + TILE - 1) / TILE;
+    const bool stager = threadIdx.x < TILE;
+    if (stager && tiles) src.put(0, threadIdx.x, ord_src(sx, sy, sg, threadIdx.x, n_src));
+    __syncthreads();
+    int b0 = 0, b1 = 1, b2 = 2;
+    for (int32_t k = 0; k <= tiles; ++k) {
+        const int b = k & 1;
+        double3 next;
+        if (stager && k + 1 < tiles) next = ord_src(sx, sy, sg, (k + 1) * TILE + (int32_t)threadIdx.x, n_src);
+        if (wv < kOrdWaves) {
+            if (k < tiles) {
+#pragma unroll
+                for (int q = 0; q < Q; ++q) {
+                    const int jj = (q * kOrdWaves + wv) * SL + slot;
+                    const double dx = ax - src.c[b0][0][jj], dy = ay - src.c[b0][1][jj], g = src.c[b0][2][jj];
+                    const double r2 = fma(dx, dx, dy * dy);
+                    double w, dist = sqrt_pos_exact(r2, g, w);
+                    if (__builtin_expect(__any(r2 > 1e300), 0)) {
+                        asm volatile("; rare: kept out of the main path");
+                        dist = sqrt(r2);
+                        w = g / dist;
+                    }
+                    const bool on = dist > thr && k * TILE + jj < n_src;
+                    const double e = exp(-dist * kd);
+                    double *o = (double *)&lt[b][0][jj >> 1][t] + (jj & 1);
+                    o[0] = on ? w * dx : 0.0;
+                    o[TILE * TG] = on ? w * dy : 0.0;
+                    o[2 * TILE * TG] = on ? e : 0.0;
+                }
+            }
+        } else if (k > 0 && lane < 2 * TG) {
+            __builtin_amdgcn_s_setprio(3);
+            const double2 *p_ = &lt[b ^ 1][slot & 1][0][t], *e_ = &lt[b ^ 1][2][0][t];
+            const double2 *g_ = (const double2 *)src.c[b2][2];
+            constexpr int H = kAhead / 2;
+            double2 p[2][H], x[2][H], g[2][H];
+#pragma unroll
+            for (int q = 0; q < H; ++q) {
+                p[0][q] = p_[q * TG];
+                x[0][q] = e_[q * TG];
+                g[0][q] = g_[q];
+            }
+#pragma unroll
+            for (int h = 0; h < TILE / 2 / H; ++h) {
+                if (h + 1 < TILE / 2 / H) {
+#pragma unroll
+                    for (int q = 0; q < H; ++q) {
+                        p[(h + 1) & 1][q] = p_[((h + 1) * H + q) * TG];
+                        x[(h + 1) & 1][q] = e_[((h + 1) * H + q) * TG];
+                        g[(h + 1) & 1][q] = g_[(h + 1) * H + q];
+                    }
+                }
+#pragma unroll
+                for (int q = 0; q < H; ++q) {
+                    acc = fma(p[h & 1][q].x, x[h & 1][q].x, acc);
+                    acc1 = fma(g[h & 1][q].x, x[h & 1][q].x, acc1);
+                    acc = fma(p[h & 1][q].y, x[h & 1][q].y, acc);
+                    acc1 = fma(g[h & 1][q].y, x[h & 1][q].y, acc1);
+                }
+            }
+            __builtin_amdgcn_s_setprio(0);
+        }
+        if (stager && k + 1 < tiles) src.put(b1, threadIdx.x, next);
+        __syncthreads();
+        const int r = b2;
+        b2 = b0;
+        b0 = b1;
+        b1 = r;
+    }
+    if (wv < kOrdWaves) return;
+    const double a2y = __shfl(acc, t + TG, 64);
+    if (slot == 0 && i < n_tgt) diff_add(i, acc, a2y, acc1, dd, nu, u, v);
 }
 
 // atan2 in FP32 for the panel right-hand side: octant reduction to
@@ -604,14 +1057,14 @@ __global__ __launch_bounds__(kTile) void k_probe_partial(const double *__restric
     const int64_t i = (int64_t)blockIdx.x * kTile + threadIdx.x;
     const int64_t c = blockIdx.y;
     const int64_t lo = c * chunk, hi = min(n_src, lo + chunk);
-    const double a0 = i < m ? px[i] : 0.0, a1 = i < m ? py[i] : 0.0;
+    const double a0 = i < m ? far_clamp(px[i]) : 0.0, a1 = i < m ? far_clamp(py[i]) : 0.0;
     double su = 0.0, sv = 0.0;
     for (int64_t base = lo; base < hi; base += kTile) {
         __syncthreads();
         const int64_t j = base + threadIdx.x;
         Src4<double> s;
-        s.x = j < hi ? sx[j] : A::kFar;
-        s.y = j < hi ? sy[j] : A::kFar;
+        s.x = j < hi ? far_clamp(sx[j]) : A::kFar;
+        s.y = j < hi ? far_clamp(sy[j]) : A::kFar;
         s.g = j < hi ? sg[j] : 0.0;
         s.pad = 0.0;
         ls[threadIdx.x] = s;
@@ -705,39 +1158,44 @@ int launch_biot_savart(vx_case *c, int64_t n_tgt, int64_t n_src, double vinf_x, 
 }
 
 // Targets per thread of the direct kernels: the case's tuning (see
-// vx_case_autotune) or the default, 4 in FP32 and 2 in FP64.  Every choice
-// sums each target's sources in the same order, so the results do not depend
-// on it.
-// Default targets per thread of the direct kernels: 4 (FP32) or 2 (FP64),
-// fewer while the grid would give the 256 CUs less than two work-groups each
-// (the sums, and so the results, do not depend on it).
-int direct_tpt_default(bool f32, int64_t n_tgt) {
-    int tpt = f32 ? 4 : 2;
-    while (tpt > 1 && (n_tgt + kTile * tpt - 1) / (kTile * tpt) < 512) tpt >>= 1;
-    return tpt;
-}
+// vx_case_autotune) or one.  Every choice sums each target's sources in the
+// same order, so the results do not depend on it.  Sources come as scalar
+// operands, so more targets per thread save no loads: 60001 vortices take
+// 1.02, 1.11, 1.44 and 1.53 ms (Biot-Savart, FP32) with 1, 2, 4 and 8, and
+// 2.42, 2.34, 2.52 and 3.00 ms in FP64.
+int direct_tpt_default(bool, int64_t) { return 1; }
 
 static int tpt_of(int want, bool f32, int64_t n_tgt) {
     if (want == 1 || want == 2 || want == 4 || want == 8) return want;
     return direct_tpt_default(f32, n_tgt);
 }
 
+// FP64: the ordered kernels up to kOrdered sources, the split ones above.  A
+// device count's bound may lie above it while the count does not: then both
+// are queued and the live count decides in the kernels.
+static bool takes_ordered(Cnt n_src) { return n_src.dev || n_src.ub <= kOrdered; }
+static bool takes_split(Cnt n_src) { return n_src.ub > kOrdered; }
+// 16 targets per ordered work-group while that makes no more than one for each
+// CU, else 32: at 4000 vortices 40 and 52 us (Biot-Savart, diffusion) against
+// 47 and 82 with 32, at 6000 (two rounds of work-groups) 114 and 151 against
+// 73 and 126.  A device count goes by the host's last count; the results do
+// not depend on the choice.
+constexpr int64_t kOrdNarrow = 4096;
+static bool ord_narrow(const vx_case *c, Cnt n_tgt) { return (n_tgt.dev ? c->n : n_tgt.ub) <= kOrdNarrow; }
+
 template <typename T, int TPT>
-static void bs_launch(vx_case *c, const T *sx, const T *sy, const T *sg, Cnt n_src, Cnt n_tgt, T eps2, double vinf_x,
-                      double vinf_y) {
-    const unsigned nb = (unsigned)((n_tgt.ub + kTile * TPT - 1) / (kTile * TPT));
-    hipLaunchKernelGGL((k_biot_savart<T, TPT>), dim3(nb), dim3(kTile), 0, c->stream, sx, sy, sg, n_src, n_tgt, eps2,
-                       vinf_x, vinf_y, c->u.p, c->v.p, c->d.p);
+static void bs_launch(vx_case *c, const T *sx, const T *sy, const T *sg, Cnt n_src, Cnt n_tgt, T eps2) {
+    hipLaunchKernelGGL((k_biot_savart<T, TPT>), dim3((unsigned)direct_blocks<T>(n_tgt, n_src, TPT)), dim3(kTile), 0,
+                       c->stream, sx, sy, sg, n_src, n_tgt, eps2, c->partial.p);
 }
 
 template <typename T>
-static void bs_dispatch(vx_case *c, int tpt, const T *sx, const T *sy, const T *sg, Cnt n_src, Cnt n_tgt, T eps2,
-                        double vinf_x, double vinf_y) {
+static void bs_dispatch(vx_case *c, int tpt, const T *sx, const T *sy, const T *sg, Cnt n_src, Cnt n_tgt, T eps2) {
     switch (tpt) {
-        case 1: bs_launch<T, 1>(c, sx, sy, sg, n_src, n_tgt, eps2, vinf_x, vinf_y); break;
-        case 2: bs_launch<T, 2>(c, sx, sy, sg, n_src, n_tgt, eps2, vinf_x, vinf_y); break;
-        case 4: bs_launch<T, 4>(c, sx, sy, sg, n_src, n_tgt, eps2, vinf_x, vinf_y); break;
-        default: bs_launch<T, 8>(c, sx, sy, sg, n_src, n_tgt, eps2, vinf_x, vinf_y); break;
+        case 1: bs_launch<T, 1>(c, sx, sy, sg, n_src, n_tgt, eps2); break;
+        case 2: bs_launch<T, 2>(c, sx, sy, sg, n_src, n_tgt, eps2); break;
+        case 4: bs_launch<T, 4>(c, sx, sy, sg, n_src, n_tgt, eps2); break;
+        default: bs_launch<T, 8>(c, sx, sy, sg, n_src, n_tgt, eps2); break;
     }
 }
 
@@ -745,13 +1203,32 @@ int launch_biot_savart(vx_case *c, Cnt n_tgt, Cnt n_src, double vinf_x, double v
     if (n_tgt.ub <= 0) return 0;
     tree_d_changed(c);  // d from direct sums: a tree's sorted copy no longer matches
     const double eps2 = c->prm.ve_size * c->prm.ve_size;
+    const dim3 gsum((unsigned)((n_tgt.ub + 63) / 64));
     if (mixed(c)) {
-        if (launch_pack_f32(c, n_src)) return 1;
+        if (c->partial.ensure(direct_partials<float>(n_tgt, n_src, 6), c->stream) || launch_pack_f32(c, n_src))
+            return 1;
         bs_dispatch<float>(c, tpt_of(c->tune.tpt_bs, true, n_tgt.ub), c->xf.p, c->yf.p, c->gf.p, n_src, n_tgt,
-                           (float)eps2, vinf_x, vinf_y);
+                           (float)eps2);
+        hipLaunchKernelGGL(k_bs_sum<float>, gsum, dim3(256), 0, c->stream, c->partial.p, n_src, n_tgt, vinf_x, vinf_y,
+                           c->u.p, c->v.p, c->d.p);
     } else {
-        bs_dispatch<double>(c, tpt_of(c->tune.tpt_bs, false, n_tgt.ub), c->x.p, c->y.p, c->g.p, n_src, n_tgt, eps2,
-                            vinf_x, vinf_y);
+        if (takes_ordered(n_src)) {
+            if (ord_narrow(c, n_tgt))
+                hipLaunchKernelGGL((k_biot_savart_ordered<16, 2>), dim3((unsigned)((n_tgt.ub + 15) / 16)), dim3(1024), 0,
+                                   c->stream, c->x.p, c->y.p, c->g.p, n_src, n_tgt, eps2, vinf_x, vinf_y, c->u.p,
+                                   c->v.p, c->d.p);
+            else
+                hipLaunchKernelGGL((k_biot_savart_ordered<32, 4>), dim3((unsigned)((n_tgt.ub + 31) / 32)), dim3(1024), 0,
+                                   c->stream, c->x.p, c->y.p, c->g.p, n_src, n_tgt, eps2, vinf_x, vinf_y, c->u.p,
+                                   c->v.p, c->d.p);
+        }
+        if (takes_split(n_src)) {
+            if (c->partial.ensure(direct_partials<double>(n_tgt, n_src, 6), c->stream)) return 1;
+            bs_dispatch<double>(c, tpt_of(c->tune.tpt_bs, false, n_tgt.ub), c->x.p, c->y.p, c->g.p, n_src, n_tgt,
+                                eps2);
+            hipLaunchKernelGGL(k_bs_sum<double>, gsum, dim3(256), 0, c->stream, c->partial.p, n_src, n_tgt, vinf_x,
+                               vinf_y, c->u.p, c->v.p, c->d.p);
+        }
     }
     VX_CHECK(hipGetLastError());
     return 0;
@@ -762,33 +1239,59 @@ int launch_diffusion(vx_case *c, int64_t n_tgt, int64_t n_src) {
 }
 
 template <typename T, int TPT>
-static void diff_launch(vx_case *c, const T *sx, const T *sy, const T *sg, Cnt n_src, Cnt n_tgt, double thr) {
-    const unsigned nb = (unsigned)((n_tgt.ub + kTile * TPT - 1) / (kTile * TPT));
-    hipLaunchKernelGGL((k_diffusion<T, TPT>), dim3(nb), dim3(kTile), 0, c->stream, sx, sy, sg, n_src, n_tgt, c->d.p,
-                       c->prm.nu, thr, c->u.p, c->v.p);
+static void diff_launch(vx_case *c, const T *sx, const T *sy, const T *sg, Cnt n_src, Cnt n_tgt, T thr2) {
+    hipLaunchKernelGGL((k_diffusion<T, TPT>), dim3((unsigned)direct_blocks<T>(n_tgt, n_src, TPT)), dim3(kTile), 0,
+                       c->stream, sx, sy, sg, n_src, n_tgt, c->d.p, thr2, c->partial.p);
 }
 
 template <typename T>
-static void diff_dispatch(vx_case *c, int tpt, const T *sx, const T *sy, const T *sg, Cnt n_src, Cnt n_tgt,
-                          double thr) {
+static void diff_dispatch(vx_case *c, int tpt, const T *sx, const T *sy, const T *sg, Cnt n_src, Cnt n_tgt, T thr2) {
     switch (tpt) {
-        case 1: diff_launch<T, 1>(c, sx, sy, sg, n_src, n_tgt, thr); break;
-        case 2: diff_launch<T, 2>(c, sx, sy, sg, n_src, n_tgt, thr); break;
-        case 4: diff_launch<T, 4>(c, sx, sy, sg, n_src, n_tgt, thr); break;
-        default: diff_launch<T, 8>(c, sx, sy, sg, n_src, n_tgt, thr); break;
+        case 1: diff_launch<T, 1>(c, sx, sy, sg, n_src, n_tgt, thr2); break;
+        case 2: diff_launch<T, 2>(c, sx, sy, sg, n_src, n_tgt, thr2); break;
+        case 4: diff_launch<T, 4>(c, sx, sy, sg, n_src, n_tgt, thr2); break;
+        default: diff_launch<T, 8>(c, sx, sy, sg, n_src, n_tgt, thr2); break;
     }
+}
+
+// The largest r^2 whose rounded square root is not above thr, so that
+// r^2 > thr2 decides as sqrt(r^2) > thr does.
+double diff_thr2(double thr) {
+    double t = thr * thr;
+    while (std::sqrt(t) > thr) t = std::nextafter(t, 0.0);
+    for (double q = std::nextafter(t, INFINITY); std::sqrt(q) <= thr; q = std::nextafter(t, INFINITY)) t = q;
+    return t;
 }
 
 int launch_diffusion(vx_case *c, Cnt n_tgt, Cnt n_src) {
     if (n_tgt.ub <= 0) return 0;
     const double thr = 0.001 * c->prm.ve_size;
+    const dim3 gsum((unsigned)((n_tgt.ub + 63) / 64));
     if (mixed(c)) {
-        if (launch_pack_f32(c, n_src)) return 1;
+        if (c->partial.ensure(direct_partials<float>(n_tgt, n_src, 3), c->stream) || launch_pack_f32(c, n_src))
+            return 1;
         diff_dispatch<float>(c, tpt_of(c->tune.tpt_diff, true, n_tgt.ub), c->xf.p, c->yf.p, c->gf.p, n_src, n_tgt,
-                             thr);
+                             (float)(thr * thr));
+        hipLaunchKernelGGL(k_diff_sum<float>, gsum, dim3(256), 0, c->stream, c->partial.p, n_src, n_tgt, c->d.p,
+                           c->prm.nu, c->u.p, c->v.p);
     } else {
-        diff_dispatch<double>(c, tpt_of(c->tune.tpt_diff, false, n_tgt.ub), c->x.p, c->y.p, c->g.p, n_src, n_tgt,
-                              thr);
+        if (takes_ordered(n_src)) {
+            if (ord_narrow(c, n_tgt))
+                hipLaunchKernelGGL((k_diffusion_ordered<16, 2>), dim3((unsigned)((n_tgt.ub + 15) / 16)), dim3(1024), 0,
+                                   c->stream, c->x.p, c->y.p, c->g.p, n_src, n_tgt, c->d.p, c->prm.nu, thr, c->u.p,
+                                   c->v.p);
+            else
+                hipLaunchKernelGGL((k_diffusion_ordered<32, 2>), dim3((unsigned)((n_tgt.ub + 31) / 32)), dim3(1024), 0,
+                                   c->stream, c->x.p, c->y.p, c->g.p, n_src, n_tgt, c->d.p, c->prm.nu, thr, c->u.p,
+                                   c->v.p);
+        }
+        if (takes_split(n_src)) {
+            if (c->partial.ensure(direct_partials<double>(n_tgt, n_src, 3), c->stream)) return 1;
+            diff_dispatch<double>(c, tpt_of(c->tune.tpt_diff, false, n_tgt.ub), c->x.p, c->y.p, c->g.p, n_src, n_tgt,
+                                  diff_thr2(thr));
+            hipLaunchKernelGGL(k_diff_sum<double>, gsum, dim3(256), 0, c->stream, c->partial.p, n_src, n_tgt, c->d.p,
+                               c->prm.nu, c->u.p, c->v.p);
+        }
     }
     VX_CHECK(hipGetLastError());
     return 0;
