@@ -88,8 +88,490 @@ int launch_panel_matrix(vx_case *c) {
 // standard choice -- largest |A[i][k]| over i >= k once columns < k are
 // eliminated, first index on ties -- is used here because the look-ahead rule
 // breaks down on the bordered system of thin closed bodies.)
-// Per column k: pivot search (one work-group), row swap, column factors,
-// rank-1 update of both A and the inverse over all columns.
+//
+// Column by column, step k swaps the pivot row up, takes the factors
+// f_k[i] = A[i][k] / A[k][k] and subtracts f_k[i] times row k from every
+// other row of A and of the growing inverse.  One column at a time that is
+// four launches and 32 m^2 bytes each (109 ms at m = 2577, 15 ms at 1001), so
+// it runs in blocks of B columns, with the same operations on every element
+// in the same order and the same rounding:
+//   k_gj_panel  one work-group takes a block's columns over all rows in
+//               registers: pivots and factors of its B steps;
+//   k_gj_rows   a thread per other column: the block's row exchanges, and the
+//               pivot rows brought to each step in turn (U: their values as
+//               the step uses them);
+//   k_gj_rank   every other row: a = ((a - f_0 U_0) - f_1 U_1) - ...
+// In place: W's columns below the block hold the inverse's columns that are
+// not zero yet (in pivot order, the order undone at the end), the others A's.
+// The rounding residues that elimination leaves in A's finished columns reach
+// the last division through the diagonal, so they are carried along (G: rows
+// below the block; D: the diagonal).
+// Bound by the panels' latency (one CU, 1.1 to 2.4 us a column) up to about
+// 2500 rows and by W's traffic through the caches, 16 m^2 bytes a block, above.
+struct GjMoves {
+    int32_t src[16];           // the row that the block's r-th pivot step brought to row K + r
+    int32_t nq;                // rows below the block that received another row:
+    int32_t qdst[16], qsrc[16];
+};
+
+// Maximum over the wave of values that are no NaN, at least 0 (v_max_f64
+// itself: fmax would quiet its operands first).
+template <int CTRL>
+__device__ __forceinline__ double dpp_max(double v) {
+    const int lo = __builtin_amdgcn_update_dpp(0, __double2loint(v), CTRL, 0xf, 0xf, true);
+    const int hi = __builtin_amdgcn_update_dpp(0, __double2hiint(v), CTRL, 0xf, 0xf, true);
+    double r;
+    asm("v_max_f64 %0, %1, %2" : "=v"(r) : "v"(v), "v"(__hiloint2double(hi, lo)));
+    return r;
+}
+__device__ __forceinline__ double row_max(double v) {  // lane 15: over the first 16 lanes
+    return dpp_max<0x118>(dpp_max<0x114>(dpp_max<0x112>(dpp_max<0x111>(v))));
+}
+__device__ __forceinline__ double lane_of(double v, int lane) {
+    return __hiloint2double(__builtin_amdgcn_readlane(__double2hiint(v), lane),
+                            __builtin_amdgcn_readlane(__double2loint(v), lane));
+}
+__device__ __forceinline__ double wave_max(double v) { return lane_of(dpp_max<0x143>(dpp_max<0x142>(row_max(v))), 63); }
+
+template <int CTRL>
+__device__ __forceinline__ int dpp_min(int v) {
+    return min(v, __builtin_amdgcn_update_dpp(0x7fffffff, v, CTRL, 0xf, 0xf, false));
+}
+// The lane of `ties` (not empty) whose pos is lowest; a body's symmetry makes
+// many entries of a column equal.
+__device__ __forceinline__ int lowest_lane(uint64_t ties, int pos) {
+    if (!(ties & (ties - 1))) return __ffsll((unsigned long long)ties) - 1;
+    const bool in = (ties >> (threadIdx.x & 63)) & 1;
+    int v = in ? pos : 0x7fffffff;
+    v = dpp_min<0x118>(dpp_min<0x114>(dpp_min<0x112>(dpp_min<0x111>(v))));
+    v = dpp_min<0x143>(dpp_min<0x142>(v));
+    const int low = __builtin_amdgcn_readlane(v, 63);
+    return __ffsll((unsigned long long)__ballot(in && pos == low)) - 1;
+}
+
+// A barrier that orders LDS accesses only: the factors' stores to memory,
+// which only their own thread reads back, need not be waited for each step.
+__device__ __forceinline__ void lds_barrier() {
+    __builtin_amdgcn_fence(__ATOMIC_RELEASE, "workgroup", "local");
+    __builtin_amdgcn_s_barrier();
+    __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "workgroup", "local");
+}
+
+// Columns [K, K + nb) of W (column by column in Pt) over all m <= T R rows.
+// A thread holds R rows; a row exchange only exchanges the positions of two
+// rows.  Each wave offers its largest candidate with its row in LDS and every
+// thread picks the winner: one barrier per step.  The step's column is always
+// a[.][0]: the update moves the others down, so that the loop stays rolled
+// (unrolled, the code is fetched anew on every launch).  Few waves of many
+// registers: the reduction is the same work for every wave of a SIMD.
+// Results: by the rows' places before the block the factors cf[kk m + i] and
+// the columns as each one's own step left them PtG; the places (slot_of), the
+// pivots D, the row moves, perm.
+template <int NW, int B>
+struct GjPanelLds {
+    double crow[2][NW][B], ub[B][B], ckey[2][NW], crec[2][NW];
+    int cpos[2][NW], nq;
+};
+
+// A block's state: a ring of two, one being written by a panel while the
+// other is read by the rank update.
+struct GjBlock {
+    double *Pt, *PtG, *cf;
+    int32_t *slot_of;
+    GjMoves *mv;
+};
+
+// `prev` (null for the first block): the block before, whose rank update the
+// panel's own columns still lack; U its pivot rows.
+template <int T, int R, int B>
+__device__ __forceinline__ void gj_panel(GjPanelLds<T / 64, B> &ls, int32_t m, int32_t K, int32_t nb,
+                                         const GjBlock &blk, const GjBlock *prev, const double *__restrict__ U,
+                                         double *__restrict__ D, int32_t *__restrict__ perm,
+                                         int32_t *__restrict__ bad) {
+    constexpr int NW = T / 64;
+    static_assert(NW <= 16, "one row of lanes picks the winner");
+    const double *__restrict__ Pt = blk.Pt;
+    double *__restrict__ cf = blk.cf, *__restrict__ PtG = blk.PtG;
+    int32_t *__restrict__ slot_of = blk.slot_of;
+    GjMoves *__restrict__ mv = blk.mv;
+    auto &ckey = ls.ckey;
+    auto &crec = ls.crec;
+    auto &cpos = ls.cpos;
+    auto &crow = ls.crow;
+    int &nq = ls.nq;
+    const int tid = threadIdx.x, lane = tid & 63, wv = tid >> 6;
+    double a[R][B];
+    int pos[R];
+#pragma unroll
+    for (int r = 0; r < R; ++r) {
+        const int s = tid + r * T;
+        pos[r] = s < m ? s : -1;
+#pragma unroll
+        for (int c = 0; c < B; ++c) a[r][c] = s < m && c < nb ? Pt[(int64_t)c * m + s] : 0.0;
+    }
+    if (tid == 0) nq = 0;
+    if (prev) {
+        const int64_t ldu = 2 * (int64_t)m;
+        for (int e = tid; e < B * B; e += T) ls.ub[e / B][e % B] = e % B < nb ? U[(e / B) * ldu + K + e % B] : 0.0;
+        int32_t ps[R];  // where a row's factors are; -1: none (the block's own rows are at their final values)
+#pragma unroll
+        for (int r = 0; r < R; ++r) {
+            const int s = tid + r * T;
+            ps[r] = s < m && !(s >= K - B && s < K) ? prev->slot_of[s] : -1;
+        }
+        __syncthreads();
+#pragma unroll 1
+        for (int kk = 0; kk < B; ++kk) {
+            double u[B];
+#pragma unroll
+            for (int c = 0; c < B; ++c) u[c] = ls.ub[kk][c];
+#pragma unroll
+            for (int r = 0; r < R; ++r) {
+                const double f = ps[r] >= 0 ? prev->cf[(int64_t)kk * m + ps[r]] : 0.0;
+#pragma unroll
+                for (int c = 0; c < B; ++c) a[r][c] = a[r][c] - f * u[c];
+            }
+        }
+    }
+#pragma unroll 1
+    for (int kk = 0; kk < nb; ++kk) {
+        const int k = K + kk, par = kk & 1;
+        double key = -1.0, cand = 1.0;
+        int kp = 0x7fffffff, kr = 0;
+#pragma unroll
+        for (int r = 0; r < R; ++r) {
+            const double v = fabs(a[r][0]);
+            if (pos[r] >= k && (v > key || (v == key && pos[r] < kp))) {
+                key = v;
+                cand = a[r][0];
+                kp = pos[r];
+                kr = r;
+            }
+        }
+        const double rec = 1.0 / cand;  // every lane's own, beside the reduction
+        const double wm = wave_max(key);
+        const uint64_t ties = __ballot(key == wm);
+        const int wl = ties ? lowest_lane(ties, kp) : 0;
+        const int wr = __builtin_amdgcn_readlane(kr, wl);
+#pragma unroll
+        for (int r = 0; r < R; ++r)
+            if (wr == r) {
+                if (lane == wl) {
+#pragma unroll
+                    for (int c = 0; c < B; ++c) crow[par][wv][c] = a[r][c];
+                    ckey[par][wv] = key;
+                    cpos[par][wv] = kp;
+                    crec[par][wv] = rec;
+                }
+            }
+        lds_barrier();
+        const double ck = ckey[par][lane & (NW - 1)];
+        const int cp = cpos[par][lane & (NW - 1)];
+        const double gm = lane_of(row_max(ck), 15);
+        const uint64_t gt = __ballot(ck == gm) & ((1ull << NW) - 1);
+        const int gw = gt ? lowest_lane(gt, cp) : 0;
+        int p = __builtin_amdgcn_readlane(cp, gw);
+        if (!(gm >= kDelt)) {  // no usable pivot: the caller reports it
+            if (tid == 0) *bad = 1;
+            if (p < k || p >= m) p = k;
+        }
+        double row[B];
+#pragma unroll
+        for (int c = 0; c < B; ++c) row[c] = crow[par][gw][c];
+        const double y = crec[par][gw];
+        if (tid == 0) D[k] = row[0];
+#pragma unroll
+        for (int r = 0; r < R; ++r) {
+            pos[r] = pos[r] == p ? k : pos[r] == k ? p : pos[r];
+            // a / pivot correctly rounded from the rounded reciprocal
+            double f = a[r][0] * y;
+            f = fma(fma(-row[0], f, a[r][0]), y, f);
+            f = pos[r] == k ? 0.0 : f;
+            const int s = tid + r * T;
+            if (s < m) {
+                cf[(int64_t)kk * m + s] = f;
+                PtG[(int64_t)kk * m + s] = a[r][0] - f * row[0];
+            }
+#pragma unroll
+            for (int c = 1; c < B; ++c) a[r][c - 1] = a[r][c] - f * row[c];
+            a[r][B - 1] = 0.0;
+        }
+    }
+    // the moves: slot_of[final position] = the row that is there now
+    int mp[R];
+#pragma unroll
+    for (int r = 0; r < R; ++r) {
+        const int s = tid + r * T;
+        mp[r] = s < m && pos[r] != s ? perm[s] : 0;
+    }
+    __syncthreads();
+#pragma unroll
+    for (int r = 0; r < R; ++r) {
+        const int s = tid + r * T;
+        if (s < m) {
+            slot_of[pos[r]] = s;
+            if (pos[r] != s) perm[pos[r]] = mp[r];
+            if (pos[r] >= K && pos[r] < K + nb) {
+                mv->src[pos[r] - K] = s;
+            } else if (pos[r] != s) {
+                const int q = atomicAdd(&nq, 1);
+                mv->qdst[q] = pos[r];
+                mv->qsrc[q] = s;
+            }
+        }
+    }
+    __syncthreads();
+    if (tid == 0) mv->nq = nq;
+}
+
+template <int T, int R, int B>
+__global__ __launch_bounds__(T) void k_gj_panel(int32_t m, int32_t nb, GjBlock blk, double *__restrict__ D,
+                                                int32_t *__restrict__ perm, int32_t *__restrict__ bad) {
+    __shared__ __align__(16) GjPanelLds<T / 64, B> ls;
+    gj_panel<T, R, B>(ls, m, 0, nb, blk, nullptr, nullptr, D, perm, bad);
+}
+
+// A thread per column: of W (q < m) or of G (q - m < K + nb).
+// nextPt: the next block's columns, which get the moves and the block's rows
+// here and the rest in the next panel; ownPt: those of the block after it,
+// which get the block's rows here and the rest from the rank update.
+template <int B>
+__global__ __launch_bounds__(64) void k_gj_rows(double *__restrict__ W, double *__restrict__ G,
+                                                double *__restrict__ D, double *__restrict__ nextPt,
+                                                double *__restrict__ ownPt, const double *__restrict__ PtG, int32_t m, int32_t K, int32_t nb,
+                                                const double *__restrict__ cf, const GjMoves *__restrict__ mv,
+                                                double *__restrict__ U) {
+    __shared__ __align__(16) double fb[B][B];  // the factors of the block's own rows
+    for (int e = threadIdx.x; e < B * B; e += 64)
+        fb[e / B][e % B] = e / B < nb && e % B < nb ? cf[(int64_t)(e / B) * m + mv->src[e % B]] : 0.0;
+    __syncthreads();
+    const int32_t q = (int32_t)(blockIdx.x * 64 + threadIdx.x);
+    if (q >= m + K + nb) return;
+    const bool inv = q < m;
+    const int32_t j = inv ? q : q - m;
+    const bool fresh = j >= K && j < K + nb;  // W: a new column of the inverse; G: one of the block's columns
+    double *X = inv ? W : G;
+    const int64_t ldu = 2 * (int64_t)m;
+    double v[B], t[B];
+    const int nq = mv->nq;
+#pragma unroll
+    for (int r = 0; r < B; ++r) {
+        if (r >= nb)
+            v[r] = 0.0;
+        else if (!fresh)
+            v[r] = X[(int64_t)mv->src[r] * m + j];
+        else
+            v[r] = inv ? (r == j - K ? 1.0 : 0.0) : (r > j - K ? PtG[(int64_t)(j - K) * m + mv->src[r]] : 0.0);
+        t[r] = !fresh && r < nq ? X[(int64_t)mv->qsrc[r] * m + j] : 0.0;
+    }
+    const bool next = inv && j >= K + B && j < K + 2 * B;
+    if (!fresh) {
+#pragma unroll
+        for (int r = 0; r < B; ++r)
+            if (r < nq) {
+                X[(int64_t)mv->qdst[r] * m + j] = t[r];
+                if (next) nextPt[(int64_t)(j - K - B) * m + mv->qdst[r]] = t[r];
+            }
+    }
+    double dj = inv ? 0.0 : D[j];
+    const int32_t jrow = !inv && fresh ? mv->src[j - K] : j;  // a finished row stays where it is
+#pragma unroll
+    for (int kk = 0; kk < B; ++kk) {
+        if (kk < nb) {
+            const double u = v[kk];
+            U[kk * ldu + q] = u;
+#pragma unroll
+            for (int r = 0; r < B; ++r)
+                if (r != kk) v[r] = v[r] - fb[kk][r] * u;
+            if (!inv && (!fresh || kk > j - K)) dj = dj - cf[(int64_t)kk * m + jrow] * u;
+        }
+    }
+    if (inv) {
+#pragma unroll
+        for (int r = 0; r < B; ++r)
+            if (r < nb) {
+                W[(int64_t)(K + r) * m + j] = v[r];
+                if (next) nextPt[(int64_t)(j - K - B) * m + K + r] = v[r];
+                if (j >= K + 2 * B && j < K + 3 * B) ownPt[(int64_t)(j - K - 2 * B) * m + K + r] = v[r];
+            }
+    } else {
+        D[j] = dj;
+    }
+}
+
+// The other rows, and the next block's panel beside them (work-group 0): the
+// panel is one CU's work and longer than the update of one below about 2500
+// rows.  T / 4 rows x 128 columns per work-group, 4 x 8 per thread; first the
+// tiles of W (all rows outside the block), then those of G (rows below it,
+// columns below K + nb).  The columns of the block after the next also go to
+// its Pt (nextPt).
+template <int T, int B>
+struct GjRankLds {
+    double ff[B][T / 4], uu[B][128];
+};
+template <int T, int R, int B>
+__global__ __launch_bounds__(T) void k_gj_rank(double *__restrict__ W, double *__restrict__ G, int32_t m, int32_t K,
+                                               int32_t nb, GjBlock blk, GjBlock next, const double *__restrict__ U,
+                                               double *__restrict__ D, int32_t *__restrict__ perm,
+                                               int32_t *__restrict__ bad, int32_t tiles_w, int32_t tx_w, int32_t tx_g) {
+    constexpr int TR = T / 4;
+    __shared__ __align__(16) union Lds {
+        GjPanelLds<T / 64, B> panel;
+        GjRankLds<T, B> rank;
+    } ls;
+    if (blockIdx.x == 0) {
+        if (K + B < m) gj_panel<T, R, B>(ls.panel, m, K + B, min(B, m - K - B), next, &blk, U, D, perm, bad);
+        return;
+    }
+    auto &ff = ls.rank.ff;
+    auto &uu = ls.rank.uu;
+    const int32_t w = (int32_t)blockIdx.x - 1;
+    const bool inv = w < tiles_w;
+    const int32_t q = inv ? w : w - tiles_w, tx_n = inv ? tx_w : tx_g;
+    const int32_t i0 = (q / tx_n) * TR + (inv ? 0 : K + nb), j0 = (q % tx_n) * 128;
+    const int32_t jn = inv ? m : K + nb;
+    if (i0 >= m || j0 >= jn) return;
+    const int64_t ldu = 2 * (int64_t)m;
+    const int tid = threadIdx.x;
+    const int32_t fi = i0 + (tid & (TR - 1)) < m ? blk.slot_of[i0 + (tid & (TR - 1))] : -1;
+    for (int e = tid; e < B * TR; e += T)
+        ff[e / TR][e & (TR - 1)] = e / TR < nb && fi >= 0 ? blk.cf[(int64_t)(e / TR) * m + fi] : 0.0;
+    for (int e = tid; e < B * 128; e += T) {
+        const int32_t j = j0 + (e & 127);
+        uu[e >> 7][e & 127] = (e >> 7) < nb && j < jn ? U[(e >> 7) * ldu + (inv ? 0 : m) + j] : 0.0;
+    }
+    // thread (ty, tx): rows 4 ty + r, columns 2 tx + 32 c + {0, 1}
+    const int tx = tid & 15, ty = tid >> 4;
+    double *X = inv ? W : G;
+    double a[4][8];
+#pragma unroll
+    for (int r = 0; r < 4; ++r) {
+        const int32_t i = i0 + 4 * ty + r;
+#pragma unroll
+        for (int c = 0; c < 8; ++c) {
+            const int32_t j = j0 + 2 * tx + 32 * (c >> 1) + (c & 1);
+            double v = 0.0;
+            if (i < m && j < jn) {
+                if (j < K || j >= K + nb)
+                    v = X[(int64_t)i * m + j];
+                else if (!inv)
+                    v = blk.PtG[(int64_t)(j - K) * m + blk.slot_of[i]];
+            }
+            a[r][c] = v;
+        }
+    }
+    __syncthreads();
+#pragma unroll 2
+    for (int kk = 0; kk < B; ++kk) {
+        double f[4], u[8];
+#pragma unroll
+        for (int r = 0; r < 4; r += 2) {
+            const double2 v = *reinterpret_cast<const double2 *>(&ff[kk][4 * ty + r]);
+            f[r] = v.x;
+            f[r + 1] = v.y;
+        }
+#pragma unroll
+        for (int c = 0; c < 8; c += 2) {
+            const double2 v = *reinterpret_cast<const double2 *>(&uu[kk][2 * tx + 16 * c]);
+            u[c] = v.x;
+            u[c + 1] = v.y;
+        }
+#pragma unroll
+        for (int r = 0; r < 4; ++r)
+#pragma unroll
+            for (int c = 0; c < 8; ++c) a[r][c] = a[r][c] - f[r] * u[c];
+    }
+#pragma unroll
+    for (int r = 0; r < 4; ++r) {
+        const int32_t i = i0 + 4 * ty + r;
+        if (i >= m || (i >= K && i < K + nb)) continue;
+#pragma unroll
+        for (int c = 0; c < 8; ++c) {
+            const int32_t j = j0 + 2 * tx + 32 * (c >> 1) + (c & 1);
+            if (j >= jn) continue;
+            X[(int64_t)i * m + j] = a[r][c];
+            if (inv && j >= K + 2 * B && j < K + 3 * B) blk.Pt[(int64_t)(j - K - 2 * B) * m + i] = a[r][c];
+        }
+    }
+}
+
+// The first two blocks' columns, and the identity permutation.
+template <int B>
+__global__ void k_gj_first(const double *__restrict__ W, int32_t m, double *__restrict__ Pt0,
+                           double *__restrict__ Pt1, int32_t *__restrict__ perm) {
+    const int32_t i = (int32_t)(blockIdx.x * blockDim.x + threadIdx.x);
+    if (i >= m) return;
+    perm[i] = i;
+    for (int c = 0; c < 2 * B && c < m; ++c) (c < B ? Pt0 : Pt1)[(int64_t)(c % B) * m + i] = W[(int64_t)i * m + c];
+}
+
+// M[i][perm[p]] = W[i][p] / D[i]: the inverse's columns back in the rows' order.
+__global__ void k_gj_finish(const double *__restrict__ W, const double *__restrict__ D,
+                            const int32_t *__restrict__ perm, int32_t m, double *__restrict__ M) {
+    const int32_t p = (int32_t)(blockIdx.x * blockDim.x + threadIdx.x);
+    const int64_t i = blockIdx.y;
+    if (p < m) M[i * m + perm[p]] = W[i * m + p] / D[i];
+}
+
+// A in W (destroyed), the inverse into M (also G's room); work holds
+// gj_work(m) doubles and ints 3 m.
+constexpr int kGjMaxB = 16;
+static size_t gj_work(int64_t m) { return (size_t)(kGjMaxB * m * 8 + m) + 2 * (sizeof(GjMoves) / sizeof(double) + 2); }
+
+template <int T, int R, int B>
+static void gj_blocks(double *W, double *M, int32_t m, double *work, int32_t *ints, int32_t *bad, hipStream_t st) {
+    static_assert(B <= kGjMaxB, "work");
+    const int64_t bm = (int64_t)B * m;
+    GjBlock ring[2];
+    double *p = work;
+    for (int b = 0; b < 2; ++b) {
+        ring[b] = GjBlock{p, p + bm, p + 2 * bm, ints + (int64_t)(1 + b) * m, nullptr};
+        p += 3 * bm;
+    }
+    double *U = p, *D = U + 2 * bm;
+    for (int b = 0; b < 2; ++b) ring[b].mv = (GjMoves *)(D + m + (m & 1)) + b;
+    int32_t *perm = ints;
+    hipLaunchKernelGGL(k_gj_first<B>, dim3((unsigned)((m + 255) / 256)), dim3(256), 0, st, W, m, ring[0].Pt,
+                       ring[1].Pt, perm);
+    hipLaunchKernelGGL((k_gj_panel<T, R, B>), dim3(1), dim3(T), 0, st, m, std::min(B, m), ring[0], D, perm, bad);
+    for (int32_t K = 0, b = 0; K < m; K += B, b ^= 1) {
+        const int32_t nb = std::min(B, m - K);
+        const GjBlock &blk = ring[b], &next = ring[b ^ 1];
+        hipLaunchKernelGGL(k_gj_rows<B>, dim3((unsigned)((m + K + nb + 63) / 64)), dim3(64), 0, st, W, M, D, next.Pt,
+                           blk.Pt, blk.PtG, m, K, nb, blk.cf, blk.mv, U);
+        constexpr int TR = T / 4;
+        const int32_t tx_w = (m + 127) / 128, ty_w = (m + TR - 1) / TR, tx_g = (K + nb + 127) / 128,
+                      ty_g = (m - K - nb + TR - 1) / TR;
+        hipLaunchKernelGGL((k_gj_rank<T, R, B>), dim3((unsigned)(1 + tx_w * ty_w + tx_g * ty_g)), dim3(T), 0, st, W, M,
+                           m, K, nb, blk, next, U, D, perm, bad, tx_w * ty_w, tx_w, tx_g);
+    }
+    hipLaunchKernelGGL(k_gj_finish, dim3((unsigned)((m + 255) / 256), (unsigned)m), dim3(256), 0, st, W, D, perm, m,
+                       M);
+}
+
+// T R rows of a panel in one work-group's registers, R B doubles a thread of
+// its 512, 256 or 128 registers (T = 256, 512, 1024).  Measured build times:
+// m = 1001: <512, 2> with B = 8, 10, 12, 16: 2.95, 2.95, 2.99, 3.20 ms, <256,
+// 4, 16> 3.54; 1501: <1024, 2, 10> 5.38, <512, 4, 12> 5.60, <512, 4, 16> 6.12;
+// 2577: <512, 6> with 10, 12, 14: 13.2, 12.6, 13.0; 4001: <512, 8, 10> 36.7,
+// <512, 8, 8> 42.4, <512, 12, 7> 48.0, <1024, 4, 9> 73; 5201: <1024, 6, 8>
+// 87, <512, 12, 7> 95, <512, 12, 5> 124.  One column at a time took 13.7
+// (1001), 28.7, 104, 339 and 913 ms.  Above kGjBlocked rows a panel no longer
+// fits: one column at a time there.
+constexpr int64_t kGjBlocked = 12288;
+
+static void gj_blocked(double *W, double *M, int64_t m, double *work, int32_t *ints, int32_t *bad, hipStream_t st) {
+    const int32_t n = (int32_t)m;
+    if (m <= 256) gj_blocks<256, 1, 16>(W, M, n, work, ints, bad, st);
+    else if (m <= 512) gj_blocks<256, 2, 16>(W, M, n, work, ints, bad, st);
+    else if (m <= 1024) gj_blocks<512, 2, 10>(W, M, n, work, ints, bad, st);
+    else if (m <= 2048) gj_blocks<1024, 2, 10>(W, M, n, work, ints, bad, st);
+    else if (m <= 3072) gj_blocks<512, 6, 12>(W, M, n, work, ints, bad, st);
+    else if (m <= 4096) gj_blocks<512, 8, 10>(W, M, n, work, ints, bad, st);
+    else if (m <= 6144) gj_blocks<1024, 6, 8>(W, M, n, work, ints, bad, st);
+    else gj_blocks<512, 24, 2>(W, M, n, work, ints, bad, st);
+}
+
 __global__ __launch_bounds__(1024) void k_gj_pivot(const double *__restrict__ A, int64_t m, int64_t k,
                                                    int64_t *__restrict__ piv, int32_t *__restrict__ bad) {
     __shared__ double bv[1024];
@@ -159,14 +641,18 @@ __global__ void k_gj_scale(const double *__restrict__ A, double *__restrict__ I,
 
 int launch_invert(vx_case *c) {
     const int64_t m = c->P + 1;
-    DBuf<double> A;
-    if (A.ensure((size_t)(m * m), c->stream) || c->M.ensure((size_t)(m * m), c->stream) ||
-        c->red.ensure((size_t)m, c->stream) || c->dcount.ensure(4, c->stream)) {
-        A.release();
-        return 1;
-    }
+    const bool blocked = m <= kGjBlocked;
+    DBuf<double> A, work;
+    DBuf<int32_t> perm;
     int rc = 0;
+    if (A.ensure((size_t)(m * m), c->stream) || c->M.ensure((size_t)(m * m), c->stream) ||
+        c->dcount.ensure(4, c->stream))
+        rc = 1;
+    if (!rc && (blocked ? work.ensure(gj_work(m), c->stream) || perm.ensure((size_t)(3 * m), c->stream)
+                        : c->red.ensure((size_t)m, c->stream)))
+        rc = 1;
     do {
+        if (rc) break;
         if (hipMemcpyAsync(A.p, c->L.p, sizeof(double) * m * m, hipMemcpyDeviceToDevice, c->stream) != hipSuccess ||
             hipMemsetAsync(c->dcount.p, 0, sizeof(int64_t) * 4, c->stream) != hipSuccess) {
             set_error("invert: staging failed");
@@ -175,16 +661,20 @@ int launch_invert(vx_case *c) {
         }
         int64_t *piv = c->dcount.p;
         int32_t *bad = (int32_t *)(c->dcount.p + 1);
-        const dim3 g2((unsigned)((m + 255) / 256), (unsigned)m);
-        const unsigned g1 = (unsigned)((m + 255) / 256);
-        hipLaunchKernelGGL(k_gj_identity, g2, dim3(256), 0, c->stream, c->M.p, m);
-        for (int64_t k = 0; k < m; ++k) {
-            hipLaunchKernelGGL(k_gj_pivot, dim3(1), dim3(1024), 0, c->stream, A.p, m, k, piv, bad);
-            hipLaunchKernelGGL(k_gj_swap_factor, dim3(g1), dim3(256), 0, c->stream, A.p, c->M.p, m, k, piv);
-            hipLaunchKernelGGL(k_gj_colfactor, dim3(g1), dim3(256), 0, c->stream, A.p, m, k, c->red.p);
-            hipLaunchKernelGGL(k_gj_update, g2, dim3(256), 0, c->stream, A.p, c->M.p, m, k, c->red.p);
+        if (blocked) {
+            gj_blocked(A.p, c->M.p, m, work.p, perm.p, bad, c->stream);
+        } else {
+            const dim3 g2((unsigned)((m + 255) / 256), (unsigned)m);
+            const unsigned g1 = (unsigned)((m + 255) / 256);
+            hipLaunchKernelGGL(k_gj_identity, g2, dim3(256), 0, c->stream, c->M.p, m);
+            for (int64_t k = 0; k < m; ++k) {
+                hipLaunchKernelGGL(k_gj_pivot, dim3(1), dim3(1024), 0, c->stream, A.p, m, k, piv, bad);
+                hipLaunchKernelGGL(k_gj_swap_factor, dim3(g1), dim3(256), 0, c->stream, A.p, c->M.p, m, k, piv);
+                hipLaunchKernelGGL(k_gj_colfactor, dim3(g1), dim3(256), 0, c->stream, A.p, m, k, c->red.p);
+                hipLaunchKernelGGL(k_gj_update, g2, dim3(256), 0, c->stream, A.p, c->M.p, m, k, c->red.p);
+            }
+            hipLaunchKernelGGL(k_gj_scale, g2, dim3(256), 0, c->stream, A.p, c->M.p, m);
         }
-        hipLaunchKernelGGL(k_gj_scale, g2, dim3(256), 0, c->stream, A.p, c->M.p, m);
         if (hipGetLastError() != hipSuccess) {
             set_error("invert: launch failed");
             rc = 1;
@@ -204,6 +694,8 @@ int launch_invert(vx_case *c) {
     } while (0);
     (void)hipStreamSynchronize(c->stream);
     A.release();
+    work.release();
+    perm.release();
     return rc;
 }
 
