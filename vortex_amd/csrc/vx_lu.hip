@@ -20,9 +20,11 @@
 // W the two inverses (strict lower: L^-1 below its unit diagonal; upper
 // with diagonal: U^-1).
 #include <cmath>
+#include <type_traits>
 
 #include "vx_internal.h"
 #include "vx_prim.h"
+#include "vx_wave.h"
 
 namespace vx {
 
@@ -49,14 +51,10 @@ struct LuBufs {
 // multiples of 64 and K a multiple of 16.  One work-group of 4 waves per
 // 64 x 64 tile of C, each wave a 32 x 32 quarter as 2 x 2 products of
 // v_mfma_f32_16x16x4_f32 (A: lane = i + 16 k; B: lane = j + 16 k; C: lane =
-// j + 16 (i / 4), register i % 4).  TRI = 1: A is lower triangular in its
-// absolute indices (a_row0 + i, a_col0 + k) and the other triangle holds
-// zeros, TRI = 2: upper; the K loop then skips whole zero steps.
-template <int TRI>
+// j + 16 (i / 4), register i % 4).
 __global__ __launch_bounds__(256) void k_gemm_f32(const float *__restrict__ A, int64_t lda, const float *__restrict__ B,
                                                   int64_t ldb, float *C, int64_t ldc, const float *Cin,
-                                                  int64_t ldcin, int64_t K, float alpha, float beta, int64_t a_row0,
-                                                  int64_t a_col0) {
+                                                  int64_t ldcin, int64_t K, float alpha, float beta) {
     __shared__ float As[64][17];
     __shared__ float Bs[16][65];
     const int tid = threadIdx.x, wave = tid >> 6, lane = tid & 63;
@@ -65,19 +63,9 @@ __global__ __launch_bounds__(256) void k_gemm_f32(const float *__restrict__ A, i
     floatx4 acc[2][2];
     for (int a = 0; a < 2; ++a)
         for (int b = 0; b < 2; ++b) acc[a][b] = floatx4{0.f, 0.f, 0.f, 0.f};
-    int64_t k_lo = 0, k_hi = K;
-    if (TRI == 1) {
-        const int64_t lim = a_row0 + bm + 64 - a_col0;  // local k beyond the tile's last row are zero
-        k_hi = lim < K ? (lim > 0 ? lim : 0) : K;
-        k_hi = (k_hi + 15) / 16 * 16;
-    } else if (TRI == 2) {
-        const int64_t lim = a_row0 + bm - a_col0;  // local k before the tile's first row are zero
-        k_lo = lim > 0 ? (lim < K ? lim : K) : 0;
-        k_lo = k_lo / 16 * 16;
-    }
     const int ar = tid >> 2, ac = (tid & 3) * 4;     // A tile: 64 rows x 16
     const int br = tid >> 4, bc = (tid & 15) * 4;    // B tile: 16 rows x 64
-    for (int64_t k0 = k_lo; k0 < k_hi; k0 += 16) {
+    for (int64_t k0 = 0; k0 < K; k0 += 16) {
         const float *ap = A + (bm + ar) * lda + k0 + ac;
         const float *bp = B + (k0 + br) * ldb + bn + bc;
         const float4 av = *reinterpret_cast<const float4 *>(ap);
@@ -107,19 +95,97 @@ __global__ __launch_bounds__(256) void k_gemm_f32(const float *__restrict__ A, i
             }
 }
 
-template <int TRI>
 static int gemm(const float *A, int64_t lda, const float *B, int64_t ldb, float *C, int64_t ldc, const float *Cin,
-                int64_t ldcin, int64_t M, int64_t N, int64_t K, float alpha, float beta, int64_t a_row0,
-                int64_t a_col0, hipStream_t st) {
+                int64_t ldcin, int64_t M, int64_t N, int64_t K, float alpha, float beta, hipStream_t st) {
     if (M <= 0 || N <= 0 || K <= 0) return 0;
     if (M % 64 || N % 64 || K % 16) {
         set_error("internal: product sizes must be multiples of 64 (M, N) and 16 (K)");
         return 1;
     }
-    hipLaunchKernelGGL(k_gemm_f32<TRI>, dim3((unsigned)(N / 64), (unsigned)(M / 64)), dim3(256), 0, st, A, lda, B,
-                       ldb, C, ldc, Cin, ldcin, K, alpha, beta, a_row0, a_col0);
+    hipLaunchKernelGGL(k_gemm_f32, dim3((unsigned)(N / 64), (unsigned)(M / 64)), dim3(256), 0, st, A, lda, B,
+                       ldb, C, ldc, Cin, ldcin, K, alpha, beta);
     VX_CHECK(hipGetLastError());
     return 0;
+}
+
+// One block column of a triangular factor's inverse, C = -(A B) D with A the
+// inverse's finished triangle (TRI 1: lower, 2: upper; A's rows and columns
+// start at the same index), B the factor's block column and D its diagonal
+// block's inverse (64 x 64).  16 rows of C per work-group, so that the few
+// thousand rows there are spread over the chip: 64 x 64 tiles made 52
+// work-groups at most (71 us a column at 3392 rows, 14 us now); each wave 16
+// columns, K in LDS chunks of 64, the next two loaded while one is
+// multiplied.  An element's products are added in the order of k_gemm_f32
+// (skipped zeros apart), the second product in the same work-group.
+template <int TRI>
+__global__ __launch_bounds__(256) void k_lu_inv_col(const float *A, int64_t ld, const float *__restrict__ B,
+                                                    const float *D, float *C, int32_t K) {
+    __shared__ __align__(16) float As[2][16][68], Bs[2][64][80];
+    const int tid = threadIdx.x, wave = tid >> 6, lane = tid & 63;
+    const int q = lane & 15, g = lane >> 4, wn = wave * 16;
+    const int32_t bm = (int32_t)blockIdx.x * 16;
+    const int32_t k_lo = TRI == 2 ? bm / 64 * 64 : 0, k_hi = TRI == 1 ? (bm / 64 + 1) * 64 : K;
+    const int32_t chunks = (k_hi - k_lo) / 64;
+    const int ar = tid >> 4, ac = (tid & 15) * 4;  // A: a float4 per thread; B: four, 16 rows apart
+    const float *ap = A + (int64_t)(bm + ar) * ld + k_lo + ac;
+    const float *bp = B + (int64_t)(k_lo + ar) * ld + ac;
+    floatx4 acc = floatx4{0.f, 0.f, 0.f, 0.f};
+    struct Chunk {
+        floatx4 a, b0, b1, b2, b3;
+    } c0, c1;
+    auto load = [&](int32_t c, Chunk &v) __attribute__((always_inline)) {
+        const int32_t cc = min(c, chunks - 1) * 64;
+        const float *bb = bp + (int64_t)cc * ld;
+        v.a = *reinterpret_cast<const floatx4 *>(ap + cc);
+        v.b0 = *reinterpret_cast<const floatx4 *>(bb);
+        v.b1 = *reinterpret_cast<const floatx4 *>(bb + 16 * ld);
+        v.b2 = *reinterpret_cast<const floatx4 *>(bb + 32 * ld);
+        v.b3 = *reinterpret_cast<const floatx4 *>(bb + 48 * ld);
+    };
+    auto step = [&](int32_t c, auto half, Chunk &v) __attribute__((always_inline)) {
+        constexpr int b = decltype(half)::value;
+        *reinterpret_cast<floatx4 *>(&As[b][ar][ac]) = v.a;
+        *reinterpret_cast<floatx4 *>(&Bs[b][ar][ac]) = v.b0;
+        *reinterpret_cast<floatx4 *>(&Bs[b][ar + 16][ac]) = v.b1;
+        *reinterpret_cast<floatx4 *>(&Bs[b][ar + 32][ac]) = v.b2;
+        *reinterpret_cast<floatx4 *>(&Bs[b][ar + 48][ac]) = v.b3;
+        load(c + 2, v);
+        lds_barrier();  // also: every wave is done with chunk c - 1, whose buffer chunk c + 1 takes
+        // all operands before the first product: each waits for the one before it alone
+        float x[16], y[16];
+#pragma unroll
+        for (int s = 0; s < 16; ++s) {
+            x[s] = As[b][q][4 * s + g];
+            y[s] = Bs[b][4 * s + g][wn + q];
+        }
+        __builtin_amdgcn_sched_barrier(0);
+#pragma unroll
+        for (int s = 0; s < 16; ++s) acc = __builtin_amdgcn_mfma_f32_16x16x4f32(x[s], y[s], acc, 0, 0, 0);
+    };
+    const std::integral_constant<int, 0> even;
+    const std::integral_constant<int, 1> odd;
+    load(0, c0);
+    load(1, c1);
+    int32_t c = 0;
+    for (; c + 2 <= chunks; c += 2) {
+        step(c, even, c0);
+        step(c + 1, odd, c1);
+    }
+    if (c < chunks) step(c, even, c0);
+    lds_barrier();
+#pragma unroll
+    for (int e = 0; e < 4; ++e)
+        *reinterpret_cast<float4 *>(&Bs[0][ar + 16 * e][ac]) =
+            *reinterpret_cast<const float4 *>(D + (int64_t)(ar + 16 * e) * ld + ac);
+#pragma unroll
+    for (int r = 0; r < 4; ++r) As[0][4 * g + r][wn + q] = acc[r];
+    lds_barrier();
+    acc = floatx4{0.f, 0.f, 0.f, 0.f};
+#pragma unroll
+    for (int s = 0; s < 16; ++s)
+        acc = __builtin_amdgcn_mfma_f32_16x16x4f32(As[0][q][4 * s + g], Bs[0][4 * s + g][wn + q], acc, 0, 0, 0);
+#pragma unroll
+    for (int r = 0; r < 4; ++r) C[(int64_t)(bm + 4 * g + r) * ld + wn + q] = -acc[r];
 }
 
 // ---- factorisation ---------------------------------------------------------------
@@ -214,6 +280,213 @@ __global__ __launch_bounds__(1024) void k_lu_panel(float *__restrict__ F, int64_
         const int64_t i = k0 + e / kLuB;
         const int c = (int)(e % kLuB);
         F[i * np + k0 + c] = Pt[c * np + i];
+    }
+}
+
+// The same panel in sub-panels of kLuS columns, bit for bit: the products and
+// differences of an element are those of k_lu_panel in the same order, so only
+// where they are done changes.  k_lu_panel walks 64 columns of up to np rows
+// through memory with one work-group (0.85 ms a panel at 3392 rows).  Here a
+// work-group holds a sub-panel's columns of all rows in registers
+// (k_lu_sub, one LDS barrier a column), and the panel's other columns take
+// the sub-panel's steps on many work-groups (k_lu_sub_apply).  Rows move
+// between two column-major copies of the panel (64 x np), so that every
+// work-group reads the old places and writes the new.
+constexpr int kLuS = 16;
+
+// Panel [k0, k0 + 64) of F, rows from k0 on, column by column into Pt.
+__global__ __launch_bounds__(256) void k_lu_in(const float *__restrict__ F, int64_t np, int64_t k0,
+                                               float *__restrict__ Pt) {
+    __shared__ float t[64][65];
+    const int64_t i0 = k0 + (int64_t)blockIdx.x * 64;
+    const int x = threadIdx.x & 63, y = threadIdx.x >> 6;
+    for (int r = y; r < 64; r += 4) t[r][x] = F[(i0 + r) * np + k0 + x];
+    __syncthreads();
+    for (int c = y; c < 64; c += 4) Pt[c * np + i0 + x] = t[x][c];
+}
+
+// Columns k .. k + 15 (c0 = k - k0 in the panel) over the rows from k on, T R
+// of them at most.  A thread holds R rows, a swap exchanges the places of two
+// rows; each wave offers its largest candidate with its row in LDS.  The
+// step's column is a[.][0], the others move down.  The columns go back to Pt
+// by the rows' old places: below the diagonal the factors, on and above it U.
+template <int T, int R>
+__global__ __launch_bounds__(T) void k_lu_sub(float *__restrict__ Pt, int32_t np, int32_t k0, int32_t k,
+                                              int32_t *__restrict__ ipiv, int32_t *__restrict__ slot_of,
+                                              unsigned long long *__restrict__ st) {
+    constexpr int NW = T / 64, B = kLuS;
+    __shared__ __align__(16) float crow[2][NW][B];
+    __shared__ float ckey[2][NW];
+    __shared__ int cpos[2][NW];
+    const int tid = threadIdx.x, lane = tid & 63, wv = tid >> 6;
+    const int64_t c0 = k - k0;
+    float a[R][B];
+    int pos[R];
+#pragma unroll
+    for (int r = 0; r < R; ++r) {
+        const int s = k + tid + r * T;
+        pos[r] = s < np ? s : -1;
+#pragma unroll
+        for (int c = 0; c < B; ++c) a[r][c] = s < np ? Pt[(c0 + c) * np + s] : 0.f;
+    }
+#pragma unroll 1
+    for (int kk = 0; kk < B; ++kk) {
+        const int col = k + kk, par = kk & 1;
+        float key = -1.f;
+        int kp = 0x7fffffff, kr = 0;
+#pragma unroll
+        for (int r = 0; r < R; ++r) {
+            const float v = fabsf(a[r][0]);
+            if (pos[r] >= col && (v > key || (v == key && pos[r] < kp))) {
+                key = v;
+                kp = pos[r];
+                kr = r;
+            }
+        }
+        const float wm = wave_max(key);
+        const uint64_t ties = __ballot(key == wm);
+        const int wl = ties ? lowest_lane(ties, kp) : 0;
+        const int wr = __builtin_amdgcn_readlane(kr, wl);
+#pragma unroll
+        for (int r = 0; r < R; ++r)
+            if (wr == r) {
+                if (lane == wl) {
+#pragma unroll
+                    for (int c = 0; c < B; ++c) crow[par][wv][c] = a[r][c];
+                    ckey[par][wv] = key;
+                    cpos[par][wv] = kp;
+                }
+            }
+        lds_barrier();
+        const float ck = ckey[par][lane & (NW - 1)];
+        const int cp = cpos[par][lane & (NW - 1)];
+        const float gm = lane_of(row_max(ck), 15);
+        const uint64_t gt = __ballot(ck == gm) & ((1ull << NW) - 1);
+        const int gw = gt ? lowest_lane(gt, cp) : 0;
+        int p = __builtin_amdgcn_readlane(cp, gw);
+        const bool none = p < col || p >= np;  // no comparable entry (NaN): the diagonal one
+        if (none) p = col;
+        float row[B];
+#pragma unroll
+        for (int c = 0; c < B; ++c) row[c] = crow[par][gw][c];
+        if (none) row[0] = __builtin_nanf("");
+        const bool zero = row[0] == 0.f;  // singular: the column stays as it is
+        if (tid == 0) {
+            ipiv[col] = p;
+            if (zero) st[4] = 1ull;
+        }
+        // an FP32 quotient is never as near a rounding boundary as the FP64
+        // product's error, so this is the correctly rounded quotient
+        const double y = 1.0 / (double)row[0];
+#pragma unroll
+        for (int r = 0; r < R; ++r) {
+            pos[r] = pos[r] == p ? col : pos[r] == col ? p : pos[r];
+            float f = (float)((double)a[r][0] * y);
+            f = zero || pos[r] <= col ? 0.f : f;
+            const int s = k + tid + r * T;
+            if (s < np) Pt[(c0 + kk) * np + s] = pos[r] > col && !zero ? f : a[r][0];
+#pragma unroll
+            for (int c = 1; c < B; ++c) a[r][c - 1] = fmaf(-f, row[c], a[r][c]);
+            a[r][B - 1] = 0.f;
+        }
+    }
+#pragma unroll
+    for (int r = 0; r < R; ++r) {
+        const int s = k + tid + r * T;
+        if (s < np) slot_of[pos[r]] = s;
+    }
+}
+
+// The panel's columns after the sub-panel at k: moved rows in their new places
+// (old -> Pt, or -> F for the last), and the columns right of the sub-panel
+// through its kLuS steps.  A row per thread, 256 per work-group; each
+// work-group solves for U's rows itself.
+__global__ __launch_bounds__(256) void k_lu_sub_apply(const float *__restrict__ old, float *__restrict__ Pt,
+                                                      float *__restrict__ F, int32_t np, int32_t k0, int32_t k,
+                                                      const int32_t *__restrict__ slot_of) {
+    constexpr int B = kLuS;
+    __shared__ __align__(16) float lb[B][B], ub[B][kLuB];  // the block's factors; U's rows, columns of the panel
+    const int32_t c0 = k - k0, c1 = c0 + B;
+    const int tid = threadIdx.x;
+    lb[tid >> 4][tid & 15] = old[(int64_t)(c0 + (tid & 15)) * np + slot_of[k + (tid >> 4)]];
+    __syncthreads();
+    if (tid >= c1 && tid < kLuB) {
+        float v[B];
+#pragma unroll
+        for (int r = 0; r < B; ++r) v[r] = old[(int64_t)tid * np + slot_of[k + r]];
+#pragma unroll
+        for (int q = 0; q < B; ++q) {
+            ub[q][tid] = v[q];
+#pragma unroll
+            for (int r = q + 1; r < B; ++r) v[r] = fmaf(-lb[r][q], v[q], v[r]);
+        }
+    }
+    __syncthreads();
+    const int32_t i = k0 + (int32_t)blockIdx.x * 256 + tid;
+    if (i >= np) return;
+    const int64_t s = i >= k ? slot_of[i] : i;
+    float l[B];
+#pragma unroll
+    for (int q = 0; q < B; ++q) l[q] = old[(c0 + q) * (int64_t)np + s];
+    for (int32_t c = 0; c < kLuB; c += 4) {
+        float v[4];
+#pragma unroll
+        for (int e = 0; e < 4; ++e) v[e] = old[(c + e) * (int64_t)np + s];
+        if (c >= c1 && i >= k) {
+            if (i < k + B) {
+#pragma unroll
+                for (int e = 0; e < 4; ++e) v[e] = ub[i - k][c + e];
+            } else {
+#pragma unroll
+                for (int q = 0; q < B; ++q) {
+                    const float4 u = *reinterpret_cast<const float4 *>(&ub[q][c]);
+                    v[0] = fmaf(-l[q], u.x, v[0]);
+                    v[1] = fmaf(-l[q], u.y, v[1]);
+                    v[2] = fmaf(-l[q], u.z, v[2]);
+                    v[3] = fmaf(-l[q], u.w, v[3]);
+                }
+            }
+        }
+        if (c1 < kLuB) {
+#pragma unroll
+            for (int e = 0; e < 4; ++e) Pt[(c + e) * (int64_t)np + i] = v[e];
+        } else {
+            *reinterpret_cast<float4 *>(&F[(int64_t)i * np + k0 + c]) = float4{v[0], v[1], v[2], v[3]};
+        }
+    }
+}
+
+template <int T, int R>
+static void lu_sub(float *Pt, int64_t np, int64_t k0, int64_t k, int32_t *ipiv, int32_t *slot_of,
+                   unsigned long long *stt, hipStream_t st) {
+    hipLaunchKernelGGL((k_lu_sub<T, R>), dim3(1), dim3(T), 0, st, Pt, (int32_t)np, (int32_t)k0, (int32_t)k, ipiv,
+                       slot_of, stt);
+}
+
+// A panel by sub-panels while its rows fit a work-group's registers (16 floats
+// a row, T R rows), else by k_lu_panel.  T: 64 np floats twice.
+constexpr int64_t kLuSubRows = 12 * 512;
+
+static void lu_panel(float *F, int64_t np, int64_t k0, int32_t *ipiv, int32_t *slot_of, unsigned long long *stt,
+                     float *T, hipStream_t st) {
+    if (np - k0 > kLuSubRows) {
+        hipLaunchKernelGGL(k_lu_panel, dim3(1), dim3(1024), 0, st, F, np, k0, ipiv, stt, T);
+        return;
+    }
+    float *P[2] = {T, T + kLuB * np};
+    hipLaunchKernelGGL(k_lu_in, dim3((unsigned)((np - k0) / 64)), dim3(256), 0, st, F, np, k0, P[0]);
+    for (int sub = 0; sub < kLuB / kLuS; ++sub) {
+        const int64_t k = k0 + sub * kLuS, rows = np - k;
+        float *A = P[sub & 1], *B = P[(sub & 1) ^ 1];
+        if (rows <= 256) lu_sub<256, 1>(A, np, k0, k, ipiv, slot_of, stt, st);
+        else if (rows <= 512) lu_sub<256, 2>(A, np, k0, k, ipiv, slot_of, stt, st);
+        else if (rows <= 1024) lu_sub<512, 2>(A, np, k0, k, ipiv, slot_of, stt, st);
+        else if (rows <= 2048) lu_sub<512, 4>(A, np, k0, k, ipiv, slot_of, stt, st);
+        else if (rows <= 3072) lu_sub<512, 6>(A, np, k0, k, ipiv, slot_of, stt, st);
+        else if (rows <= 4096) lu_sub<512, 8>(A, np, k0, k, ipiv, slot_of, stt, st);
+        else lu_sub<512, 12>(A, np, k0, k, ipiv, slot_of, stt, st);
+        hipLaunchKernelGGL(k_lu_sub_apply, dim3((unsigned)((np - k0 + 255) / 256)), dim3(256), 0, st, A, B, F,
+                           (int32_t)np, (int32_t)k0, (int32_t)k, slot_of);
     }
 }
 
@@ -424,7 +697,7 @@ int launch_lu_setup(vx_case *c) {
     b.np = np;
     const size_t nn = (size_t)(np * np);
     if (b.F.ensure(nn, st) || b.Wl.ensure(nn, st) || b.Wu.ensure(nn, st) || b.W.ensure(nn, st) ||
-        b.T.ensure((size_t)(np * kLuB), st) || b.A.ensure((size_t)(n * n), st) || b.x.ensure((size_t)np, st) ||
+        b.T.ensure((size_t)(2 * np * kLuB), st) || b.A.ensure((size_t)(n * n), st) || b.x.ensure((size_t)np, st) ||
         b.rp.ensure((size_t)np, st) || b.t.ensure((size_t)np, st) || b.ipiv.ensure((size_t)np, st) ||
         b.perm.ensure((size_t)np, st) || b.pinv.ensure((size_t)np, st) || b.st.ensure(8, st) || b.nrm.ensure(2, st))
         return 1;
@@ -439,7 +712,7 @@ int launch_lu_setup(vx_case *c) {
     hipLaunchKernelGGL(k_lu_perm_init, dim3(g1), dim3(256), 0, st, b.perm.p, np);
     // right-looking LU: panel, swaps, block row, trailing product
     for (int64_t k0 = 0; k0 < np; k0 += kLuB) {
-        hipLaunchKernelGGL(k_lu_panel, dim3(1), dim3(1024), 0, st, b.F.p, np, k0, b.ipiv.p, b.st.p, b.T.p);
+        lu_panel(b.F.p, np, k0, b.ipiv.p, b.pinv.p, b.st.p, b.T.p, st);
         hipLaunchKernelGGL(k_lu_swap, dim3(g1), dim3(256), 0, st, b.F.p, np, k0, b.ipiv.p, b.perm.p);
         const int64_t rest = np - k0 - kLuB;
         if (rest > 0) {
@@ -447,7 +720,7 @@ int launch_lu_setup(vx_case *c) {
             float *A21 = b.F.p + (k0 + kLuB) * np + k0;
             float *A12 = b.F.p + k0 * np + k0 + kLuB;
             float *A22 = b.F.p + (k0 + kLuB) * np + k0 + kLuB;
-            if (gemm<0>(A21, np, A12, np, A22, np, A22, np, rest, rest, kLuB, -1.f, 1.f, 0, 0, st)) return 1;
+            if (gemm(A21, np, A12, np, A22, np, A22, np, rest, rest, kLuB, -1.f, 1.f, st)) return 1;
         }
     }
     VX_CHECK(hipGetLastError());
@@ -459,18 +732,12 @@ int launch_lu_setup(vx_case *c) {
     for (int64_t j0 = np - kLuB; j0 >= 0; j0 -= kLuB) {
         const int64_t r0 = j0 + kLuB, m = np - r0;
         if (m <= 0) continue;
-        if (gemm<1>(b.Wl.p + r0 * np + r0, np, b.F.p + r0 * np + j0, np, b.T.p, kLuB, b.T.p, kLuB, m, kLuB, m, 1.f,
-                    0.f, r0, r0, st) ||
-            gemm<0>(b.T.p, kLuB, b.Wl.p + j0 * np + j0, np, b.Wl.p + r0 * np + j0, np, b.Wl.p, np, m, kLuB, kLuB,
-                    -1.f, 0.f, 0, 0, st))
-            return 1;
+        hipLaunchKernelGGL(k_lu_inv_col<1>, dim3((unsigned)(m / 16)), dim3(256), 0, st, b.Wl.p + r0 * np + r0, np,
+                           b.F.p + r0 * np + j0, b.Wl.p + j0 * np + j0, b.Wl.p + r0 * np + j0, (int32_t)m);
     }
-    for (int64_t j0 = kLuB; j0 < np; j0 += kLuB) {
-        if (gemm<2>(b.Wu.p, np, b.F.p + j0, np, b.T.p, kLuB, b.T.p, kLuB, j0, kLuB, j0, 1.f, 0.f, 0, 0, st) ||
-            gemm<0>(b.T.p, kLuB, b.Wu.p + j0 * np + j0, np, b.Wu.p + j0, np, b.Wu.p, np, j0, kLuB, kLuB, -1.f, 0.f,
-                    0, 0, st))
-            return 1;
-    }
+    for (int64_t j0 = kLuB; j0 < np; j0 += kLuB)
+        hipLaunchKernelGGL(k_lu_inv_col<2>, dim3((unsigned)(j0 / 16)), dim3(256), 0, st, b.Wu.p, np, b.F.p + j0,
+                           b.Wu.p + j0 * np + j0, b.Wu.p + j0, (int32_t)j0);
     hipLaunchKernelGGL(k_lu_merge, g2, dim3(256), 0, st, b.Wl.p, b.Wu.p, np, b.W.p);
     VX_CHECK(hipGetLastError());
     unsigned long long sing = 0;
