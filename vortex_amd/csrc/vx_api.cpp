@@ -643,8 +643,7 @@ int vx_step(vx_case *c, double out4[4]) {
     VX_ARG(c && out4, "null pointer");
     Timer t(c, &c->tm.step_ms, 4);
     const int64_t n_ub = c->n;
-    if (launch_set_dn(c, n_ub) || launch_step_move(c) || launch_compact(c, n_ub) || launch_step_collapse(c, n_ub))
-        return 1;
+    if (launch_set_dn(c, n_ub) || launch_step_move(c) || launch_step_tail(c, n_ub)) return 1;
     int err = 0;
     if (step_readback(c, out4, &err)) return 1;
     if (err) {
@@ -806,9 +805,7 @@ static int device_step(vx_case *c, double vinf_x, double vinf_y) {
     const Cnt s = cnt_s(c);
     if (launch_biot_savart(c, s, s, vinf_x, vinf_y) || launch_diffusion(c, s, s) || launch_diffusion_wall(c, s))
         return 1;
-    if (launch_set_dn(c, n_ub) || launch_step_move(c) || launch_compact(c, n_ub) ||
-        launch_step_collapse(c, n_ub))
-        return 1;
+    if (launch_set_dn(c, n_ub) || launch_step_move(c) || launch_step_tail(c, n_ub)) return 1;
     return launch_step_record(c);
 }
 
@@ -817,7 +814,28 @@ static void graph_release(vx_case *c) {
     if (c->graph) (void)hipGraphDestroy(c->graph);
     c->graph_exec = nullptr;
     c->graph = nullptr;
-    c->graph_cap = -1;
+    c->graph_key.clear();
+}
+
+// All that a captured device_step holds fixed: the bound of its grids, the
+// free stream, its form, and every buffer it may use.  A call between two
+// runs (a probe over many points, a host-count step) can grow a workspace,
+// and a replay would then use the memory it had before.
+static void step_key(vx_case *c, double vinf_x, double vinf_y, std::vector<uint64_t> &k) {
+    uint64_t w[2];
+    memcpy(w, &vinf_x, 8);
+    memcpy(w + 1, &vinf_y, 8);
+    k.insert(k.end(), {(uint64_t)c->n_ub, (uint64_t)step_tail_fits(c, c->n_ub), w[0], w[1], (uint64_t)c->prb_m,
+                       (uint64_t)c->have_inverse, (uint64_t)c->tune.tpt_bs, (uint64_t)c->tune.tpt_diff,
+                       (uint64_t)c->tune.col_share_min, (uint64_t)c->gr_cap});
+    for (const void *p : std::initializer_list<const void *>{
+             c->x.p,     c->y.p,     c->g.p,      c->u.p,      c->v.p,        c->d.p,      c->xf.p,    c->yf.p,
+             c->gf.p,    c->L.p,     c->M.p,      c->lu,       c->rp.p,       c->gsheet.p, c->partial.p, c->red.p,
+             c->rhs_s.p, c->tx.p,    c->ty.p,     c->tg.p,     c->flags.p,    c->scan.p,   c->lists.p, c->col.p,
+             c->misc.p,  c->keys.p,  c->keys_alt.p, c->vals.p, c->vals_alt.p, c->cnode.p,  c->ptmp.p,  c->gridp.p,
+             c->dcount.p, c->colseg.p, c->wlist.p, c->wtmp.p,  c->wstage.p,   c->prb_x.p,  c->prb_y.p, c->prb_u.p,
+             c->prb_v.p, c->prb_part.p, c->gr_ring.p})
+        k.push_back((uint64_t)(uintptr_t)p);
 }
 
 __global__ void k_graph_begin(int64_t *__restrict__ dcount, int64_t n) {
@@ -829,7 +847,7 @@ __global__ void k_graph_begin(int64_t *__restrict__ dcount, int64_t n) {
 // Prepares c for `steps` device-count steps: capacity for every step, the
 // record ring, the count, error flag and ring slot on the device, and the
 // absorbed circulation in red[0].  Returns with c->devcount set.
-static int devcount_begin(vx_case *c, int64_t steps, bool *ring_moved) {
+static int devcount_begin(vx_case *c, int64_t steps) {
     VX_ARG(c->have_matrix, "no panel matrix");
     VX_ARG(!c->timing, "stage timing synchronises the host; switch it off for graph steps");
     const int64_t n_max = c->n + steps * c->P;
@@ -838,11 +856,9 @@ static int devcount_begin(vx_case *c, int64_t steps, bool *ring_moved) {
     if (reserve(c, ceil32(n_max + c->P) + 32)) return 1;
     hipStream_t s = c->stream;
     if (c->red.ensure(8, s) || c->dcount.ensure(16, s)) return 1;
-    *ring_moved = false;
     if (steps > c->gr_cap) {
         if (c->gr_ring.ensure((size_t)(5 * steps), s)) return 1;
         c->gr_cap = (int64_t)(c->gr_ring.n / 5);
-        *ring_moved = true;  // the ring's address is part of captured launches
     }
     c->n_ub = c->cap;
     VX_CHECK(hipMemcpyAsync(c->red.p, &c->d_g, sizeof(double), hipMemcpyHostToDevice, s));
@@ -898,15 +914,15 @@ static int instantiate(hipGraph_t g, hipGraphExec_t *exec) {
 int vx_run_steps_graph(vx_case *c, int64_t steps, double vinf_x, double vinf_y, double *f4, int64_t *counts) {
     VX_ARG(c && steps >= 0, "steps");
     if (steps == 0) return 0;
-    bool moved = false;
-    if (devcount_begin(c, steps, &moved)) {
+    if (devcount_begin(c, steps)) {
         c->devcount = false;
         return 1;
     }
-    if (moved || c->graph_cap != c->cap || c->graph_vinf[0] != vinf_x || c->graph_vinf[1] != vinf_y)
-        graph_release(c);
     hipStream_t s = c->stream;
     int rc = device_step(c, vinf_x, vinf_y);
+    std::vector<uint64_t> key;
+    step_key(c, vinf_x, vinf_y, key);
+    if (!rc && key != c->graph_key) graph_release(c);
     if (!rc && steps > 1 && !c->graph_exec) {
         VX_CHECK(hipStreamBeginCapture(s, hipStreamCaptureModeThreadLocal));
         rc = device_step(c, vinf_x, vinf_y);
@@ -921,9 +937,7 @@ int vx_run_steps_graph(vx_case *c, int64_t steps, double vinf_x, double vinf_y, 
             if (g) (void)hipGraphDestroy(g);
         } else {
             c->graph = g;
-            c->graph_cap = c->cap;
-            c->graph_vinf[0] = vinf_x;
-            c->graph_vinf[1] = vinf_y;
+            c->graph_key = key;
         }
     }
     for (int64_t k = 1; !rc && k < steps; ++k) {
@@ -955,8 +969,7 @@ struct vx_batch {
     std::vector<hipEvent_t> join;
     hipGraph_t graph = nullptr;
     hipGraphExec_t exec = nullptr;
-    std::vector<int64_t> caps;
-    std::vector<double> vinf;
+    std::vector<uint64_t> key;  // the cases' step_keys, in turn
 };
 
 static void batch_graph_release(vx_batch *b) {
@@ -1007,19 +1020,14 @@ int vx_batch_run_steps(vx_batch *b, int64_t steps, const double *vinf, double *f
     VX_ARG(b && vinf && steps >= 0, "batch arguments");
     if (steps == 0) return 0;
     const size_t k = b->cases.size();
-    bool stale = b->caps.size() != k || b->vinf.size() != 2 * k;
     int rc = 0;
-    for (size_t i = 0; i < k && !rc; ++i) {
-        vx_case *c = b->cases[i];
-        bool moved = false;
-        rc = devcount_begin(c, steps, &moved);
-        stale = stale || moved || b->caps[i] != c->cap || b->vinf[2 * i] != vinf[2 * i] ||
-                b->vinf[2 * i + 1] != vinf[2 * i + 1];
-    }
+    for (size_t i = 0; i < k && !rc; ++i) rc = devcount_begin(b->cases[i], steps);
     // the first step of every case on its own stream, uncaptured
     for (size_t i = 0; i < k && !rc; ++i) rc = device_step(b->cases[i], vinf[2 * i], vinf[2 * i + 1]);
     if (!rc && steps > 1) {
-        if (stale) batch_graph_release(b);
+        std::vector<uint64_t> key;
+        for (size_t i = 0; i < k; ++i) step_key(b->cases[i], vinf[2 * i], vinf[2 * i + 1], key);
+        if (key != b->key) batch_graph_release(b);
         // the batch stream waits for every case's first step
         for (size_t i = 0; i < k && !rc; ++i)
             if (hipEventRecord(b->join[i], b->cases[i]->stream) != hipSuccess ||
@@ -1050,9 +1058,7 @@ int vx_batch_run_steps(vx_batch *b, int64_t steps, const double *vinf, double *f
                 if (g) (void)hipGraphDestroy(g);
             } else {
                 b->graph = g;
-                b->caps.resize(k);
-                b->vinf.assign(vinf, vinf + 2 * k);
-                for (size_t i = 0; i < k; ++i) b->caps[i] = b->cases[i]->cap;
+                b->key = key;
             }
         }
         for (int64_t s = 1; !rc && s < steps; ++s)

@@ -208,8 +208,7 @@ struct vx_case {
     int64_t gr_cap = 0;
     hipGraph_t graph = nullptr;
     hipGraphExec_t graph_exec = nullptr;
-    int64_t graph_cap = -1;                           // capacity the graph was captured for
-    double graph_vinf[2] = {0.0, 0.0};
+    std::vector<uint64_t> graph_key;                  // what the graph was captured for (step_key)
     // timing
     bool timing = false;
     hipEvent_t ev[18] = {};
@@ -365,5 +364,9 @@ int launch_collapse(vx_case *c, int kind, int64_t n_ub, bool prepared, const Gri
 // compactions), from 2^17 slots on over a grid kept from pass to pass.
 // Collapse error flag in dcount[3] (bit 2: the grid's node pool was full).
 int launch_step_collapse(vx_case *c, int64_t n_ub);
+// The compaction after the move and launch_step_collapse, at small counts as
+// one launch with the same results.
+int launch_step_tail(vx_case *c, int64_t n_ub);
+bool step_tail_fits(const vx_case *c, int64_t n_ub);  // as one launch
 
 }  // namespace vx

@@ -1110,4 +1110,393 @@ int launch_step_collapse(vx_case *c, int64_t n_ub) {
     }
     return 0;
 }
+// ---- the tail of a step at small counts -----------------------------------------
+// The compaction after the move and every collapse pass with its compaction
+// in one launch of one work-group: at a few thousand vortices the stage is
+// about 40 launches of which each has next to nothing to do.  The decisions
+// and the arithmetic are those of the kernels above, slot by slot, so the
+// results are the same bit for bit: the closed form of the compaction, the
+// smallest partner index whatever the cells, the leaf-first resolution, the
+// merge.  x, y, g and the work arrays live in LDS up to kTailLds vortices
+// (the whole Step at 300, 2500 and 3300 vortices 141, 173 and 182 -> 57, 93
+// and 108 us); a graph's count may grow beyond, up to kTailMax, and is worked
+// on in place then, no faster than the launches (4000: 169 against 191,
+// 7900: 286 against 198), so a run that starts above kTailLds keeps those.
+// Bound by the one work-group's instructions.
+constexpr int kTailT = 1024, kTailHeads = 4096;
+constexpr int kTailLds = 3584;
+constexpr int64_t kTailMax = 8192;
+
+struct TailArgs {
+    double *x, *y, *g;
+    double *tx, *ty, *tg;          // compaction staging, 2 n slots
+    int32_t *holes, *donors;       // n slots each
+    const int64_t *dn;
+    int64_t *dn_out;
+    const double *box;             // live box after the move
+    int32_t *err;
+    double r2[2], max_ve_g;
+    int64_t n_col;
+};
+
+struct TailShared {
+    Grid grid[2];
+    int32_t wc[kTailMax / kTailT][kTailT / 64], woff[kTailMax / kTailT][kTailT / 64];
+    int32_t live, any, undecided;
+};
+
+// The list of a cell: cells are as small as the search allows, so that the
+// vortices crowded at a body spread over the lists, and share kTailHeads
+// lists by a hash; what else a list holds is too far to pair.
+__device__ __forceinline__ uint32_t tail_bucket(int32_t cx, int32_t cy) {
+    static_assert(kTailHeads == 1 << 12, "twelve bits");
+    return ((uint32_t)cx * 0x9E3779B1u + (uint32_t)cy * 0x85EBCA77u) >> 20;
+}
+// cell_of along one axis of at most 2^30 cells (one work-group walks every
+// slot, so its conversions count: 64-bit ones take twenty instructions each):
+// the cell, and the neighbour on the side of its half that holds v.
+__device__ __forceinline__ int32_t tail_cell(double v, double v0, double inv_s, int32_t n, int32_t &side) {
+    double f = (v - v0) * inv_s;
+    if (!(f >= 0.0)) f = 0.0;
+    const int32_t c = f >= (double)(n - 1) ? n - 1 : (int32_t)f;
+    side = f - (double)c < 0.5 ? c - 1 : c + 1;
+    return c;
+}
+
+// lds: heads, then next (also the scan), S, first, col of C ints, C bits,
+// then with IN_LDS x, y and g.  S holds the state bits of k_col_pass (1
+// active, 2 inactive, 4 killed by an active child, 16 published) and, from bit
+// 8, the count of unpublished candidates pointing at the slot.
+template <bool IN_LDS, int C>
+__device__ void tail_run(const TailArgs &A, TailShared &sh, int32_t *lds, int32_t n) {
+    int32_t *head = lds, *next = head + kTailHeads, *S = next + C, *first = S + C, *col = first + C;
+    uint32_t *bits = (uint32_t *)(col + C);
+    double *x, *y, *g;
+    if constexpr (IN_LDS) {
+        x = (double *)(bits + C / 32);
+        y = x + C;
+        g = y + C;
+    } else {
+        x = A.x;
+        y = A.y;
+        g = A.g;
+    }
+    const int tid = threadIdx.x, lane = tid & 63, wv = tid >> 6;
+    const int32_t n0 = n;
+    for (int32_t i = tid; i < n; i += kTailT) {
+        if constexpr (IN_LDS) {
+            x[i] = A.x[i];
+            y[i] = A.y[i];
+            g[i] = A.g[i];
+        }
+        S[i] = 0;
+        first[i] = INT32_MAX;
+    }
+    for (int32_t i = tid; i < C / 32; i += kTailT) bits[i] = 0u;
+    if (tid < 2) sh.grid[tid] = grid_params(A.box, A.r2[tid], (int64_t)1 << 30);
+    __syncthreads();
+
+    auto live = [&](int32_t i) { return i < n && !(fabs(g[i]) < kDelt); };
+    // k_compact_*: swap-with-last removal in closed form
+    auto compact = [&]() {
+        uint64_t bal[kTailMax / kTailT];
+#pragma unroll
+        for (int r = 0; r < (int)(kTailMax / kTailT); ++r) {
+            bal[r] = 0;
+            if (r * kTailT < n) {
+                bal[r] = __ballot(live(r * kTailT + tid));
+                if (lane == 0) sh.wc[r][wv] = __popcll(bal[r]);
+            } else if (lane == 0) {
+                sh.wc[r][wv] = 0;
+            }
+        }
+        __syncthreads();
+        if (tid < 64) {  // exclusive scan of the 128 wave counts, two per lane
+            constexpr int W = kTailT / 64;
+            int32_t *f = &sh.wc[0][0], *o = &sh.woff[0][0];
+            static_assert(kTailMax / kTailT * W == 128, "two counts per lane");
+            const int32_t a = f[2 * lane], b = f[2 * lane + 1];
+            int32_t inc = a + b;
+            for (int d = 1; d < 64; d <<= 1) {
+                const int32_t q = __shfl_up(inc, d, 64);
+                if (lane >= d) inc += q;
+            }
+            o[2 * lane] = inc - a - b;
+            o[2 * lane + 1] = inc - b;
+            if (lane == 63) sh.live = inc;
+        }
+        __syncthreads();
+        const int32_t n1 = sh.live;
+        if (n1 == n) return;  // every slot is live
+        const int32_t T = n - n1;
+        // at most T holes and donors: in the heads' room, else in memory
+        const bool small = T <= kTailHeads / 2;
+        int32_t *s = next;
+        int32_t *holes = small ? head : A.holes, *donors = small ? head + kTailHeads / 2 : A.donors;
+#pragma unroll
+        for (int r = 0; r < (int)(kTailMax / kTailT); ++r) {
+            const int32_t i = r * kTailT + tid;
+            if (i < n) {
+                const int32_t pos = sh.woff[r][wv] + __popcll(bal[r] & ((1ull << lane) - 1));
+                s[i] = pos;
+                const bool f = (bal[r] >> lane) & 1;
+                if (i < n1) {
+                    if (!f) holes[i - pos] = i;
+                } else if (f) {
+                    donors[n1 - pos - 1] = i;
+                }
+            }
+        }
+        __syncthreads();
+        const int32_t K = n1 > 0 ? n1 - s[n1] : 0;
+        auto source = [&](int32_t t) {
+            if (t < K) return donors[t];
+            const int32_t e = n1 + (t - K);
+            const int32_t above = n1 - (s[e] + (live(e) ? 1 : 0));
+            const int32_t start = above < K ? holes[above] : n1;
+            return e + 1 < n && !live(e + 1) ? e + 1 : start;
+        };
+        if (K + T <= kTailT) {  // a value per thread
+            double vx = 0.0, vy = 0.0, vg = 0.0;
+            if (tid < K + T) {
+                const int32_t src = source(tid);
+                vx = x[src];
+                vy = y[src];
+                vg = tid < K ? g[src] : 0.0;
+            }
+            __syncthreads();
+            if (tid < K + T) {
+                const int32_t dst = tid < K ? holes[tid] : n1 + (tid - K);
+                x[dst] = vx;
+                y[dst] = vy;
+                g[dst] = vg;
+            }
+        } else {
+            for (int32_t t = tid; t < K + T; t += kTailT) {
+                const int32_t src = source(t);
+                A.tx[t] = x[src];
+                A.ty[t] = y[src];
+                A.tg[t] = t < K ? g[src] : 0.0;
+            }
+            __syncthreads();
+            for (int32_t t = tid; t < K + T; t += kTailT) {
+                const int32_t dst = t < K ? holes[t] : n1 + (t - K);
+                x[dst] = A.tx[t];
+                y[dst] = A.ty[t];
+                g[dst] = A.tg[t];
+            }
+        }
+        n = n1;
+        __syncthreads();
+    };
+
+    compact();
+    for (int kind = 1; kind <= 2; ++kind) {
+        const Grid G = sh.grid[kind - 1];
+        const int32_t gx = (int32_t)G.nx, gy = (int32_t)G.ny;
+        const double r2 = A.r2[kind - 1];
+        int32_t n_before = -1;
+        for (int64_t cc = 0; cc < A.n_col; ++cc) {
+            // nothing to find, or the last pass of this kind changed nothing
+            if (!G.valid || n == n_before) break;
+            n_before = n;
+            for (int32_t t = tid; t < kTailHeads; t += kTailT) head[t] = -1;
+            if (tid == 0) sh.any = 0;
+            __syncthreads();
+            for (int32_t i = tid; i < n; i += kTailT)
+                if (g[i] != 0) {
+                    int32_t ox, oy;
+                    const int32_t cx = tail_cell(x[i], G.x0, G.inv_s, gx, ox);
+                    const int32_t cy = tail_cell(y[i], G.y0, G.inv_s, gy, oy);
+                    next[i] = atomicExch(&head[tail_bucket(cx, cy)], i);
+                }
+            __syncthreads();
+            // k_setka_nodes: the smallest partner above i in four cells.  A
+            // thread keeps its own candidates, bit r for slot r kTailT + tid.
+            uint32_t mine = 0;
+            for (int32_t r = 0; r * kTailT < n; ++r) {
+                const int32_t i = r * kTailT + tid;
+                int32_t best = INT32_MAX;
+                const double gi = i < n ? g[i] : 0.0;
+                if (gi != 0) {
+                    const double r0 = x[i], r1 = y[i];
+                    int32_t ox, oy;
+                    const int32_t cx = tail_cell(r0, G.x0, G.inv_s, gx, ox);
+                    const int32_t cy = tail_cell(r1, G.y0, G.inv_s, gy, oy);
+                    for (int q = 0; q < 4; ++q) {
+                        const int32_t xx = q & 1 ? ox : cx, yy = q >> 1 ? oy : cy;
+                        if ((uint32_t)xx >= (uint32_t)gx || (uint32_t)yy >= (uint32_t)gy) continue;
+                        for (int32_t j = head[tail_bucket(xx, yy)]; j >= 0; j = next[j]) {
+                            if (j <= i || j >= best) continue;
+                            const double gj = g[j];
+                            bool hit;
+                            if (kind == 1)
+                                hit = (gi * gj < 0) && (dist2(r0, r1, x[j], y[j]) < r2);
+                            else
+                                hit = (gi * gj > 0) && (dist2(r0, r1, x[j], y[j]) < r2) && (fabs(gi + gj) < A.max_ve_g);
+                            if (hit) best = j;
+                        }
+                    }
+                }
+                if (best != INT32_MAX) {
+                    col[i] = best;
+                    atomicOr(&bits[best >> 5], 1u << (best & 31));
+                    atomicAdd(&S[best], 1 << 8);
+                    mine |= 1u << r;
+                }
+            }
+            if (mine) sh.any = 1;
+            __syncthreads();
+            if (!sh.any) break;  // nothing merges: no compaction, and the next pass would find the same
+            // k_col_pass: leaves, rounds, merge
+            auto each = [&](uint32_t m, auto f) __attribute__((always_inline)) {
+                for (; m; m &= m - 1) f((__ffs((int)m) - 1) * kTailT + tid);
+            };
+            uint32_t rest = 0;
+            each(mine, [&](int32_t i) __attribute__((always_inline)) {
+                if ((bits[i >> 5] >> (i & 31)) & 1) {
+                    rest |= 1u << (i / kTailT);
+                    return;
+                }
+                const int32_t j = col[i];
+                atomicOr(&S[i], 1 | 16);
+                atomicOr(&S[j], 4);
+                atomicMin(&first[j], i);
+                atomicSub(&S[j], 1 << 8);
+            });
+            for (int32_t round = 0;; ++round) {
+                if (tid == 0) sh.undecided = 0;
+                __syncthreads();
+                bool open = false;
+                each(rest, [&](int32_t i) __attribute__((always_inline)) {
+                    const int32_t st = atomicOr(&S[i], 0);
+                    if (st & 3) return;
+                    if (st >> 8 == 0)
+                        atomicOr(&S[i], (st & 4) ? 2 : 1);
+                    else
+                        open = true;
+                });
+                if (open) sh.undecided = 1;
+                __syncthreads();
+                each(rest, [&](int32_t i) __attribute__((always_inline)) {
+                    const int32_t st = atomicOr(&S[i], 0);
+                    if ((st & 3) && !(st & 16)) {
+                        const int32_t j = col[i];
+                        if (st & 1) {
+                            atomicOr(&S[j], 4);
+                            atomicMin(&first[j], i);
+                        }
+                        atomicOr(&S[i], 16);
+                        atomicSub(&S[j], 1 << 8);
+                    }
+                });
+                const int more = sh.undecided;
+                __syncthreads();
+                if (!more) break;
+                if (round > n + 1) {
+                    if (tid == 0) atomicOr(A.err, 1);
+                    break;
+                }
+            }
+            each(mine, [&](int32_t i) __attribute__((always_inline)) {
+                if (!(S[i] & 1)) return;
+                const int32_t j = col[i];
+                const bool fst = first[j] == i;
+                double xj = 1e+10, yj = 1e+10, gj = 0.0;
+                if (fst) {
+                    xj = x[j];
+                    yj = y[j];
+                    gj = g[j];
+                }
+                const double xi = x[i], yi = y[i], gi = g[i];
+                const double ng = gi + gj;
+                double nx, ny;
+                if (kind == 1) {
+                    const double mn = fabs(gi) + fabs(gj);
+                    nx = (xi * fabs(gi) + xj * fabs(gj)) / fabs(mn);
+                    ny = (yi * fabs(gi) + yj * fabs(gj)) / fabs(mn);
+                } else {
+                    nx = (xi * gi + xj * gj) / ng;
+                    ny = (yi * gi + yj * gj) / ng;
+                }
+                x[i] = nx;
+                y[i] = ny;
+                g[i] = ng;
+                if (fst) {
+                    x[j] = 1e+10;
+                    y[j] = 1e+10;
+                    g[j] = 0.0;
+                }
+            });
+            __syncthreads();
+            each(mine, [&](int32_t i) __attribute__((always_inline)) {
+                const int32_t j = col[i];
+                S[i] = S[j] = 0;
+                first[i] = first[j] = INT32_MAX;
+            });
+            for (int32_t i = tid; i < C / 32; i += kTailT) bits[i] = 0u;
+            compact();
+            __syncthreads();
+        }
+    }
+    if constexpr (IN_LDS) {
+        __syncthreads();
+        for (int32_t i = tid; i < n0; i += kTailT) {
+            A.x[i] = x[i];
+            A.y[i] = y[i];
+            A.g[i] = g[i];
+        }
+    }
+    if (tid == 0) *A.dn_out = n;
+}
+
+constexpr size_t tail_ints(int64_t c) { return (size_t)(kTailHeads + 4 * c + c / 32); }
+constexpr size_t kTailBytes = std::max(sizeof(int32_t) * tail_ints(kTailLds) + 24 * (size_t)kTailLds,
+                                       sizeof(int32_t) * tail_ints(kTailMax));
+
+__global__ __launch_bounds__(kTailT) void k_step_tail(TailArgs A) {
+    __shared__ __align__(16) int32_t lds[kTailBytes / sizeof(int32_t)];
+    __shared__ TailShared sh;
+    const int32_t n = (int32_t)*A.dn;
+    if (n <= kTailLds)
+        tail_run<true, kTailLds>(A, sh, lds, n);
+    else
+        tail_run<false, (int)kTailMax>(A, sh, lds, n);
+}
+
+// The compaction after the move and the collapse (both kinds), by count.
+bool step_tail_fits(const vx_case *c, int64_t n_ub) { return n_ub <= kTailMax && c->n <= kTailLds; }
+
+int launch_step_tail(vx_case *c, int64_t n_ub) {
+    if (!step_tail_fits(c, n_ub)) return launch_compact(c, n_ub) || launch_step_collapse(c, n_ub);
+    if (n_ub <= 0) return 0;
+    hipStream_t st = c->stream;
+    if (c->lists.ensure((size_t)(2 * n_ub), st) || c->tx.ensure((size_t)(2 * n_ub), st) ||
+        c->ty.ensure((size_t)(2 * n_ub), st) || c->tg.ensure((size_t)(2 * n_ub), st) || c->dcount.ensure(16, st))
+        return 1;
+    const double ve2 = c->prm.ve_size * c->prm.ve_size;
+    int32_t *l = c->lists.p;
+    TailArgs A{};
+    A.x = c->x.p;
+    A.y = c->y.p;
+    A.g = c->g.p;
+    A.tx = c->tx.p;
+    A.ty = c->ty.p;
+    A.tg = c->tg.p;
+    A.holes = l;
+    A.donors = l + n_ub;
+    A.dn = step_dn(c);
+    A.dn_out = c->dcount.p + (c->dn_slot == 1 ? 8 : 1);
+    A.box = c->red.p + 4;
+    A.err = (int32_t *)(c->dcount.p + 3);
+    A.r2[0] = c->prm.r_col_diff_sign * c->prm.r_col_diff_sign * ve2;  // src/unit_1.cu:1228-1229
+    A.r2[1] = c->prm.r_col_same_sign * c->prm.r_col_same_sign * ve2;
+    A.max_ve_g = c->prm.max_ve_g;
+    A.n_col = c->prm.n_col;
+    hipLaunchKernelGGL(k_step_tail, dim3(1), dim3(kTailT), 0, st, A);
+    VX_CHECK(hipGetLastError());
+    c->dn_slot = c->dn_slot == 1 ? 8 : 1;
+    return 0;
+}
+
 }  // namespace vx
