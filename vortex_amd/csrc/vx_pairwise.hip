@@ -17,6 +17,7 @@
 #include "vx_internal.h"
 #include "vx_math.h"
 #include "vx_prim.h"
+#include "vx_wave.h"
 
 namespace vx {
 
@@ -923,57 +924,150 @@ __global__ __launch_bounds__(256) void k_right_part_terms(const double *__restri
         part[(c * 2 + (tid & 1)) * pan.P + S.first + p0 + (tid >> 1)] = acc;
 }
 
-// Far sources: per work-group partial S_k (FP64), k < kLoc, grid-stride over
-// the sources; spart[(blk * kLoc + k) * 2 + {0,1}].
-__global__ __launch_bounds__(256) void k_rhs_far_partial(const double *__restrict__ x, const double *__restrict__ y,
-                                                         const double *__restrict__ g, Cnt cn_src, double cx,
-                                                         double cy, double r2, double *__restrict__ spart) {
-    __shared__ double red[16][256];
-    const int64_t n_src = cn_src.get();
+// Sums of g w^{k+1}, w = 1 / (z_j - c), k < kLoc, over a work-group's sources
+// (FP64; item(j, g, dx, dy) gives source j, or false to leave it out), in a
+// fixed order: each thread its own sources, then the binary tree over the
+// 256 threads, strides 128 to 1.  out gets the kLoc complex sums.
+//
+// Eight terms at a time go through LDS.  The tree used to be walked there,
+// eight levels with a barrier and 16 read-add-writes each; now sixteen
+// threads take a row, sixteen values each in the tree's order, and the last
+// four levels are lane exchanges: the same sums.  A work-group whose threads
+// have one source each (all of them, up to 131072 sources and 8192 listed
+// ones) runs the terms as a loop with nothing kept in registers: the 48
+// unrolled terms are 8 KB of code read once.  Both launches of a step at 2785
+// vortices: 41 -> 6.4 us.
+constexpr int kRedRow = 256 + 16;  // a row of the LDS stage: 16 doubles of padding split two rows over the banks
+
+__device__ __forceinline__ void rhs_rows_out(const double *red, double *__restrict__ out) {
+    const int tid = threadIdx.x, e = tid & 15;
+    const double *row = red + (tid >> 4) * kRedRow + e;
+    double a[16];
+#pragma unroll
+    for (int m = 0; m < 16; ++m) a[m] = row[16 * m];
+#pragma unroll
+    for (int st = 8; st > 0; st >>= 1)
+#pragma unroll
+        for (int m = 0; m < st; ++m) a[m] += a[m + st];
+    double r = a[0];
+    for (int st = 8; st > 0; st >>= 1) r += __shfl_xor(r, st, 16);
+    if (e == 0) out[tid >> 4] = r;
+}
+
+template <class Item>
+__device__ __forceinline__ void rhs_expand(Item item, int64_t n, int64_t first, int64_t stride,
+                                           double (*red)[16 * kRedRow], double *__restrict__ out) {
+    const int tid = threadIdx.x;
+    if (n <= stride) {
+        double pr = 0.0, pi = 0.0, wr = 0.0, wi = 0.0, gj, dx, dy;
+        if (first < n && item(first, gj, dx, dy)) {
+            const double q2 = dx * dx + dy * dy;
+            wr = dx / q2;
+            wi = -dy / q2;
+            pr = gj * wr;
+            pi = gj * wi;
+        }
+#pragma unroll 1
+        for (int k0 = 0; k0 < kLoc; k0 += 8) {
+            double *r = red[(k0 >> 3) & 1];
+#pragma unroll
+            for (int q = 0; q < 8; ++q) {
+                r[2 * q * kRedRow + tid] = 0.0 + pr;
+                r[(2 * q + 1) * kRedRow + tid] = 0.0 + pi;
+                const double npr = fma(wr, pr, -(wi * pi));
+                pi = fma(wi, pr, wr * pi);
+                pr = npr;
+            }
+            lds_barrier();  // the other buffer was last read before this one was written
+            rhs_rows_out(r, out + 2 * k0);
+        }
+        return;
+    }
     double sr[kLoc], si[kLoc];
 #pragma unroll
     for (int k = 0; k < kLoc; ++k) sr[k] = si[k] = 0.0;
-    for (int64_t j = (int64_t)blockIdx.x * blockDim.x + threadIdx.x; j < n_src; j += (int64_t)gridDim.x * blockDim.x) {
-        const double gj = g[j];
-        const double dx = x[j] - cx, dy = y[j] - cy;
+    for (int64_t j = first; j < n; j += stride) {
+        double gj, dx, dy;
+        if (!item(j, gj, dx, dy)) continue;
         const double q2 = dx * dx + dy * dy;
-        if (gj == 0 || !(q2 >= r2)) continue;
-        const double wr = dx / q2, wi = -dy / q2;  // w = 1 / (z_j - c)
-        double pr = gj * wr, pi = gj * wi;           // g w^{k+1}
+        const double wr = dx / q2, wi = -dy / q2;
+        double pr = gj * wr, pi = gj * wi;
 #pragma unroll
         for (int k = 0; k < kLoc; ++k) {
             sr[k] += pr;
             si[k] += pi;
-            const double npr = pr * wr - pi * wi;
-            pi = pr * wi + pi * wr;
+            const double npr = fma(wr, pr, -(wi * pi));
+            pi = fma(wi, pr, wr * pi);
             pr = npr;
         }
     }
-    // block sums, eight terms at a time, in a fixed order
 #pragma unroll
     for (int k0 = 0; k0 < kLoc; k0 += 8) {
-        __syncthreads();
+        double *r = red[(k0 >> 3) & 1];
 #pragma unroll
         for (int q = 0; q < 8; ++q) {
-            red[2 * q][threadIdx.x] = sr[k0 + q];
-            red[2 * q + 1][threadIdx.x] = si[k0 + q];
+            r[2 * q * kRedRow + tid] = sr[k0 + q];
+            r[(2 * q + 1) * kRedRow + tid] = si[k0 + q];
         }
-        __syncthreads();
-        for (int st = 128; st > 0; st >>= 1) {
-            if ((int)threadIdx.x < st)
-                for (int q = 0; q < 16; ++q) red[q][threadIdx.x] += red[q][threadIdx.x + st];
-            __syncthreads();
-        }
-        if (threadIdx.x < 16) spart[((int64_t)blockIdx.x * kLoc + k0) * 2 + threadIdx.x] = red[threadIdx.x][0];
+        lds_barrier();
+        rhs_rows_out(r, out + 2 * k0);
+    }
+}
+
+// The global expansion (far sources, work-groups [0, nfar)) and the segments'
+// own (then nseg work-groups for each segment: listed sources at least 2 R_s
+// from its centre) in one launch, neither needs the other.  Work-groups
+// without a source leave no partial, rhs_groups counts those that do.
+constexpr int kFarBlocks = 512;
+constexpr int kSegBlocks = 32;
+
+__host__ __device__ __forceinline__ int64_t rhs_groups(int64_t n, int64_t most) {
+    const int64_t b = (n + 255) / 256;
+    return b < most ? b : most;
+}
+
+__global__ __launch_bounds__(256) void k_rhs_expand(const double *__restrict__ x, const double *__restrict__ y,
+                                                    const double *__restrict__ g, Cnt cn_src, double cx, double cy,
+                                                    double r2, const int32_t *__restrict__ list,
+                                                    const int32_t *__restrict__ nlist,
+                                                    const RhsSeg *__restrict__ segs, int64_t nfar, int64_t nseg,
+                                                    double *__restrict__ spart, double *__restrict__ spart_seg) {
+    __shared__ double red[2][16 * kRedRow];
+    if ((int64_t)blockIdx.x < nfar) {
+        const int64_t n = cn_src.get(), first = (int64_t)blockIdx.x * 256;
+        if (first >= n) return;
+        rhs_expand(
+            [&](int64_t j, double &gj, double &dx, double &dy) {
+                gj = g[j];
+                dx = x[j] - cx;
+                dy = y[j] - cy;
+                return !(gj == 0 || !(dx * dx + dy * dy >= r2));
+            },
+            n, first + threadIdx.x, nfar * 256, red, spart + (int64_t)blockIdx.x * kLoc * 2);
+    } else {
+        const int64_t b = (int64_t)blockIdx.x - nfar, s = b / nseg, first = b % nseg * 256, n = *nlist;
+        if (first >= n) return;
+        const RhsSeg S = segs[s];
+        const double rn2 = 4.0 * S.r * S.r;
+        rhs_expand(
+            [&](int64_t t, double &gj, double &dx, double &dy) {
+                const int32_t j = list[t];
+                gj = g[j];
+                dx = x[j] - S.cx;
+                dy = y[j] - S.cy;
+                return dx * dx + dy * dy >= rn2;
+            },
+            n, first + threadIdx.x, nseg * 256, red, spart_seg + (s * kSegBlocks + first / 256) * kLoc * 2);
     }
 }
 
 // S_k over the work-group partials: one work-group per real/imaginary part of
 // each term, a strided pass per thread and a tree in LDS (fixed order).
-__global__ __launch_bounds__(256) void k_rhs_far_final(const double *__restrict__ spart, int64_t nblk,
+__global__ __launch_bounds__(256) void k_rhs_far_final(const double *__restrict__ spart, Cnt cn_src, int64_t nfar,
                                                        double *__restrict__ S) {
     __shared__ double r[256];
     const int t = blockIdx.x;
+    const int64_t nblk = rhs_groups(cn_src.get(), nfar);  // the others would add exact zeros
     double a = 0.0;
     for (int64_t b = threadIdx.x; b < nblk; b += 256) a += spart[b * 2 * kLoc + t];
     r[threadIdx.x] = a;
@@ -985,82 +1079,52 @@ __global__ __launch_bounds__(256) void k_rhs_far_final(const double *__restrict_
     if (threadIdx.x == 0) S[t] = r[0];
 }
 
-// Listed sources at least 2 R_s from a segment's centre: their terms
-// g w^{m+1}, w = 1 / (z_j - c_s), for m < kLoc, per work-group (blockIdx.y
-// of kSegBlocks for segment blockIdx.x, grid-stride over the list), summed in
-// a fixed order; spart[((s * kSegBlocks + blk) * kLoc + m) * 2 + {0,1}].
-constexpr int kSegBlocks = 32;
-
-__global__ __launch_bounds__(256) void k_rhs_seg_partial(const double *__restrict__ x, const double *__restrict__ y,
-                                                         const double *__restrict__ g,
-                                                         const int32_t *__restrict__ list,
-                                                         const int32_t *__restrict__ nlist,
-                                                         const RhsSeg *__restrict__ segs,
-                                                         double *__restrict__ spart) {
-    __shared__ double red[16][256];
-    const RhsSeg S = segs[blockIdx.x];
-    const double rn2 = 4.0 * S.r * S.r;
-    const int64_t n = *nlist;
-    double sr[kLoc], si[kLoc];
-#pragma unroll
-    for (int k = 0; k < kLoc; ++k) sr[k] = si[k] = 0.0;
-    for (int64_t t = (int64_t)blockIdx.y * blockDim.x + threadIdx.x; t < n; t += (int64_t)gridDim.y * blockDim.x) {
-        const int32_t j = list[t];
-        const double dx = x[j] - S.cx, dy = y[j] - S.cy;
-        const double q2 = dx * dx + dy * dy;
-        if (!(q2 >= rn2)) continue;
-        const double wr = dx / q2, wi = -dy / q2;
-        double pr = g[j] * wr, pi = g[j] * wi;
-#pragma unroll
-        for (int k = 0; k < kLoc; ++k) {
-            sr[k] += pr;
-            si[k] += pi;
-            const double npr = pr * wr - pi * wi;
-            pi = pr * wi + pi * wr;
-            pr = npr;
-        }
+// Binomials C(k, m), m <= k < kLoc (below 2^44, so exact).
+struct Binom {
+    double c[kLoc][kLoc];
+};
+constexpr Binom binomials() {
+    Binom b{};
+    for (int k = 0; k < kLoc; ++k) {
+        b.c[k][0] = 1.0;
+        for (int m = 1; m <= k; ++m) b.c[k][m] = b.c[k - 1][m - 1] + (m < k ? b.c[k - 1][m] : 0.0);
     }
-    const int64_t blk = (int64_t)blockIdx.x * gridDim.y + blockIdx.y;
-#pragma unroll
-    for (int k0 = 0; k0 < kLoc; k0 += 8) {
-        __syncthreads();
-#pragma unroll
-        for (int q = 0; q < 8; ++q) {
-            red[2 * q][threadIdx.x] = sr[k0 + q];
-            red[2 * q + 1][threadIdx.x] = si[k0 + q];
-        }
-        __syncthreads();
-        for (int st = 128; st > 0; st >>= 1) {
-            if ((int)threadIdx.x < st)
-                for (int q = 0; q < 16; ++q) red[q][threadIdx.x] += red[q][threadIdx.x + st];
-            __syncthreads();
-        }
-        if (threadIdx.x < 16) spart[(blk * kLoc + k0) * 2 + threadIdx.x] = red[threadIdx.x][0];
-    }
+    return b;
 }
+__device__ const Binom kBinom = binomials();
 
 // Each segment's coefficients about c_s: the global S shifted exactly,
 //   sum_{k >= m} S_k C(k, m) (c_s - c)^{k - m},
 // plus its own sources' partials (fixed order).  Thread m < kLoc.
-__global__ void k_rhs_seg_final(const double *__restrict__ spart, const double *__restrict__ S, double cx,
-                                double cy, const RhsSeg *__restrict__ segs, double *__restrict__ Ss) {
+__global__ __launch_bounds__(64) void k_rhs_seg_final(const double *__restrict__ spart, const double *__restrict__ S,
+                                                      double cx, double cy, const RhsSeg *__restrict__ segs,
+                                                      const int32_t *__restrict__ nlist, int64_t nseg,
+                                                      double *__restrict__ Ss) {
+    __shared__ double lS[2 * kLoc];
+    for (int t = threadIdx.x; t < 2 * kLoc; t += 64) lS[t] = S[t];
+    __syncthreads();
     const int m = threadIdx.x;
     if (m >= kLoc) return;
     const RhsSeg G = segs[blockIdx.x];
+    const int nb = (int)rhs_groups(*nlist, nseg);
     const double er = G.cx - cx, ei = G.cy - cy;  // c_s - c
     double ar = 0.0, ai = 0.0;
-    double bin = 1.0;              // C(k, m)
-    double pr = 1.0, pi = 0.0;     // (c_s - c)^{k - m}
-    for (int k = m; k < kLoc; ++k) {
+    double pr = 1.0, pi = 0.0;  // (c_s - c)^{k - m}
+#pragma unroll 4
+    for (int q = 0; q < kLoc; ++q) {
+        const int k = m + q < kLoc ? m + q : kLoc - 1;
+        const double bin = kBinom.c[k][m];
         const double tr = pr * bin, ti = pi * bin;
-        ar += S[2 * k] * tr - S[2 * k + 1] * ti;
-        ai += S[2 * k] * ti + S[2 * k + 1] * tr;
-        bin = bin * (double)(k + 1) / (double)(k + 1 - m);
-        const double npr = pr * er - pi * ei;
-        pi = pr * ei + pi * er;
+        const double sr = ar + fma(tr, lS[2 * k], -(ti * lS[2 * k + 1]));
+        const double si = ai + fma(ti, lS[2 * k], tr * lS[2 * k + 1]);
+        ar = m + q < kLoc ? sr : ar;
+        ai = m + q < kLoc ? si : ai;
+        const double npr = fma(er, pr, -(ei * pi));
+        pi = fma(ei, pr, er * pi);
         pr = npr;
     }
-    for (int b = 0; b < kSegBlocks; ++b) {
+#pragma unroll 8
+    for (int b = 0; b < nb; ++b) {
         const double *q = spart + (((int64_t)blockIdx.x * kSegBlocks + b) * kLoc + m) * 2;
         ar += q[0];
         ai += q[1];
@@ -1078,6 +1142,17 @@ __device__ __forceinline__ void chunk_sum2(const double *__restrict__ part, int6
     for (int64_t c = threadIdx.x; c < nchunk; c += kTile) {
         x0 += part[(c * 2 + 0) * m + i];
         x1 += part[(c * 2 + 1) * m + i];
+    }
+    if (nchunk <= 64) {  // the tree's first two levels would add zeros
+        if (threadIdx.x < 64) {
+            for (int st = 32; st > 0; st >>= 1) {
+                x0 += __shfl_xor(x0, st, 64);
+                x1 += __shfl_xor(x1, st, 64);
+            }
+        }
+        a = x0;  // of thread 0, the one that goes on
+        b = x1;
+        return;
     }
     r[0][threadIdx.x] = x0;
     r[1][threadIdx.x] = x1;
@@ -1103,14 +1178,17 @@ __global__ __launch_bounds__(kTile) void k_right_part_final(const double *__rest
                                                             const RhsSeg *__restrict__ segs,
                                                             const int32_t *__restrict__ seg_of, double vinf_x,
                                                             double vinf_y, double *__restrict__ R) {
+    __shared__ double S[2 * kLoc], inv[kLoc];
     const int64_t i = blockIdx.x;
     const int64_t used = ((int64_t)*nlist + kRhsChunk - 1) / kRhsChunk;
+    const int32_t sg = seg_of[i];
+    if (threadIdx.x < 2 * kLoc) S[threadIdx.x] = Ss[(int64_t)sg * 2 * kLoc + threadIdx.x];
+    if (threadIdx.x < kLoc) inv[threadIdx.x] = 1.0 / (double)(threadIdx.x + 1);
+    __syncthreads();
     double y0, y1;
     chunk_sum2(part, used < nchunk ? used : nchunk, pan.P, i, y0, y1);
     if (threadIdx.x != 0) return;
-    const int32_t sg = seg_of[i];
     const double cx = segs[sg].cx, cy = segs[sg].cy;
-    const double *S = Ss + (int64_t)sg * 2 * kLoc;
     const double d0 = pan.rx[i] - pan.lx[i], d1 = pan.ry[i] - pan.ly[i];
     const double mnog = 1 / (2 * kPi * (d0 * d0 + d1 * d1));
     // W = sum_k (i S_k / 2 pi) Q_k / (k + 1), u = Re W, v = -Im W
@@ -1119,20 +1197,19 @@ __global__ __launch_bounds__(kTile) void k_right_part_final(const double *__rest
     double qr = 1.0, qi = 0.0;                               // Q_0
     double bkr = 1.0, bki = 0.0;                             // b^k
     double wr = 0.0, wi = 0.0;
-#pragma unroll
+#pragma unroll 4
     for (int k = 0; k < kLoc; ++k) {
         if (k > 0) {
-            const double nbr = bkr * br - bki * bi;
-            bki = bkr * bi + bki * br;
+            const double nbr = fma(br, bkr, -(bi * bki));
+            bki = fma(br, bki, bi * bkr);
             bkr = nbr;
-            const double nqr = ar * qr - ai * qi + bkr;
-            qi = ar * qi + ai * qr + bki;
+            const double nqr = fma(ar, qr, -(ai * qi)) + bkr;
+            qi = fma(ar, qi, ai * qr) + bki;
             qr = nqr;
         }
         const double sr = S[2 * k], si = S[2 * k + 1];
-        const double inv = 1.0 / (double)(k + 1);
-        wr += (sr * qr - si * qi) * inv;
-        wi += (sr * qi + si * qr) * inv;
+        wr = fma(fma(qr, sr, -(qi * si)), inv[k], wr);
+        wi = fma(fma(sr, qi, si * qr), inv[k], wi);
     }
     // times i / (2 pi)
     const double uf = -wi / (2 * kPi), vf = -(wr / (2 * kPi));
@@ -1399,7 +1476,6 @@ int launch_right_part(vx_case *c, Cnt cn_src, double vinf_x, double vinf_y) {
     hipStream_t st = c->stream;
     const int64_t n_src = cn_src.ub;  // bound: grids, list and partial sizes
     const int64_t nchunk = n_src > 0 ? (n_src + kRhsChunk - 1) / kRhsChunk : 1;
-    constexpr int64_t kFarBlocks = 512;
     const size_t ns_far = (size_t)(2 * kLoc * kFarBlocks), ns_glob = 2 * kLoc,
                  ns_seg = (size_t)(2 * kLoc * kSegBlocks * K), ns_segS = (size_t)(2 * kLoc * K);
     if (c->partial.ensure((size_t)(2 * nchunk * P), st) || c->rp.ensure((size_t)P, st) ||
@@ -1435,12 +1511,12 @@ int launch_right_part(vx_case *c, Cnt cn_src, double vinf_x, double vinf_y) {
     }
     // the global expansion (sources beyond 2 R_b), the segments' own
     // sources, and each segment's total about c_s
-    hipLaunchKernelGGL(k_rhs_far_partial, dim3((unsigned)kFarBlocks), dim3(256), 0, st, c->x.p, c->y.p, c->g.p, cn_src,
-                       cx, cy, rnear2, c->rhs_s.p);
-    hipLaunchKernelGGL(k_rhs_far_final, dim3(2 * kLoc), dim3(256), 0, st, c->rhs_s.p, kFarBlocks, S);
-    hipLaunchKernelGGL(k_rhs_seg_partial, dim3((unsigned)K, (unsigned)kSegBlocks), dim3(256), 0, st, c->x.p, c->y.p,
-                       c->g.p, c->lists.p, nlist, c->segs, spart);
-    hipLaunchKernelGGL(k_rhs_seg_final, dim3((unsigned)K), dim3(64), 0, st, spart, S, cx, cy, c->segs, Ss);
+    const int64_t nfar = rhs_groups(n_src, kFarBlocks), nseg = rhs_groups(n_src, kSegBlocks);
+    if (nfar > 0)
+        hipLaunchKernelGGL(k_rhs_expand, dim3((unsigned)(nfar + K * nseg)), dim3(256), 0, st, c->x.p, c->y.p, c->g.p,
+                           cn_src, cx, cy, rnear2, c->lists.p, nlist, c->segs, nfar, nseg, c->rhs_s.p, spart);
+    hipLaunchKernelGGL(k_rhs_far_final, dim3(2 * kLoc), dim3(256), 0, st, c->rhs_s.p, cn_src, nfar, S);
+    hipLaunchKernelGGL(k_rhs_seg_final, dim3((unsigned)K), dim3(64), 0, st, spart, S, cx, cy, c->segs, nlist, nseg, Ss);
     VX_CHECK(hipGetLastError());
     hipLaunchKernelGGL(k_right_part_final, dim3((unsigned)P), dim3(kTile), 0, st, c->partial.p, nchunk, nlist, c->pan,
                        Ss, c->segs, c->seg_of, vinf_x, vinf_y, c->rp.p);
