@@ -127,31 +127,6 @@ __device__ __forceinline__ void keep4(T &m0, T &m1, T &m2, T &m3, T r) {
     m0 = A::min_(m0, r);
 }
 
-__device__ __forceinline__ void order2(double &a, double &b) {
-    const double lo = fmin(a, b), hi = fmax(a, b);
-    a = lo;
-    b = hi;
-}
-
-// Four values at a time: they are sorted (5 exchanges), the pairwise minima
-// with the kept ones in reverse are the four smallest of the eight, a bitonic
-// run that 4 exchanges sort.  FP64 has no med3: 5.5 min/max a value against 13.
-__device__ __forceinline__ void keep4x4(double &m0, double &m1, double &m2, double &m3, double a, double b, double c,
-                                        double d) {
-    order2(a, b);
-    order2(c, d);
-    order2(a, c);
-    order2(b, d);
-    order2(b, c);
-    m0 = fmin(m0, d);
-    m1 = fmin(m1, c);
-    m2 = fmin(m2, b);
-    m3 = fmin(m3, a);
-    order2(m0, m2);
-    order2(m1, m3);
-    order2(m0, m1);
-    order2(m2, m3);
-}
 // Two values at a time, the same way (6 min/max a value).
 __device__ __forceinline__ void keep4x2(double &m0, double &m1, double &m2, double &m3, double a, double b) {
     order2(a, b);

@@ -33,6 +33,7 @@
 #include <vector>
 
 #include "vx_internal.h"
+#include "vx_math.h"
 #include "vx_prim.h"
 
 namespace vx {
@@ -959,7 +960,7 @@ template <typename T>
 struct PairMath;
 template <>
 struct PairMath<double> {
-    __device__ static __forceinline__ double div(double a, double b) { return a / b; }
+    __device__ static __forceinline__ double div(double a, double b) { return div_pos(a, b); }
     __device__ static __forceinline__ double sqrt_bound(double a) { return sqrt(a); }
     __device__ static __forceinline__ double med3(double a, double b, double c) {
         return fmax(fmin(a, b), fmin(fmax(a, b), c));
@@ -1099,6 +1100,23 @@ __device__ __forceinline__ void p2p_leaf(const Src4T<T> *lds, int cnt, T ox, T o
             pu -= w * dy;
             pv += v * ex;
             pu -= v * ey;
+        }
+    }
+    if constexpr (sizeof(T) == 8) {
+        // four sources at a time: their quotients' chains overlap, and the
+        // smallest distances take 5.5 min/max a pair against 13
+        for (; jj + 3 < cnt; jj += 4) {
+            T r2[4];
+#pragma unroll
+            for (int e = 0; e < 4; ++e) {
+                const Src4T<T> q = lds[jj + e];
+                const T dx = ox - q.x, dy = oy - q.y;
+                r2[e] = dx * dx + dy * dy;
+                const T w = PM::div(q.g, CLAMP ? fmax(r2[e], eps2) : r2[e]);
+                pv += w * dx;
+                pu -= w * dy;
+            }
+            if constexpr (TRACK) keep4x4(m0, m1, m2, m3, r2[0], r2[1], r2[2], r2[3]);
         }
     }
     for (; jj < cnt; ++jj) {
@@ -1389,7 +1407,15 @@ __device__ __forceinline__ int64_t xcd_block() {
 constexpr int kBsStack = 256;  // traversal stack entries per wave
 constexpr int kFarQ = 512;     // FP32: far nodes queued per wave before any M2L
 
-template <typename T, int ORDER, int STRIDE>
+// S waves per bucket.  FP64 takes four up to kBsSplit buckets, each with every
+// fourth far node and near leaf: one each are three waves a SIMD at 131103
+// vortices, and the longest chain sets the time (0.54 -> 0.42 ms; 500000: 1.53
+// -> 1.46).  Each walks the tree by itself, which costs more than the balance
+// gives where there are waves enough (2^20: 2.89 -> 3.11).  FP32's far
+// nodes are translated 16 at a time, which wants them together.
+constexpr int64_t kBsSplit = 14336;
+
+template <typename T, int ORDER, int STRIDE, int S>
 __device__ __forceinline__ void bs_wave(const TreeDev &t, double theta, double eps, double vinf_x, double vinf_y,
                                         double *__restrict__ u, double *__restrict__ v, double *__restrict__ d,
                                         double *__restrict__ sdo,
@@ -1399,6 +1425,7 @@ __device__ __forceinline__ void bs_wave(const TreeDev &t, double theta, double e
                                         unsigned long long &cm2l) {
     using PM = PairMath<T>;
     constexpr bool F32 = sizeof(T) == 4;
+    static_assert(S == 1 || (S == 4 && !F32), "a work-group holds whole groups of waves");
     __shared__ Src4T<T> lds_all[4][kLeaf];
     __shared__ int32_t fq_all[4][kFarQ];  // FP32: far nodes waiting for M2L
     __shared__ int32_t stk_all[4][kBsStack];
@@ -1409,7 +1436,8 @@ __device__ __forceinline__ void bs_wave(const TreeDev &t, double theta, double e
     // targets: one bucket per wave (a compact node, which keeps the MAC's
     // opening radius small; runs of 64 particles of the Morton order fill
     // more lanes but open about 1.6 times as many pairs)
-    const int leaf = __builtin_amdgcn_readfirstlane((int)(xcd_block() * 4 + (threadIdx.x >> 6)));
+    const int leaf = __builtin_amdgcn_readfirstlane((int)(S == 1 ? xcd_block() * 4 + (threadIdx.x >> 6) : xcd_block()));
+    const int part = S == 1 ? 0 : __builtin_amdgcn_readfirstlane((int)(threadIdx.x >> 6));
     if (leaf >= t.nleaf) return;
     const NodeRec L = t.rec[leaf];
     const int nvalid = L.b;
@@ -1444,7 +1472,7 @@ __device__ __forceinline__ void bs_wave(const TreeDev &t, double theta, double e
     const float rT = fmaxf((float)rA, 1e-30f);  // FP32: kTiny would round to zero
     // the own bucket first: its particles are usually the nearest, which
     // tightens the bound that lets most other leaves skip the nearest-3 updates
-    {
+    if (part == 0) {
         stage_leaf<T>(lds, lane, -1 - L.a, nvalid, t);
         T pu = 0, pv = 0;
         const int h = share_len(ls, nvalid);
@@ -1453,6 +1481,14 @@ __device__ __forceinline__ void bs_wave(const TreeDev &t, double theta, double e
         npairs += nvalid;
         su += (double)pu;
         sv += (double)pv;
+    }
+    // (the other waves of the bucket keep lists of their own, under its bound)
+    T bound = T(1e5);
+    if constexpr (S > 1) {
+        __shared__ T bound_s[64];
+        if (part == 0) bound_s[lane] = m3;
+        __syncthreads();
+        bound = bound_s[lane];
     }
     // Traversal: a stack in the wave's LDS slot, popped up to 64 nodes at a
     // time, one per lane, which tests its node's MAC; far nodes are queued
@@ -1513,7 +1549,7 @@ __device__ __forceinline__ void bs_wave(const TreeDev &t, double theta, double e
         if (isleaf) lq[__popcll(lm & ((1ull << lane) - 1))] = node;
         const int nl = __popcll(lm);
         const uint64_t fm = __ballot(isfar);
-        nfar += __popcll(fm);
+        if (part == 0) nfar += __popcll(fm);
         if constexpr (F32) {
             if (isfar) fq[nq + __popcll(fm & ((1ull << lane) - 1))] = node;
             nq += __popcll(fm);
@@ -1539,18 +1575,17 @@ __device__ __forceinline__ void bs_wave(const TreeDev &t, double theta, double e
                 fv += sr * qx - si * qy;
                 farmin = fmin(farmin, PM::sqrt_bound(den) - (T)nd.r);
             };
-            if (ls.per == 1) {
-                for (uint64_t m = fm; m; m &= m - 1) m2p(__builtin_amdgcn_readlane(node, __builtin_ctzll(m)));
-            } else {
-                // a target's lanes take the far nodes in turn
-                if (isfar) fq[__popcll(fm & ((1ull << lane) - 1))] = node;
-                __builtin_amdgcn_wave_barrier();
-                const int nf = __popcll(fm);
-                for (int fi = ls.sub; fi < nf; fi += ls.per) m2p(fq[fi]);
-            }
+            // the bucket's waves, and a target's lanes, take the far nodes in turn
+            if (isfar) fq[__popcll(fm & ((1ull << lane) - 1))] = node;
+            __builtin_amdgcn_wave_barrier();
+            const int nf = __popcll(fm);
+            if (ls.per == 1)
+                for (int fi = part; fi < nf; fi += S) m2p(__builtin_amdgcn_readfirstlane(fq[fi]));
+            else
+                for (int fi = part * ls.per + ls.sub; fi < nf; fi += S * ls.per) m2p(fq[fi]);
         }
         __builtin_amdgcn_wave_barrier();
-        for (int li = 0; li < nl; ++li) {
+        for (int li = part; li < nl; li += S) {
             const int lnode = __builtin_amdgcn_readfirstlane(lq[li]);
             const NodeRec nd = t.rec[lnode];
             const double ddx = nd.cx - cAx, ddy = nd.cy - cAy;
@@ -1576,7 +1611,7 @@ __device__ __forceinline__ void bs_wave(const TreeDev &t, double theta, double e
             // eps of some target
             const T cx_ = F32 ? ox : ax - (T)nd.cx, cy_ = F32 ? oy : ay - (T)nd.cy;
             const T dc2 = cx_ * cx_ + cy_ * cy_;
-            const T reach = (T)nd.r + PM::sqrt_bound(m3), reache = (T)nd.r + (T)eps;
+            const T reach = (T)nd.r + PM::sqrt_bound(S == 1 ? m3 : fmin(m3, bound)), reache = (T)nd.r + (T)eps;
             const bool near3 = ok && !(dc2 > reach * reach * T(1.002));
             const bool neare = ok && !(dc2 > reache * reache * T(1.002));
             if (__ballot(near3))
@@ -1593,6 +1628,30 @@ __device__ __forceinline__ void bs_wave(const TreeDev &t, double theta, double e
     }
     su += (double)fu;
     sv += (double)fv;
+    if constexpr (S > 1) {  // the waves' shares, in wave order
+        __shared__ T sh_[S - 1][7][64];
+        if (part > 0) {
+            T(&o)[7][64] = sh_[part - 1];
+            o[0][lane] = su;
+            o[1][lane] = sv;
+            o[2][lane] = m0;
+            o[3][lane] = m1;
+            o[4][lane] = m2;
+            o[5][lane] = m3;
+            o[6][lane] = farmin;
+        }
+        cpairs = (unsigned long long)(npairs * nvalid);
+        __syncthreads();
+        if (part > 0) return;
+#pragma unroll
+        for (int q = 0; q < S - 1; ++q) {
+            const T(&o)[7][64] = sh_[q];
+            su += o[0][lane];
+            sv += o[1][lane];
+            keep4x4(m0, m1, m2, m3, o[2][lane], o[3][lane], o[4][lane], o[5][lane]);
+            farmin = fmin(farmin, o[6][lane]);
+        }
+    }
     // the target's shares: sums added in the same order on each of its
     // lanes, the four smallest distances merged, the far bound the least
     for (int o = ls.tpw; o < 64; o <<= 1) {
@@ -1646,7 +1705,7 @@ __device__ __forceinline__ void bs_wave(const TreeDev &t, double theta, double e
 }
 
 // ORDER terms of coefficients stored STRIDE per node.
-template <typename T, int ORDER, int STRIDE>
+template <typename T, int ORDER, int STRIDE, int S>
 __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(sizeof(T) == 4 && ORDER == 16 ? 6 : 1)))
 void k_tree_bs(TreeDev t, double theta, double eps, double vinf_x, double vinf_y,
                                                  double *__restrict__ u, double *__restrict__ v,
@@ -1654,7 +1713,7 @@ void k_tree_bs(TreeDev t, double theta, double eps, double vinf_x, double vinf_y
                                                  int32_t *__restrict__ fb, double *__restrict__ fbr2,
                                                  unsigned long long *__restrict__ nfb, int exact_all) {
     unsigned long long cp = 0, cf = 0, cl = 0;
-    bs_wave<T, ORDER, STRIDE>(t, theta, eps, vinf_x, vinf_y, u, v, d, sdo, fb, fbr2, nfb, exact_all, cp, cf, cl);
+    bs_wave<T, ORDER, STRIDE, S>(t, theta, eps, vinf_x, vinf_y, u, v, d, sdo, fb, fbr2, nfb, exact_all, cp, cf, cl);
     block_count_add(cp, cf, nfb + 1, nfb + 2);
     block_count_add(cl, 0ull, nfb + 7, nullptr);
 }
@@ -1852,7 +1911,8 @@ __global__ __launch_bounds__(1024) void k_tree_nearest_fallback(TreeDev t, const
 // Diffusion pair terms (src/kernel.cu:1011-1019): s1 += g e, (s2x, s2y) +=
 // g e (dx, dy) / r with e = exp(-r / d), for r above the threshold.  FP32:
 // kd = -log2(e) / d and a below-threshold r^2 is pushed to 1e30, whose
-// weight underflows to zero; FP64: kd = 1 / d.
+// weight underflows to zero.  FP64: the same kd and one inverse square root
+// for r and 1 / r (vx_math.h); a below-threshold pair's g counts as 0.
 template <typename T>
 struct DiffPair;
 template <>
@@ -1897,33 +1957,43 @@ __device__ __forceinline__ void diff_pair_log(float dx, float dy, float lg, floa
 template <>
 struct DiffPair<double> {
     template <bool GUARD>
-    __device__ static __forceinline__ void add(double dx, double dy, double g, double kd, double thr,
+    __device__ static __forceinline__ void add(double dx, double dy, double g, double kd, double thr2,
                                                double &s2x, double &s2y, double &s1) {
-        const double dist = sqrt(dx * dx + dy * dy);
-        if (!GUARD || dist > thr) {
-            const double w = g / dist;
-            const double e = exp(-dist * kd);
-            s2x += w * dx * e;
-            s2y += w * dy * e;
-            s1 += g * e;
-        }
+        const double r2 = dx * dx + dy * dy;
+        const bool far = !GUARD || r2 > thr2;
+        double rs, r;
+        rsqrt_sqrt_pos(far ? r2 : 1.0, rs, r);
+        const double ge = (far ? g : 0.0) * exp2_neg(r * kd);
+        const double w = ge * rs;
+        s2x += w * dx;
+        s2y += w * dy;
+        s1 += ge;
     }
 };
 
-// Radius beyond which a diffusion target is summed by k_diff_far: 5 % of
-// the root's radius.  At most t.fcap targets are listed (the most of kFarCap,
-// one in 16 included vortices and a quarter more than the last diffusion
-// found: sparse wakes have many); further ones stay in their group's wave.
+// Radius beyond which a diffusion target is summed by k_diff_far, as a part
+// of the root's radius: in a group it would widen the group's wave to much of
+// the wake, a long serial chain.  A wave for a target and 64 buckets costs
+// more per pair than a group's wave, though, and a sparse wake has many wide
+// targets side by side, which share their group's sources.  So FP64, whose
+// groups have four waves, draws the line at 10 % (66000, 90000 and 131103
+// vortices of a 10 x 4 wake: speed stage 2.52, 3.12 and 3.40 ms with 5 %, which
+// listed half of the targets and more; 1.23, 1.62 and 1.94 with 10 %, 1.25,
+// 1.58 and 1.94 with 20 %), FP32 at 5 %.  At most t.fcap targets are listed
+// (the most of kFarCap, one in 16 included vortices and a quarter more than
+// the last diffusion found); further ones stay in their group's wave.
 constexpr int64_t kFarCap = 4096;
+template <typename T>
+constexpr double far_part() {
+    return sizeof(T) == 4 ? 0.05 : 0.1;
+}
 // A target goes to k_diff_far when kFarCut d (or its cut-off times d, if
-// smaller) exceeds far_radius(): the same targets for both cut-offs, so the
-// FP64 path's 30 d widens some group waves rather than listing a large part
-// of a sparse wake.
+// smaller) exceeds far_radius().
 constexpr double kFarCut = 18.0;
-__device__ __forceinline__ double far_radius(const TreeDev &t) {
+__device__ __forceinline__ double far_radius(const TreeDev &t, double part) {
     const double4 b = t.nbb[t.root];
     const double rr = 0.5 * sqrt((b.y - b.x) * (b.y - b.x) + (b.w - b.z) * (b.w - b.z));
-    return fmax(0.05 * rr, 1e-300);
+    return fmax(part * rr, 1e-300);
 }
 
 __device__ __forceinline__ int64_t far_count(const unsigned long long *cnt, int64_t cap) {
@@ -1937,14 +2007,21 @@ __device__ __forceinline__ int64_t far_count(const unsigned long long *cnt, int6
 // largest radius of its lanes reaches it and, lane by lane, when some lane's
 // own radius reaches it.  A lane whose radius exceeds far_radius() is listed for
 // k_diff_far instead and does not widen the wave's radius.  A group of at
-// most 32 targets gives each several lanes (LaneSplit).  cnt[0] +=
+// most 32 targets gives each several lanes (LaneSplit).  In FP64 a group has
+// four waves, each with every fourth of the listed leaves: one each are two
+// waves a SIMD at 131103 vortices, and the longest chain sets the time (with the wider
+// groups of far_part, 1.46 -> 1.03 ms; the FP64 pair terms of vx_math.h
+// before that, 1.66 -> 1.06 ms).  cnt[0] +=
 // evaluated pairs, cnt[2] the list length.
+constexpr int kDiffWaves = 4;  // per target group
+
 template <typename T, bool CENSUS>
-__device__ __forceinline__ void diffusion_wave(const TreeDev &t, double cut, double nu, double thr,
+__device__ __forceinline__ void diffusion_wave(const TreeDev &t, double cut, double nu, double thr, double thr2d,
                                                const double *__restrict__ sd, double *__restrict__ u,
                                                double *__restrict__ v, unsigned long long *__restrict__ cnt,
                                                unsigned long long &cpairs, unsigned long long &cin) {
     constexpr bool F32 = sizeof(T) == 4;
+    constexpr int S = kDiffWaves;
     __shared__ Src4T<T> lds_all[4][kLeaf];
     __shared__ int32_t stk_all[4][kBsStack];
     __shared__ double4 lbox_all[4][64];  // the popped leaves: box,
@@ -1959,7 +2036,8 @@ __device__ __forceinline__ void diffusion_wave(const TreeDev &t, double cut, dou
     int2 *lrng = lrng_all[wid];
     int32_t *lsel = lsel_all[wid];
     const uint64_t below = (1ull << lane) - 1;
-    const int64_t grp = __builtin_amdgcn_readfirstlane((int)(xcd_block() * 4 + wid));
+    const int64_t grp = __builtin_amdgcn_readfirstlane((int)xcd_block());
+    const int part = __builtin_amdgcn_readfirstlane(wid);
     if (grp >= t.ngroup) return;
     const TargetGroup G = target_group(t, grp, lane);
     const int64_t ti = G.ti;
@@ -1981,10 +2059,10 @@ __device__ __forceinline__ void diffusion_wave(const TreeDev &t, double cut, dou
     } else {
         ax = ok ? t.sx[ti] : cAx;
         ay = ok ? t.sy[ti] : cAy;
-        kd = 1.0 / (ok ? di : 1.0);
+        kd = -1.4426950408889634 / (ok ? di : 1.0);
         ri2 = mine ? cut * di * cut * di : -1.0;
     }
-    const T thr2 = F32 ? (T)(thr * thr) : (T)thr;
+    const T thr2 = (T)thr2d;
     const T gap2 = (T)(4.0 * thr * thr);
     // sources farther than R from the group's box reach no target's radius
     const T Rs2 = F32 ? (T)(R2 * (1.0 + 1e-4)) : (T)R2;
@@ -2035,7 +2113,7 @@ __device__ __forceinline__ void diffusion_wave(const TreeDev &t, double cut, dou
         __builtin_amdgcn_wave_barrier();
         // the leaves some lane's own radius reaches, in list order
         int nr = 0;
-        for (int li = 0; li < nl; ++li) {
+        for (int li = part; li < nl; li += S) {
             const double4 lb = lbox[li];
             T lx, ly;
             if constexpr (F32) {
@@ -2182,11 +2260,13 @@ __device__ __forceinline__ void diffusion_wave(const TreeDev &t, double cut, dou
                     }
             }
             if (sel >> 8) {
+#pragma unroll 4
                 for (int jj = 0; jj < h; ++jj) {
                     const Src4T<T> q = sh[jj];
                     DiffPair<T>::template add<true>(ox - q.x, oy - q.y, q.g, kd, thr2, s2x, s2y, s1);
                 }
             } else {
+#pragma unroll 4
                 for (int jj = 0; jj < h; ++jj) {
                     const Src4T<T> q = sh[jj];
                     DiffPair<T>::template add<false>(ox - q.x, oy - q.y, q.g, kd, thr2, s2x, s2y, s1);
@@ -2204,6 +2284,23 @@ __device__ __forceinline__ void diffusion_wave(const TreeDev &t, double cut, dou
         for (int o = 32; o > 0; o >>= 1) nin += __shfl_xor(nin, o, 64);
         cin = (unsigned long long)nin;
     }
+    // the waves' shares, in wave order, through the slots of the leaf boxes
+    static_assert(sizeof(lbox_all[0]) >= 3 * 64 * sizeof(double), "three sums a lane");
+    if (part > 0) {
+        double *o = reinterpret_cast<double *>(lbox);
+        o[lane] = a2x;
+        o[64 + lane] = a2y;
+        o[128 + lane] = a1;
+    }
+    __syncthreads();
+    if (part > 0) return;
+#pragma unroll
+    for (int q = 1; q < S; ++q) {
+        const double *o = reinterpret_cast<const double *>(lbox_all[q]);
+        a2x += o[lane];
+        a2y += o[64 + lane];
+        a1 += o[128 + lane];
+    }
     // the target's shares, added in the same order on each of its lanes
     for (int o = G.ls.tpw; o < 64; o <<= 1) {
         a2x += __shfl_xor(a2x, o, 64);
@@ -2220,12 +2317,12 @@ __device__ __forceinline__ void diffusion_wave(const TreeDev &t, double cut, dou
 // CENSUS also counts the pairs within each target's own radius (cnt[5]).
 template <typename T, bool CENSUS>
 __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(sizeof(T) == 4 ? 6 : 1)))
-void k_tree_diffusion(TreeDev t, double cut, double nu, double thr,
+void k_tree_diffusion(TreeDev t, double cut, double nu, double thr, double thr2d,
                                                         const double *__restrict__ sd,
                                                         double *__restrict__ u, double *__restrict__ v,
                                                         unsigned long long *__restrict__ cnt) {
     unsigned long long cp = 0, ci = 0;
-    diffusion_wave<T, CENSUS>(t, cut, nu, thr, sd, u, v, cnt, cp, ci);
+    diffusion_wave<T, CENSUS>(t, cut, nu, thr, thr2d, sd, u, v, cnt, cp, ci);
     block_count_add(cp, ci, cnt, CENSUS ? cnt + 5 : nullptr);
 }
 
@@ -2236,9 +2333,9 @@ void k_tree_diffusion(TreeDev t, double cut, double nu, double thr,
 // targets past the capacity stay with their group's wave.
 struct FarFlag {
     TreeDev t;
-    double cut;
+    double cut, part;
     const double *sd;  // d in sorted order (all positive before the selection)
-    __device__ int operator()(int64_t ti) const { return fmin(cut, kFarCut) * sd[ti] > far_radius(t); }
+    __device__ int operator()(int64_t ti) const { return fmin(cut, kFarCut) * sd[ti] > far_radius(t, part); }
 };
 struct FarWrite {
     TreeDev t;
@@ -2356,14 +2453,13 @@ __global__ void k_far_zero(double *__restrict__ a, int64_t nchunk, const unsigne
 
 template <typename T>
 __device__ void diff_far_pair(const TreeDev &t, const double4 *__restrict__ ftgt, int64_t H, int64_t k, int64_t ch,
-                              double cut, double thr, double *__restrict__ part, unsigned long long &cpairs) {
-    constexpr bool F32 = sizeof(T) == 4;
+                              double cut, double thr2d, double *__restrict__ part, unsigned long long &cpairs) {
     const int lane = threadIdx.x & 63;
     const double4 tg = ftgt[k];
     const double ax = tg.x, ay = tg.y, di = tg.z;
     const double R2 = (cut * di) * (cut * di);
-    const T kd = F32 ? (T)(-1.4426950408889634 / di) : (T)(1.0 / di);
-    const T thr2 = F32 ? (T)(thr * thr) : (T)thr;
+    const T kd = (T)(-1.4426950408889634 / di);
+    const T thr2 = (T)thr2d;
     // the chunk's buckets, one per lane: box test and the record in one load
     const int64_t b = ch * 64 + lane;
     const bool inb = b < t.nleaf;
@@ -2419,14 +2515,14 @@ template <typename T>
 __global__ __launch_bounds__(256) void k_diff_far(TreeDev t, const double4 *__restrict__ ftgt,
                                                   const int2 *__restrict__ pairs,
                                                   const unsigned long long *__restrict__ npair_list, double cut,
-                                                  double thr, double *__restrict__ part,
+                                                  double thr2d, double *__restrict__ part,
                                                   unsigned long long *__restrict__ cnt) {
     const int64_t H = far_count(cnt, t.fcap);
     const int64_t total = (int64_t)*npair_list;
     const int64_t nw = (int64_t)gridDim.x * 4;
     unsigned long long cp = 0;
     for (int64_t w = (int64_t)blockIdx.x * 4 + (threadIdx.x >> 6); w < total; w += nw)
-        diff_far_pair<T>(t, ftgt, H, pairs[w].x, pairs[w].y, cut, thr, part, cp);
+        diff_far_pair<T>(t, ftgt, H, pairs[w].x, pairs[w].y, cut, thr2d, part, cp);
     block_count_add(cp, 0ull, cnt, nullptr);
 }
 
@@ -2917,30 +3013,32 @@ int launch_tree_biot_savart(vx_case *c, int64_t s, double vinf_x, double vinf_y)
     if (t.m == 0) return 0;
     if (t.sd.ensure((size_t)t.m, st)) return 1;
     const TreeDev tv = view(t);
-    const unsigned lb = (unsigned)((t.nleaf + 3) / 4 + 7) / 8 * 8;  // padded for xcd_block()
+    const bool mixed = c->prm.precision == VX_PREC_MIXED;
+    const bool split = !mixed && t.nleaf <= kBsSplit;
+    const int64_t wgs = split ? t.nleaf : (t.nleaf + 3) / 4;
+    const unsigned lb = (unsigned)(wgs + 7) / 8 * 8;  // padded for xcd_block()
     const double th = theta_of(c), eps = c->prm.ve_size;
     unsigned long long *nfb = t.cnt.p + 1;
-    const bool mixed = c->prm.precision == VX_PREC_MIXED;
     const int exact_all = (c->prm.flags & VX_FLAG_EXACT_NEAREST) ? 1 : 0;
     Timer tk(c, &c->tm.bs_kernel_ms, 6);
-#define VX_TREE_BS(T_, P_, S_)                                                                                       \
-    hipLaunchKernelGGL((k_tree_bs<T_, P_, S_>), dim3(lb), dim3(256), 0, st, tv, th, eps, vinf_x, vinf_y, c->u.p,     \
-                       c->v.p, c->d.p, t.sd.p, t.fb.p, t.fbr2.p, nfb, exact_all)
+#define VX_TREE_BS(T_, P_, ST_, S_)                                                                                  \
+    hipLaunchKernelGGL((k_tree_bs<T_, P_, ST_, S_>), dim3(lb), dim3(256), 0, st, tv, th, eps, vinf_x, vinf_y,        \
+                       c->u.p, c->v.p, c->d.p, t.sd.p, t.fb.p, t.fbr2.p, nfb, exact_all)
+#define VX_TREE_BS_ORDERS(T_, S_)    \
+    if (t.terms == 32)               \
+        VX_TREE_BS(T_, 32, 32, S_);  \
+    else if (t.terms == 20)          \
+        VX_TREE_BS(T_, 20, 32, S_);  \
+    else                             \
+        VX_TREE_BS(T_, 16, 16, S_)
     if (mixed) {
-        if (t.terms == 32)
-            VX_TREE_BS(float, 32, 32);
-        else if (t.terms == 20)
-            VX_TREE_BS(float, 20, 32);
-        else
-            VX_TREE_BS(float, 16, 16);
+        VX_TREE_BS_ORDERS(float, 1);
+    } else if (split) {
+        VX_TREE_BS_ORDERS(double, 4);
     } else {
-        if (t.terms == 32)
-            VX_TREE_BS(double, 32, 32);
-        else if (t.terms == 20)
-            VX_TREE_BS(double, 20, 32);
-        else
-            VX_TREE_BS(double, 16, 16);
+        VX_TREE_BS_ORDERS(double, 1);
     }
+#undef VX_TREE_BS_ORDERS
 #undef VX_TREE_BS
     tk.stop();
     hipLaunchKernelGGL(k_tree_nearest_fallback, dim3(512), dim3(1024), 0, st, tv, t.arr.p, t.cnt.p + 10, t.fb.p,
@@ -2966,6 +3064,7 @@ int tree_diffusion_pre(vx_case *c) {
     if (!c->tree || c->tree->m == 0) return 0;
     TreeBufs &t = *c->tree;
     hipStream_t st = c->stream;
+    const bool mixed = c->prm.precision == VX_PREC_MIXED;
     const int64_t nchunk = (t.nleaf + 63) / 64;
     // The last diffusion's count comes from pinned memory, copied at the end
     // of its far part; a caller that has not synchronised since reads an
@@ -2995,7 +3094,7 @@ int tree_diffusion_pre(vx_case *c) {
         hipLaunchKernelGGL(k_sd_gather, dim3((unsigned)((t.m + 255) / 256)), dim3(256), 0, st, t.perm.p, c->d.p, t.m,
                            t.sd.p);
     t.sd_fresh = false;
-    VX_CHECK(prim::select_flags(FarFlag{tv, diff_cut_of(c), t.sd.p}, t.m, FarWrite{tv, t.sd.p, t.fb.p}, c->ptmp.p,
+    VX_CHECK(prim::select_flags(FarFlag{tv, diff_cut_of(c), mixed ? far_part<float>() : far_part<double>(), t.sd.p}, t.m, FarWrite{tv, t.sd.p, t.fb.p}, c->ptmp.p,
                                 cnt + 2, st));
     return 0;
 }
@@ -3005,7 +3104,7 @@ int tree_diffusion_far(vx_case *c, hipStream_t st) {
     TreeBufs &t = *c->tree;
     const TreeDev tv = view(t);
     const bool mixed = c->prm.precision == VX_PREC_MIXED;
-    const double cut = diff_cut_of(c), thr = 0.001 * c->prm.ve_size;
+    const double cut = diff_cut_of(c), thr = 0.001 * c->prm.ve_size, thr2 = mixed ? thr * thr : diff_thr2(thr);
     unsigned long long *cnt = t.cnt.p + 4;
     // all counts stay on the device (grid-stride kernels sized for the list's capacity)
     const int64_t nchunk = (t.nleaf + 63) / 64;
@@ -3016,10 +3115,10 @@ int tree_diffusion_far(vx_case *c, hipStream_t st) {
                        t.fpairs.p, cnt + 3, t.ftgt.p);
     if (mixed)
         hipLaunchKernelGGL(k_diff_far<float>, dim3(4096), dim3(256), 0, st, tv, t.ftgt.p, t.fpairs.p, cnt + 3, cut,
-                           thr, t.hpart.p, cnt);
+                           thr2, t.hpart.p, cnt);
     else
         hipLaunchKernelGGL(k_diff_far<double>, dim3(4096), dim3(256), 0, st, tv, t.ftgt.p, t.fpairs.p, cnt + 3, cut,
-                           thr, t.hpart.p, cnt);
+                           thr2, t.hpart.p, cnt);
     hipLaunchKernelGGL(k_diff_far_final, dim3(1024), dim3(256), 0, st, tv, t.fb.p, cnt, nchunk, t.hpart.p, c->d.p,
                        c->prm.nu, c->u.p, c->v.p);
     VX_CHECK(hipGetLastError());
@@ -3030,24 +3129,24 @@ int tree_diffusion_main(vx_case *c) {
     if (!c->tree || c->tree->m == 0) return 0;
     TreeBufs &t = *c->tree;
     hipStream_t st = c->stream;
-    const unsigned lb8 = (unsigned)((t.ngroup + 3) / 4 + 7) / 8 * 8;  // target groups, padded for xcd_block()
     const bool mixed = c->prm.precision == VX_PREC_MIXED;
-    const double cut = diff_cut_of(c), thr = 0.001 * c->prm.ve_size;
+    const unsigned lb8 = (unsigned)(t.ngroup + 7) / 8 * 8;  // target groups, padded for xcd_block()
+    const double cut = diff_cut_of(c), thr = 0.001 * c->prm.ve_size, thr2 = mixed ? thr * thr : diff_thr2(thr);
     unsigned long long *cnt = t.cnt.p + 4;
     Timer tk(c, &c->tm.diff_kernel_ms, 8);
     if (c->census) {
         if (mixed)
             hipLaunchKernelGGL((k_tree_diffusion<float, true>), dim3(lb8), dim3(256), 0, st, view(t), cut, c->prm.nu,
-                               thr, t.sd.p, c->u.p, c->v.p, cnt);
+                               thr, thr2, t.sd.p, c->u.p, c->v.p, cnt);
         else
             hipLaunchKernelGGL((k_tree_diffusion<double, true>), dim3(lb8), dim3(256), 0, st, view(t), cut,
-                               c->prm.nu, thr, t.sd.p, c->u.p, c->v.p, cnt);
+                               c->prm.nu, thr, thr2, t.sd.p, c->u.p, c->v.p, cnt);
     } else if (mixed) {
         hipLaunchKernelGGL((k_tree_diffusion<float, false>), dim3(lb8), dim3(256), 0, st, view(t), cut, c->prm.nu,
-                           thr, t.sd.p, c->u.p, c->v.p, cnt);
+                           thr, thr2, t.sd.p, c->u.p, c->v.p, cnt);
     } else {
         hipLaunchKernelGGL((k_tree_diffusion<double, false>), dim3(lb8), dim3(256), 0, st, view(t), cut, c->prm.nu,
-                           thr, t.sd.p, c->u.p, c->v.p, cnt);
+                           thr, thr2, t.sd.p, c->u.p, c->v.p, cnt);
     }
     VX_CHECK(hipGetLastError());
     return 0;
