@@ -592,50 +592,112 @@ __global__ void k_lu_pinv(const int32_t *__restrict__ perm, int64_t np, int32_t 
 __device__ __forceinline__ unsigned long long dbits(double v) { return (unsigned long long)__double_as_longlong(v); }
 __device__ __forceinline__ double bitsd(unsigned long long v) { return __longlong_as_double((long long)v); }
 
-__global__ void k_lu_begin(double *__restrict__ x, int64_t np, unsigned long long *__restrict__ st) {
-    const int64_t i = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
-    if (i < np) x[i] = 0.0;
-    if (i < 4) st[i] = 0ull;
-}
-
-// r = b - A x with b = [R; d_g], one wave per row, written permuted and in
-// FP32 (rp[pinv[i]]); the largest |r_i| into st[2].
-__global__ __launch_bounds__(256) void k_lu_resid(const double *__restrict__ A, const double *__restrict__ R,
-                                                  double d_g_host, const double *__restrict__ d_g_dev, int64_t n,
-                                                  int64_t np, const double *__restrict__ x,
-                                                  const int32_t *__restrict__ pinv, float *__restrict__ rp,
-                                                  unsigned long long *__restrict__ st) {
-    if (st[0]) return;
-    const double d_g = d_g_dev ? *d_g_dev : d_g_host;
-    const int lane = threadIdx.x & 63;
-    const int64_t i = (int64_t)blockIdx.x * 4 + (threadIdx.x >> 6);
-    if (i >= np) return;
-    if (i >= n) {
-        if (lane == 0) rp[pinv[i]] = 0.f;
-        return;
-    }
-    const double *a = A + i * n;
-    double s = 0.0;
-    for (int64_t j = lane; j < n; j += 64) s += a[j] * x[j];
-    for (int o = 32; o > 0; o >>= 1) s += __shfl_xor(s, o, 64);
-    if (lane == 0) {
-        const double b = i < n - 1 ? R[i] : d_g;
-        const double r = b - s;
-        rp[pinv[i]] = (float)r;
-        atomicMax(st + 2, dbits(fabs(r)));
-    }
-}
-
 // Convergence test (LAPACK dsgesv): done when ||r|| <= ||x|| ||A|| eps sqrt(n);
-// else one more correction is counted.  Resets the maxima for the next pass.
-__global__ void k_lu_check(unsigned long long *__restrict__ st, double *__restrict__ nrm, int64_t n) {
-    if (st[0]) return;
-    const double r = bitsd(st[2]), xm = bitsd(st[3]), an = bitsd(st[5]);
+// else one more correction is counted.  One thread; r and xm are the maxima
+// of |r_i| and |x_i|.
+__device__ __forceinline__ void lu_check(unsigned long long *__restrict__ st, double *__restrict__ nrm, int64_t n,
+                                         double r, double xm) {
+    const double an = bitsd(st[5]);
     const double cte = an * 1.1102230246251565e-16 * sqrt((double)n);
     nrm[1] = (xm > 0.0 && an > 0.0) ? r / (xm * an) : r;
     if (r <= xm * cte) st[0] = 1ull;
     else st[1] += 1ull;
+}
+
+// The largest of a value per thread (as bits of a non-negative double), valid
+// in thread 0.
+template <int W>
+__device__ __forceinline__ unsigned long long block_max_bits(unsigned long long v) {
+    __shared__ unsigned long long s[W];
+    for (int o = 32; o > 0; o >>= 1) {
+        const unsigned long long q = __shfl_xor(v, o, 64);
+        v = q > v ? q : v;
+    }
+    if ((threadIdx.x & 63) == 0) s[threadIdx.x >> 6] = v;
+    __syncthreads();
+    if (threadIdx.x == 0)
+        for (int w = 1; w < W; ++w) v = s[w] > v ? s[w] : v;
+    return v;
+}
+
+// sum_j w[j] v[j] over the lane's j = lo + lane, lo + lane + 64, ... < hi, in
+// order, with eight loads of each in flight.
+template <typename T>
+__device__ __forceinline__ T row_dot(const T *__restrict__ w, const T *__restrict__ v, int64_t lo, int64_t hi,
+                                     int lane) {
+    T s = T(0);
+    int64_t j = lo + lane;
+    for (; j + 7 * 64 < hi; j += 8 * 64) {
+        T a[8], b[8];
+#pragma unroll
+        for (int e = 0; e < 8; ++e) {
+            a[e] = w[j + 64 * e];
+            b[e] = v[j + 64 * e];
+        }
+#pragma unroll
+        for (int e = 0; e < 8; ++e) s += a[e] * b[e];
+    }
+    for (; j < hi; j += 64) s += w[j] * v[j];
+    return s;
+}
+
+// x = 0, so r = b = [R; d_g], permuted and in FP32, and its test, in one
+// work-group: no pass over A for it.
+__global__ __launch_bounds__(1024) void k_lu_begin(double *__restrict__ x, int64_t n, int64_t np,
+                                                   const double *__restrict__ R, double d_g_host,
+                                                   const double *__restrict__ d_g_dev,
+                                                   const int32_t *__restrict__ pinv, float *__restrict__ rp,
+                                                   unsigned long long *__restrict__ st, double *__restrict__ nrm) {
+    const double d_g = d_g_dev ? *d_g_dev : d_g_host;
+    unsigned long long m = 0ull;
+    for (int64_t i = threadIdx.x; i < np; i += 1024) {
+        x[i] = 0.0;
+        const double b = i < n - 1 ? R[i] : (i < n ? d_g : 0.0);
+        rp[pinv[i]] = (float)b;
+        const unsigned long long q = dbits(fabs(b));
+        m = q > m ? q : m;
+    }
+    m = block_max_bits<16>(m);
+    if (threadIdx.x != 0) return;
+    st[0] = st[1] = st[2] = st[3] = st[6] = 0ull;
+    lu_check(st, nrm, n, bitsd(m), 0.0);
+}
+
+// r = b - A x with b = [R; d_g], one wave per row, written permuted and in
+// FP32 (rp[pinv[i]]); the largest |r_i| into st[2].  The last work-group to
+// end (st[6] counts them) tests for convergence and clears both for the next
+// pass.  Bound by the read of A: with eight loads in flight, without the
+// first pass and the test's launches a birth of 1000, 2040 and 3320 panels (three
+// corrections) takes 144, 194 and 289 us with its copies, 208, 342 and 517
+// before.
+__global__ __launch_bounds__(256) void k_lu_resid(const double *__restrict__ A, const double *__restrict__ R,
+                                                  double d_g_host, const double *__restrict__ d_g_dev, int64_t n,
+                                                  int64_t np, const double *__restrict__ x,
+                                                  const int32_t *__restrict__ pinv, float *__restrict__ rp,
+                                                  unsigned long long *__restrict__ st, double *__restrict__ nrm) {
+    if (st[0]) return;
+    const double d_g = d_g_dev ? *d_g_dev : d_g_host;
+    const int lane = threadIdx.x & 63;
+    const int64_t i = (int64_t)blockIdx.x * 4 + (threadIdx.x >> 6);
+    unsigned long long m = 0ull;
+    if (i >= n && i < np) {
+        if (lane == 0) rp[pinv[i]] = 0.f;
+    } else if (i < n) {
+        double s = row_dot(A + i * n, x, 0, n, lane);
+        for (int o = 32; o > 0; o >>= 1) s += __shfl_xor(s, o, 64);
+        const double r = (i < n - 1 ? R[i] : d_g) - s;
+        if (lane == 0) rp[pinv[i]] = (float)r;
+        m = dbits(fabs(r));
+    }
+    m = block_max_bits<4>(m);
+    if (threadIdx.x != 0) return;
+    atomicMax(st + 2, m);
+    __threadfence();
+    if (atomicAdd(st + 6, 1ull) + 1 != gridDim.x) return;
+    __threadfence();
+    lu_check(st, nrm, n, bitsd(atomicMax(st + 2, 0ull)), bitsd(atomicMax(st + 3, 0ull)));
     st[2] = 0ull;
+    st[6] = 0ull;
 }
 
 // t = L^-1 (P r): row i sums W's strict lower part (one wave per row).
@@ -646,9 +708,7 @@ __global__ __launch_bounds__(256) void k_lu_apply_l(const float *__restrict__ W,
     const int lane = threadIdx.x & 63;
     const int64_t i = (int64_t)blockIdx.x * 4 + (threadIdx.x >> 6);
     if (i >= np) return;
-    const float *w = W + i * np;
-    float s = 0.f;
-    for (int64_t j = lane; j < i; j += 64) s += w[j] * rp[j];
+    float s = row_dot(W + i * np, rp, 0, i, lane);
     for (int o = 32; o > 0; o >>= 1) s += __shfl_xor(s, o, 64);
     if (lane == 0) t[i] = s + rp[i];
 }
@@ -660,16 +720,16 @@ __global__ __launch_bounds__(256) void k_lu_apply_u(const float *__restrict__ W,
     if (st[0]) return;
     const int lane = threadIdx.x & 63;
     const int64_t i = (int64_t)blockIdx.x * 4 + (threadIdx.x >> 6);
-    if (i >= np) return;
-    const float *w = W + i * np;
-    float s = 0.f;
-    for (int64_t j = i + lane; j < np; j += 64) s += w[j] * t[j];
-    for (int o = 32; o > 0; o >>= 1) s += __shfl_xor(s, o, 64);
-    if (lane == 0) {
+    unsigned long long m = 0ull;
+    if (i < np) {
+        float s = row_dot(W + i * np, t, i, np, lane);
+        for (int o = 32; o > 0; o >>= 1) s += __shfl_xor(s, o, 64);
         const double xi = x[i] + (double)s;
-        x[i] = xi;
-        atomicMax(st + 3, dbits(fabs(xi)));
+        if (lane == 0) x[i] = xi;
+        m = dbits(fabs(xi));
     }
+    m = block_max_bits<4>(m);
+    if (threadIdx.x == 0) atomicMax(st + 3, m);
 }
 
 // ---- host side ------------------------------------------------------------------------
@@ -759,16 +819,13 @@ int launch_lu_solve(vx_case *c, const double *R, double d_g, const double *d_g_d
     hipStream_t st = c->stream;
     const int64_t n = b.n, np = b.np;
     const unsigned gw = (unsigned)((np + 3) / 4);
-    hipLaunchKernelGGL(k_lu_begin, dim3((unsigned)((np + 255) / 256)), dim3(256), 0, st, b.x.p, np, b.st.p);
-    hipLaunchKernelGGL(k_lu_resid, dim3(gw), dim3(256), 0, st, b.A.p, R, d_g, d_g_dev, n, np, b.x.p, b.pinv.p,
-                       b.rp.p, b.st.p);
-    hipLaunchKernelGGL(k_lu_check, dim3(1), dim3(1), 0, st, b.st.p, b.nrm.p, n);
+    hipLaunchKernelGGL(k_lu_begin, dim3(1), dim3(1024), 0, st, b.x.p, n, np, R, d_g, d_g_dev, b.pinv.p, b.rp.p,
+                       b.st.p, b.nrm.p);
     for (int it = 0; it < kLuMaxIt; ++it) {
         hipLaunchKernelGGL(k_lu_apply_l, dim3(gw), dim3(256), 0, st, b.W.p, np, b.rp.p, b.t.p, b.st.p);
         hipLaunchKernelGGL(k_lu_apply_u, dim3(gw), dim3(256), 0, st, b.W.p, np, b.t.p, b.x.p, b.st.p);
         hipLaunchKernelGGL(k_lu_resid, dim3(gw), dim3(256), 0, st, b.A.p, R, d_g, d_g_dev, n, np, b.x.p, b.pinv.p,
-                           b.rp.p, b.st.p);
-        hipLaunchKernelGGL(k_lu_check, dim3(1), dim3(1), 0, st, b.st.p, b.nrm.p, n);
+                           b.rp.p, b.st.p, b.nrm.p);
     }
     VX_CHECK(hipGetLastError());
     return 0;
