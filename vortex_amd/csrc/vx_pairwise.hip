@@ -806,27 +806,32 @@ __global__ __launch_bounds__(kSegTile) void k_right_part_partial(
     }
 }
 
-// The FP64 pairs with kRhsPG panels per work-group.  A pair takes two arc
-// tangents, a logarithm and five quotients (about 500 instructions), and the
-// list is short at the counts where a step is short: one thread per panel
+// The pairs with kRhsPG panels per work-group.  An FP64 pair takes two arc
+// tangents, a logarithm and five quotients (about 500 instructions; FP32 50), and
+// the list is short at the counts where a step is short: one thread per panel
 // over a chunk's sources kept 2 work-groups busy for 90 to 200 us.  Here a
 // tile's terms are evaluated by all 256 threads, each on one panel and every
 // 64th near source, and added in list order by a lane per panel and
-// component, with the operations of the loop above: the same partials, bit
-// for bit.  200 panels, 2785 vortices: 200 -> 12 us.
+// component, with the operations of the loop above (FP32: sums over kSegTile
+// listed sources, added in FP64): the same partials, bit for bit.  FP64, 200
+// panels, 2785 vortices: 200 -> 12 us; FP32, a batch of plates with up to
+// 2040 panels: 35 -> 9.7 us.
 constexpr int kRhsPG = 4;
 // Larger bounds keep the kernel above: its segments and chunks fill the chip
 // by themselves there, and a grid for the bound would be mostly idle groups.
 constexpr int64_t kRhsSplitSrc = 32768;
 
-__global__ __launch_bounds__(256) void k_right_part_terms(const double *__restrict__ x, const double *__restrict__ y,
-                                                          const double *__restrict__ g,
+template <typename T>
+__global__ __launch_bounds__(256) void k_right_part_terms(const T *__restrict__ sg, const double *__restrict__ x,
+                                                          const double *__restrict__ y,
                                                           const int32_t *__restrict__ list,
                                                           const int32_t *__restrict__ nlist, PanelsSoA pan,
                                                           const RhsSeg *__restrict__ segs, double *__restrict__ part) {
     constexpr int kPer = kSegTile / kRhsPG;
-    __shared__ double lx[256], ly[256], lg[256];
-    __shared__ double lt[256][kRhsPG][2];
+    constexpr bool F32 = sizeof(T) == 4;
+    static_assert(kSegTile == 128, "two tiles of the sums in 256 sources");
+    __shared__ T lx[256], ly[256], lg[256];
+    __shared__ T lt[256][kRhsPG][2];
     __shared__ int wcount[4];
     const RhsSeg S = segs[blockIdx.x / kPer];
     const int p0 = (int)(blockIdx.x % kPer) * kRhsPG;
@@ -836,26 +841,50 @@ __global__ __launch_bounds__(256) void k_right_part_terms(const double *__restri
     const int tid = threadIdx.x, lane = tid & 63, wv = tid >> 6;
     const int pp = tid & (kRhsPG - 1), slot = tid / kRhsPG;
     const int64_t i = S.first + min(p0 + pp, S.count - 1);
-    const double l0 = pan.lx[i], l1 = pan.ly[i], r0 = pan.rx[i], r1 = pan.ry[i];
-    const double d0 = r0 - l0, d1 = r1 - l1;
+    const double ox = F32 ? S.cx : 0.0, oy = F32 ? S.cy : 0.0;
+    const T l0 = (T)(pan.lx[i] - ox), l1 = (T)(pan.ly[i] - oy);
+    const T r0 = (T)(pan.rx[i] - ox), r1 = (T)(pan.ry[i] - oy);
+    const T d0 = F32 ? (T)(pan.rx[i] - pan.lx[i]) : r0 - l0, d1 = F32 ? (T)(pan.ry[i] - pan.ly[i]) : r1 - l1;
+    const T dd2 = fma(d0, d0, d1 * d1);
     const double rn2 = 4.0 * S.r * S.r;
-    double acc = 0.0;  // lane (panel, component) of the first wave
+    T acc = 0;  // lane (panel, component) of the first wave
+    double sum = 0.0;
+    auto add_terms = [&](int jj, int end) {
+        const T *t = &lt[0][tid >> 1][tid & 1];
+        for (; jj + 8 <= end; jj += 8) {
+            T v[8], w[8];
+#pragma unroll
+            for (int e = 0; e < 8; ++e) {
+                v[e] = t[(jj + e) * 2 * kRhsPG];
+                w[e] = lg[jj + e];
+            }
+#pragma unroll
+            for (int e = 0; e < 8; ++e) acc = fma(w[e], v[e], acc);
+        }
+        for (; jj < end; ++jj) acc = fma(lg[jj], t[jj * 2 * kRhsPG], acc);
+        if (F32) {
+            sum += (double)acc;
+            acc = 0;
+        }
+    };
     for (int64_t base = lo; base < hi; base += 256) {
         const int64_t j = base + tid;
         bool near = false;
-        double qx = 0.0, qy = 0.0, qg = 0.0;
+        T qx = 0, qy = 0, qg = 0;
         if (j < hi) {
             const int32_t k = list[j];
-            qx = x[k];
-            qy = y[k];
-            qg = g[k];
-            const double ex = qx - S.cx, ey = qy - S.cy;
+            const double px = x[k], py = y[k];
+            qg = sg[k];
+            const double ex = px - S.cx, ey = py - S.cy;
             near = ex * ex + ey * ey < rn2;
+            qx = F32 ? (T)ex : (T)px;
+            qy = F32 ? (T)ey : (T)py;
         }
         const uint64_t m = __ballot(near);
         if (lane == 0) wcount[wv] = __popcll(m);
         __syncthreads();
         int pos = __popcll(m & ((1ull << lane) - 1)), cnt = 0;
+        const int half = wcount[0] + wcount[1];
         for (int q = 0; q < 4; ++q) {
             pos += q < wv ? wcount[q] : 0;
             cnt += wcount[q];
@@ -867,36 +896,36 @@ __global__ __launch_bounds__(256) void k_right_part_terms(const double *__restri
         }
         __syncthreads();
         for (int jj = slot; jj < cnt; jj += 256 / kRhsPG) {
-            const double s00 = l0 - lx[jj], s01 = l1 - ly[jj];
-            const double s10 = r0 - lx[jj], s11 = r1 - ly[jj];
-            const double z = fma(d0, s01, -(d1 * s00));
-            const double A = fma(d0, s00, d1 * s01);
-            const double B = fma(d0, s10, d1 * s11);
-            const double alpha = atan(A / z) - atan(B / z);
-            const double beta = 0.5 * log(fma(s10, s10, s11 * s11) / fma(s00, s00, s01 * s01));
-            lt[jj][pp][0] = fma(d0, alpha, -(d1 * beta));
-            lt[jj][pp][1] = fma(d1, alpha, d0 * beta);
+            const T s00 = l0 - lx[jj], s01 = l1 - ly[jj];
+            const T s10 = r0 - lx[jj], s11 = r1 - ly[jj];
+            if constexpr (F32) {
+                const T z = fma(s01, d0, -(s00 * d1));
+                const T A = fma(s00, d0, s01 * d1);
+                const T B = fma(s10, d0, s11 * d1);
+                const T alpha = vx_atan2f(-dd2 * z, fma(z, z, A * B));
+                const T q0 = fma(s00, s00, s01 * s01), q1 = fma(s10, s10, s11 * s11);
+                const T beta = 0.34657359027997264f * __builtin_amdgcn_logf(q1 * __builtin_amdgcn_rcpf(q0));
+                lt[jj][pp][0] = fma(alpha, d0, -(beta * d1));
+                lt[jj][pp][1] = fma(beta, d0, alpha * d1);
+            } else {
+                const T z = fma(d0, s01, -(d1 * s00));
+                const T A = fma(d0, s00, d1 * s01);
+                const T B = fma(d0, s10, d1 * s11);
+                const T alpha = atan(A / z) - atan(B / z);
+                const T beta = 0.5 * log(fma(s10, s10, s11 * s11) / fma(s00, s00, s01 * s01));
+                lt[jj][pp][0] = fma(d0, alpha, -(d1 * beta));
+                lt[jj][pp][1] = fma(d1, alpha, d0 * beta);
+            }
         }
         __syncthreads();
         if (tid < 2 * kRhsPG) {
-            const double *t = &lt[0][tid >> 1][tid & 1];
-            int jj = 0;
-            for (; jj + 8 <= cnt; jj += 8) {
-                double v[8], w[8];
-#pragma unroll
-                for (int e = 0; e < 8; ++e) {
-                    v[e] = t[(jj + e) * 2 * kRhsPG];
-                    w[e] = lg[jj + e];
-                }
-#pragma unroll
-                for (int e = 0; e < 8; ++e) acc = fma(w[e], v[e], acc);
-            }
-            for (; jj < cnt; ++jj) acc = fma(lg[jj], t[jj * 2 * kRhsPG], acc);
+            if (F32) add_terms(0, half);
+            add_terms(F32 ? half : 0, cnt);
         }
         __syncthreads();
     }
     if (tid < 2 * kRhsPG && p0 + (tid >> 1) < S.count)
-        part[(c * 2 + (tid & 1)) * pan.P + S.first + p0 + (tid >> 1)] = acc;
+        part[(c * 2 + (tid & 1)) * pan.P + S.first + p0 + (tid >> 1)] = F32 ? sum : (double)acc;
 }
 
 // Sums of g w^{k+1}, w = 1 / (z_j - c), k < kLoc, over a work-group's sources
@@ -1471,18 +1500,21 @@ int launch_right_part(vx_case *c, Cnt cn_src, double vinf_x, double vinf_y) {
                                     nlist, st));
     }
     // pairs within 2 R_s of each segment
-    if (mixed(c)) {
-        if (launch_pack_f32(c, cn_src)) return 1;
-        hipLaunchKernelGGL(k_right_part_partial<float>, dim3((unsigned)K, (unsigned)nchunk), dim3(kSegTile), 0, st,
-                           c->xf.p, c->yf.p, c->gf.p, c->x.p, c->y.p, c->lists.p, nlist, c->pan, c->segs,
-                           c->partial.p);
-    } else if (n_src <= kRhsSplitSrc) {
-        hipLaunchKernelGGL(k_right_part_terms, dim3((unsigned)(K * (kSegTile / kRhsPG)), (unsigned)nchunk), dim3(256), 0,
-                           st, c->x.p, c->y.p, c->g.p, c->lists.p, nlist, c->pan, c->segs, c->partial.p);
+    if (mixed(c) && launch_pack_f32(c, cn_src)) return 1;
+    const dim3 gterms((unsigned)(K * (kSegTile / kRhsPG)), (unsigned)nchunk), gseg((unsigned)K, (unsigned)nchunk);
+    if (n_src <= kRhsSplitSrc) {
+        if (mixed(c))
+            hipLaunchKernelGGL(k_right_part_terms<float>, gterms, dim3(256), 0, st, c->gf.p, c->x.p, c->y.p,
+                               c->lists.p, nlist, c->pan, c->segs, c->partial.p);
+        else
+            hipLaunchKernelGGL(k_right_part_terms<double>, gterms, dim3(256), 0, st, c->g.p, c->x.p, c->y.p,
+                               c->lists.p, nlist, c->pan, c->segs, c->partial.p);
+    } else if (mixed(c)) {
+        hipLaunchKernelGGL(k_right_part_partial<float>, gseg, dim3(kSegTile), 0, st, c->xf.p, c->yf.p, c->gf.p, c->x.p,
+                           c->y.p, c->lists.p, nlist, c->pan, c->segs, c->partial.p);
     } else {
-        hipLaunchKernelGGL(k_right_part_partial<double>, dim3((unsigned)K, (unsigned)nchunk), dim3(kSegTile), 0, st,
-                           c->x.p, c->y.p, c->g.p, c->x.p, c->y.p, c->lists.p, nlist, c->pan, c->segs,
-                           c->partial.p);
+        hipLaunchKernelGGL(k_right_part_partial<double>, gseg, dim3(kSegTile), 0, st, c->x.p, c->y.p, c->g.p, c->x.p,
+                           c->y.p, c->lists.p, nlist, c->pan, c->segs, c->partial.p);
     }
     // the global expansion (sources beyond 2 R_b), the segments' own
     // sources, and each segment's total about c_s
