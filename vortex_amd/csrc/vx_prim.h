@@ -205,49 +205,71 @@ __global__ __launch_bounds__(kT) void k_flag_apply(F f, int64_t n, const int32_t
 
 // Count, scan and apply in one launch of one work-group: a small selection is
 // all launch and latency (at 2785 of 8192 items, the hit candidates 23 -> 6.1 us,
-// the near sources 19 -> 5.4 us, the wall targets 16 -> 5.1 us).  Two tiles
-// are the most that one work-group reads as fast as two do.  The flags of a thread's items (r * 1024 + t) are
-// kept in a mask between the count and the writer, which sees each item
-// once, as above.
-constexpr int64_t kOneMax = 8192;
+// the near sources 19 -> 5.4 us, the wall targets 16 -> 5.1 us; in a batch of
+// some 20000 each, 20 to 22 us -> 10 to 12).  The flags of a thread's items are
+// kept in a mask between the count and the writer, which sees each item once,
+// as above; its 32 bits set the limit.
+constexpr int64_t kOneMax = 32768;
 constexpr int kOneT = 1024, kOneR = (int)(kOneMax / kOneT);
+static_assert(kOneR == 32, "a mask bit a round");
 
-template <class F, class Wr, class TT, bool GRAND>
-__global__ __launch_bounds__(kOneT) void k_flag_one(F f, int64_t n, Wr wr, TT *total) {
-    __shared__ int32_t wc[kOneR * 16 + 1];
+// Flags of items [0, n), n <= kOneMax, by one work-group of kOneT threads:
+// the thread's own as a mask (bit r: item r * kOneT + threadIdx.x), eight
+// rounds' loads in flight, and in wc[r * 16 + w] the flagged items before
+// wave w of round r; wc[kOneR * 16] = all of them.
+template <class F>
+__device__ __forceinline__ uint32_t one_flags(F f, int64_t n, int32_t (&wc)[kOneR * 16 + 1]) {
     const int lane = lane_id(), w = threadIdx.x >> 6;
     const int rounds = (int)((n + kOneT - 1) / kOneT);
     uint32_t mine = 0;
+    for (int r0 = 0; r0 < rounds; r0 += 8) {
 #pragma unroll
-    for (int r = 0; r < kOneR; ++r) {
-        const int64_t i = (int64_t)r * kOneT + threadIdx.x;
-        const int fl = i < n ? f(i) : 0;
-        const uint64_t bal = __ballot(fl);
-        mine |= (uint32_t)fl << r;
-        if (lane == 0) wc[r * 16 + w] = __popcll(bal);
-    }
-    __syncthreads();
-    if (w == 0) {  // exclusive scan of the 128 counts, two a lane
-        const int32_t a = wc[2 * lane], b = wc[2 * lane + 1];
-        const int32_t inc = wave_inclusive(a + b, OpSum());
-        wc[2 * lane] = inc - a - b;
-        wc[2 * lane + 1] = inc - b;
-        if (lane == 63) {
-            wc[kOneR * 16] = inc;
-            if (total) *total = (TT)inc;
+        for (int e = 0; e < 8; ++e) {
+            const int64_t i = (int64_t)(r0 + e) * kOneT + threadIdx.x;
+            const int fl = i < n ? f(i) : 0;
+            const uint64_t bal = __ballot(fl);
+            mine |= (uint32_t)fl << (r0 + e);
+            if (lane == 0) wc[(r0 + e) * 16 + w] = __popcll(bal);
         }
     }
     __syncthreads();
+    if (w == 0) {  // exclusive scan, eight counts a lane
+        const int end = (rounds + 7) / 8 * 8 * 16;
+        int32_t v[8], sum = 0;
+#pragma unroll
+        for (int e = 0; e < 8; ++e) {
+            v[e] = lane * 8 + e < end ? wc[lane * 8 + e] : 0;
+            sum += v[e];
+        }
+        const int32_t inc = wave_inclusive(sum, OpSum());
+        int32_t pre = inc - sum;
+#pragma unroll
+        for (int e = 0; e < 8; ++e) {
+            wc[lane * 8 + e] = pre;
+            pre += v[e];
+        }
+        if (lane == 63) wc[kOneR * 16] = inc;
+    }
+    __syncthreads();
+    return mine;
+}
+
+// Rank of the thread's item of round r among the flagged items (or the
+// flagged items before it); every lane of the wave takes part.
+__device__ __forceinline__ int32_t one_rank(uint32_t mine, int r, const int32_t (&wc)[kOneR * 16 + 1]) {
+    return wc[r * 16 + (threadIdx.x >> 6)] + (int32_t)__popcll(__ballot((mine >> r) & 1) & lanes_below());
+}
+
+template <class F, class Wr, class TT>
+__global__ __launch_bounds__(kOneT) void k_flag_one(F f, int64_t n, Wr wr, TT *total) {
+    __shared__ int32_t wc[kOneR * 16 + 1];
+    const uint32_t mine = one_flags(f, n, wc);
+    if (total && threadIdx.x == 0) *total = (TT)wc[kOneR * 16];
+    const int rounds = (int)((n + kOneT - 1) / kOneT);
     for (int r = 0; r < rounds; ++r) {
         const int64_t i = (int64_t)r * kOneT + threadIdx.x;
-        const int fl = (mine >> r) & 1;
-        const int32_t pos = wc[r * 16 + w] + (int32_t)__popcll(__ballot(fl) & lanes_below());
-        if (i < n) {
-            if constexpr (GRAND)
-                wr(i, pos, fl, wc[kOneR * 16]);
-            else
-                wr(i, pos, fl);
-        }
+        const int32_t pos = one_rank(mine, r, wc);
+        if (i < n) wr(i, pos, (int)((mine >> r) & 1));
     }
 }
 
@@ -317,7 +339,7 @@ template <class F, class Wr, class TT>
 inline hipError_t select_flags(F f, int64_t n, Wr wr, int32_t *tmp, TT *total, hipStream_t st) {
     const int64_t nt = tiles_of(n);
     if (n > 0 && n <= kOneMax) {
-        hipLaunchKernelGGL((k_flag_one<F, Wr, TT, false>), dim3(1), dim3(kOneT), 0, st, f, n, wr, total);
+        hipLaunchKernelGGL((k_flag_one<F, Wr, TT>), dim3(1), dim3(kOneT), 0, st, f, n, wr, total);
         return hipGetLastError();
     }
     if (nt > 0) hipLaunchKernelGGL(k_flag_count<F>, dim3((unsigned)nt), dim3(kT), 0, st, f, n, tmp);
@@ -339,10 +361,6 @@ inline hipError_t select_flags(F f, int64_t n, Wr wr, int32_t *tmp, TT *total, h
 template <class F, class Wr>
 inline hipError_t select_flags_counted(F f, int64_t n, Wr wr, int32_t *tmp, int32_t *total, hipStream_t st) {
     const int64_t nt = tiles_of(n);
-    if (n > 0 && n <= kOneMax) {
-        hipLaunchKernelGGL((k_flag_one<F, Wr, int32_t, true>), dim3(1), dim3(kOneT), 0, st, f, n, wr, total);
-        return hipGetLastError();
-    }
     if (nt > 0) hipLaunchKernelGGL(k_flag_count<F>, dim3((unsigned)nt), dim3(kT), 0, st, f, n, tmp);
     if (nt > 0 && nt <= kFuseTiles) {
         hipLaunchKernelGGL((k_flag_apply<F, Wr, true, int32_t, true>), dim3((unsigned)nt), dim3(kT), 0, st, f, n,

@@ -438,9 +438,102 @@ __global__ void k_compact_scatter(double *__restrict__ x, double *__restrict__ y
     if (gp.grid && t < K) grid_push(gp, (int32_t)dst, tx[t], ty[t]);
 }
 
+// The compaction in one work-group of prim::kOneT threads, for up to
+// prim::kOneMax slots: ranks as in prim::k_flag_one, the holes and donors in LDS,
+// the moved slots staged in tx, ty, tg.  Every thread of the work-group calls
+// it, with its writes to g done.
+struct CompactOne {
+    const int64_t *dn;
+    int64_t *dn1;
+    double *tx, *ty, *tg;
+};
+
+__device__ void compact_one(double *x, double *y, double *g, const CompactOne &A) {
+    __shared__ int32_t wc[prim::kOneR * 16 + 1], K_s;
+    __shared__ uint16_t holes[prim::kOneMax / 2], donors[prim::kOneMax / 2];
+    const int32_t n = (int32_t)*A.dn, tid = (int32_t)threadIdx.x;
+    const uint32_t mine = prim::one_flags([&](int64_t i) { return (int)live_at(g, i, n); }, n, wc);
+    const int32_t n1 = wc[prim::kOneR * 16];
+    if (tid == 0) *A.dn1 = n1;
+    if (n1 == n) return;
+    const int rounds = (n + prim::kOneT - 1) / prim::kOneT;
+    for (int r = 0; r < rounds; ++r) {
+        const int32_t i = r * prim::kOneT + tid, pos = prim::one_rank(mine, r, wc);
+        const bool f = (mine >> r) & 1;
+        if (i < n1) {
+            if (!f) holes[i - pos] = (uint16_t)i;
+        } else if (f) {
+            donors[n1 - pos - 1] = (uint16_t)i;
+        }
+        if (i == n1) K_s = n1 - pos;  // live entries of [n1, n), as many as holes
+    }
+    __syncthreads();
+    const int32_t K = K_s;
+    for (int32_t t = tid; t < K; t += prim::kOneT) {
+        const int32_t src = donors[t];
+        A.tx[t] = x[src];
+        A.ty[t] = y[src];
+        A.tg[t] = g[src];
+    }
+    for (int r = n1 / prim::kOneT; r < rounds; ++r) {
+        const int32_t e = r * prim::kOneT + tid, pos = prim::one_rank(mine, r, wc);
+        if (e < n1 || e >= n) continue;
+        const int32_t above = n1 - pos - (int32_t)((mine >> r) & 1);  // live entries of [n1, n) above e
+        const int32_t start = above < K ? (int32_t)holes[above] : n1;
+        const int32_t src = (e + 1 < n && !live_at(g, e + 1, n)) ? e + 1 : start;
+        A.tx[K + e - n1] = x[src];
+        A.ty[K + e - n1] = y[src];
+    }
+    __syncthreads();
+    for (int32_t t = tid; t < K; t += prim::kOneT) {
+        const int32_t h = holes[t];
+        x[h] = A.tx[t];
+        y[h] = A.ty[t];
+        g[h] = A.tg[t];
+    }
+    for (int r = n1 / prim::kOneT; r < rounds; ++r) {
+        const int32_t e = r * prim::kOneT + tid;
+        if (e < n1 || e >= n) continue;
+        x[e] = A.tx[K + e - n1];
+        y[e] = A.ty[K + e - n1];
+        g[e] = 0.0;
+    }
+}
+
+__global__ __launch_bounds__(prim::kOneT) void k_compact_one(double *x, double *y, double *g, CompactOne A,
+                                                             const int64_t *__restrict__ merged) {
+    if (compact_skip(merged)) {
+        if (threadIdx.x == 0) *A.dn1 = *A.dn;
+        return;
+    }
+    compact_one(x, y, g, A);
+}
+
+// Buffers and counts of a compaction in one work-group.
+static int compact_one_args(vx_case *c, int64_t n_ub, CompactOne *A) {
+    hipStream_t st = c->stream;
+    if (c->tx.ensure((size_t)(2 * n_ub), st) || c->ty.ensure((size_t)(2 * n_ub), st) ||
+        c->tg.ensure((size_t)(2 * n_ub), st) || c->dcount.ensure(16, st))
+        return 1;
+    *A = CompactOne{step_dn(c), c->dcount.p + (c->dn_slot == 1 ? 8 : 1), c->tx.p, c->ty.p, c->tg.p};
+    return 0;
+}
+
 int launch_compact(vx_case *c, int64_t n_ub, const int64_t *merged, const GridPush *gp) {
     if (n_ub <= 0) return 0;
     hipStream_t st = c->stream;
+    // Small bounds in one launch of one work-group: four launches of 4 to 9 us
+    // have little to do in each (the whole Step at 5000, 16000 and 31000
+    // vortices: 200 to 212 -> 111, 128 and 159 us; beyond, more slots than a
+    // thread's mask holds).
+    if (n_ub <= prim::kOneMax && !gp) {
+        CompactOne A;
+        if (compact_one_args(c, n_ub, &A)) return 1;
+        hipLaunchKernelGGL(k_compact_one, dim3(1), dim3(prim::kOneT), 0, st, c->x.p, c->y.p, c->g.p, A, merged);
+        VX_CHECK(hipGetLastError());
+        c->dn_slot = c->dn_slot == 1 ? 8 : 1;
+        return 0;
+    }
     if (c->scan.ensure((size_t)n_ub, st) || c->lists.ensure((size_t)(2 * n_ub), st) ||
         c->tx.ensure((size_t)(2 * n_ub), st) || c->ty.ensure((size_t)(2 * n_ub), st) ||
         c->tg.ensure((size_t)(2 * n_ub), st) || c->dcount.ensure(16, st))
@@ -900,12 +993,12 @@ struct ColCandidate {
 //     targets) gets its prepared work-array values back and the list counts
 //     are zeroed, so the next pass's search needs no preparation.
 // The candidates are the cb.nseg segments of the search's lists; *merged
-// receives their count.
-template <int KIND>
-__global__ __launch_bounds__(1024) void k_col_pass(double *__restrict__ x, double *__restrict__ y,
-                                                   double *__restrict__ g, const int32_t *__restrict__ col, ColBufs cb,
-                                                   int64_t *__restrict__ merged, int32_t *__restrict__ err,
-                                                   GridPush gp, int reset) {
+// receives their count.  With ONE, the pass's compaction (small counts) follows
+// in the same launch; without a candidate the count is only passed on.
+template <int KIND, bool ONE>
+__global__ __launch_bounds__(1024) void k_col_pass(double *x, double *y, double *g, const int32_t *__restrict__ col,
+                                                   ColBufs cb, int64_t *__restrict__ merged, int32_t *__restrict__ err,
+                                                   GridPush gp, int reset, CompactOne A) {
     __shared__ int64_t segoff[kColSeg + 1];
     __shared__ int32_t nrest;
     __shared__ int undecided;
@@ -921,6 +1014,10 @@ __global__ __launch_bounds__(1024) void k_col_pass(double *__restrict__ x, doubl
     }
     __syncthreads();
     const int64_t K = segoff[cb.nseg];
+    if (ONE && K == 0) {
+        if (threadIdx.x == 0) *A.dn1 = *A.dn;
+        return;
+    }
     auto cand = [&](int64_t t) -> int32_t {
         int q = 0;
         while (segoff[q + 1] <= t) ++q;
@@ -1009,6 +1106,12 @@ __global__ __launch_bounds__(1024) void k_col_pass(double *__restrict__ x, doubl
         }
         if (gp.grid) grid_push(gp, i, nx, ny);  // the survivor may have left its cell
     }
+    if constexpr (ONE) {  // the next pass clears the work arrays itself
+        static_assert(prim::kOneT == 1024, "one work-group for both");
+        __syncthreads();
+        compact_one(x, y, g, A);
+        return;
+    }
     if (!reset) return;
     __syncthreads();
     for (int64_t t = threadIdx.x; t < K; t += blockDim.x) {
@@ -1026,7 +1129,7 @@ __global__ __launch_bounds__(1024) void k_col_pass(double *__restrict__ x, doubl
     if (threadIdx.x == 0) *cb.nrest = 0;
 }
 
-int launch_collapse(vx_case *c, int kind, int64_t n_ub, bool prepared, const GridPush *gp, bool reset) {
+int launch_collapse(vx_case *c, int kind, int64_t n_ub, bool prepared, const GridPush *gp, bool reset, bool compact) {
     if (n_ub <= 0) return 0;
     hipStream_t st = c->stream;
     ColBufs cb{};
@@ -1041,14 +1144,27 @@ int launch_collapse(vx_case *c, int kind, int64_t n_ub, bool prepared, const Gri
     }
     const GridPush push = gp ? *gp : GridPush{};
     int32_t *err = (int32_t *)(c->dcount.p + 3);
+    if (compact && n_ub <= prim::kOneMax && !gp && !reset) {
+        CompactOne A;
+        if (compact_one_args(c, n_ub, &A)) return 1;
+        if (kind == 1)
+            hipLaunchKernelGGL((k_col_pass<1, true>), dim3(1), dim3(1024), 0, st, c->x.p, c->y.p, c->g.p, c->col.p, cb,
+                               col_merged(c), err, push, 0, A);
+        else
+            hipLaunchKernelGGL((k_col_pass<2, true>), dim3(1), dim3(1024), 0, st, c->x.p, c->y.p, c->g.p, c->col.p, cb,
+                               col_merged(c), err, push, 0, A);
+        VX_CHECK(hipGetLastError());
+        c->dn_slot = c->dn_slot == 1 ? 8 : 1;
+        return 0;
+    }
     if (kind == 1)
-        hipLaunchKernelGGL(k_col_pass<1>, dim3(1), dim3(1024), 0, st, c->x.p, c->y.p, c->g.p, c->col.p, cb,
-                           col_merged(c), err, push, (int)reset);
+        hipLaunchKernelGGL((k_col_pass<1, false>), dim3(1), dim3(1024), 0, st, c->x.p, c->y.p, c->g.p, c->col.p, cb,
+                           col_merged(c), err, push, (int)reset, CompactOne{});
     else
-        hipLaunchKernelGGL(k_col_pass<2>, dim3(1), dim3(1024), 0, st, c->x.p, c->y.p, c->g.p, c->col.p, cb,
-                           col_merged(c), err, push, (int)reset);
+        hipLaunchKernelGGL((k_col_pass<2, false>), dim3(1), dim3(1024), 0, st, c->x.p, c->y.p, c->g.p, c->col.p, cb,
+                           col_merged(c), err, push, (int)reset, CompactOne{});
     VX_CHECK(hipGetLastError());
-    return 0;
+    return compact ? launch_compact(c, n_ub, col_merged(c), gp) : 0;
 }
 
 // Below this many slots (the default of tune.col_share_min) a grid costs
@@ -1111,8 +1227,7 @@ int launch_step_collapse(vx_case *c, int64_t n_ub) {
             VX_CHECK(hipGetLastError());
             // a rebuilt grid needs no pushes, and its clear prepares the work arrays
             const GridPush *push = keep ? &gp : nullptr;
-            if (launch_collapse(c, kind, n_ub, true, push, keep) || launch_compact(c, n_ub, col_merged(c), push))
-                return 1;
+            if (launch_collapse(c, kind, n_ub, true, push, keep, true)) return 1;
         }
     }
     return 0;
@@ -1120,15 +1235,15 @@ int launch_step_collapse(vx_case *c, int64_t n_ub) {
 // ---- the tail of a step at small counts -----------------------------------------
 // The compaction after the move and every collapse pass with its compaction
 // in one launch of one work-group: at a few thousand vortices the stage is
-// about 40 launches of which each has next to nothing to do.  The decisions
+// about 20 launches of which each has next to nothing to do.  The decisions
 // and the arithmetic are those of the kernels above, slot by slot, so the
 // results are the same bit for bit: the closed form of the compaction, the
 // smallest partner index whatever the cells, the leaf-first resolution, the
 // merge.  x, y, g and the work arrays live in LDS up to kTailLds vortices
-// (the whole Step at 300, 2500 and 3300 vortices 141, 173 and 182 -> 57, 93
-// and 108 us); a graph's count may grow beyond, up to kTailMax, and is worked
-// on in place then, no faster than the launches (4000: 169 against 191,
-// 7900: 286 against 198), so a run that starts above kTailLds keeps those.
+// (the whole Step at 300, 2500 and 3300 vortices 89, 96 and 97 us as
+// launches, 44, 76 and 89 here); a graph's count may grow beyond, up to
+// kTailMax, and is worked on in place then, slower than the launches (4000: 169
+// against 110), so a run that starts above kTailLds keeps those.
 // Bound by the one work-group's instructions.
 constexpr int kTailT = 1024, kTailHeads = 4096;
 constexpr int kTailLds = 3584;
