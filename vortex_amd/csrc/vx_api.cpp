@@ -617,7 +617,7 @@ int vx_speed(vx_case *c, double vinf_x, double vinf_y) {
         if ((tree && tree_diffusion_pre(c)) || side_fork(c)) return 1;
         // the long main-stream kernel is issued first; the side stream's
         // work is ordered after the fork point only
-        rc = tree ? tree_diffusion_main(c) : launch_diffusion(c, s, s);
+        rc = tree ? tree_diffusion_main(c) : launch_diffusion(c, host_cnt(s), host_cnt(s), true);
         if (c->timing) (void)hipEventRecord(c->ev[14], c->side);
         if (!rc) rc = launch_wall_side(c, s, c->side);
         if (c->timing) (void)hipEventRecord(c->ev[15], c->side);
@@ -643,7 +643,8 @@ int vx_step(vx_case *c, double out4[4]) {
     VX_ARG(c && out4, "null pointer");
     Timer t(c, &c->tm.step_ms, 4);
     const int64_t n_ub = c->n;
-    if (launch_set_dn(c, n_ub) || launch_step_move(c) || launch_step_tail(c, n_ub)) return 1;
+    if (launch_set_dn(c, n_ub) || launch_step_move(c, !step_tail_fits(c, n_ub)) || launch_step_tail(c, n_ub, false))
+        return 1;
     int err = 0;
     if (step_readback(c, out4, &err)) return 1;
     if (err) {
@@ -803,10 +804,10 @@ static int device_step(vx_case *c, double vinf_x, double vinf_y) {
         launch_step_probes(c, vinf_x, vinf_y))
         return 1;
     const Cnt s = cnt_s(c);
-    if (launch_biot_savart(c, s, s, vinf_x, vinf_y) || launch_diffusion(c, s, s) || launch_diffusion_wall(c, s))
+    if (launch_biot_savart(c, s, s, vinf_x, vinf_y) || launch_diffusion(c, s, s, true) || launch_diffusion_wall(c, s))
         return 1;
-    if (launch_set_dn(c, n_ub) || launch_step_move(c) || launch_step_tail(c, n_ub)) return 1;
-    return launch_step_record(c);
+    return launch_set_dn(c, n_ub) || launch_step_move(c, !step_tail_fits(c, n_ub)) ||
+           launch_step_tail(c, n_ub, true);
 }
 
 static void graph_release(vx_case *c) {

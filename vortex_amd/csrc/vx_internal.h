@@ -252,7 +252,6 @@ int side_join(vx_case *c);  // the main stream waits for the work queued so far 
 int aux_streams(vx_case *c);  // creates aux[] and their events once
 int launch_pack_f32(vx_case *c, int64_t count);
 int launch_pack_f32(vx_case *c, Cnt count);
-int launch_count_add(vx_case *c, int64_t *a, int64_t v);  // *a += v (stream-ordered)
 int launch_step_record(vx_case *c);  // count back to slot 1; forces and count into gr_ring
 // The counts of the current stage: host values, or in device-count mode the
 // count slot dcount[1] (n, or rounded up to a multiple of 32: s).
@@ -269,7 +268,8 @@ int launch_biot_savart(vx_case *c, int64_t n_tgt, int64_t n_src, double vinf_x, 
 int launch_biot_savart(vx_case *c, Cnt n_tgt, Cnt n_src, double vinf_x, double vinf_y);
 int launch_diffusion(vx_case *c, int64_t n_tgt, int64_t n_src);
 double diff_thr2(double thr);  // r^2 > diff_thr2(thr) decides as sqrt(r^2) > thr
-int launch_diffusion(vx_case *c, Cnt n_tgt, Cnt n_src);
+// packed: launch_biot_savart over the same sources just left their FP32 copies
+int launch_diffusion(vx_case *c, Cnt n_tgt, Cnt n_src, bool packed = false);
 int launch_right_part(vx_case *c, int64_t n_src, double vinf_x, double vinf_y);  // -> c->rp
 int launch_right_part(vx_case *c, Cnt n_src, double vinf_x, double vinf_y);
 int launch_probe(vx_case *c, int64_t m, int64_t n_src, double vinf_x, double vinf_y); // c->px.. -> c->pu,pv
@@ -292,12 +292,11 @@ int launch_tree_probes(vx_case *c, const double *px, const double *py, int64_t m
 int launch_probe_noalloc(vx_case *c, const double *px, const double *py, int64_t m, double vinf_x, double vinf_y,
                          double *pu, double *pv);
 // vx_wall.hip
-// launch_wall_side queues the wall term on stream st (the main stream, or the
-// side stream after side_fork), into per-target staging; launch_wall_add
-// (main stream, after side_join if st was the side stream) adds the terms to
-// u, v.  launch_diffusion_wall is the two in a row on the main stream.
+// launch_wall_side queues the wall term on stream st (the side stream after
+// side_fork), into per-target staging; launch_wall_add (main stream, after
+// side_join) adds the terms to u, v.  launch_diffusion_wall does both on the main
+// stream in one pass.
 int launch_wall_side(vx_case *c, int64_t n_tgt, hipStream_t st);
-int launch_wall_side(vx_case *c, Cnt n_tgt, hipStream_t st);
 int launch_wall_add(vx_case *c);
 int launch_diffusion_wall(vx_case *c, int64_t n_tgt);
 int launch_diffusion_wall(vx_case *c, Cnt n_tgt);
@@ -334,7 +333,7 @@ void tree_release(vx_case *c);
 // n_ub is an upper bound of it (n never grows inside Step), used for grids.
 int64_t *step_dn(vx_case *c);                          // the device count
 int launch_set_dn(vx_case *c, int64_t n);              // *dn = n (stream-ordered)
-int launch_step_move(vx_case *c);                      // sums and live box -> c->red[0..7]
+int launch_step_move(vx_case *c, bool sums = true);    // with sums: they and the live box -> c->red[0..7]
 int launch_points_move(vx_case *c, int64_t m);         // c->px, py, pg moved by c->pu, pv
 // A collapse grid kept over the passes of one step (launch_step_collapse):
 // a kernel that gives a slot new data (a merge's survivor, a compaction's
@@ -365,9 +364,10 @@ int launch_collapse(vx_case *c, int kind, int64_t n_ub, bool prepared, const Gri
 // compactions), from 2^17 slots on over a grid kept from pass to pass.
 // Collapse error flag in dcount[3] (bit 2: the grid's node pool was full).
 int launch_step_collapse(vx_case *c, int64_t n_ub);
-// The compaction after the move and launch_step_collapse, at small counts as
-// one launch with the same results.
-int launch_step_tail(vx_case *c, int64_t n_ub);
+// The compaction after the move and launch_step_collapse, and with record
+// launch_step_record; at small counts (step_tail_fits) as one launch with the
+// same results, which makes the move's sums too.
+int launch_step_tail(vx_case *c, int64_t n_ub, bool record);
 bool step_tail_fits(const vx_case *c, int64_t n_ub);  // as one launch
 
 }  // namespace vx

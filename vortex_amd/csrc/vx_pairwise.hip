@@ -1437,12 +1437,13 @@ double diff_thr2(double thr) {
     return t;
 }
 
-int launch_diffusion(vx_case *c, Cnt n_tgt, Cnt n_src) {
+int launch_diffusion(vx_case *c, Cnt n_tgt, Cnt n_src, bool packed) {
     if (n_tgt.ub <= 0) return 0;
     const double thr = 0.001 * c->prm.ve_size;
     const dim3 gsum((unsigned)((n_tgt.ub + 63) / 64));
     if (mixed(c)) {
-        if (c->partial.ensure(direct_partials<float>(n_tgt, n_src, 3), c->stream) || launch_pack_f32(c, n_src))
+        if (c->partial.ensure(direct_partials<float>(n_tgt, n_src, 3), c->stream) ||
+            (!packed && launch_pack_f32(c, n_src)))
             return 1;
         diff_dispatch<float>(c, tpt_of(c->tune.tpt_diff, true, n_tgt.ub), c->xf.p, c->yf.p, c->gf.p, n_src, n_tgt,
                              (float)(thr * thr));

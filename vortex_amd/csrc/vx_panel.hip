@@ -693,15 +693,23 @@ int launch_birth_positions(vx_case *c) {
     return 0;
 }
 
-__global__ void k_birth_place(const double *__restrict__ gs, PanelsSoA pan, const double *__restrict__ bp, Cnt cn,
-                              int64_t cap, double *__restrict__ x, double *__restrict__ y, double *__restrict__ g) {
-    const int64_t i = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
+// With grow (one work-group then, which has read the count before), the device
+// count becomes *grow + P.
+__global__ __launch_bounds__(1024) void k_birth_place(const double *__restrict__ gs, PanelsSoA pan,
+                                                      const double *__restrict__ bp, Cnt cn, int64_t cap,
+                                                      double *__restrict__ x, double *__restrict__ y,
+                                                      double *__restrict__ g, int64_t *grow) {
     const int64_t n = cn.get();
-    if (i >= pan.P || n + i >= cap) return;
-    const int64_t nx = pan.rp[i];
-    x[n + i] = bp[i];
-    y[n + i] = bp[pan.P + i];
-    g[n + i] = 0.5 * (gs[i] * pan.len[i] + gs[nx] * pan.len[nx]);
+    for (int64_t i = (int64_t)blockIdx.x * blockDim.x + threadIdx.x; i < pan.P; i += (int64_t)gridDim.x * blockDim.x) {
+        if (n + i >= cap) break;
+        const int64_t nx = pan.rp[i];
+        x[n + i] = bp[i];
+        y[n + i] = bp[pan.P + i];
+        g[n + i] = 0.5 * (gs[i] * pan.len[i] + gs[nx] * pan.len[nx]);
+    }
+    if (!grow) return;
+    __syncthreads();
+    if (threadIdx.x == 0) *grow += pan.P;
 }
 
 // The sheet strengths of the last birth: the inverse's product, or with the
@@ -721,10 +729,10 @@ int launch_birth(vx_case *c, double d_g) {
         hipLaunchKernelGGL(k_birth_gemv, dim3((unsigned)((P + 3) / 4)), dim3(256), 0, c->stream, c->M.p, c->rp.p,
                            d_g, dgp, P, c->gsheet.p);
     }
-    hipLaunchKernelGGL(k_birth_place, dim3((unsigned)((P + 255) / 256)), dim3(256), 0, c->stream, birth_sheet(c),
-                       c->pan, c->bpos, cnt_n(c), c->cap, c->x.p, c->y.p, c->g.p);
+    const dim3 grid(c->devcount ? 1u : (unsigned)((P + 255) / 256)), wg(c->devcount ? 1024u : 256u);
+    hipLaunchKernelGGL(k_birth_place, grid, wg, 0, c->stream, birth_sheet(c), c->pan, c->bpos, cnt_n(c), c->cap, c->x.p,
+                       c->y.p, c->g.p, c->devcount ? c->dcount.p + 1 : nullptr);
     VX_CHECK(hipGetLastError());
-    if (c->devcount && launch_count_add(c, c->dcount.p + 1, P)) return 1;
     return 0;
 }
 

@@ -93,10 +93,8 @@ int launch_pack_f32(vx_case *c, Cnt count) {
 
 int launch_pack_f32(vx_case *c, int64_t count) { return launch_pack_f32(c, host_cnt(count)); }
 
-// Device-count helpers for captured steps: *a += v; the step's count back to
-// slot 1 and the step's forces and count into the ring (slot k = st[0]++).
-__global__ void k_count_add(int64_t *__restrict__ a, int64_t v) { *a += v; }
-
+// For captured steps: the step's count back to slot 1 and the step's forces
+// and count into the ring (slot k = st[0]++).
 __global__ void k_step_record(int64_t *__restrict__ dcount, int slot, const double *__restrict__ red,
                               double *__restrict__ ring, int64_t *__restrict__ nring, int64_t *__restrict__ k) {
     const int64_t n = dcount[slot];
@@ -105,12 +103,6 @@ __global__ void k_step_record(int64_t *__restrict__ dcount, int slot, const doub
     for (int q = 0; q < 4; ++q) ring[4 * s + q] = red[q];
     nring[s] = n;
     *k = s + 1;
-}
-
-int launch_count_add(vx_case *c, int64_t *a, int64_t v) {
-    hipLaunchKernelGGL(k_count_add, dim3(1), dim3(1), 0, c->stream, a, v);
-    VX_CHECK(hipGetLastError());
-    return 0;
 }
 
 int launch_step_record(vx_case *c) {

@@ -228,7 +228,7 @@ int launch_set_dn(vx_case *c, int64_t n) {
     return 0;
 }
 
-int launch_step_move(vx_case *c) {
+int launch_step_move(vx_case *c, bool sums) {
     const Cnt cn = cnt_n(c);
     const int64_t n = cn.ub;  // bound: grids and list sizes
     const int64_t nb = n > 0 ? (n + 255) / 256 : 1;
@@ -250,7 +250,7 @@ int launch_step_move(vx_case *c) {
     }
     hipLaunchKernelGGL(k_step_move, dim3((unsigned)nb), dim3(256), 0, st, c->x.p, c->y.p, c->g.p, c->u.p, c->v.p, cn,
                        c->P, c->pan, k, hitp, c->partial.p);
-    hipLaunchKernelGGL(k_sum4, dim3(1), dim3(256), 0, st, c->partial.p, nb, p.rho, p.dt, c->red.p);
+    if (sums) hipLaunchKernelGGL(k_sum4, dim3(1), dim3(256), 0, st, c->partial.p, nb, p.rho, p.dt, c->red.p);
     VX_CHECK(hipGetLastError());
     return 0;
 }
@@ -1255,7 +1255,16 @@ struct TailArgs {
     int32_t *holes, *donors;       // n slots each
     const int64_t *dn;
     int64_t *dn_out;
-    const double *box;             // live box after the move
+    // k_sum4's sums of the move's nb <= 32 partials go to red (the live box to
+    // red[4..7])
+    const double *part;
+    double *red;
+    int64_t nb;
+    double rho, dt;
+    // with ring, the step's record (k_step_record): forces and count, the
+    // count back to *dn_first
+    double *ring;
+    int64_t *nring, *kring, *dn_first;
     int32_t *err;
     double r2[2], max_ve_g;
     int64_t n_col;
@@ -1315,7 +1324,7 @@ __device__ void tail_run(const TailArgs &A, TailShared &sh, int32_t *lds, int32_
         first[i] = INT32_MAX;
     }
     for (int32_t i = tid; i < C / 32; i += kTailT) bits[i] = 0u;
-    if (tid < 2) sh.grid[tid] = grid_params(A.box, A.r2[tid], (int64_t)1 << 30);
+    if (tid < 2) sh.grid[tid] = grid_params((A.red + 4), A.r2[tid], (int64_t)1 << 30);
     __syncthreads();
 
     auto live = [&](int32_t i) { return i < n && !(fabs(g[i]) < kDelt); };
@@ -1569,29 +1578,64 @@ __device__ void tail_run(const TailArgs &A, TailShared &sh, int32_t *lds, int32_
             A.g[i] = g[i];
         }
     }
-    if (tid == 0) *A.dn_out = n;
+    if (tid != 0) return;
+    *A.dn_out = n;
+    if (!A.ring) return;
+    const int64_t k = *A.kring;
+    for (int q = 0; q < 4; ++q) A.ring[4 * k + q] = A.red[q];
+    A.nring[k] = n;
+    *A.kring = k + 1;
+    *A.dn_first = n;
 }
 
 constexpr size_t tail_ints(int64_t c) { return (size_t)(kTailHeads + 4 * c + c / 32); }
 constexpr size_t kTailBytes = std::max(sizeof(int32_t) * tail_ints(kTailLds) + 24 * (size_t)kTailLds,
                                        sizeof(int32_t) * tail_ints(kTailMax));
 
+// k_sum4 by one wave: its tree's levels of 128 to 32 would add zeros.
+__device__ __forceinline__ void tail_sums(const TailArgs &A) {
+    const int lane = (int)(threadIdx.x & 63);
+    double a[8];
+#pragma unroll
+    for (int q = 0; q < 8; ++q) {
+        const double p = lane < A.nb ? A.part[lane * 8 + q] : (q < 4 ? 0.0 : 1e300);
+        a[q] = q < 4 ? 0.0 + p : p;
+        for (int o = 16; o > 0; o >>= 1) {
+            const double b = __shfl_xor(a[q], o, 64);
+            a[q] = q < 4 ? a[q] + b : fmin(a[q], b);
+        }
+    }
+    if (lane != 0) return;
+    A.red[0] = a[0];
+    A.red[1] = a[1] * (A.rho / A.dt);
+    A.red[2] = a[2] * (A.rho / A.dt);
+    A.red[3] = a[3] * (A.rho / (2 * A.dt));
+    A.red[4] = a[4];
+    A.red[5] = -a[5];
+    A.red[6] = a[6];
+    A.red[7] = -a[7];
+}
+
 __global__ __launch_bounds__(kTailT) void k_step_tail(TailArgs A) {
     __shared__ __align__(16) int32_t lds[kTailBytes / sizeof(int32_t)];
     __shared__ TailShared sh;
     const int32_t n = (int32_t)*A.dn;
+    if (threadIdx.x < 64) tail_sums(A);
+    __syncthreads();
     if (n <= kTailLds)
         tail_run<true, kTailLds>(A, sh, lds, n);
     else
         tail_run<false, (int)kTailMax>(A, sh, lds, n);
 }
 
-// The compaction after the move and the collapse (both kinds), by count.
-bool step_tail_fits(const vx_case *c, int64_t n_ub) { return n_ub <= kTailMax && c->n <= kTailLds; }
+// The compaction after the move and the collapse (both kinds), by count; in
+// one launch also the move's sums (launch_step_move without them) and, for a
+// step on device counts, the step's record.
+bool step_tail_fits(const vx_case *c, int64_t n_ub) { return n_ub > 0 && n_ub <= kTailMax && c->n <= kTailLds; }
 
-int launch_step_tail(vx_case *c, int64_t n_ub) {
-    if (!step_tail_fits(c, n_ub)) return launch_compact(c, n_ub) || launch_step_collapse(c, n_ub);
-    if (n_ub <= 0) return 0;
+int launch_step_tail(vx_case *c, int64_t n_ub, bool record) {
+    if (!step_tail_fits(c, n_ub))
+        return launch_compact(c, n_ub) || launch_step_collapse(c, n_ub) || (record && launch_step_record(c));
     hipStream_t st = c->stream;
     if (c->lists.ensure((size_t)(2 * n_ub), st) || c->tx.ensure((size_t)(2 * n_ub), st) ||
         c->ty.ensure((size_t)(2 * n_ub), st) || c->tg.ensure((size_t)(2 * n_ub), st) || c->dcount.ensure(16, st))
@@ -1609,7 +1653,17 @@ int launch_step_tail(vx_case *c, int64_t n_ub) {
     A.donors = l + n_ub;
     A.dn = step_dn(c);
     A.dn_out = c->dcount.p + (c->dn_slot == 1 ? 8 : 1);
-    A.box = c->red.p + 4;
+    A.part = c->partial.p;
+    A.red = c->red.p;
+    A.nb = (n_ub + 255) / 256;
+    A.rho = c->prm.rho;
+    A.dt = c->prm.dt;
+    if (record) {
+        A.ring = c->gr_ring.p;
+        A.nring = (int64_t *)(c->gr_ring.p + 4 * c->gr_cap);
+        A.kring = c->dcount.p + 9;
+        A.dn_first = c->dcount.p + 1;
+    }
     A.err = (int32_t *)(c->dcount.p + 3);
     A.r2[0] = c->prm.r_col_diff_sign * c->prm.r_col_diff_sign * ve2;  // src/unit_1.cu:1228-1229
     A.r2[1] = c->prm.r_col_same_sign * c->prm.r_col_same_sign * ve2;
@@ -1617,7 +1671,7 @@ int launch_step_tail(vx_case *c, int64_t n_ub) {
     A.n_col = c->prm.n_col;
     hipLaunchKernelGGL(k_step_tail, dim3(1), dim3(kTailT), 0, st, A);
     VX_CHECK(hipGetLastError());
-    c->dn_slot = c->dn_slot == 1 ? 8 : 1;
+    c->dn_slot = record ? 1 : (c->dn_slot == 1 ? 8 : 1);
     return 0;
 }
 
