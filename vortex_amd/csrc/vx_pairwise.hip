@@ -420,10 +420,12 @@ __global__ __launch_bounds__(256) void k_diff_sum(const double *__restrict__ par
 // 64 / TG sources per wave and pass, into LDS, and one adds the tile before
 // in order, the components of a target on lanes of their own.  The term
 // arithmetic is correctly rounded as the plain expressions are, so the
-// results are those of the plain loop bit for bit.  Bound by the adding
-// wave's reads and adds (about 10 ns a source while there is a CU for each
-// work-group).  2500 vortices: Biot-Savart 243 -> 26 us, diffusion 475 -> 34
-// us against one lane per target over all sources.  Above kOrdered the split
+// results are those of the plain loop bit for bit.  Bound by the LDS while
+// there is a CU for each work-group: Biot-Savart takes 24 cycles a source, the
+// adding wave alone 21 (two 16-byte reads a pair of sources), the evaluating
+// ones alone 15; the reads of the next batch stand between the adds (all
+// before them: 3 % more).  2500 vortices: Biot-Savart 243 -> 25 us, diffusion
+// 475 -> 33 us against one lane per target over all sources.  Above kOrdered the split
 // sums are faster: at 17000 0.26 and 0.40 ms against 0.62 and 1.05 ms.
 constexpr int kOrdWaves = 15;
 constexpr int kAhead = 6;  // pairs of terms per batch: the LDS latency of one is covered by the adds of another
@@ -515,15 +517,12 @@ __global__ __launch_bounds__(1024) void k_biot_savart_ordered(const double *__re
             }
 #pragma unroll
             for (int h = 0; h < TILE / 2 / kAhead; ++h) {
-                if (h + 1 < TILE / 2 / kAhead) {
 #pragma unroll
-                    for (int e = 0; e < kAhead; ++e) {
+                for (int e = 0; e < kAhead; ++e) {
+                    if (h + 1 < TILE / 2 / kAhead) {
                         w[(h + 1) & 1][e] = w_[((h + 1) * kAhead + e) * TG];
                         p[(h + 1) & 1][e] = s_[(h + 1) * kAhead + e];
                     }
-                }
-#pragma unroll
-                for (int e = 0; e < kAhead; ++e) {
                     acc = fma(w[h & 1][e].x, fma(p[h & 1][e].x, c1, c0), acc);
                     acc = fma(w[h & 1][e].y, fma(p[h & 1][e].y, c1, c0), acc);
                 }
@@ -626,16 +625,13 @@ __global__ __launch_bounds__(1024) void k_diffusion_ordered(const double *__rest
             }
 #pragma unroll
             for (int h = 0; h < TILE / 2 / H; ++h) {
-                if (h + 1 < TILE / 2 / H) {
 #pragma unroll
-                    for (int q = 0; q < H; ++q) {
+                for (int q = 0; q < H; ++q) {
+                    if (h + 1 < TILE / 2 / H) {
                         p[(h + 1) & 1][q] = p_[((h + 1) * H + q) * TG];
                         x[(h + 1) & 1][q] = e_[((h + 1) * H + q) * TG];
                         g[(h + 1) & 1][q] = g_[(h + 1) * H + q];
                     }
-                }
-#pragma unroll
-                for (int q = 0; q < H; ++q) {
                     acc = fma(p[h & 1][q].x, x[h & 1][q].x, acc);
                     acc1 = fma(g[h & 1][q].x, x[h & 1][q].x, acc1);
                     acc = fma(p[h & 1][q].y, x[h & 1][q].y, acc);
