@@ -818,20 +818,27 @@ constexpr int kRhsPG = 4;
 constexpr int64_t kRhsSplitSrc = 32768;
 
 template <typename T>
-__global__ __launch_bounds__(256) void k_right_part_terms(const T *__restrict__ sg, const double *__restrict__ x,
-                                                          const double *__restrict__ y,
-                                                          const int32_t *__restrict__ list,
-                                                          const int32_t *__restrict__ nlist, PanelsSoA pan,
-                                                          const RhsSeg *__restrict__ segs, double *__restrict__ part) {
+struct RhsTermsLds {
+    T lx[256], ly[256], lg[256];
+    T lt[256][kRhsPG][2];
+    int wcount[4];
+};
+
+template <typename T>
+__device__ __forceinline__ void rhs_terms(RhsTermsLds<T> &L, int64_t group, int64_t c, const T *__restrict__ sg,
+                                          const double *__restrict__ x, const double *__restrict__ y,
+                                          const int32_t *__restrict__ list, int64_t n_src, const PanelsSoA &pan,
+                                          const RhsSeg *__restrict__ segs, double *__restrict__ part) {
     constexpr int kPer = kSegTile / kRhsPG;
     constexpr bool F32 = sizeof(T) == 4;
     static_assert(kSegTile == 128, "two tiles of the sums in 256 sources");
-    __shared__ T lx[256], ly[256], lg[256];
-    __shared__ T lt[256][kRhsPG][2];
-    __shared__ int wcount[4];
-    const RhsSeg S = segs[blockIdx.x / kPer];
-    const int p0 = (int)(blockIdx.x % kPer) * kRhsPG;
-    const int64_t c = blockIdx.y, n_src = *nlist;
+    auto &lx = L.lx;
+    auto &ly = L.ly;
+    auto &lg = L.lg;
+    auto &lt = L.lt;
+    auto &wcount = L.wcount;
+    const RhsSeg S = segs[group / kPer];
+    const int p0 = (int)(group % kPer) * kRhsPG;
     const int64_t lo = c * kRhsChunk, hi = min(n_src, lo + kRhsChunk);
     if (p0 >= S.count || (lo >= n_src && lo > 0)) return;
     const int tid = threadIdx.x, lane = tid & 63, wv = tid >> 6;
@@ -1026,16 +1033,15 @@ __host__ __device__ __forceinline__ int64_t rhs_groups(int64_t n, int64_t most) 
     return b < most ? b : most;
 }
 
-__global__ __launch_bounds__(256) void k_rhs_expand(const double *__restrict__ x, const double *__restrict__ y,
-                                                    const double *__restrict__ g, Cnt cn_src, double cx, double cy,
-                                                    double r2, const int32_t *__restrict__ list,
-                                                    const int32_t *__restrict__ nlist,
-                                                    const RhsSeg *__restrict__ segs, int64_t nfar, int64_t nseg,
-                                                    double *__restrict__ spart, double *__restrict__ spart_seg) {
-    __shared__ double red[2][16 * kRedRow];
-    if ((int64_t)blockIdx.x < nfar) {
-        const int64_t n = cn_src.get(), first = (int64_t)blockIdx.x * 256;
-        if (first >= n) return;
+__device__ __forceinline__ void rhs_expand_group(double (*red)[16 * kRedRow], int64_t group,
+                                                 const double *__restrict__ x, const double *__restrict__ y,
+                                                 const double *__restrict__ g, int64_t n_src, double cx, double cy,
+                                                 double r2, const int32_t *__restrict__ list, int64_t n_list,
+                                                 const RhsSeg *__restrict__ segs, int64_t nfar, int64_t nseg,
+                                                 double *__restrict__ spart, double *__restrict__ spart_seg) {
+    if (group < nfar) {
+        const int64_t first = group * 256;
+        if (first >= n_src) return;
         rhs_expand(
             [&](int64_t j, double &gj, double &dx, double &dy) {
                 gj = g[j];
@@ -1043,10 +1049,10 @@ __global__ __launch_bounds__(256) void k_rhs_expand(const double *__restrict__ x
                 dy = y[j] - cy;
                 return !(gj == 0 || !(dx * dx + dy * dy >= r2));
             },
-            n, first + threadIdx.x, nfar * 256, red, spart + (int64_t)blockIdx.x * kLoc * 2);
+            n_src, first + threadIdx.x, nfar * 256, red, spart + group * kLoc * 2);
     } else {
-        const int64_t b = (int64_t)blockIdx.x - nfar, s = b / nseg, first = b % nseg * 256, n = *nlist;
-        if (first >= n) return;
+        const int64_t b = group - nfar, s = b / nseg, first = b % nseg * 256;
+        if (first >= n_list) return;
         const RhsSeg S = segs[s];
         const double rn2 = 4.0 * S.r * S.r;
         rhs_expand(
@@ -1057,8 +1063,54 @@ __global__ __launch_bounds__(256) void k_rhs_expand(const double *__restrict__ x
                 dy = y[j] - S.cy;
                 return dx * dx + dy * dy >= rn2;
             },
-            n, first + threadIdx.x, nseg * 256, red, spart_seg + (s * kSegBlocks + first / 256) * kLoc * 2);
+            n_list, first + threadIdx.x, nseg * 256, red, spart_seg + (s * kSegBlocks + first / 256) * kLoc * 2);
     }
+}
+
+struct RhsExpand {
+    const double *x, *y, *g;
+    Cnt cn_src;
+    double cx, cy, r2;
+    const int32_t *list, *nlist;
+    const RhsSeg *segs;
+    int64_t nfar, nseg;
+    double *spart, *spart_seg;
+};
+
+__global__ __launch_bounds__(256) void k_rhs_expand(RhsExpand A) {
+    __shared__ double red[2][16 * kRedRow];
+    rhs_expand_group(red, blockIdx.x, A.x, A.y, A.g, A.cn_src.get(), A.cx, A.cy, A.r2, A.list, *A.nlist, A.segs, A.nfar,
+                     A.nseg, A.spart, A.spart_seg);
+}
+
+template <typename T>
+__global__ __launch_bounds__(256) void k_right_part_terms(const T *__restrict__ sg, PanelsSoA pan,
+                                                          double *__restrict__ part, RhsExpand A) {
+    __shared__ RhsTermsLds<T> L;
+    rhs_terms<T>(L, blockIdx.x, blockIdx.y, sg, A.x, A.y, A.list, *A.nlist, pan, A.segs, part);
+}
+
+// The pairs by terms (work-groups [0, nterm): nx groups of panels for each
+// chunk) and the expansions in one launch: up to kRhsOneSrc sources neither
+// fills the chip, and the expansions' 6 us pass beside the pairs.  The pairs
+// then run with the expansions' registers and LDS, which a longer list would
+// feel (a batch with some 20000 sources each: 23 us against 9.4 + 8).
+constexpr int64_t kRhsOneSrc = 8192;
+
+template <typename T>
+__global__ __launch_bounds__(256) void k_right_part_all(const T *__restrict__ sg, PanelsSoA pan, int64_t nx,
+                                                        int64_t nterm, double *__restrict__ part, RhsExpand A) {
+    __shared__ __align__(16) union Lds {
+        RhsTermsLds<T> terms;
+        double red[2][16 * kRedRow];
+        __device__ Lds() {}
+    } L;
+    const int64_t w = blockIdx.x;
+    if (w < nterm)
+        rhs_terms<T>(L.terms, w % nx, w / nx, sg, A.x, A.y, A.list, *A.nlist, pan, A.segs, part);
+    else
+        rhs_expand_group(L.red, w - nterm, A.x, A.y, A.g, A.cn_src.get(), A.cx, A.cy, A.r2, A.list, *A.nlist, A.segs,
+                         A.nfar, A.nseg, A.spart, A.spart_seg);
 }
 
 // S_k over the work-group partials: one work-group per real/imaginary part of
@@ -1079,16 +1131,16 @@ __global__ __launch_bounds__(256) void k_rhs_far_final(const double *__restrict_
     if (threadIdx.x == 0) S[t] = r[0];
 }
 
-// Binomials C(k, m), m <= k < kLoc (below 2^44, so exact).
+// Binomials c[q][m] = C(m + q, m) for m + q < kLoc (below 2^44, so exact),
+// else 0; a step of the shift reads a row.
 struct Binom {
     double c[kLoc][kLoc];
 };
 constexpr Binom binomials() {
     Binom b{};
-    for (int k = 0; k < kLoc; ++k) {
-        b.c[k][0] = 1.0;
-        for (int m = 1; m <= k; ++m) b.c[k][m] = b.c[k - 1][m - 1] + (m < k ? b.c[k - 1][m] : 0.0);
-    }
+    for (int m = 0; m < kLoc; ++m) b.c[0][m] = 1.0;
+    for (int q = 1; q < kLoc; ++q)
+        for (int m = 0; m + q < kLoc; ++m) b.c[q][m] = b.c[q - 1][m] + (m > 0 ? b.c[q][m - 1] : 0.0);
     return b;
 }
 __device__ const Binom kBinom = binomials();
@@ -1096,24 +1148,14 @@ __device__ const Binom kBinom = binomials();
 // Each segment's coefficients about c_s: the global S shifted exactly,
 //   sum_{k >= m} S_k C(k, m) (c_s - c)^{k - m},
 // plus its own sources' partials (fixed order).  Thread m < kLoc.
-__global__ __launch_bounds__(64) void k_rhs_seg_final(const double *__restrict__ spart, const double *__restrict__ S,
-                                                      double cx, double cy, const RhsSeg *__restrict__ segs,
-                                                      const int32_t *__restrict__ nlist, int64_t nseg,
-                                                      double *__restrict__ Ss) {
-    __shared__ double lS[2 * kLoc];
-    for (int t = threadIdx.x; t < 2 * kLoc; t += 64) lS[t] = S[t];
-    __syncthreads();
-    const int m = threadIdx.x;
-    if (m >= kLoc) return;
-    const RhsSeg G = segs[blockIdx.x];
-    const int nb = (int)rhs_groups(*nlist, nseg);
-    const double er = G.cx - cx, ei = G.cy - cy;  // c_s - c
-    double ar = 0.0, ai = 0.0;
+__device__ __forceinline__ void rhs_seg_coeff(const double *__restrict__ spart, int nb, const double *lS, double er,
+                                              double ei, int m, double &ar, double &ai) {
+    ar = ai = 0.0;
     double pr = 1.0, pi = 0.0;  // (c_s - c)^{k - m}
-#pragma unroll 4
+#pragma unroll 12
     for (int q = 0; q < kLoc; ++q) {
         const int k = m + q < kLoc ? m + q : kLoc - 1;
-        const double bin = kBinom.c[k][m];
+        const double bin = kBinom.c[q][m];
         const double tr = pr * bin, ti = pi * bin;
         const double sr = ar + fma(tr, lS[2 * k], -(ti * lS[2 * k + 1]));
         const double si = ai + fma(ti, lS[2 * k], tr * lS[2 * k + 1]);
@@ -1125,10 +1167,25 @@ __global__ __launch_bounds__(64) void k_rhs_seg_final(const double *__restrict__
     }
 #pragma unroll 8
     for (int b = 0; b < nb; ++b) {
-        const double *q = spart + (((int64_t)blockIdx.x * kSegBlocks + b) * kLoc + m) * 2;
+        const double *q = spart + ((int64_t)b * kLoc + m) * 2;
         ar += q[0];
         ai += q[1];
     }
+}
+
+__global__ __launch_bounds__(64) void k_rhs_seg_final(const double *__restrict__ spart, const double *__restrict__ S,
+                                                      double cx, double cy, const RhsSeg *__restrict__ segs,
+                                                      const int32_t *__restrict__ nlist, int64_t nseg,
+                                                      double *__restrict__ Ss) {
+    __shared__ double lS[2 * kLoc];
+    for (int t = threadIdx.x; t < 2 * kLoc; t += 64) lS[t] = S[t];
+    __syncthreads();
+    const int m = threadIdx.x;
+    if (m >= kLoc) return;
+    const RhsSeg G = segs[blockIdx.x];
+    double ar, ai;
+    rhs_seg_coeff(spart + (int64_t)blockIdx.x * kSegBlocks * kLoc * 2, (int)rhs_groups(*nlist, nseg), lS, G.cx - cx,
+                  G.cy - cy, m, ar, ai);
     Ss[((int64_t)blockIdx.x * kLoc + m) * 2] = ar;
     Ss[((int64_t)blockIdx.x * kLoc + m) * 2 + 1] = ai;
 }
@@ -1168,29 +1225,12 @@ __device__ __forceinline__ void chunk_sum2(const double *__restrict__ part, int6
     b = r[1][0];
 }
 
-// One work-group per panel: the near chunk partials, plus the panel average
-// of its segment's expansion (thread 0).  Only the chunks of the near list's
-// length hold partials (the grid is sized for its bound); the others would
-// add exact zeros.
-__global__ __launch_bounds__(kTile) void k_right_part_final(const double *__restrict__ part, int64_t nchunk,
-                                                            const int32_t *__restrict__ nlist, PanelsSoA pan,
-                                                            const double *__restrict__ Ss,
-                                                            const RhsSeg *__restrict__ segs,
-                                                            const int32_t *__restrict__ seg_of, double vinf_x,
-                                                            double vinf_y, double *__restrict__ R) {
-    __shared__ double S[2 * kLoc], inv[kLoc];
-    const int64_t i = blockIdx.x;
-    const int64_t used = ((int64_t)*nlist + kRhsChunk - 1) / kRhsChunk;
-    const int32_t sg = seg_of[i];
-    if (threadIdx.x < 2 * kLoc) S[threadIdx.x] = Ss[(int64_t)sg * 2 * kLoc + threadIdx.x];
-    if (threadIdx.x < kLoc) inv[threadIdx.x] = 1.0 / (double)(threadIdx.x + 1);
-    __syncthreads();
-    double y0, y1;
-    chunk_sum2(part, used < nchunk ? used : nchunk, pan.P, i, y0, y1);
-    if (threadIdx.x != 0) return;
-    const double cx = segs[sg].cx, cy = segs[sg].cy;
+// Panel i's entry from its near sums (y0, y1) and its segment's coefficients
+// S about (cx, cy); inv[k] = 1 / (k + 1).
+__device__ __forceinline__ double rhs_entry(const PanelsSoA &pan, int64_t i, double cx, double cy, const double *S,
+                                            const double *inv, double y0, double y1, double vinf_x, double vinf_y) {
     const double d0 = pan.rx[i] - pan.lx[i], d1 = pan.ry[i] - pan.ly[i];
-    const double mnog = 1 / (2 * kPi * (d0 * d0 + d1 * d1));
+    const double mnog = 1 / (2 * kPi * fma(d0, d0, d1 * d1));
     // W = sum_k (i S_k / 2 pi) Q_k / (k + 1), u = Re W, v = -Im W
     const double ar = pan.rx[i] - cx, ai = pan.ry[i] - cy;  // a = z_r - c_s
     const double br = pan.lx[i] - cx, bi = pan.ly[i] - cy;  // b = z_l - c_s
@@ -1213,7 +1253,86 @@ __global__ __launch_bounds__(kTile) void k_right_part_final(const double *__rest
     }
     // times i / (2 pi)
     const double uf = -wi / (2 * kPi), vf = -(wr / (2 * kPi));
-    R[i] = -((mnog * y0 + uf + vinf_x) * pan.tx[i] + (mnog * y1 + vf + vinf_y) * pan.ty[i]);
+    const double u = fma(mnog, y0, uf) + vinf_x, v = fma(mnog, y1, vf) + vinf_y;
+    return -fma(u, pan.tx[i], v * pan.ty[i]);
+}
+
+// One work-group per panel: the near chunk partials, plus the panel average
+// of its segment's expansion (thread 0).  Only the chunks of the near list's
+// length hold partials (the grid is sized for its bound); the others would
+// add exact zeros.
+__global__ __launch_bounds__(kTile) void k_right_part_final(const double *__restrict__ part, int64_t nchunk,
+                                                            const int32_t *__restrict__ nlist, PanelsSoA pan,
+                                                            const double *__restrict__ Ss,
+                                                            const RhsSeg *__restrict__ segs,
+                                                            const int32_t *__restrict__ seg_of, double vinf_x,
+                                                            double vinf_y, double *__restrict__ R) {
+    __shared__ double S[2 * kLoc], inv[kLoc];
+    const int64_t i = blockIdx.x;
+    const int64_t used = ((int64_t)*nlist + kRhsChunk - 1) / kRhsChunk;
+    const int32_t sg = seg_of[i];
+    if (threadIdx.x < 2 * kLoc) S[threadIdx.x] = Ss[(int64_t)sg * 2 * kLoc + threadIdx.x];
+    if (threadIdx.x < kLoc) inv[threadIdx.x] = 1.0 / (double)(threadIdx.x + 1);
+    __syncthreads();
+    double y0, y1;
+    chunk_sum2(part, used < nchunk ? used : nchunk, pan.P, i, y0, y1);
+    if (threadIdx.x != 0) return;
+    R[i] = rhs_entry(pan, i, segs[sg].cx, segs[sg].cy, S, inv, y0, y1, vinf_x, vinf_y);
+}
+
+// The three finals in one launch for at most kFewGroups work-groups of far
+// sources: every panel's work-group adds up the global coefficients (32 lanes
+// each, the tree of k_rhs_far_final without its levels of zeros), shifts them
+// to the panel's segment while another wave adds the near partials, and takes
+// the average.  200 panels, 2785 vortices: 4.5 + 5.1 + 5.8 us and two gaps -> 12.3
+// us.
+constexpr int64_t kFewGroups = 32;
+
+__global__ __launch_bounds__(256) void k_right_part_final_few(
+    const double *__restrict__ part, int64_t nchunk, const int32_t *__restrict__ nlist, PanelsSoA pan,
+    const double *__restrict__ spart, const double *__restrict__ spart_seg, Cnt cn_src, int64_t nfar, int64_t nseg,
+    double cx, double cy, const RhsSeg *__restrict__ segs, const int32_t *__restrict__ seg_of, double vinf_x,
+    double vinf_y, double *__restrict__ R) {
+    __shared__ double S[2 * kLoc], Ss[2 * kLoc], inv[kLoc], y[2];
+    const int64_t i = blockIdx.x;
+    const int tid = threadIdx.x, lane = tid & 63, wv = tid >> 6;
+    const int32_t sg = seg_of[i], nl = *nlist;
+    const RhsSeg G = segs[sg];
+    const int nblk = (int)rhs_groups(cn_src.get(), nfar), b = tid & 31;
+    double v[2 * kLoc / 8];
+#pragma unroll
+    for (int r = 0; r < 2 * kLoc / 8; ++r)
+        v[r] = b < nblk ? 0.0 + spart[(int64_t)b * 2 * kLoc + 8 * r + (tid >> 5)] : 0.0;
+#pragma unroll
+    for (int r = 0; r < 2 * kLoc / 8; ++r) {
+        for (int st = 16; st > 0; st >>= 1) v[r] += __shfl_xor(v[r], st, 32);
+        if (b == 0) S[8 * r + (tid >> 5)] = v[r];
+    }
+    __syncthreads();
+    if (wv == 0 && lane < kLoc) {
+        double ar, ai;
+        rhs_seg_coeff(spart_seg + (int64_t)sg * kSegBlocks * kLoc * 2, (int)rhs_groups(nl, nseg), S, G.cx - cx,
+                      G.cy - cy, lane, ar, ai);
+        Ss[2 * lane] = ar;
+        Ss[2 * lane + 1] = ai;
+    } else if (wv == 1) {
+        const int64_t used = ((int64_t)nl + kRhsChunk - 1) / kRhsChunk;
+        const bool on = lane < (used < nchunk ? used : nchunk);
+        double x0 = on ? 0.0 + part[((int64_t)lane * 2 + 0) * pan.P + i] : 0.0;
+        double x1 = on ? 0.0 + part[((int64_t)lane * 2 + 1) * pan.P + i] : 0.0;
+        for (int st = 32; st > 0; st >>= 1) {
+            x0 += __shfl_xor(x0, st, 64);
+            x1 += __shfl_xor(x1, st, 64);
+        }
+        if (lane == 0) {
+            y[0] = x0;
+            y[1] = x1;
+        }
+    } else if (wv == 2 && lane < kLoc) {
+        inv[lane] = 1.0 / (double)(lane + 1);
+    }
+    __syncthreads();
+    if (tid == 0) R[i] = rhs_entry(pan, i, G.cx, G.cy, Ss, inv, y[0], y[1], vinf_x, vinf_y);
 }
 
 // ---- A19: src/kernel.cu:1434-1475, split over source chunks ---------------
@@ -1498,27 +1617,43 @@ int launch_right_part(vx_case *c, Cnt cn_src, double vinf_x, double vinf_y) {
     }
     // pairs within 2 R_s of each segment
     if (mixed(c) && launch_pack_f32(c, cn_src)) return 1;
-    const dim3 gterms((unsigned)(K * (kSegTile / kRhsPG)), (unsigned)nchunk), gseg((unsigned)K, (unsigned)nchunk);
-    if (n_src <= kRhsSplitSrc) {
-        if (mixed(c))
-            hipLaunchKernelGGL(k_right_part_terms<float>, gterms, dim3(256), 0, st, c->gf.p, c->x.p, c->y.p,
-                               c->lists.p, nlist, c->pan, c->segs, c->partial.p);
-        else
-            hipLaunchKernelGGL(k_right_part_terms<double>, gterms, dim3(256), 0, st, c->g.p, c->x.p, c->y.p,
-                               c->lists.p, nlist, c->pan, c->segs, c->partial.p);
-    } else if (mixed(c)) {
-        hipLaunchKernelGGL(k_right_part_partial<float>, gseg, dim3(kSegTile), 0, st, c->xf.p, c->yf.p, c->gf.p, c->x.p,
-                           c->y.p, c->lists.p, nlist, c->pan, c->segs, c->partial.p);
-    } else {
-        hipLaunchKernelGGL(k_right_part_partial<double>, gseg, dim3(kSegTile), 0, st, c->x.p, c->y.p, c->g.p, c->x.p,
-                           c->y.p, c->lists.p, nlist, c->pan, c->segs, c->partial.p);
-    }
     // the global expansion (sources beyond 2 R_b), the segments' own
-    // sources, and each segment's total about c_s
+    // sources, and below each segment's total about c_s
     const int64_t nfar = rhs_groups(n_src, kFarBlocks), nseg = rhs_groups(n_src, kSegBlocks);
-    if (nfar > 0)
-        hipLaunchKernelGGL(k_rhs_expand, dim3((unsigned)(nfar + K * nseg)), dim3(256), 0, st, c->x.p, c->y.p, c->g.p,
-                           cn_src, cx, cy, rnear2, c->lists.p, nlist, c->segs, nfar, nseg, c->rhs_s.p, spart);
+    const RhsExpand E{c->x.p, c->y.p, c->g.p, cn_src, cx, cy, rnear2, c->lists.p, nlist, c->segs, nfar, nseg,
+                      c->rhs_s.p, spart};
+    const int64_t nx = K * (kSegTile / kRhsPG), nterm = nx * nchunk;
+    if (n_src <= kRhsOneSrc) {
+        const dim3 grid((unsigned)(nterm + nfar + K * nseg));
+        if (mixed(c))
+            hipLaunchKernelGGL(k_right_part_all<float>, grid, dim3(256), 0, st, c->gf.p, c->pan, nx, nterm,
+                               c->partial.p, E);
+        else
+            hipLaunchKernelGGL(k_right_part_all<double>, grid, dim3(256), 0, st, c->g.p, c->pan, nx, nterm,
+                               c->partial.p, E);
+    } else {
+        const dim3 gterms((unsigned)nx, (unsigned)nchunk), gseg((unsigned)K, (unsigned)nchunk);
+        if (n_src <= kRhsSplitSrc && mixed(c))
+            hipLaunchKernelGGL(k_right_part_terms<float>, gterms, dim3(256), 0, st, c->gf.p, c->pan, c->partial.p, E);
+        else if (n_src <= kRhsSplitSrc)
+            hipLaunchKernelGGL(k_right_part_terms<double>, gterms, dim3(256), 0, st, c->g.p, c->pan, c->partial.p, E);
+        else if (mixed(c))
+            hipLaunchKernelGGL(k_right_part_partial<float>, gseg, dim3(kSegTile), 0, st, c->xf.p, c->yf.p, c->gf.p,
+                               c->x.p, c->y.p, c->lists.p, nlist, c->pan, c->segs, c->partial.p);
+        else
+            hipLaunchKernelGGL(k_right_part_partial<double>, gseg, dim3(kSegTile), 0, st, c->x.p, c->y.p, c->g.p,
+                               c->x.p, c->y.p, c->lists.p, nlist, c->pan, c->segs, c->partial.p);
+        hipLaunchKernelGGL(k_rhs_expand, dim3((unsigned)(nfar + K * nseg)), dim3(256), 0, st, E);
+    }
+    VX_CHECK(hipGetLastError());
+    if (nfar <= kFewGroups) {
+        static_assert(kFewGroups * 256 <= 64 * kRhsChunk, "the near chunks fit a wave");
+        hipLaunchKernelGGL(k_right_part_final_few, dim3((unsigned)P), dim3(256), 0, st, c->partial.p, nchunk, nlist,
+                           c->pan, c->rhs_s.p, spart, cn_src, nfar, nseg, cx, cy, c->segs, c->seg_of, vinf_x, vinf_y,
+                           c->rp.p);
+        VX_CHECK(hipGetLastError());
+        return 0;
+    }
     hipLaunchKernelGGL(k_rhs_far_final, dim3(2 * kLoc), dim3(256), 0, st, c->rhs_s.p, cn_src, nfar, S);
     hipLaunchKernelGGL(k_rhs_seg_final, dim3((unsigned)K), dim3(64), 0, st, spart, S, cx, cy, c->segs, nlist, nseg, Ss);
     VX_CHECK(hipGetLastError());

@@ -192,6 +192,31 @@ __global__ __launch_bounds__(256) void k_diffusion_wall(const double *__restrict
     }
 }
 
+// The wall pass on the main stream without a list, for bounds up to
+// kScanMax: wave w looks at targets w, w + nw, ... (at most 64) and takes those in
+// the box in turn.  2785 vortices: 5.1 us for the list and 9.9 for its targets ->
+// 10.5 us.
+constexpr int64_t kScanMax = 32768;
+
+template <typename T>
+__global__ __launch_bounds__(256) void k_wall_scan(InWallBox pred, Cnt cn, const double *__restrict__ d, PanelsSoA pan,
+                                                   double nu, int32_t npts, double *__restrict__ u,
+                                                   double *__restrict__ v) {
+    __shared__ WallLds<T> lds[4];
+    const int lane = threadIdx.x & 63;
+    const int64_t n = cn.get(), nw = (int64_t)gridDim.x * 4, w = (int64_t)blockIdx.x * 4 + (threadIdx.x >> 6);
+    const int64_t mine = w + nw * lane;
+    for (uint64_t m = __ballot(mine < n && pred((int32_t)mine)); m; m &= m - 1) {
+        const int64_t i = w + nw * __builtin_ctzll(m);
+        double II0, II30, II31;
+        wave_wall<T>(pan, lane, pred.x[i], pred.y[i], (T)d[i], npts, lds[threadIdx.x >> 6], II0, II30, II31);
+        if (lane == 0) {
+            u[i] += nu * II30 / II0;
+            v[i] += nu * II31 / II0;
+        }
+    }
+}
+
 __global__ __launch_bounds__(256) void k_wall_add(const int32_t *__restrict__ list, const int32_t *__restrict__ cnt,
                                                   const double *__restrict__ wst, double *__restrict__ u,
                                                   double *__restrict__ v) {
@@ -212,9 +237,20 @@ static int wall_pass(vx_case *c, Cnt cn_tgt, hipStream_t st) {
     if (c->wlist.ensure((size_t)n_tgt, c->stream) || c->dcount.ensure(16, c->stream) ||
         (!ADD && c->wstage.ensure((size_t)(2 * n_tgt), c->stream)))
         return 1;
-    int32_t *cnt = (int32_t *)(c->dcount.p + 5);
     const int32_t npts = (int32_t)std::clamp<int64_t>(c->prm.n_of_points, 0, 1 << 24);
     const InWallBox pred{c->x.p, c->y.p, c->wall_box};
+    if (ADD && n_tgt <= kScanMax) {
+        const dim3 grid((unsigned)std::min<int64_t>(1024, (n_tgt + 3) / 4));
+        if (c->prm.precision == VX_PREC_MIXED)
+            hipLaunchKernelGGL(k_wall_scan<float>, grid, dim3(256), 0, st, pred, cn_tgt, c->d.p, c->pan, c->prm.nu, npts,
+                               c->u.p, c->v.p);
+        else
+            hipLaunchKernelGGL(k_wall_scan<double>, grid, dim3(256), 0, st, pred, cn_tgt, c->d.p, c->pan, c->prm.nu, npts,
+                               c->u.p, c->v.p);
+        VX_CHECK(hipGetLastError());
+        return 0;
+    }
+    int32_t *cnt = (int32_t *)(c->dcount.p + 5);
     if (c->wtmp.ensure((size_t)prim::tiles_of(n_tgt) + 1, c->stream)) return 1;
     VX_CHECK(prim::select_flags(prim::pred_flag(pred, cn_tgt), n_tgt, prim::WriteIndex{c->wlist.p}, c->wtmp.p, cnt,
                                 st));
