@@ -595,7 +595,7 @@ def main():
         "roofline": {"bound": "valu", "achieved": achieved, "peak": PEAK_FP32, "unit": "TFLOP/s",
                      "frac": achieved / PEAK_FP32, "traffic": traffic_from_profiles(kname),
                      "kernel": kname + {"k_tree_bs": f"<float,{ORDER}>", "k_tree_diffusion": "<float>"}.get(
-                         kname, "<float,4>"),
+                         kname, "<float,1>"),
                      "pipe": "VALU FP32", "flop_per_launch": kflop,
                      "avg_launch_ms": kms},
         "cpu_baseline": cpu and {k: cpu[k] for k in ("value", "unit", "cores", "kind", "sample",
