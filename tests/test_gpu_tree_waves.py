@@ -1,9 +1,10 @@
 """The tree's velocity stages with several waves a target group (diffusion) or
-bucket (FP64 Biot-Savart up to 14336 buckets): edges of the groups, pairs
-around the diffusion's threshold, and counts on both sides of the limit.
+bucket (Biot-Savart up to 14336 buckets in FP64, 8192 in mixed precision):
+edges of the groups, pairs around the diffusion's threshold, and counts on both
+sides of the limits.
 Tolerances as stated in test_gpu_tree.py: diffusion FP64 1e-9, mixed 1e-3 (one
 sign of circulation, so the weight sums do not cancel); Biot-Savart FP64 with
-32 terms 1e-8."""
+32 terms 1e-8, mixed with 16 terms 3e-4 (nearest-3 distance 1e-4)."""
 import numpy as np
 import pytest
 
@@ -59,3 +60,28 @@ def test_biot_savart_around_the_split_limit(n):
     c.close()
     for a, b in ((u[k], up), (v[k], vp)):
         assert np.max(np.abs(a - b)) <= 1e-8 * np.max(np.abs(b))
+
+
+@pytest.mark.parametrize("n", [250000, 700000])
+def test_biot_savart_mixed_around_the_split_limit(n):
+    """The same for the mixed tree; the nearest-3 distances against the FP64
+    tree's, whose searches are exact."""
+    rng = np.random.default_rng(n)
+    x, y = rng.uniform(0.7, 9.5, n), rng.uniform(-4.0, 4.0, n)
+    g = rng.uniform(-0.004, 0.004, n)
+    pan = geo.circle(64, 0.5)
+    res = {}
+    for prec in (VX_PREC_MIXED, VX_PREC_F64):
+        c = Case(make_params(pan, precision=prec, ve_size=0.004, order=16), pan)
+        c.set_state(x, y, g)
+        c.tree_biot_savart((n + 31) // 32 * 32, (0.0, 0.0))
+        res[prec] = c.velocity(n)
+        assert (c.tree_stats()["leaves"] > 8192) == (n == 700000)
+        if prec == VX_PREC_F64:
+            k = np.arange(0, n, 1000)
+            up, vp = c.velocity_probe(x[k], y[k], (0.0, 0.0))
+        c.close()
+    u, v, d = res[VX_PREC_MIXED]
+    for a, b in ((u[k], up), (v[k], vp)):
+        assert np.max(np.abs(a - b)) <= 3e-4 * np.max(np.abs(b))
+    np.testing.assert_allclose(d, res[VX_PREC_F64][2], rtol=1e-4, atol=0)

@@ -1411,9 +1411,12 @@ constexpr int kFarQ = 512;     // FP32: far nodes queued per wave before any M2L
 // fourth far node and near leaf: one each are three waves a SIMD at 131103
 // vortices, and the longest chain sets the time (0.54 -> 0.42 ms; 500000: 1.53
 // -> 1.46).  Each walks the tree by itself, which costs more than the balance
-// gives where there are waves enough (2^20: 2.89 -> 3.11).  FP32's far
-// nodes are translated 16 at a time, which wants them together.
-constexpr int64_t kBsSplit = 14336;
+// gives where there are waves enough (2^20: 2.89 -> 3.11).  FP32's far nodes
+// are translated 16 at a time, which wants them together: its first wave takes
+// them all, the near leaves are dealt over the four (66000 vortices: 142 ->
+// 120 us, 131103: 228 -> 177, 262177: 305 -> 290, 524288 the same, 2^20: 868
+// -> 1030, hence kBsSplitF).
+constexpr int64_t kBsSplit = 14336, kBsSplitF = 8192;
 
 template <typename T, int ORDER, int STRIDE, int S>
 __device__ __forceinline__ void bs_wave(const TreeDev &t, double theta, double eps, double vinf_x, double vinf_y,
@@ -1425,7 +1428,7 @@ __device__ __forceinline__ void bs_wave(const TreeDev &t, double theta, double e
                                         unsigned long long &cm2l) {
     using PM = PairMath<T>;
     constexpr bool F32 = sizeof(T) == 4;
-    static_assert(S == 1 || (S == 4 && !F32), "a work-group holds whole groups of waves");
+    static_assert(S == 1 || S == 4, "a work-group holds whole groups of waves");
     __shared__ Src4T<T> lds_all[4][kLeaf];
     __shared__ int32_t fq_all[4][kFarQ];  // FP32: far nodes waiting for M2L
     __shared__ int32_t stk_all[4][kBsStack];
@@ -1551,8 +1554,10 @@ __device__ __forceinline__ void bs_wave(const TreeDev &t, double theta, double e
         const uint64_t fm = __ballot(isfar);
         if (part == 0) nfar += __popcll(fm);
         if constexpr (F32) {
-            if (isfar) fq[nq + __popcll(fm & ((1ull << lane) - 1))] = node;
-            nq += __popcll(fm);
+            if (part == 0) {  // the far nodes stay together
+                if (isfar) fq[nq + __popcll(fm & ((1ull << lane) - 1))] = node;
+                nq += __popcll(fm);
+            }
         } else {
             // M2P: S = (1/D) sum_k b_k (R/D)^k, D = z - c_node; u += Im S, v += Re S
             auto m2p = [&](int fnode) {
@@ -1629,27 +1634,32 @@ __device__ __forceinline__ void bs_wave(const TreeDev &t, double theta, double e
     su += (double)fu;
     sv += (double)fv;
     if constexpr (S > 1) {  // the waves' shares, in wave order
-        __shared__ T sh_[S - 1][7][64];
+        __shared__ double sh_s[S - 1][2][64];
+        __shared__ T sh_m[S - 1][5][64];
         if (part > 0) {
-            T(&o)[7][64] = sh_[part - 1];
-            o[0][lane] = su;
-            o[1][lane] = sv;
-            o[2][lane] = m0;
-            o[3][lane] = m1;
-            o[4][lane] = m2;
-            o[5][lane] = m3;
-            o[6][lane] = farmin;
+            sh_s[part - 1][0][lane] = su;
+            sh_s[part - 1][1][lane] = sv;
+            T(&o)[5][64] = sh_m[part - 1];
+            o[0][lane] = m0;
+            o[1][lane] = m1;
+            o[2][lane] = m2;
+            o[3][lane] = m3;
+            o[4][lane] = farmin;
         }
         cpairs = (unsigned long long)(npairs * nvalid);
         __syncthreads();
         if (part > 0) return;
 #pragma unroll
         for (int q = 0; q < S - 1; ++q) {
-            const T(&o)[7][64] = sh_[q];
-            su += o[0][lane];
-            sv += o[1][lane];
-            keep4x4(m0, m1, m2, m3, o[2][lane], o[3][lane], o[4][lane], o[5][lane]);
-            farmin = fmin(farmin, o[6][lane]);
+            const T(&o)[5][64] = sh_m[q];
+            su += sh_s[q][0][lane];
+            sv += sh_s[q][1][lane];
+            if constexpr (F32) {
+                for (int e = 0; e < 4; ++e) near4_insert<T>(o[e][lane], m0, m1, m2, m3);
+            } else {
+                keep4x4(m0, m1, m2, m3, o[0][lane], o[1][lane], o[2][lane], o[3][lane]);
+                farmin = fmin(farmin, o[4][lane]);
+            }
         }
     }
     // the target's shares: sums added in the same order on each of its
@@ -3014,7 +3024,7 @@ int launch_tree_biot_savart(vx_case *c, int64_t s, double vinf_x, double vinf_y)
     if (t.sd.ensure((size_t)t.m, st)) return 1;
     const TreeDev tv = view(t);
     const bool mixed = c->prm.precision == VX_PREC_MIXED;
-    const bool split = !mixed && t.nleaf <= kBsSplit;
+    const bool split = t.nleaf <= (mixed ? kBsSplitF : kBsSplit);
     const int64_t wgs = split ? t.nleaf : (t.nleaf + 3) / 4;
     const unsigned lb = (unsigned)(wgs + 7) / 8 * 8;  // padded for xcd_block()
     const double th = theta_of(c), eps = c->prm.ve_size;
@@ -3031,7 +3041,9 @@ int launch_tree_biot_savart(vx_case *c, int64_t s, double vinf_x, double vinf_y)
         VX_TREE_BS(T_, 20, 32, S_);  \
     else                             \
         VX_TREE_BS(T_, 16, 16, S_)
-    if (mixed) {
+    if (mixed && split) {
+        VX_TREE_BS_ORDERS(float, 4);
+    } else if (mixed) {
         VX_TREE_BS_ORDERS(float, 1);
     } else if (split) {
         VX_TREE_BS_ORDERS(double, 4);
