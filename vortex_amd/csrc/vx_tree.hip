@@ -69,6 +69,7 @@ struct TreeBufs {
     DBuf<float> fx, fy, fg;
     DBuf<double4> nbb, part, cbox, ftgt;
     DBuf<int2> fpairs;
+    DBuf<uint64_t> fmask;
     DBuf<double2> cd;
     DBuf<float2> cf;
     DBuf<NodeRec> rec;
@@ -2371,8 +2372,8 @@ __global__ void k_sd_gather(const int32_t *__restrict__ perm, const double *__re
 // box each; k_far_pairs lists the (target, chunk) pairs whose boxes meet, and
 // one wave per pair tests the chunk's 64 bucket boxes at once, then sums the
 // buckets in range with one source per lane, eight buckets' loads in flight.
-// Partial sums go to part[(chunk * 3 + q) * H + k] (zero for pairs not
-// listed).
+// Partial sums go to part[(chunk * 3 + q) * H + k]; fmask[(chunk / 64) * H + k]
+// holds a bit for each chunk listed with target k.
 template <typename T>
 __device__ __forceinline__ void far_load(const TreeDev &t, int64_t j0, int cnt, double bcx, double bcy, int lane,
                                          double ax, double ay, T &dx, T &dy, T &g) {
@@ -2413,52 +2414,58 @@ __global__ __launch_bounds__(256) void k_chunk_box(TreeDev t, int64_t nchunk, do
     if (lane == 0) cbox[ch] = r;
 }
 
-// One wave per listed target: the chunks whose box lies within its radius,
-// appended as (target, chunk) pairs, one atomic per wave and 64 chunks.
-__device__ void far_pairs_of(const TreeDev &t, const int32_t *__restrict__ list, int64_t k, int64_t nchunk,
-                             const double4 *__restrict__ cbox, double cut, const double *__restrict__ dd,
-                             int2 *__restrict__ pairs, unsigned long long *__restrict__ npairs,
-                             double4 *__restrict__ ftgt, int lane) {
-    const int64_t ti = list[k];
-    const double di = dd[t.perm[ti]];
-    const double R2 = (cut * di) * (cut * di);
-    const double ax = t.sx[ti], ay = t.sy[ti];
-    if (lane == 0) ftgt[k] = make_double4(ax, ay, di, 0.0);  // for the pair kernel
-    for (int64_t c0 = 0; c0 < nchunk; c0 += 64) {
-        const int64_t ch = c0 + lane;
-        const bool need = ch < nchunk && box_d2(cbox[ch], ax, ay) < R2;
-        const uint64_t m = __ballot(need);
-        if (m == 0) continue;
-        unsigned long long base = 0;
-        if (lane == 0) base = atomicAdd(npairs, (unsigned long long)__popcll(m));
-        base = __shfl(base, 0, 64);
-        if (need) pairs[base + __popcll(m & ((1ull << lane) - 1))] = make_int2((int)k, (int)ch);
-    }
-}
-
+// One wave per 64 listed targets and 64 chunks: the chunks whose box lies
+// within each target's radius, appended as (target, chunk) pairs, a chunk's
+// targets together (their waves then read the same buckets), with one atomic
+// for all of them.  One atomic and one chain of loads per target took 870 us
+// for the 78993 listed of 100000 vortices in mixed precision, more than their
+// sums (290); now 23.
 __global__ __launch_bounds__(256) void k_far_pairs(TreeDev t, const int32_t *__restrict__ list,
                                                    const unsigned long long *__restrict__ cnt, int64_t nchunk,
                                                    const double4 *__restrict__ cbox, double cut,
                                                    const double *__restrict__ dd, int2 *__restrict__ pairs,
                                                    unsigned long long *__restrict__ npairs,
-                                                   double4 *__restrict__ ftgt) {
+                                                   double4 *__restrict__ ftgt, uint64_t *__restrict__ fmask) {
     const int lane = threadIdx.x & 63;
     const int64_t H = far_count(cnt, t.fcap);
-    for (int64_t k = (int64_t)blockIdx.x * 4 + (threadIdx.x >> 6); k < H; k += (int64_t)gridDim.x * 4)
-        far_pairs_of(t, list, k, nchunk, cbox, cut, dd, pairs, npairs, ftgt, lane);
+    const int64_t nwin = (nchunk + 63) / 64, units = (H + 63) / 64 * nwin;
+    const int64_t w0 = (int64_t)blockIdx.x * 4 + __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+    for (int64_t w = w0; w < units; w += (int64_t)gridDim.x * 4) {
+        const int64_t win = w % nwin, k = w / nwin * 64 + lane;
+        const bool ok = k < H;
+        double ax = 0.0, ay = 0.0, R2 = -1.0;
+        if (ok) {
+            const int64_t ti = list[k];
+            const double di = dd[t.perm[ti]];
+            R2 = (cut * di) * (cut * di);
+            ax = t.sx[ti];
+            ay = t.sy[ti];
+            if (win == 0) ftgt[k] = make_double4(ax, ay, di, 0.0);  // for the pair kernel
+        }
+        const int64_t c0 = win * 64;
+        const int nc = (int)min((int64_t)64, nchunk - c0);
+        uint64_t mine = 0;
+#pragma unroll 4
+        for (int q = 0; q < nc; ++q) mine |= (uint64_t)(box_d2(cbox[c0 + q], ax, ay) < R2) << q;
+        int total = __popcll(mine);
+        for (int o = 32; o > 0; o >>= 1) total += __shfl_xor(total, o, 64);
+        if (ok) fmask[win * H + k] = mine;
+        if (total == 0) continue;
+        unsigned long long base = 0;
+        if (lane == 0) base = atomicAdd(npairs, (unsigned long long)total);
+        base = __shfl(base, 0, 64);
+        for (int q = 0; q < nc; ++q) {
+            const bool need = (mine >> q) & 1u;
+            const uint64_t m = __ballot(need);
+            if (need) pairs[base + __popcll(m & ((1ull << lane) - 1))] = make_int2((int)k, (int)(c0 + q));
+            base += __popcll(m);
+        }
+    }
 }
 
 // Zero the counters a[q] whose bit q is set in mask.
 __global__ void k_zero_u64(unsigned long long *__restrict__ a, unsigned mask) {
     if (threadIdx.x < 32 && ((mask >> threadIdx.x) & 1u)) a[threadIdx.x] = 0ull;
-}
-
-// Zero the partials of the listed targets (grid-stride; H on the device).
-__global__ void k_far_zero(double *__restrict__ a, int64_t nchunk, const unsigned long long *__restrict__ cnt,
-                           int64_t cap) {
-    const int64_t count = 3 * nchunk * far_count(cnt, cap);
-    for (int64_t t = (int64_t)blockIdx.x * blockDim.x + threadIdx.x; t < count; t += (int64_t)gridDim.x * blockDim.x)
-        a[t] = 0.0;
 }
 
 template <typename T>
@@ -2536,43 +2543,79 @@ __global__ __launch_bounds__(256) void k_diff_far(TreeDev t, const double4 *__re
     block_count_add(cp, 0ull, cnt, nullptr);
 }
 
-// One work-group per listed target: the chunk partials summed in a fixed
-// order (strided per thread, then a tree in LDS), then the velocity update.
-__device__ void far_final_of(const TreeDev &t, const int32_t *__restrict__ list, int64_t H, int64_t k,
-                             int64_t nchunk, const double *__restrict__ part, const double *__restrict__ dd,
-                             double nu, double *__restrict__ u, double *__restrict__ v) {
-    __shared__ double r[3][256];
-    double a2x = 0.0, a2y = 0.0, a1 = 0.0;
-    for (int64_t ch = threadIdx.x; ch < nchunk; ch += 256) {
-        a2x += part[(ch * 3 + 0) * H + k];
-        a2y += part[(ch * 3 + 1) * H + k];
-        a1 += part[(ch * 3 + 2) * H + k];
-    }
-    r[0][threadIdx.x] = a2x;
-    r[1][threadIdx.x] = a2y;
-    r[2][threadIdx.x] = a1;
-    __syncthreads();
-    for (int st = 128; st > 0; st >>= 1) {
-        if ((int)threadIdx.x < st)
-            for (int q = 0; q < 3; ++q) r[q][threadIdx.x] += r[q][threadIdx.x + st];
-        __syncthreads();
-    }
-    if (threadIdx.x != 0) return;
-    const int32_t i = t.perm[list[k]];
-    if (fabs(r[2][0]) > 1e-5) {
-        const double di = dd[i];
-        u[i] += nu * r[0][0] / (r[2][0] * di);
-        v[i] += nu * r[1][0] / (r[2][0] * di);
-    }
-}
+// Sixteen listed targets a work-group, sixteen threads each: the partials of
+// the target's listed chunks, then the velocity update.  Thread j takes chunks
+// j, j + 16, ..., all loads in flight, and the sum is the tree over 256 slots
+// (chunk mod 256) whatever the count, so a chunk not listed is an exact zero
+// and its partial is neither cleared before nor read.  One work-group a target
+// left most threads idle and read a word of each line: 146 -> 54 us for
+// 78993 targets and 37 chunks.
+constexpr int kFarTgts = 16;
 
 __global__ __launch_bounds__(256) void k_diff_far_final(TreeDev t, const int32_t *__restrict__ list,
                                                         const unsigned long long *__restrict__ cnt,
-                                                        int64_t nchunk, const double *__restrict__ part,
+                                                        int64_t nchunk, const uint64_t *__restrict__ fmask,
+                                                        const double *__restrict__ part,
                                                         const double *__restrict__ dd, double nu,
                                                         double *__restrict__ u, double *__restrict__ v) {
+    constexpr int kPer = 256 / kFarTgts;  // slots per thread
+    __shared__ double r[3][kFarTgts][kFarTgts + 1];
     const int64_t H = far_count(cnt, t.fcap);
-    for (int64_t k = blockIdx.x; k < H; k += gridDim.x) far_final_of(t, list, H, k, nchunk, part, dd, nu, u, v);
+    const int kt = threadIdx.x % kFarTgts, j = threadIdx.x / kFarTgts;
+    for (int64_t k0 = (int64_t)blockIdx.x * kFarTgts; k0 < H; k0 += (int64_t)gridDim.x * kFarTgts) {
+        const int64_t k = k0 + kt;
+        int32_t i = 0;
+        double di = 1.0, ui = 0.0, vi = 0.0;
+        if (j == 0 && k < H) {
+            i = t.perm[list[k]];
+            di = dd[i];
+            ui = u[i];
+            vi = v[i];
+        }
+        double a[3][kPer] = {};
+        for (int64_t c0 = 0; c0 < nchunk; c0 += 256) {
+#pragma unroll
+            for (int g = 0; g < 4; ++g) {  // a mask word's chunks
+                const int64_t w0 = c0 + g * 64;
+                if (w0 >= nchunk) break;
+                const uint64_t m = k < H ? fmask[(w0 >> 6) * H + k] >> j : 0;
+                double x[3][kPer / 4];
+#pragma unroll
+                for (int q = 0; q < kPer / 4; ++q)
+#pragma unroll
+                    for (int e = 0; e < 3; ++e)  // an unlisted chunk's load goes to the first word
+                        x[e][q] = part[(m >> (q * kFarTgts)) & 1u ? ((w0 + q * kFarTgts + j) * 3 + e) * H + k : 0];
+#pragma unroll
+                for (int q = 0; q < kPer / 4; ++q)
+#pragma unroll
+                    for (int e = 0; e < 3; ++e)
+                        a[e][g * (kPer / 4) + q] += (m >> (q * kFarTgts)) & 1u ? x[e][q] : 0.0;
+            }
+        }
+#pragma unroll
+        for (int st = kPer / 2; st > 0; st >>= 1)
+#pragma unroll
+            for (int q = 0; q < st; ++q)
+#pragma unroll
+                for (int e = 0; e < 3; ++e) a[e][q] += a[e][q + st];
+#pragma unroll
+        for (int e = 0; e < 3; ++e) r[e][j][kt] = a[e][0];
+        __syncthreads();
+        if (threadIdx.x < 64) {  // threads j < 4: j and j + 8, then j and j + 4, the rest over the lanes
+            double f[3];
+#pragma unroll
+            for (int e = 0; e < 3; ++e) {
+                f[e] = (r[e][j][kt] + r[e][j + 8][kt]) + (r[e][j + 4][kt] + r[e][j + 12][kt]);
+                f[e] += __shfl_down(f[e], 2 * kFarTgts, 64);
+                f[e] += __shfl_down(f[e], kFarTgts, 64);
+            }
+            if (j == 0 && k < H && fabs(f[2]) > 1e-5) {
+                u[i] = ui + nu * f[0] / (f[2] * di);
+                v[i] = vi + nu * f[1] / (f[2] * di);
+            }
+        }
+        __syncthreads();  // r is written again
+    }
 }
 
 // Slots left out of the tree (dead and far from the box) see no neighbour.
@@ -2606,7 +2649,7 @@ void tree_release(vx_case *c) {
     t.bstart.release(); t.bscan.release(); t.upper.release(); t.uscan.release(); t.toplist.release();
     t.sx.release(); t.sy.release(); t.sg.release(); t.ncx.release(); t.ncy.release(); t.nr.release();
     t.fx.release(); t.fy.release(); t.fg.release(); t.nbb.release(); t.part.release(); t.rec.release();
-    t.cbox.release(); t.fpairs.release(); t.ftgt.release();
+    t.cbox.release(); t.fpairs.release(); t.fmask.release(); t.ftgt.release();
     t.gcs.release(); t.gcs2.release(); t.gflag.release(); t.gscan.release(); t.gfirst.release(); t.pcount.release(); t.arr.release(); t.sizes.release();
     t.cd.release(); t.cf.release(); t.cnt.release(); t.tmp.release(); t.tmp2.release(); t.fbr2.release(); t.hpart.release();
     t.sd.release();
@@ -3091,7 +3134,8 @@ int tree_diffusion_pre(vx_case *c) {
     const int64_t grow = std::min<int64_t>({last + last / 4, t.m, budget});
     t.fcap = std::max<int64_t>({kFarCap, t.m / 16, grow});
     if (t.hpart.ensure((size_t)(3 * nchunk * t.fcap), st) || t.cbox.ensure((size_t)nchunk, st) ||
-        t.fpairs.ensure((size_t)(nchunk * t.fcap), st) || t.ftgt.ensure((size_t)t.fcap, st) ||
+        t.fpairs.ensure((size_t)(nchunk * t.fcap), st) ||
+        t.fmask.ensure((size_t)((nchunk + 63) / 64 * t.fcap), st) || t.ftgt.ensure((size_t)t.fcap, st) ||
         t.sd.ensure((size_t)t.m, st))
         return 1;
     // pairs, overflow, far targets, far (target, chunk) pairs; [4] is the
@@ -3120,19 +3164,18 @@ int tree_diffusion_far(vx_case *c, hipStream_t st) {
     unsigned long long *cnt = t.cnt.p + 4;
     // all counts stay on the device (grid-stride kernels sized for the list's capacity)
     const int64_t nchunk = (t.nleaf + 63) / 64;
-    hipLaunchKernelGGL(k_far_zero, dim3(512), dim3(256), 0, st, t.hpart.p, nchunk, cnt, t.fcap);
     VX_CHECK(hipMemcpyAsync(t.h_far, cnt + 2, sizeof(unsigned long long), hipMemcpyDeviceToHost, st));
     hipLaunchKernelGGL(k_chunk_box, dim3((unsigned)((nchunk + 3) / 4)), dim3(256), 0, st, tv, nchunk, t.cbox.p);
-    hipLaunchKernelGGL(k_far_pairs, dim3(256), dim3(256), 0, st, tv, t.fb.p, cnt, nchunk, t.cbox.p, cut, c->d.p,
-                       t.fpairs.p, cnt + 3, t.ftgt.p);
+    hipLaunchKernelGGL(k_far_pairs, dim3(1024), dim3(256), 0, st, tv, t.fb.p, cnt, nchunk, t.cbox.p, cut, c->d.p,
+                       t.fpairs.p, cnt + 3, t.ftgt.p, t.fmask.p);
     if (mixed)
         hipLaunchKernelGGL(k_diff_far<float>, dim3(4096), dim3(256), 0, st, tv, t.ftgt.p, t.fpairs.p, cnt + 3, cut,
                            thr2, t.hpart.p, cnt);
     else
         hipLaunchKernelGGL(k_diff_far<double>, dim3(4096), dim3(256), 0, st, tv, t.ftgt.p, t.fpairs.p, cnt + 3, cut,
                            thr2, t.hpart.p, cnt);
-    hipLaunchKernelGGL(k_diff_far_final, dim3(1024), dim3(256), 0, st, tv, t.fb.p, cnt, nchunk, t.hpart.p, c->d.p,
-                       c->prm.nu, c->u.p, c->v.p);
+    hipLaunchKernelGGL(k_diff_far_final, dim3(1024), dim3(256), 0, st, tv, t.fb.p, cnt, nchunk, t.fmask.p, t.hpart.p,
+                       c->d.p, c->prm.nu, c->u.p, c->v.p);
     VX_CHECK(hipGetLastError());
     return 0;
 }
