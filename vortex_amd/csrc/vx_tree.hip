@@ -835,15 +835,20 @@ __device__ bool build_sub_lds(int32_t r, Desc desc, SubLds<ORDER> &L, const int3
 // kCut - 1 internal nodes).  At 16 coefficients the subtree stays in LDS
 // until it is complete (SubLds), so a level waits on LDS rather than on
 // global memory; at 32 it is built through global memory (build_levels).
+// Its time is that of its chain of levels, the work-groups being few: with 16
+// waves each level of up to 64 nodes is one round (four waves had sixteen
+// nodes a round: 57 -> 39 us at 262177 vortices).
+constexpr int kUpperWaves = 16;
+
 template <int ORDER>
-__global__ __launch_bounds__(256) void k_upper_local(const int32_t *__restrict__ cut,
+__global__ __launch_bounds__(64 * kUpperWaves) void k_upper_local(const int32_t *__restrict__ cut,
                                                      const unsigned long long *__restrict__ ncut,
                                                      int64_t nb, const int32_t *__restrict__ child0,
                                                      const int32_t *__restrict__ child1, double *__restrict__ ncx,
                                                      double *__restrict__ ncy, double *__restrict__ nr,
                                                      double4 *__restrict__ nbb, double2 *__restrict__ cd,
                                                      float2 *__restrict__ cf) {
-    __shared__ double2 ws_all[4][64];
+    __shared__ double2 ws_all[kUpperWaves][64];
     __shared__ double bin[ORDER][ORDER];
     fill_binomials<ORDER>(bin);
     double2 *ws = ws_all[threadIdx.x >> 6] + ((threadIdx.x & 63) / ORDER) * ORDER;
@@ -853,7 +858,7 @@ __global__ __launch_bounds__(256) void k_upper_local(const int32_t *__restrict__
         for (int w = blockIdx.x; w < n; w += gridDim.x) {
             const int32_t r = cut[w];
             if (r < nb) continue;  // a bucket: nothing to build (the same for every thread)
-            (void)build_sub_lds<ORDER, 4>(r, IsInternal{nb}, L, child0, child1, ncx, ncy, nr, nbb, cd, cf, ws, bin);
+            (void)build_sub_lds<ORDER, kUpperWaves>(r, IsInternal{nb}, L, child0, child1, ncx, ncy, nr, nbb, cd, cf, ws, bin);
         }
     } else {
         __shared__ int32_t lst[kCut];
@@ -862,7 +867,7 @@ __global__ __launch_bounds__(256) void k_upper_local(const int32_t *__restrict__
         for (int w = blockIdx.x; w < n; w += gridDim.x) {
             const int32_t r = cut[w];
             if (r < nb) continue;  // a bucket: nothing to build (the same for every thread)
-            build_levels<ORDER, 4>(r, IsInternal{nb}, lst, lev, &ntot, child0, child1, ncx, ncy, nr, nbb, cd, cf,
+            build_levels<ORDER, kUpperWaves>(r, IsInternal{nb}, lst, lev, &ntot, child0, child1, ncx, ncy, nr, nbb, cd, cf,
                                    ws, bin);
         }
     }
@@ -2822,7 +2827,7 @@ static int tree_build_b(vx_case *c, hipStream_t st, Births B) {
         hipLaunchKernelGGL(k_bucket_build<32>, dim3(lb), dim3(256), 0, st, t.sx.p, t.sy.p, t.sg.p, nb, t.first.p,
                            t.count.p, t.fx.p, t.fy.p, t.fg.p, t.ncx.p, t.ncy.p, t.nr.p, t.nbb.p, t.child0.p,
                            t.child1.p, t.cd.p, t.cf.p);
-        hipLaunchKernelGGL(k_upper_local<32>, dim3(gc), dim3(256), 0, st, cut, ncut, nb, t.child0.p, t.child1.p,
+        hipLaunchKernelGGL(k_upper_local<32>, dim3(gc), dim3(64 * kUpperWaves), 0, st, cut, ncut, nb, t.child0.p, t.child1.p,
                            t.ncx.p, t.ncy.p, t.nr.p, t.nbb.p, t.cd.p, t.cf.p);
         hipLaunchKernelGGL(k_upper_top<32>, dim3(1), dim3(1024), 0, st, t.root, nb, m, t.first.p, t.count.p,
                            t.bscan.p, t.toplist.p, t.child0.p, t.child1.p, t.ncx.p, t.ncy.p, t.nr.p, t.nbb.p, t.cd.p,
@@ -2831,7 +2836,7 @@ static int tree_build_b(vx_case *c, hipStream_t st, Births B) {
         hipLaunchKernelGGL(k_bucket_build<16>, dim3(lb), dim3(256), 0, st, t.sx.p, t.sy.p, t.sg.p, nb, t.first.p,
                            t.count.p, t.fx.p, t.fy.p, t.fg.p, t.ncx.p, t.ncy.p, t.nr.p, t.nbb.p, t.child0.p,
                            t.child1.p, t.cd.p, t.cf.p);
-        hipLaunchKernelGGL(k_upper_local<16>, dim3(gc), dim3(256), 0, st, cut, ncut, nb, t.child0.p, t.child1.p,
+        hipLaunchKernelGGL(k_upper_local<16>, dim3(gc), dim3(64 * kUpperWaves), 0, st, cut, ncut, nb, t.child0.p, t.child1.p,
                            t.ncx.p, t.ncy.p, t.nr.p, t.nbb.p, t.cd.p, t.cf.p);
         hipLaunchKernelGGL(k_upper_top<16>, dim3(1), dim3(1024), 0, st, t.root, nb, m, t.first.p, t.count.p,
                            t.bscan.p, t.toplist.p, t.child0.p, t.child1.p, t.ncx.p, t.ncy.p, t.nr.p, t.nbb.p, t.cd.p,
