@@ -443,16 +443,20 @@ struct WriteIndex {  // out[pos] = i for flagged items (ordered selection of ind
 
 // ---- LSD radix sort: 32-bit keys, 32-bit values, 8-bit digits ---------------------------
 // Four stable passes of one launch each, after one launch that counts every
-// pass's digits over all the keys.  A pass takes tiles of kSortTile keys; a
-// tile counts its digits (one LDS add per run of equal digits in a wave,
-// found with 8 ballots), publishes the counts in its status words, ranks its
-// keys in LDS by digit (the wave's earlier lanes with the same digit, plus
-// the tile's earlier waves and rounds) and writes them out digit run by digit
-// run.  A run's output offset is the global count of the smaller digits plus
-// the digit's count in the earlier tiles, which the tile reads back from
+// pass's digits over all the keys.  A pass takes tiles of kSortTile keys, a
+// quarter of consecutive ones for each wave, which ranks them by itself: the
+// lanes of equal digit come from 8 ballots, and the wave's count of the digit
+// so far from its own row of LDS counters.  The rows give the tile's digit
+// counts, published in its status words, and each wave's first slot of a
+// digit; so a tile has five barriers (a rank over the tile's rounds, counted
+// before, took 28: 30 -> 24 us a pass at 2^20 keys).
+// The keys are written out digit run by digit run.  A run's output offset is
+// the global count of the smaller digits plus the digit's count in the earlier
+// tiles, which the tile reads back from
 // their status words: a word holds a tile's own count (kStAgg) or its count
 // including every earlier tile (kStInc); the look-back adds own counts until
-// it meets an inclusive one, then publishes its own inclusive count.
+// it meets an inclusive one (four words in flight), then publishes its own
+// inclusive count.
 // Progress: a work-group takes its tile by ticket, so every tile it reads
 // belongs to a work-group that took its ticket earlier and is resident, and
 // a tile publishes its own counts before it reads any other tile's, so each
@@ -489,7 +493,9 @@ __device__ __forceinline__ uint64_t digit_peers(int d, bool ok) {
     return peers;
 }
 
-// Every pass's digit counts over all n keys, added into ghist (zeroed).
+// Every pass's digit counts over all n keys, added into ghist (zeroed).  Plain
+// LDS adds: 64 equal digits cost 64 cycles, less than the ballots that would
+// merge them.
 template <int DUMMY = 0>
 __global__ __launch_bounds__(kT) void k_radix_counts(const uint32_t *__restrict__ key, int64_t n,
                                                      int32_t *__restrict__ ghist) {
@@ -497,16 +503,17 @@ __global__ __launch_bounds__(kT) void k_radix_counts(const uint32_t *__restrict_
     for (int p = 0; p < kSortPasses; ++p) h[p][threadIdx.x] = 0;
     __syncthreads();
     const int64_t base = (int64_t)blockIdx.x * kSortTile;
+    uint32_t k[kSortIPT];
+#pragma unroll
     for (int r = 0; r < kSortIPT; ++r) {
         const int64_t i = base + r * kT + threadIdx.x;
-        const bool ok = i < n;
-        const uint32_t k = ok ? key[i] : 0u;
+        k[r] = i < n ? key[i] : 0u;
+    }
 #pragma unroll
-        for (int p = 0; p < kSortPasses; ++p) {
-            const int d = (int)((k >> (p * kRadixBits)) & (kBins - 1));
-            const uint64_t peers = digit_peers(d, ok);
-            if (ok && (peers & lanes_below()) == 0) atomicAdd(&h[p][d], (int32_t)__popcll(peers));
-        }
+    for (int r = 0; r < kSortIPT; ++r) {
+        if (base + r * kT + threadIdx.x >= n) continue;
+#pragma unroll
+        for (int p = 0; p < kSortPasses; ++p) atomicAdd(&h[p][(k[r] >> (p * kRadixBits)) & (kBins - 1)], 1);
     }
     __syncthreads();
     for (int p = 0; p < kSortPasses; ++p) {
@@ -525,36 +532,43 @@ __global__ __launch_bounds__(kT) void k_radix_onesweep(const uint32_t *__restric
                                                        int32_t *__restrict__ vout, int32_t *__restrict__ err) {
     __shared__ uint32_t sk[kSortTile];   // the tile sorted by digit
     __shared__ int32_t sv[kSortTile];
-    __shared__ int32_t cnt[kBins];       // the tile's count of each digit
     __shared__ int32_t loc[kBins];       // first slot of each digit in sk
-    __shared__ int32_t run[kBins];       // next free slot of each digit in sk
     __shared__ int32_t gbase[kBins];     // first output position of each digit's run
-    __shared__ int32_t wcnt[kW][kBins];
+    __shared__ int32_t wcnt[kW][kBins];  // each wave's count of a digit, then its first slot in sk
     __shared__ int32_t ws[2][kW];
     __shared__ int32_t tile_s;
     const int w = threadIdx.x >> 6, dd = threadIdx.x;  // thread dd handles digit dd in the per-digit steps
     if (threadIdx.x == 0) tile_s = atomicAdd(ticket, 1);
-    cnt[dd] = 0;
+#pragma unroll
+    for (int q = 0; q < kW; ++q) wcnt[q][dd] = 0;
     __syncthreads();
     const int64_t tile = tile_s;
     const int64_t base = tile * kSortTile;
+    const int64_t i0 = base + w * (64 * kSortIPT) + lane_id();  // the wave's keys, 64 a round
     uint32_t kr[kSortIPT];
-    int32_t vr[kSortIPT];
+    int32_t vr[kSortIPT], rank[kSortIPT];
 #pragma unroll
     for (int r = 0; r < kSortIPT; ++r) {
-        const int64_t i = base + r * kT + threadIdx.x;
+        const int64_t i = i0 + r * 64;
         kr[r] = i < n ? kin[i] : 0u;
         vr[r] = i < n ? vin[i] : 0;
     }
 #pragma unroll
     for (int r = 0; r < kSortIPT; ++r) {
-        const bool ok = base + r * kT + threadIdx.x < n;
+        const bool ok = i0 + r * 64 < n;
         const int d = (int)((kr[r] >> shift) & (kBins - 1));
         const uint64_t peers = digit_peers(d, ok);
-        if (ok && (peers & lanes_below()) == 0) atomicAdd(&cnt[d], (int32_t)__popcll(peers));
+        const int32_t below = (int32_t)__popcll(peers & lanes_below());
+        const int32_t before = wcnt[w][d];
+        __builtin_amdgcn_wave_barrier();
+        if (ok && below == 0) wcnt[w][d] = before + (int32_t)__popcll(peers);  // the digit's first lane
+        __builtin_amdgcn_wave_barrier();
+        rank[r] = before + below;
     }
     __syncthreads();
-    const int32_t c = cnt[dd];
+    int32_t c = 0;
+#pragma unroll
+    for (int q = 0; q < kW; ++q) c += wcnt[q][dd];
     uint64_t *own = status + tile * kBins + dd;
     __hip_atomic_store(own, (tile == 0 ? kStInc : kStAgg) | (uint64_t)(uint32_t)c, __ATOMIC_RELAXED,
                        __HIP_MEMORY_SCOPE_AGENT);
@@ -572,47 +586,49 @@ __global__ __launch_bounds__(kT) void k_radix_onesweep(const uint32_t *__restric
         gpre += ws[1][k];
     }
     loc[dd] = pre;
-    run[dd] = pre;
+#pragma unroll
+    for (int q = 0; q < kW; ++q) {
+        const int32_t o = wcnt[q][dd];
+        wcnt[q][dd] = pre;
+        pre += o;
+    }
+    __syncthreads();
+#pragma unroll
     for (int r = 0; r < kSortIPT; ++r) {
-        for (int k = 0; k < kW; ++k) wcnt[k][threadIdx.x] = 0;
-        const bool ok = base + r * kT + threadIdx.x < n;
-        const uint32_t k = kr[r];
-        const int d = (int)((k >> shift) & (kBins - 1));
-        const uint64_t peers = digit_peers(d, ok);
-        const int32_t below = (int32_t)__popcll(peers & lanes_below());
-        __syncthreads();  // wcnt cleared, run up to date
-        if (ok && below == 0) wcnt[w][d] = (int32_t)__popcll(peers);  // the digit's first lane in this wave
-        __syncthreads();
-        if (ok) {
-            int32_t pos = run[d] + below;
-            for (int q = 0; q < w; ++q) pos += wcnt[q][d];
-            sk[pos] = k;
+        if (i0 + r * 64 < n) {
+            const int32_t pos = wcnt[w][(kr[r] >> shift) & (kBins - 1)] + rank[r];
+            sk[pos] = kr[r];
             sv[pos] = vr[r];
         }
-        __syncthreads();
-        int32_t add = 0;
-#pragma unroll
-        for (int q = 0; q < kW; ++q) add += wcnt[q][threadIdx.x];
-        run[threadIdx.x] += add;
     }
     // the digit's count in the earlier tiles
     int64_t excl = 0;
     if (tile > 0) {
         int64_t t = tile - 1, polls = 0;
         for (;;) {
-            const uint64_t sw = __hip_atomic_load(status + t * kBins + dd, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-            const uint64_t st = sw & kStMask;
-            if (st == 0) {
-                if (++polls > kSpinMax) {
-                    if (err) atomicOr(err, 1);
-                    break;
-                }
-                __builtin_amdgcn_s_sleep(1);
-                continue;
+            uint64_t sw[4];
+#pragma unroll
+            for (int q = 0; q < 4; ++q)
+                sw[q] = __hip_atomic_load(status + (t > q ? t - q : 0) * kBins + dd, __ATOMIC_RELAXED,
+                                          __HIP_MEMORY_SCOPE_AGENT);
+            int used = 0;
+            bool done = false;
+#pragma unroll
+            for (int q = 0; q < 4; ++q) {
+                const uint64_t st = sw[q] & kStMask;
+                if (done || used < q || st == 0) continue;
+                excl += (int64_t)(sw[q] & kStCount);
+                used = q + 1;
+                done = st == kStInc || t == q;
             }
-            excl += (int64_t)(sw & kStCount);
-            if (st == kStInc || t == 0) break;
-            --t;
+            if (done) break;
+            t -= used;
+            if (used > 0) continue;
+            if (++polls > kSpinMax) {
+                if (err) atomicOr(err, 1);
+                break;
+            }
+            __builtin_amdgcn_s_sleep(1);
         }
         __hip_atomic_store(own, kStInc | (uint64_t)(uint32_t)(excl + c), __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
     }
