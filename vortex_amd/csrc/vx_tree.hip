@@ -2548,14 +2548,16 @@ __global__ __launch_bounds__(256) void k_diff_far(TreeDev t, const double4 *__re
     block_count_add(cp, 0ull, cnt, nullptr);
 }
 
-// Sixteen listed targets a work-group, sixteen threads each: the partials of
-// the target's listed chunks, then the velocity update.  Thread j takes chunks
-// j, j + 16, ..., all loads in flight, and the sum is the tree over 256 slots
-// (chunk mod 256) whatever the count, so a chunk not listed is an exact zero
-// and its partial is neither cleared before nor read.  One work-group a target
-// left most threads idle and read a word of each line: 146 -> 54 us for
-// 78993 targets and 37 chunks.
-constexpr int kFarTgts = 16;
+// Eight listed targets a work-group, 32 threads each: the partials of the
+// target's listed chunks, then the velocity update.  Thread j takes chunks
+// j, j + 32, ..., and the sum is the tree over 256 slots (chunk mod 256)
+// whatever the count, so a chunk not listed is an exact zero and its partial
+// is neither cleared before nor read.  One work-group a target left most
+// threads idle and read a word of each line: 146 -> 33 us for 78993 targets and
+// 37 chunks.  The slots are added one after the other: all in registers, the
+// work-groups, idle ones too, waited for room beside the groups' waves (0.76 ms
+// at 2^20 vortices, now 0.04).
+constexpr int kFarTgts = 8, kFarThr = 256 / kFarTgts;
 
 __global__ __launch_bounds__(256) void k_diff_far_final(TreeDev t, const int32_t *__restrict__ list,
                                                         const unsigned long long *__restrict__ cnt,
@@ -2563,8 +2565,7 @@ __global__ __launch_bounds__(256) void k_diff_far_final(TreeDev t, const int32_t
                                                         const double *__restrict__ part,
                                                         const double *__restrict__ dd, double nu,
                                                         double *__restrict__ u, double *__restrict__ v) {
-    constexpr int kPer = 256 / kFarTgts;  // slots per thread
-    __shared__ double r[3][kFarTgts][kFarTgts + 1];
+    __shared__ double r[3][kFarThr][kFarTgts + 1];
     const int64_t H = far_count(cnt, t.fcap);
     const int kt = threadIdx.x % kFarTgts, j = threadIdx.x / kFarTgts;
     for (int64_t k0 = (int64_t)blockIdx.x * kFarTgts; k0 < H; k0 += (int64_t)gridDim.x * kFarTgts) {
@@ -2577,42 +2578,43 @@ __global__ __launch_bounds__(256) void k_diff_far_final(TreeDev t, const int32_t
             ui = u[i];
             vi = v[i];
         }
-        double a[3][kPer] = {};
-        for (int64_t c0 = 0; c0 < nchunk; c0 += 256) {
-#pragma unroll
-            for (int g = 0; g < 4; ++g) {  // a mask word's chunks
-                const int64_t w0 = c0 + g * 64;
-                if (w0 >= nchunk) break;
-                const uint64_t m = k < H ? fmask[(w0 >> 6) * H + k] >> j : 0;
-                double x[3][kPer / 4];
-#pragma unroll
-                for (int q = 0; q < kPer / 4; ++q)
-#pragma unroll
-                    for (int e = 0; e < 3; ++e)  // an unlisted chunk's load goes to the first word
-                        x[e][q] = part[(m >> (q * kFarTgts)) & 1u ? ((w0 + q * kFarTgts + j) * 3 + e) * H + k : 0];
-#pragma unroll
-                for (int q = 0; q < kPer / 4; ++q)
-#pragma unroll
-                    for (int e = 0; e < 3; ++e)
-                        a[e][g * (kPer / 4) + q] += (m >> (q * kFarTgts)) & 1u ? x[e][q] : 0.0;
+        // slot q of this thread's eight: its chunks, 256 apart
+        auto slot = [&](int q, double (&f)[3]) {
+#pragma unroll 1
+            for (int64_t ch = q * kFarThr + j; ch < nchunk; ch += 256) {
+                if (k < H && ((fmask[(ch >> 6) * H + k] >> (ch & 63)) & 1u)) {
+                    const double *p = part + ch * 3 * H + k;
+                    const double x0 = p[0], x1 = p[H], x2 = p[2 * H];
+                    f[0] += x0;
+                    f[1] += x1;
+                    f[2] += x2;
+                }
             }
+        };
+        double a[3] = {};  // (q and q + 4), then q and q + 2, then q and q + 1
+#pragma unroll 1
+        for (int q1 = 0; q1 < 2; ++q1) {
+            double b[3] = {};
+#pragma unroll 1
+            for (int q2 = q1; q2 < 4; q2 += 2) {
+                double f[3] = {}, g[3] = {};
+                slot(q2, f);
+                slot(q2 + 4, g);
+#pragma unroll
+                for (int e = 0; e < 3; ++e) b[e] += f[e] + g[e];
+            }
+#pragma unroll
+            for (int e = 0; e < 3; ++e) a[e] += b[e];
         }
 #pragma unroll
-        for (int st = kPer / 2; st > 0; st >>= 1)
-#pragma unroll
-            for (int q = 0; q < st; ++q)
-#pragma unroll
-                for (int e = 0; e < 3; ++e) a[e][q] += a[e][q + st];
-#pragma unroll
-        for (int e = 0; e < 3; ++e) r[e][j][kt] = a[e][0];
+        for (int e = 0; e < 3; ++e) r[e][j][kt] = a[e];
         __syncthreads();
-        if (threadIdx.x < 64) {  // threads j < 4: j and j + 8, then j and j + 4, the rest over the lanes
+        if (threadIdx.x < 64) {  // threads j < 8: j and j + 16, then j and j + 8, the rest over the lanes
             double f[3];
 #pragma unroll
             for (int e = 0; e < 3; ++e) {
-                f[e] = (r[e][j][kt] + r[e][j + 8][kt]) + (r[e][j + 4][kt] + r[e][j + 12][kt]);
-                f[e] += __shfl_down(f[e], 2 * kFarTgts, 64);
-                f[e] += __shfl_down(f[e], kFarTgts, 64);
+                f[e] = (r[e][j][kt] + r[e][j + 16][kt]) + (r[e][j + 8][kt] + r[e][j + 24][kt]);
+                for (int st = 4; st > 0; st >>= 1) f[e] += __shfl_down(f[e], st * kFarTgts, 64);
             }
             if (j == 0 && k < H && fabs(f[2]) > 1e-5) {
                 u[i] = ui + nu * f[0] / (f[2] * di);
