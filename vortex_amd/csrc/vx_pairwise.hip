@@ -1553,7 +1553,9 @@ double diff_thr2(double thr) {
 }
 
 int launch_diffusion(vx_case *c, Cnt n_tgt, Cnt n_src, bool packed) {
-    if (n_tgt.ub <= 0) return 0;
+    // No sources (vx_diffusion takes any count below the capacity): nothing to
+    // add, and the split and the ordered kernels' staging need one at least.
+    if (n_tgt.ub <= 0 || n_src.ub <= 0) return 0;
     const double thr = 0.001 * c->prm.ve_size;
     const dim3 gsum((unsigned)((n_tgt.ub + 63) / 64));
     if (mixed(c)) {
