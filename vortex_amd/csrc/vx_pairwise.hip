@@ -92,29 +92,29 @@ __host__ __device__ __forceinline__ DirectSplit direct_split(int64_t n_tgt, int6
     return DirectSplit{(int32_t)(per * unit), (int32_t)((units + per - 1) / per)};
 }
 
-// Blocks of kTile * tpt targets times runs: exact for host counts, else a
-// bound over all smaller counts (kernels leave surplus blocks at once).  The
-// runs of n sources number at most max(kDirectWork / tb + 1, kOrdered units).
-template <typename T>
-static int64_t direct_runs_max(int64_t n_tgt, int64_t n_src) {
-    constexpr int64_t unit = sizeof(T) == 4 ? kTile : kTile / 4;
-    const int64_t units = (n_src + unit - 1) / unit, tb = (n_tgt + kTile - 1) / kTile;
-    return std::max<int64_t>(std::min(units, kOrdered / unit), std::min(units, kDirectWork / std::max<int64_t>(tb, 1) + 1));
-}
+// Work-groups of kTile * tpt targets times runs, and doubles of partials for q
+// values per target and run: exact for host counts.  A device count (the same
+// for targets and sources) gets a bound over all counts up to its own; kernels
+// leave surplus work-groups at once.  With tb blocks of kTile targets, n
+// sources above kOrdered make at most (kDirectWork - 1) / tb + 1 runs, so n
+// times runs stays below kTile * kDirectWork + n, and (tb + tpt - 1) / tpt
+// times runs below kDirectWork / tpt + tb / tpt + 64 (tb > 64).  Up to kOrdered
+// the runs are the units: both products grow with n, to kTile * kDirectWork and
+// kDirectWork / tpt in FP32, while FP64 leaves those counts to the ordered kernels.
+static_assert(kOrdered == 64 * kTile && kOrdered * 64 == kTile * kDirectWork, "the bounds of both ranges meet");
 
 template <typename T>
 static int64_t direct_blocks(Cnt n_tgt, Cnt n_src, int tpt) {
     const int64_t w = kTile * tpt, tb = (n_tgt.ub + w - 1) / w;
-    if (!n_tgt.dev && !n_src.dev) return tb * direct_split<T>(n_tgt.ub, n_src.ub).runs;
-    return tb * direct_runs_max<T>(n_tgt.ub, n_src.ub) + kDirectWork / tpt;
+    if (!n_tgt.dev || n_src.ub <= kOrdered) return tb * direct_split<T>(n_tgt.ub, n_src.ub).runs;
+    return tb + kDirectWork / tpt + 64;
 }
 
-// Doubles of partials for q values per target and run.
 template <typename T>
 static size_t direct_partials(Cnt n_tgt, Cnt n_src, int q) {
-    const int64_t t = n_tgt.ub > 0 ? n_tgt.ub : 1;
-    if (!n_tgt.dev && !n_src.dev) return (size_t)(q * t * direct_split<T>(n_tgt.ub, n_src.ub).runs);
-    return (size_t)(q * (t * direct_runs_max<T>(t, n_src.ub) + kTile * kDirectWork));
+    if (!n_tgt.dev || n_src.ub <= kOrdered)
+        return (size_t)(q * n_tgt.ub * direct_split<T>(n_tgt.ub, n_src.ub).runs);
+    return (size_t)(q * (n_tgt.ub + kTile * kDirectWork));
 }
 
 // The four smallest values seen so far, m0 <= m1 <= m2 <= m3.
