@@ -10,14 +10,6 @@
 
 namespace vx {
 
-// g / a for a normal a > 0 (|g / a| in range): within 1.5 ulp.
-__device__ __forceinline__ double div_pos(double g, double a) {
-    const double y = __builtin_amdgcn_rcp(a);
-    const double e = fma(-a, y, 1.0);
-    const double w = g * y;
-    return fma(w, fma(e, e, e), w);
-}
-
 // g / a for a normal a > 0, correctly rounded as `/` gives it: a reciprocal
 // within 1 ulp, then the quotient's exact residual.
 __device__ __forceinline__ double div_pos_exact(double g, double a) {

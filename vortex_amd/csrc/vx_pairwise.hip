@@ -32,7 +32,7 @@ struct Arith;
 template <>
 struct Arith<double> {
     static constexpr double kFar = 1e30;  // padding sources: squared distance stays finite
-    __device__ static __forceinline__ double div(double a, double b) { return div_pos(a, b); }
+    __device__ static __forceinline__ double div(double a, double b) { return div_pos_exact(a, b); }
     __device__ static __forceinline__ double med3(double a, double b, double c) {
         return fmax(fmin(a, b), fmin(fmax(a, b), c));
     }
