@@ -28,3 +28,19 @@ def test_diffusion_without_sources_adds_nothing(prec, n_src):
     c.close()
     for a, b in zip(got, (u, v, d)):
         assert np.array_equal(a, b)
+
+
+@pytest.mark.parametrize("prec", [VX_PREC_F64, VX_PREC_MIXED])
+@pytest.mark.parametrize("n", [500, 20000])
+def test_diffusion_threshold_without_bound(prec, n):
+    """ve_size has no upper limit; no distance is above an infinite threshold."""
+    pan = geo.circle(64, 0.5)
+    c = Case(make_params(pan, precision=prec, ve_size=np.inf, nu=NU), pan)
+    c.set_state(*uniform_wake(n, seed=2))
+    u, v, d = np.full(n, 0.25), np.full(n, -0.5), np.full(n, 0.1)
+    c.set_velocity(u, v, d)
+    c.diffusion(n, n)
+    got = c.velocity(n)
+    c.close()
+    for a, b in zip(got, (u, v, d)):
+        assert np.array_equal(a, b)

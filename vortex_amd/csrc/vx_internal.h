@@ -267,7 +267,6 @@ inline Cnt cnt_s(const vx_case *c) {
 int launch_biot_savart(vx_case *c, int64_t n_tgt, int64_t n_src, double vinf_x, double vinf_y);
 int launch_biot_savart(vx_case *c, Cnt n_tgt, Cnt n_src, double vinf_x, double vinf_y);
 int launch_diffusion(vx_case *c, int64_t n_tgt, int64_t n_src);
-double diff_thr2(double thr);  // r^2 > diff_thr2(thr) decides as sqrt(r^2) > thr
 // packed: launch_biot_savart over the same sources just left their FP32 copies
 int launch_diffusion(vx_case *c, Cnt n_tgt, Cnt n_src, bool packed = false);
 int launch_right_part(vx_case *c, int64_t n_src, double vinf_x, double vinf_y);  // -> c->rp

@@ -1,8 +1,7 @@
-// FP64 quotient, inverse square root and exponential for the pair kernels.
-// The compiler's division, sqrt and the library's exp take about 60, 60 and
-// 150 SIMD cycles per wave64 with their scaling and special cases; the pair
-// kernels know their ranges, so these take Newton steps from the hardware's
-// approximation.
+// FP64 quotient and square root for the pair kernels.  The compiler's division
+// and sqrt take about 60 SIMD cycles per wave64 each with their scaling and
+// special cases; the pair kernels know their ranges, so these take Newton steps
+// from the hardware's approximation.
 #pragma once
 
 #include <hip/hip_runtime.h>
@@ -34,41 +33,6 @@ __device__ __forceinline__ double sqrt_pos_exact(double a, double g, double &q) 
     const double w = g * y;
     q = fma(fma(-s, w, g), y, w);
     return s;
-}
-
-// 1 / sqrt(a) and sqrt(a) for a normal a > 0: within 1.5 ulp each.
-// With a y^2 = 1 - e: 1/sqrt(1 - e) = 1 + e/2 + 3 e^2/8 + O(e^3).
-__device__ __forceinline__ void rsqrt_sqrt_pos(double a, double &rs, double &s) {
-    const double y = __builtin_amdgcn_rsq(a);
-    const double t = a * y;
-    const double e = fma(-t, y, 1.0);
-    const double p = e * fma(0.375, e, 0.5);
-    rs = fma(y, p, y);
-    s = fma(t, p, t);
-}
-
-// 2^t for t <= 1020; below -1100 (where 2^t rounds to zero) the result is 0.
-// t = k + f, |f| <= 1/2, k from adding 3 * 2^51; 2^f by a polynomial of degree
-// 11, the Chebyshev interpolant on [-1/2, 1/2] computed for this library in
-// 40 digits (3e-18 relative before, 2e-17 after its coefficients are rounded).
-__device__ __forceinline__ double exp2_neg(double t) {
-    constexpr double kRound = 6755399441055744.0;
-    t = fmax(t, -1100.0);
-    const double s = t + kRound;
-    const double f = t - (s - kRound);
-    double p = 4.4558179083360645e-10;
-    p = fma(p, f, 7.074194297288521e-09);
-    p = fma(p, f, 1.0178057087733941e-07);
-    p = fma(p, f, 1.3215432535912375e-06);
-    p = fma(p, f, 1.5252733841556773e-05);
-    p = fma(p, f, 1.5403530463724353e-04);
-    p = fma(p, f, 1.333355814640647e-03);
-    p = fma(p, f, 9.618129107587256e-03);
-    p = fma(p, f, 5.5504108664821625e-02);
-    p = fma(p, f, 2.4022650695910158e-01);
-    p = fma(p, f, 6.931471805599453e-01);
-    p = fma(p, f, 1.0);
-    return __builtin_amdgcn_ldexp(p, __double2loint(s));
 }
 
 __device__ __forceinline__ void order2(double &a, double &b) {

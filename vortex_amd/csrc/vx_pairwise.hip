@@ -289,13 +289,38 @@ __global__ __launch_bounds__(256) void k_bs_sum(const double *__restrict__ part,
 // ---- A7: src/kernel.cu:985-1029 -------------------------------------------
 // Over j with r_ij > 0.001 ve_size: I2 += -g_j (r_i - r_j)/r e^{-r/d_i},
 // I1 += g_j e^{-r/d_i}; if |I1| > 1e-5: V_i += -nu I2 / (I1 d_i).
-// thr2 is the largest r^2 that the test leaves out.  Sources and partials as
-// in k_biot_savart: part[(3 s + q) n_tgt + i], q = x and y of the weighted
-// separations, then I1.
+// Sources and partials as in k_biot_savart: part[(3 s + q) n_tgt + i], q = x
+// and y of the weighted separations, then I1.
+//
+// FP64 takes four sources at a time through expressions for ordinary
+// separations; where some lane comes near the threshold (its own source among
+// others) or a coordinate or circulation is huge or no number, the four go
+// through the plain ones.  Both round alike.
+template <typename T>
+struct DiffSums {
+    T x, y, i1;
+};
+
+__device__ __forceinline__ void diff_pair_plain(double dx, double dy, double g, double kd, double thr,
+                                                DiffSums<double> &s) {
+    const double dist = sqrt(fma(dx, dx, dy * dy));
+    if (dist > thr) {
+        const double w = g / dist, e = exp(-dist * kd);
+        s.x = fma(w * dx, e, s.x);
+        s.y = fma(w * dy, e, s.y);
+        s.i1 = fma(g, e, s.i1);
+    }
+}
+
+// Neither NaN nor an infinity nor above 2^500, so that squares of differences
+// stay in range.  Integer compares only: on wave-uniform values they run on the
+// scalar unit.
+__device__ __forceinline__ bool ordinary(double v) { return (__double2hiint(v) & 0x7fffffff) < 0x5f300000; }
+
 template <typename T, int TPT>
 __global__ __launch_bounds__(kTile) void k_diffusion(const T *__restrict__ sx, const T *__restrict__ sy,
                                                      const T *__restrict__ sg, Cnt cn_src, Cnt cn_tgt,
-                                                     const double *__restrict__ dd, T thr2,
+                                                     const double *__restrict__ dd, T thr,
                                                      double *__restrict__ part) {
     const int32_t n_src = (int32_t)cn_src.get(), n_tgt = (int32_t)cn_tgt.get();
     if (sizeof(T) == 8 && n_src <= kOrdered) return;  // the ordered kernel's
@@ -306,53 +331,93 @@ __global__ __launch_bounds__(kTile) void k_diffusion(const T *__restrict__ sx, c
     if (s >= (uint32_t)sp.runs) return;
     const int32_t lo = (int32_t)s * sp.len, hi = min(n_src, lo + sp.len);
     const int32_t t0 = (int32_t)(t * (kTile * TPT) + threadIdx.x);
-    T ax[TPT], ay[TPT], kd[TPT], s2x[TPT], s2y[TPT], s1[TPT];
+    T ax[TPT], ay[TPT], kd[TPT];
+    DiffSums<T> sum[TPT];
     double a2x[TPT], a2y[TPT], a1[TPT];
+    bool tame = true;
 #pragma unroll
     for (int k = 0; k < TPT; ++k) {
         const int32_t i = t0 + k * kTile;
-        ax[k] = i < n_tgt ? far_clamp(sx[i]) : T(0);
-        ay[k] = i < n_tgt ? far_clamp(sy[i]) : T(0);
+        ax[k] = i < n_tgt ? sx[i] : T(0);
+        ay[k] = i < n_tgt ? sy[i] : T(0);
         const double di = i < n_tgt ? dd[i] : 1.0;
-        kd[k] = (T)(-1.4426950408889634 / di);  // exp(-r/d) = exp2(r * kd)
-        s2x[k] = s2y[k] = s1[k] = T(0);
+        // FP32: exp(-r/d) = exp2(r * kd)
+        kd[k] = (T)((sizeof(T) == 4 ? -1.4426950408889634 : 1.0) / di);
+        sum[k] = DiffSums<T>{T(0), T(0), T(0)};
         a2x[k] = a2y[k] = a1[k] = 0.0;
+        if constexpr (sizeof(T) == 8) tame = tame && ordinary(ax[k]) && ordinary(ay[k]);
     }
-    for (int32_t base = lo; base < hi; base += kTile) {
-        const int32_t end = min(hi, base + kTile);
-#pragma unroll 4
-        for (int32_t j = base; j < end; ++j) {
-            const T x = far_clamp(sx[j]), y = far_clamp(sy[j]), g = sg[j];
+    if constexpr (sizeof(T) == 8) {
+        tame = !__any(!tame);
+        const double gap2 = fmax(4.0 * thr * thr, 0x1p-900);  // no rounding brings a distance above 2 thr to thr
+        int32_t j = lo;
+        for (; j + 4 <= hi; j += 4) {
+            double x[4], y[4], g[4];
+            bool plain = !tame;
+#pragma unroll
+            for (int q = 0; q < 4; ++q) {
+                x[q] = sx[j + q];
+                y[q] = sy[j + q];
+                g[q] = sg[j + q];
+                plain = plain || !ordinary(x[q]) || !ordinary(y[q]) || !ordinary(g[q]);
+            }
 #pragma unroll
             for (int k = 0; k < TPT; ++k) {
-                const T dx = ax[k] - x, dy = ay[k] - y;
-                const T r2 = dx * dx + dy * dy;
-                T e, rs;
-                if constexpr (sizeof(T) == 4) {
-                    const T r2c = r2 > thr2 ? r2 : T(1e30f);
-                    rs = __builtin_amdgcn_rsqf(r2c);
-                    e = __builtin_amdgcn_exp2f((r2c * rs) * kd[k]);
-                } else {
-                    // left out: a distance of 1e150, whose exponential is zero
-                    const double r2c = r2 > thr2 ? r2 : __hiloint2double(0x7e37e43c, __double2loint(r2));
-                    double dist;
-                    rsqrt_sqrt_pos(r2c, rs, dist);
-                    e = exp2_neg(dist * kd[k]);
+                double r2[4];
+                bool near = plain;
+#pragma unroll
+                for (int q = 0; q < 4; ++q) {
+                    const double dx = ax[k] - x[q], dy = ay[k] - y[q];
+                    r2[q] = fma(dx, dx, dy * dy);
+                    near = near || !(r2[q] > gap2);
                 }
-                const T ge = g * e;
-                const T w = ge * rs;
-                s2x[k] += w * dx;
-                s2y[k] += w * dy;
-                s1[k] += ge;
+                if (__builtin_expect(__any(near), 0)) {
+#pragma unroll 1
+                    for (int q = 0; q < 4; ++q)
+                        diff_pair_plain(ax[k] - sx[j + q], ay[k] - sy[j + q], sg[j + q], kd[k], thr, sum[k]);
+                    continue;
+                }
+#pragma unroll
+                for (int q = 0; q < 4; ++q) {
+                    const double dx = ax[k] - x[q], dy = ay[k] - y[q];
+                    double w;
+                    const double dist = sqrt_pos_exact(r2[q], g[q], w), e = exp(-dist * kd[k]);
+                    sum[k].x = fma(w * dx, e, sum[k].x);
+                    sum[k].y = fma(w * dy, e, sum[k].y);
+                    sum[k].i1 = fma(g[q], e, sum[k].i1);
+                }
             }
         }
-        if constexpr (sizeof(T) == 4) {
+        for (; j < hi; ++j)
+#pragma unroll
+            for (int k = 0; k < TPT; ++k) diff_pair_plain(ax[k] - sx[j], ay[k] - sy[j], sg[j], kd[k], thr, sum[k]);
+    } else {
+        const T thr2 = thr;  // squared by the caller, in FP64
+        for (int32_t base = lo; base < hi; base += kTile) {
+            const int32_t end = min(hi, base + kTile);
+#pragma unroll 4
+            for (int32_t j = base; j < end; ++j) {
+                const T x = sx[j], y = sy[j], g = sg[j];
+#pragma unroll
+                for (int k = 0; k < TPT; ++k) {
+                    const T dx = ax[k] - x, dy = ay[k] - y;
+                    const T r2 = dx * dx + dy * dy;
+                    const T r2c = r2 > thr2 ? r2 : T(1e30f);
+                    const T rs = __builtin_amdgcn_rsqf(r2c);
+                    const T e = __builtin_amdgcn_exp2f((r2c * rs) * kd[k]);
+                    const T ge = g * e;
+                    const T w = ge * rs;
+                    sum[k].x += w * dx;
+                    sum[k].y += w * dy;
+                    sum[k].i1 += ge;
+                }
+            }
 #pragma unroll
             for (int k = 0; k < TPT; ++k) {
-                a2x[k] += (double)s2x[k];
-                a2y[k] += (double)s2y[k];
-                a1[k] += (double)s1[k];
-                s2x[k] = s2y[k] = s1[k] = T(0);
+                a2x[k] += (double)sum[k].x;
+                a2y[k] += (double)sum[k].y;
+                a1[k] += (double)sum[k].i1;
+                sum[k] = DiffSums<T>{T(0), T(0), T(0)};
             }
         }
     }
@@ -361,9 +426,9 @@ __global__ __launch_bounds__(kTile) void k_diffusion(const T *__restrict__ sx, c
     for (int k = 0; k < TPT; ++k) {
         const int32_t i = t0 + k * kTile;
         if (i >= n_tgt) continue;
-        o[i] = sizeof(T) == 8 ? (double)s2x[k] : a2x[k];
-        o[(int64_t)n_tgt + i] = sizeof(T) == 8 ? (double)s2y[k] : a2y[k];
-        o[(int64_t)2 * n_tgt + i] = sizeof(T) == 8 ? (double)s1[k] : a1[k];
+        o[i] = sizeof(T) == 8 ? (double)sum[k].x : a2x[k];
+        o[(int64_t)n_tgt + i] = sizeof(T) == 8 ? (double)sum[k].y : a2y[k];
+        o[(int64_t)2 * n_tgt + i] = sizeof(T) == 8 ? (double)sum[k].i1 : a1[k];
     }
 }
 
@@ -1528,28 +1593,19 @@ int launch_diffusion(vx_case *c, int64_t n_tgt, int64_t n_src) {
 }
 
 template <typename T, int TPT>
-static void diff_launch(vx_case *c, const T *sx, const T *sy, const T *sg, Cnt n_src, Cnt n_tgt, T thr2) {
+static void diff_launch(vx_case *c, const T *sx, const T *sy, const T *sg, Cnt n_src, Cnt n_tgt, T thr) {
     hipLaunchKernelGGL((k_diffusion<T, TPT>), dim3((unsigned)direct_blocks<T>(n_tgt, n_src, TPT)), dim3(kTile), 0,
-                       c->stream, sx, sy, sg, n_src, n_tgt, c->d.p, thr2, c->partial.p);
+                       c->stream, sx, sy, sg, n_src, n_tgt, c->d.p, thr, c->partial.p);
 }
 
 template <typename T>
-static void diff_dispatch(vx_case *c, int tpt, const T *sx, const T *sy, const T *sg, Cnt n_src, Cnt n_tgt, T thr2) {
+static void diff_dispatch(vx_case *c, int tpt, const T *sx, const T *sy, const T *sg, Cnt n_src, Cnt n_tgt, T thr) {
     switch (tpt) {
-        case 1: diff_launch<T, 1>(c, sx, sy, sg, n_src, n_tgt, thr2); break;
-        case 2: diff_launch<T, 2>(c, sx, sy, sg, n_src, n_tgt, thr2); break;
-        case 4: diff_launch<T, 4>(c, sx, sy, sg, n_src, n_tgt, thr2); break;
-        default: diff_launch<T, 8>(c, sx, sy, sg, n_src, n_tgt, thr2); break;
+        case 1: diff_launch<T, 1>(c, sx, sy, sg, n_src, n_tgt, thr); break;
+        case 2: diff_launch<T, 2>(c, sx, sy, sg, n_src, n_tgt, thr); break;
+        case 4: diff_launch<T, 4>(c, sx, sy, sg, n_src, n_tgt, thr); break;
+        default: diff_launch<T, 8>(c, sx, sy, sg, n_src, n_tgt, thr); break;
     }
-}
-
-// The largest r^2 whose rounded square root is not above thr, so that
-// r^2 > thr2 decides as sqrt(r^2) > thr does.
-double diff_thr2(double thr) {
-    double t = thr * thr;
-    while (std::sqrt(t) > thr) t = std::nextafter(t, 0.0);
-    for (double q = std::nextafter(t, INFINITY); std::sqrt(q) <= thr; q = std::nextafter(t, INFINITY)) t = q;
-    return t;
 }
 
 int launch_diffusion(vx_case *c, Cnt n_tgt, Cnt n_src, bool packed) {
@@ -1580,7 +1636,7 @@ int launch_diffusion(vx_case *c, Cnt n_tgt, Cnt n_src, bool packed) {
         if (takes_split(n_src)) {
             if (c->partial.ensure(direct_partials<double>(n_tgt, n_src, 3), c->stream)) return 1;
             diff_dispatch<double>(c, tpt_of(c->tune.tpt_diff, false, n_tgt.ub), c->x.p, c->y.p, c->g.p, n_src, n_tgt,
-                                  diff_thr2(thr));
+                                  thr);
             hipLaunchKernelGGL(k_diff_sum<double>, gsum, dim3(256), 0, c->stream, c->partial.p, n_src, n_tgt, c->d.p,
                                c->prm.nu, c->u.p, c->v.p);
         }

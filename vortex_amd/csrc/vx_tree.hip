@@ -1927,8 +1927,7 @@ __global__ __launch_bounds__(1024) void k_tree_nearest_fallback(TreeDev t, const
 // Diffusion pair terms (src/kernel.cu:1011-1019): s1 += g e, (s2x, s2y) +=
 // g e (dx, dy) / r with e = exp(-r / d), for r above the threshold.  FP32:
 // kd = -log2(e) / d and a below-threshold r^2 is pushed to 1e30, whose
-// weight underflows to zero.  FP64: the same kd and one inverse square root
-// for r and 1 / r (vx_math.h); a below-threshold pair's g counts as 0.
+// weight underflows to zero.  FP64: kd = 1 / d, thr the threshold itself.
 template <typename T>
 struct DiffPair;
 template <>
@@ -1973,17 +1972,17 @@ __device__ __forceinline__ void diff_pair_log(float dx, float dy, float lg, floa
 template <>
 struct DiffPair<double> {
     template <bool GUARD>
-    __device__ static __forceinline__ void add(double dx, double dy, double g, double kd, double thr2,
+    __device__ static __forceinline__ void add(double dx, double dy, double g, double kd, double thr,
                                                double &s2x, double &s2y, double &s1) {
         const double r2 = dx * dx + dy * dy;
-        const bool far = !GUARD || r2 > thr2;
-        double rs, r;
-        rsqrt_sqrt_pos(far ? r2 : 1.0, rs, r);
-        const double ge = (far ? g : 0.0) * exp2_neg(r * kd);
-        const double w = ge * rs;
-        s2x += w * dx;
-        s2y += w * dy;
-        s1 += ge;
+        double w;
+        const double dist = sqrt_pos_exact(r2, g, w);  // r2 = 0 or infinite: NaN, not above the threshold
+        if (!GUARD || dist > thr) {
+            const double e = exp(-dist * kd);
+            s2x += w * dx * e;
+            s2y += w * dy * e;
+            s1 += g * e;
+        }
     }
 };
 
@@ -2032,7 +2031,7 @@ __device__ __forceinline__ int64_t far_count(const unsigned long long *cnt, int6
 constexpr int kDiffWaves = 4;  // per target group
 
 template <typename T, bool CENSUS>
-__device__ __forceinline__ void diffusion_wave(const TreeDev &t, double cut, double nu, double thr, double thr2d,
+__device__ __forceinline__ void diffusion_wave(const TreeDev &t, double cut, double nu, double thr,
                                                const double *__restrict__ sd, double *__restrict__ u,
                                                double *__restrict__ v, unsigned long long *__restrict__ cnt,
                                                unsigned long long &cpairs, unsigned long long &cin) {
@@ -2075,10 +2074,10 @@ __device__ __forceinline__ void diffusion_wave(const TreeDev &t, double cut, dou
     } else {
         ax = ok ? t.sx[ti] : cAx;
         ay = ok ? t.sy[ti] : cAy;
-        kd = -1.4426950408889634 / (ok ? di : 1.0);
+        kd = 1.0 / (ok ? di : 1.0);
         ri2 = mine ? cut * di * cut * di : -1.0;
     }
-    const T thr2 = (T)thr2d;
+    const T thr2 = F32 ? (T)(thr * thr) : (T)thr;
     const T gap2 = (T)(4.0 * thr * thr);
     // sources farther than R from the group's box reach no target's radius
     const T Rs2 = F32 ? (T)(R2 * (1.0 + 1e-4)) : (T)R2;
@@ -2145,7 +2144,8 @@ __device__ __forceinline__ void diffusion_wave(const TreeDev &t, double cut, dou
             if (__ballot(l2 < ri2) == 0) continue;
             // the threshold test is needed only where a pair can come within
             // it: a leaf box nearer than twice the threshold to some target
-            const int guard = __ballot(mine && !(l2 > gap2)) != 0;
+            // (it also drops a pair whose squared distance is not finite)
+            const int guard = __ballot(mine && !(l2 > gap2 && l2 < T(3e38))) != 0;
             if (lane == 0) lsel[nr] = li | (guard << 8);
             ++nr;
         }
@@ -2333,12 +2333,12 @@ __device__ __forceinline__ void diffusion_wave(const TreeDev &t, double cut, dou
 // CENSUS also counts the pairs within each target's own radius (cnt[5]).
 template <typename T, bool CENSUS>
 __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(sizeof(T) == 4 ? 6 : 1)))
-void k_tree_diffusion(TreeDev t, double cut, double nu, double thr, double thr2d,
+void k_tree_diffusion(TreeDev t, double cut, double nu, double thr,
                                                         const double *__restrict__ sd,
                                                         double *__restrict__ u, double *__restrict__ v,
                                                         unsigned long long *__restrict__ cnt) {
     unsigned long long cp = 0, ci = 0;
-    diffusion_wave<T, CENSUS>(t, cut, nu, thr, thr2d, sd, u, v, cnt, cp, ci);
+    diffusion_wave<T, CENSUS>(t, cut, nu, thr, sd, u, v, cnt, cp, ci);
     block_count_add(cp, ci, cnt, CENSUS ? cnt + 5 : nullptr);
 }
 
@@ -2475,13 +2475,14 @@ __global__ void k_zero_u64(unsigned long long *__restrict__ a, unsigned mask) {
 
 template <typename T>
 __device__ void diff_far_pair(const TreeDev &t, const double4 *__restrict__ ftgt, int64_t H, int64_t k, int64_t ch,
-                              double cut, double thr2d, double *__restrict__ part, unsigned long long &cpairs) {
+                              double cut, double thr, double *__restrict__ part, unsigned long long &cpairs) {
     const int lane = threadIdx.x & 63;
     const double4 tg = ftgt[k];
     const double ax = tg.x, ay = tg.y, di = tg.z;
     const double R2 = (cut * di) * (cut * di);
-    const T kd = (T)(-1.4426950408889634 / di);
-    const T thr2 = (T)thr2d;
+    constexpr bool F32 = sizeof(T) == 4;
+    const T kd = (T)((F32 ? -1.4426950408889634 : 1.0) / di);
+    const T thr2 = F32 ? (T)(thr * thr) : (T)thr;
     // the chunk's buckets, one per lane: box test and the record in one load
     const int64_t b = ch * 64 + lane;
     const bool inb = b < t.nleaf;
@@ -2537,14 +2538,14 @@ template <typename T>
 __global__ __launch_bounds__(256) void k_diff_far(TreeDev t, const double4 *__restrict__ ftgt,
                                                   const int2 *__restrict__ pairs,
                                                   const unsigned long long *__restrict__ npair_list, double cut,
-                                                  double thr2d, double *__restrict__ part,
+                                                  double thr, double *__restrict__ part,
                                                   unsigned long long *__restrict__ cnt) {
     const int64_t H = far_count(cnt, t.fcap);
     const int64_t total = (int64_t)*npair_list;
     const int64_t nw = (int64_t)gridDim.x * 4;
     unsigned long long cp = 0;
     for (int64_t w = (int64_t)blockIdx.x * 4 + (threadIdx.x >> 6); w < total; w += nw)
-        diff_far_pair<T>(t, ftgt, H, pairs[w].x, pairs[w].y, cut, thr2d, part, cp);
+        diff_far_pair<T>(t, ftgt, H, pairs[w].x, pairs[w].y, cut, thr, part, cp);
     block_count_add(cp, 0ull, cnt, nullptr);
 }
 
@@ -3167,7 +3168,7 @@ int tree_diffusion_far(vx_case *c, hipStream_t st) {
     TreeBufs &t = *c->tree;
     const TreeDev tv = view(t);
     const bool mixed = c->prm.precision == VX_PREC_MIXED;
-    const double cut = diff_cut_of(c), thr = 0.001 * c->prm.ve_size, thr2 = mixed ? thr * thr : diff_thr2(thr);
+    const double cut = diff_cut_of(c), thr = 0.001 * c->prm.ve_size;
     unsigned long long *cnt = t.cnt.p + 4;
     // all counts stay on the device (grid-stride kernels sized for the list's capacity)
     const int64_t nchunk = (t.nleaf + 63) / 64;
@@ -3177,10 +3178,10 @@ int tree_diffusion_far(vx_case *c, hipStream_t st) {
                        t.fpairs.p, cnt + 3, t.ftgt.p, t.fmask.p);
     if (mixed)
         hipLaunchKernelGGL(k_diff_far<float>, dim3(4096), dim3(256), 0, st, tv, t.ftgt.p, t.fpairs.p, cnt + 3, cut,
-                           thr2, t.hpart.p, cnt);
+                           thr, t.hpart.p, cnt);
     else
         hipLaunchKernelGGL(k_diff_far<double>, dim3(4096), dim3(256), 0, st, tv, t.ftgt.p, t.fpairs.p, cnt + 3, cut,
-                           thr2, t.hpart.p, cnt);
+                           thr, t.hpart.p, cnt);
     hipLaunchKernelGGL(k_diff_far_final, dim3(1024), dim3(256), 0, st, tv, t.fb.p, cnt, nchunk, t.fmask.p, t.hpart.p,
                        c->d.p, c->prm.nu, c->u.p, c->v.p);
     VX_CHECK(hipGetLastError());
@@ -3193,22 +3194,22 @@ int tree_diffusion_main(vx_case *c) {
     hipStream_t st = c->stream;
     const bool mixed = c->prm.precision == VX_PREC_MIXED;
     const unsigned lb8 = (unsigned)(t.ngroup + 7) / 8 * 8;  // target groups, padded for xcd_block()
-    const double cut = diff_cut_of(c), thr = 0.001 * c->prm.ve_size, thr2 = mixed ? thr * thr : diff_thr2(thr);
+    const double cut = diff_cut_of(c), thr = 0.001 * c->prm.ve_size;
     unsigned long long *cnt = t.cnt.p + 4;
     Timer tk(c, &c->tm.diff_kernel_ms, 8);
     if (c->census) {
         if (mixed)
             hipLaunchKernelGGL((k_tree_diffusion<float, true>), dim3(lb8), dim3(256), 0, st, view(t), cut, c->prm.nu,
-                               thr, thr2, t.sd.p, c->u.p, c->v.p, cnt);
+                               thr, t.sd.p, c->u.p, c->v.p, cnt);
         else
             hipLaunchKernelGGL((k_tree_diffusion<double, true>), dim3(lb8), dim3(256), 0, st, view(t), cut,
-                               c->prm.nu, thr, thr2, t.sd.p, c->u.p, c->v.p, cnt);
+                               c->prm.nu, thr, t.sd.p, c->u.p, c->v.p, cnt);
     } else if (mixed) {
         hipLaunchKernelGGL((k_tree_diffusion<float, false>), dim3(lb8), dim3(256), 0, st, view(t), cut, c->prm.nu,
-                           thr, thr2, t.sd.p, c->u.p, c->v.p, cnt);
+                           thr, t.sd.p, c->u.p, c->v.p, cnt);
     } else {
         hipLaunchKernelGGL((k_tree_diffusion<double, false>), dim3(lb8), dim3(256), 0, st, view(t), cut, c->prm.nu,
-                           thr, thr2, t.sd.p, c->u.p, c->v.p, cnt);
+                           thr, t.sd.p, c->u.p, c->v.p, cnt);
     }
     VX_CHECK(hipGetLastError());
     return 0;
