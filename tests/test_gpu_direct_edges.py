@@ -44,3 +44,65 @@ def test_diffusion_threshold_without_bound(prec, n):
     c.close()
     for a, b in zip(got, (u, v, d)):
         assert np.array_equal(a, b)
+
+
+def velocity_of(x, y, g, prec=VX_PREC_F64, tree=False):
+    n = x.size
+    c = case(prec)
+    c.set_state(x, y, g)
+    if tree:
+        c.tree_biot_savart((n + 31) // 32 * 32)
+    else:
+        c.biot_savart(n, n)
+    out = c.velocity(n)
+    q = c.velocity_probe(np.linspace(0.6, 4.0, 300), np.linspace(-1.0, 1.0, 300), (0.0, 0.0))
+    c.close()
+    return out, q
+
+
+def odd_wake(n, px, py, at=None):
+    """A wake and the same with vortices at (px, py); in the first those slots
+    are dead and far."""
+    x, y, g = uniform_wake(n, seed=n)
+    at = np.array([5, n // 2, n - 3][:len(px)])
+    x[at], y[at] = 1e10, 1e10
+    g0 = g.copy()
+    g0[at] = 0.0
+    x1, y1 = x.copy(), y.copy()
+    x1[at], y1[at] = px, py
+    rest = np.ones(n, bool)
+    rest[at] = False
+    return (x, y, g0), (x1, y1, g), at, rest
+
+
+@pytest.mark.parametrize("n", [100, 5000, 20000])
+@pytest.mark.parametrize("px,py", [((np.nan,), (0.5,)), ((1.0, 1.0), (np.nan, np.nan)), ((np.inf, np.inf), (1.0, 1.0)),
+                                   ((-np.inf, np.inf, 2.0), (0.0, 0.0, np.inf))])
+def test_sources_without_a_place(n, px, py):
+    """Every velocity is NaN then; a NaN or infinite distance is no near one."""
+    plain, odd, at, rest = odd_wake(n, px, py)
+    (_, _, d0), _ = velocity_of(*plain)
+    (u, v, d), q = velocity_of(*odd)
+    assert np.all(np.isnan(u)) or np.all(np.isnan(v))
+    assert np.array_equal(d[rest], d0[rest])
+    # (the padding slots are far, not nowhere)
+    np.testing.assert_allclose(d[at], np.sqrt(1e5), rtol=1e-15)
+    assert np.all(np.isnan(q[0])) or np.all(np.isnan(q[1]))
+
+
+@pytest.mark.parametrize("n,tree", [(100, False), (5000, False), (20000, False), (60, True), (300, True)])
+@pytest.mark.parametrize("px,py", [((1e200,), (0.0,)), ((1e200, 2e200, -1e180), (0.0, 0.0, 1e190)),
+                                   ((1e151, 1.2e151), (3e154, -3e154))])
+def test_sources_beyond_the_square_root_of_the_range(n, tree, px, py):
+    """Their squared distances are infinite or as good as: they add nothing."""
+    plain, odd, at, rest = odd_wake(n, px, py)
+    (u0, v0, d0), q0 = velocity_of(*plain, tree=tree)
+    (u, v, d), q = velocity_of(*odd, tree=tree)
+    tol = 1e-12 if tree else 0.0  # the trees differ
+    for a, b in ((u, u0), (v, v0), (d, d0)):
+        np.testing.assert_allclose(a[rest], b[rest], rtol=0, atol=tol * np.max(np.abs(b[rest])))
+    assert not u[at].any() and not v[at].any()
+    np.testing.assert_allclose(d[at], np.sqrt(1e5), rtol=1e-15)
+    for a, b in zip(q, q0):
+        assert np.array_equal(a, b)
+    assert np.all(np.isfinite(q[0]))

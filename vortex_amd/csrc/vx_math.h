@@ -20,6 +20,12 @@ __device__ __forceinline__ double div_pos_exact(double g, double a) {
     return fma(fma(-a, w, g), y, w);
 }
 
+// g / a for any a >= 0 that is no denormal number: infinities, zeros and NaN as
+// `/` has them.
+__device__ __forceinline__ double div_nonneg(double g, double a) {
+    return __builtin_amdgcn_div_fixup(div_pos_exact(g, a), a, g);
+}
+
 // sqrt(a) for a normal a > 0, correctly rounded as sqrt() gives it, and g over
 // it, correctly rounded, by the same steps (the start's e = (1 - a y^2) / 2 is
 // below 2^-24; 2^30 random pairs: no difference from sqrt and `/`).
@@ -44,6 +50,7 @@ __device__ __forceinline__ void order2(double &a, double &b) {
 // Four values at a time: they are sorted (5 exchanges), the pairwise minima
 // with the kept ones in reverse are the four smallest of the eight, a bitonic
 // run that 4 exchanges sort.  FP64 has no med3: 5.5 min/max a value against 13.
+// The values must be no NaN (an exchange would double its neighbour).
 __device__ __forceinline__ void keep4x4(double &m0, double &m1, double &m2, double &m3, double a, double b, double c,
                                         double d) {
     order2(a, b);
@@ -60,15 +67,19 @@ __device__ __forceinline__ void keep4x4(double &m0, double &m1, double &m2, doub
     order2(m0, m1);
     order2(m2, m3);
 }
-// A finite coordinate held within 1e150, so that squared distances stay
-// finite (such a source then counts as it did: weight 0, never near).
-// Infinities and NaN pass.  Integer compares only: on wave-uniform values
-// they run on the scalar unit.
-__device__ __forceinline__ double far_clamp(double v) {
-    const int hi = __double2hiint(v), a = hi & 0x7fffffff;
-    constexpr int kHi = 0x5f138d35;  // high word of 1e150
-    return a > kHi && a < 0x7ff00000 ? __hiloint2double((hi & (int)0x80000000) | kHi, 0) : v;
-}
-__device__ __forceinline__ float far_clamp(float v) { return v; }
+
+// Neither NaN nor an infinity nor above 2^500, so that squares of differences
+// stay in range: the sizes (high words without sign) of several values are
+// compared at once by their maximum.  Integer operations only: on wave-uniform
+// values they run on the scalar unit.
+constexpr int kOrdinary = 0x5f300000;
+__device__ __forceinline__ int size_of(double v) { return __double2hiint(v) & 0x7fffffff; }
+__device__ __forceinline__ int size_of(float) { return 0; }  // FP32 takes every value through one path
+template <typename T>
+__device__ __forceinline__ bool ordinary(T v) { return size_of(v) < kOrdinary; }
+
+// A softening eps^2 that div_pos_exact divides by.
+__device__ __forceinline__ bool ordinary_eps2(double v) { return v > 0x1p-1000 && v < 0x1p1000; }
+__device__ __forceinline__ bool ordinary_eps2(float) { return true; }
 
 }  // namespace vx

@@ -12,7 +12,7 @@
 #include <cmath>
 #include <mutex>
 #include <string>
-
+#include <type_traits>
 
 #include "vx_internal.h"
 #include "vx_math.h"
@@ -171,47 +171,59 @@ __global__ __launch_bounds__(kTile) void k_biot_savart(const T *__restrict__ sx,
     const int32_t t0 = (int32_t)(t * (kTile * TPT) + threadIdx.x);
     T ax[TPT], ay[TPT], m0[TPT], m1[TPT], m2[TPT], m3[TPT], su[TPT], sv[TPT];
     double au[TPT], av[TPT];
+    bool tame = ordinary_eps2(eps2);
 #pragma unroll
     for (int k = 0; k < TPT; ++k) {
         const int32_t i = t0 + k * kTile;
-        ax[k] = i < n_tgt ? far_clamp(sx[i]) : T(0);
-        ay[k] = i < n_tgt ? far_clamp(sy[i]) : T(0);
+        ax[k] = i < n_tgt ? sx[i] : T(0);
+        ay[k] = i < n_tgt ? sy[i] : T(0);
+        tame = tame && ordinary(ax[k]) && ordinary(ay[k]);
         m0[k] = m1[k] = m2[k] = m3[k] = T(1e5);
         su[k] = sv[k] = T(0);
         au[k] = av[k] = 0.0;
     }
-    auto pair = [&](int k, T x, T y, T g) {
+    tame = !__any(!tame);
+    auto pair = [&](int k, T x, T y, T g, auto plain) {
         const T dx = ax[k] - x, dy = ay[k] - y;
         const T r2 = dx * dx + dy * dy;
-        const T w = A::div(g, A::max_(r2, eps2));
+        const T a = A::max_(r2, eps2);
+        T w;
+        if constexpr (decltype(plain)::value)
+            w = g / a;
+        else
+            w = A::div(g, a);
         sv[k] += w * dx;
         su[k] -= w * dy;
         return r2;
     };
+    constexpr std::integral_constant<bool, sizeof(T) == 8> plain64;
     for (int32_t base = lo; base < hi; base += kTile) {
         const int32_t end = min(hi, base + kTile);
         int32_t j = base;
         for (; j + 4 <= end; j += 4) {
             T x[4], y[4], g[4];
+            int size = 0;
 #pragma unroll
             for (int q = 0; q < 4; ++q) {
-                x[q] = far_clamp(sx[j + q]);
-                y[q] = far_clamp(sy[j + q]);
+                x[q] = sx[j + q];
+                y[q] = sy[j + q];
                 g[q] = sg[j + q];
+                size = max(size, max(size_of(x[q]), size_of(y[q])));
             }
+            if (__builtin_expect(!tame || size >= kOrdinary, 0)) break;
 #pragma unroll
             for (int k = 0; k < TPT; ++k) {
                 T r2[4];
 #pragma unroll
-                for (int q = 0; q < 4; ++q) r2[q] = pair(k, x[q], y[q], g[q]);
+                for (int q = 0; q < 4; ++q) r2[q] = pair(k, x[q], y[q], g[q], std::false_type());
                 keep4x4(m0[k], m1[k], m2[k], m3[k], r2[0], r2[1], r2[2], r2[3]);
             }
         }
-        for (; j < end; ++j) {
-            const T x = far_clamp(sx[j]), y = far_clamp(sy[j]), g = sg[j];
+        for (; j < end; ++j) {  // the last ones, and the rest of a tile with unordinary values
+            const T x = sx[j], y = sy[j], g = sg[j];
 #pragma unroll
             for (int k = 0; k < TPT; ++k) {
-                const T r2 = pair(k, x, y, g);
+                const T r2 = pair(k, x, y, g, plain64);
                 keep4(m0[k], m1[k], m2[k], m3[k], r2);
             }
         }
@@ -312,11 +324,6 @@ __device__ __forceinline__ void diff_pair_plain(double dx, double dy, double g, 
     }
 }
 
-// Neither NaN nor an infinity nor above 2^500, so that squares of differences
-// stay in range.  Integer compares only: on wave-uniform values they run on the
-// scalar unit.
-__device__ __forceinline__ bool ordinary(double v) { return (__double2hiint(v) & 0x7fffffff) < 0x5f300000; }
-
 template <typename T, int TPT>
 __global__ __launch_bounds__(kTile) void k_diffusion(const T *__restrict__ sx, const T *__restrict__ sy,
                                                      const T *__restrict__ sg, Cnt cn_src, Cnt cn_tgt,
@@ -353,14 +360,15 @@ __global__ __launch_bounds__(kTile) void k_diffusion(const T *__restrict__ sx, c
         int32_t j = lo;
         for (; j + 4 <= hi; j += 4) {
             double x[4], y[4], g[4];
-            bool plain = !tame;
+            int size = 0;
 #pragma unroll
             for (int q = 0; q < 4; ++q) {
                 x[q] = sx[j + q];
                 y[q] = sy[j + q];
                 g[q] = sg[j + q];
-                plain = plain || !ordinary(x[q]) || !ordinary(y[q]) || !ordinary(g[q]);
+                size = max(size, max(size_of(x[q]), max(size_of(y[q]), size_of(g[q]))));
             }
+            const bool plain = !tame || size >= kOrdinary;
 #pragma unroll
             for (int k = 0; k < TPT; ++k) {
                 double r2[4];
@@ -533,6 +541,7 @@ __global__ __launch_bounds__(1024) void k_biot_savart_ordered(const double *__re
     const int32_t i = (int32_t)blockIdx.x * TG + t, ic = min(i, n_tgt - 1);
     const double ax = sx[ic], ay = sy[ic];
     double m0 = 1e5, m1 = 1e5, m2 = 1e5, m3 = 1e5;
+    const bool plain = !ordinary_eps2(eps2);
     // the chain of lane (t, slot): sv of dx for even slots, su of -dy for odd
     const bool xr = !(slot & 1);
     const double c1 = xr ? -1.0 : 1.0, c0 = xr ? ax : -ay;
@@ -556,13 +565,13 @@ __global__ __launch_bounds__(1024) void k_biot_savart_ordered(const double *__re
                     r2[q] = fma(dx, dx, dy * dy);
                     const double a = fmax(r2[q], eps2);
                     double w = div_pos_exact(g, a);
-                    if (__builtin_expect(__any(!(a < 1e300)), 0)) {
+                    if (__builtin_expect(plain || __any(!(a < 1e300)), 0)) {
                         asm volatile("; rare: kept out of the main path");
                         w = g / a;
                     }
                     const bool in = k * TILE + jj < n_src;
                     w_[(jj >> 1) * (2 * TG) + 2 * t + (jj & 1)] = in ? w : 0.0;
-                    r2[q] = in ? r2[q] : 1e5;
+                    r2[q] = in ? fmin(r2[q], 1e5) : 1e5;  // no NaN in the lists, which start at 1e5
                 }
                 if constexpr (Q == 4)
                     keep4x4(m0, m1, m2, m3, r2[0], r2[1], r2[2], r2[3]);
@@ -1411,19 +1420,30 @@ __global__ __launch_bounds__(kTile) void k_probe_partial(const double *__restric
     const int64_t i = (int64_t)blockIdx.x * kTile + threadIdx.x;
     const int64_t c = blockIdx.y;
     const int64_t lo = c * chunk, hi = min(n_src, lo + chunk);
-    const double a0 = i < m ? far_clamp(px[i]) : 0.0, a1 = i < m ? far_clamp(py[i]) : 0.0;
+    const double a0 = i < m ? px[i] : 0.0, a1 = i < m ? py[i] : 0.0;
+    const bool tame = ordinary(a0) && ordinary(a1) && ordinary_eps2(eps2);
     double su = 0.0, sv = 0.0;
     for (int64_t base = lo; base < hi; base += kTile) {
         __syncthreads();
         const int64_t j = base + threadIdx.x;
         Src4<double> s;
-        s.x = j < hi ? far_clamp(sx[j]) : A::kFar;
-        s.y = j < hi ? far_clamp(sy[j]) : A::kFar;
+        s.x = j < hi ? sx[j] : A::kFar;
+        s.y = j < hi ? sy[j] : A::kFar;
         s.g = j < hi ? sg[j] : 0.0;
         s.pad = 0.0;
         ls[threadIdx.x] = s;
-        __syncthreads();
+        const bool plain = __syncthreads_or(!(tame && ordinary(s.x) && ordinary(s.y)));
         const int cnt = (int)min((int64_t)kTile, hi - base);
+        if (plain) {
+            for (int jj = 0; jj < cnt; ++jj) {
+                const Src4<double> q = ls[jj];
+                const double dx = a0 - q.x, dy = a1 - q.y;
+                const double w = q.g / A::max_(dx * dx + dy * dy, eps2);
+                sv += w * dx;
+                su -= w * dy;
+            }
+            continue;
+        }
         for (int jj = 0; jj < cnt; ++jj) {
             const Src4<double> q = ls[jj];
             const double dx = a0 - q.x, dy = a1 - q.y;

@@ -966,7 +966,9 @@ template <typename T>
 struct PairMath;
 template <>
 struct PairMath<double> {
-    __device__ static __forceinline__ double div(double a, double b) { return div_pos_exact(a, b); }
+    // (vortices with circulation are included however far they are: squared
+    // distances may be infinite)
+    __device__ static __forceinline__ double div(double a, double b) { return div_nonneg(a, b); }
     __device__ static __forceinline__ double sqrt_bound(double a) { return sqrt(a); }
     __device__ static __forceinline__ double med3(double a, double b, double c) {
         return fmax(fmin(a, b), fmin(fmax(a, b), c));
