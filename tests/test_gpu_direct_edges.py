@@ -106,3 +106,32 @@ def test_sources_beyond_the_square_root_of_the_range(n, tree, px, py):
     for a, b in zip(q, q0):
         assert np.array_equal(a, b)
     assert np.all(np.isfinite(q[0]))
+
+
+@pytest.mark.parametrize("big", [np.inf, -np.inf, np.nan])
+@pytest.mark.parametrize("n,k", [(100, 50), (100, 99), (5000, 7), (5000, 4999), (20000, 123), (20001, 20000)])
+def test_circulation_without_bound(n, k, big):
+    """Velocities follow its sign (or are NaN); in the diffusion it counts for the
+    others alone, whose quotient of sums it makes NaN (or leaves out)."""
+    x, y, g = uniform_wake(n, seed=n)
+    rest = np.arange(n) != k
+    g[k] = big
+    (u, v, _), q = velocity_of(x, y, g)
+    dx, dy = x - x[k], y - y[k]
+    with np.errstate(invalid="ignore"):
+        for got, want in ((u, -big * np.sign(dy)), (v, big * np.sign(dx)),
+                          (q[0], -big * np.sign(np.linspace(-1.0, 1.0, 300) - y[k])),
+                          (q[1], big * np.sign(np.linspace(0.6, 4.0, 300) - x[k]))):
+            assert np.array_equal(got, want, equal_nan=True)
+    res = []
+    for gk in (big, 0.0):
+        g[k] = gk
+        c = case(VX_PREC_F64)
+        c.set_state(x, y, g)
+        c.set_velocity(np.full(n, 0.25), np.full(n, -0.5), np.full(n, 0.1))
+        c.diffusion(n, n)
+        res.append(c.velocity(n)[:2])
+        c.close()
+    for a, b, z in zip(res[0], res[1], (0.25, -0.5)):
+        assert a[k] == b[k] != z
+        assert np.all(a[rest] == z) if np.isnan(big) else np.all(np.isnan(a[rest]))

@@ -208,7 +208,7 @@ __global__ __launch_bounds__(kTile) void k_biot_savart(const T *__restrict__ sx,
                 x[q] = sx[j + q];
                 y[q] = sy[j + q];
                 g[q] = sg[j + q];
-                size = max(size, max(size_of(x[q]), size_of(y[q])));
+                size = max(size, max(size_of(x[q]), max(size_of(y[q]), size_of(g[q]))));
             }
             if (__builtin_expect(!tame || size >= kOrdinary, 0)) break;
 #pragma unroll
@@ -565,7 +565,7 @@ __global__ __launch_bounds__(1024) void k_biot_savart_ordered(const double *__re
                     r2[q] = fma(dx, dx, dy * dy);
                     const double a = fmax(r2[q], eps2);
                     double w = div_pos_exact(g, a);
-                    if (__builtin_expect(plain || __any(!(a < 1e300)), 0)) {
+                    if (__builtin_expect(plain || __any(!(a < 1e300) || !(fabs(g) < 1e300)), 0)) {
                         asm volatile("; rare: kept out of the main path");
                         w = g / a;
                     }
@@ -638,7 +638,11 @@ __global__ __launch_bounds__(1024) void k_biot_savart_ordered(const double *__re
 
 // The diffusion's three chains: x and y terms (w dx) e, (w dy) e with w = g /
 // r on lanes of their own, and I1's g e beside both.  A pair within the
-// threshold, or past the end, has e = 0.
+// threshold, or past the end, has e = 0.  A circulation that is no finite
+// number is staged as kNoNumber, which leaves such pairs' products zero; its own
+// value then comes with e.
+constexpr double kNoNumber = 0x1p-1074;
+
 template <int TG, int Q>
 __global__ __launch_bounds__(1024) void k_diffusion_ordered(const double *__restrict__ sx,
                                                             const double *__restrict__ sy,
@@ -657,13 +661,18 @@ __global__ __launch_bounds__(1024) void k_diffusion_ordered(const double *__rest
     double acc = 0.0, acc1 = 0.0;
     const int32_t tiles = (n_src + TILE - 1) / TILE;
     const bool stager = threadIdx.x < TILE;
-    if (stager && tiles) src.put(0, threadIdx.x, ord_src(sx, sy, sg, threadIdx.x, n_src));
+    auto source = [&](int32_t j) {
+        double3 q = ord_src(sx, sy, sg, j, n_src);
+        if (!(fabs(q.z) < INFINITY)) q.z = kNoNumber;
+        return q;
+    };
+    if (stager && tiles) src.put(0, threadIdx.x, source(threadIdx.x));
     __syncthreads();
     int b0 = 0, b1 = 1, b2 = 2;
     for (int32_t k = 0; k <= tiles; ++k) {
         const int b = k & 1;
         double3 next;
-        if (stager && k + 1 < tiles) next = ord_src(sx, sy, sg, (k + 1) * TILE + (int32_t)threadIdx.x, n_src);
+        if (stager && k + 1 < tiles) next = source((k + 1) * TILE + (int32_t)threadIdx.x);
         if (wv < kOrdWaves) {
             if (k < tiles) {
 #pragma unroll
@@ -671,14 +680,18 @@ __global__ __launch_bounds__(1024) void k_diffusion_ordered(const double *__rest
                     const int jj = (q * kOrdWaves + wv) * SL + slot;
                     const double dx = ax - src.c[b0][0][jj], dy = ay - src.c[b0][1][jj], g = src.c[b0][2][jj];
                     const double r2 = fma(dx, dx, dy * dy);
-                    double w, dist = sqrt_pos_exact(r2, g, w);
-                    if (__builtin_expect(__any(r2 > 1e300), 0)) {
+                    double w, dist = sqrt_pos_exact(r2, g, w), own = 1.0;
+                    const bool rare = __any(r2 > 1e300 || g == kNoNumber);
+                    if (__builtin_expect(rare, 0)) {
                         asm volatile("; rare: kept out of the main path");
+                        const double gj = g == kNoNumber ? sg[min(k * TILE + jj, n_src - 1)] : g;
+                        own = fabs(gj) < INFINITY ? 1.0 : gj;
                         dist = sqrt(r2);
-                        w = g / dist;
+                        w = gj / dist;
                     }
                     const bool on = dist > thr && k * TILE + jj < n_src;
-                    const double e = exp(-dist * kd);
+                    double e = exp(-dist * kd);
+                    if (__builtin_expect(rare, 0)) e *= own;
                     double *o = (double *)&lt[b][0][jj >> 1][t] + (jj & 1);
                     o[0] = on ? w * dx : 0.0;
                     o[TILE * TG] = on ? w * dy : 0.0;
@@ -1432,7 +1445,7 @@ __global__ __launch_bounds__(kTile) void k_probe_partial(const double *__restric
         s.g = j < hi ? sg[j] : 0.0;
         s.pad = 0.0;
         ls[threadIdx.x] = s;
-        const bool plain = __syncthreads_or(!(tame && ordinary(s.x) && ordinary(s.y)));
+        const bool plain = __syncthreads_or(!(tame && ordinary(s.x) && ordinary(s.y) && ordinary(s.g)));
         const int cnt = (int)min((int64_t)kTile, hi - base);
         if (plain) {
             for (int jj = 0; jj < cnt; ++jj) {
