@@ -45,8 +45,13 @@ struct WallLds {
     T prod[64], ex[64];
 };
 
-template <typename T>
-__device__ void wave_wall(const PanelsSoA &pan, int lane, double x, double y, T dd, int32_t N, WallLds<T> &L,
+//
+// I counts points: 32 bits while a round's 64 N points fit them (kShortPoints),
+// whose quotient by N is a few instructions against some hundred in 64 bits.
+constexpr int64_t kShortPoints = 1 << 24;
+
+template <typename T, typename I>
+__device__ void wave_wall(const PanelsSoA &pan, int lane, double x, double y, T dd, I N, WallLds<T> &L,
                           double &II0, double &II30, double &II31) {
     constexpr bool F32 = sizeof(T) == 4;
     const double ox = F32 ? x : 0.0, oy = F32 ? y : 0.0;
@@ -97,10 +102,10 @@ __device__ void wave_wall(const PanelsSoA &pan, int lane, double x, double y, T 
             __builtin_amdgcn_wave_barrier();
             const WallPanel<T> mine = L.p[lane < cnt ? lane : 0];  // the panel whose terms this lane adds
             T s0 = 0, s30 = 0, s31 = 0;
-            const int32_t total = cnt * N;
-            for (int32_t t0 = 0; t0 < total; t0 += 64) {
-                const int32_t t = t0 + lane < total ? t0 + lane : total - 1;
-                const int32_t e = t / N, k = t - e * N;
+            const I total = cnt * N;
+            for (I t0 = 0; t0 < total; t0 += 64) {
+                const I t = t0 + lane < total ? t0 + lane : total - 1;
+                const I e = t / N, k = t - e * N;
                 const WallPanel<T> &q = L.p[e];
                 const T rk0 = fma((T)(k + 1), q.dR0, fma((T)k, q.dR0, q.ra0) + q.ra0);
                 const T rk1 = fma((T)(k + 1), q.dR1, fma((T)k, q.dR1, q.ra1) + q.ra1);
@@ -112,9 +117,9 @@ __device__ void wave_wall(const PanelsSoA &pan, int lane, double x, double y, T 
                 L.prod[lane] = fma(e1, q.n1, e0 * q.n0) / e2 * (me + T(1)) * ex;
                 L.ex[lane] = ex;
                 __builtin_amdgcn_wave_barrier();
-                const int32_t lo = max(lane * N, t0), hi = lane < cnt ? min(lane * N + N, t0 + 64) : 0;
+                const I lo = max(lane * N, t0), hi = lane < cnt ? min(lane * N + N, t0 + 64) : 0;
 #pragma unroll 4
-                for (int32_t u = lo; u < hi; ++u) {
+                for (I u = lo; u < hi; ++u) {
                     const T pr = L.prod[u - t0], xk = L.ex[u - t0];
                     s0 = fma(mine.delt, pr, s0);
                     s30 = fma(mine.delt, mine.n0 * xk, s30);
@@ -164,13 +169,14 @@ struct InWallBox {
 // wst (u term at 2t, v term at 2t + 1) and k_wall_add adds them; with ADD (no
 // other stream is writing u and v) the wave adds its own: a launch of 4.7 us less
 // in a captured step.
-template <typename T, bool ADD>
+template <typename T, bool ADD, typename I>
 __global__ __launch_bounds__(256) void k_diffusion_wall(const double *__restrict__ x,
                                                         const double *__restrict__ y,
                                                         const double *__restrict__ d,
                                                         const int32_t *__restrict__ list,
                                                         const int32_t *__restrict__ cnt, PanelsSoA pan,
-                                                        double nu, int32_t npts, double *__restrict__ wst, double *__restrict__ u,
+                                                        double nu, I npts, double *__restrict__ wst,
+                                                        double *__restrict__ u,
                                                         double *__restrict__ v) {
     __shared__ WallLds<T> lds[4];
     const int lane = threadIdx.x & 63;
@@ -179,7 +185,7 @@ __global__ __launch_bounds__(256) void k_diffusion_wall(const double *__restrict
     for (int64_t t = (int64_t)blockIdx.x * 4 + (threadIdx.x >> 6); t < total; t += nw) {
         const int64_t i = list[t];
         double II0, II30, II31;
-        wave_wall<T>(pan, lane, x[i], y[i], (T)d[i], npts, lds[threadIdx.x >> 6], II0, II30, II31);
+        wave_wall<T, I>(pan, lane, x[i], y[i], (T)d[i], npts, lds[threadIdx.x >> 6], II0, II30, II31);
         if (lane == 0) {
             if constexpr (ADD) {
                 u[i] += nu * II30 / II0;
@@ -198,9 +204,9 @@ __global__ __launch_bounds__(256) void k_diffusion_wall(const double *__restrict
 // 10.5 us.
 constexpr int64_t kScanMax = 32768;
 
-template <typename T>
+template <typename T, typename I>
 __global__ __launch_bounds__(256) void k_wall_scan(InWallBox pred, Cnt cn, const double *__restrict__ d, PanelsSoA pan,
-                                                   double nu, int32_t npts, double *__restrict__ u,
+                                                   double nu, I npts, double *__restrict__ u,
                                                    double *__restrict__ v) {
     __shared__ WallLds<T> lds[4];
     const int lane = threadIdx.x & 63;
@@ -209,7 +215,7 @@ __global__ __launch_bounds__(256) void k_wall_scan(InWallBox pred, Cnt cn, const
     for (uint64_t m = __ballot(mine < n && pred((int32_t)mine)); m; m &= m - 1) {
         const int64_t i = w + nw * __builtin_ctzll(m);
         double II0, II30, II31;
-        wave_wall<T>(pan, lane, pred.x[i], pred.y[i], (T)d[i], npts, lds[threadIdx.x >> 6], II0, II30, II31);
+        wave_wall<T, I>(pan, lane, pred.x[i], pred.y[i], (T)d[i], npts, lds[threadIdx.x >> 6], II0, II30, II31);
         if (lane == 0) {
             u[i] += nu * II30 / II0;
             v[i] += nu * II31 / II0;
@@ -228,25 +234,20 @@ __global__ __launch_bounds__(256) void k_wall_add(const int32_t *__restrict__ li
     }
 }
 
-template <bool ADD>
-static int wall_pass(vx_case *c, Cnt cn_tgt, hipStream_t st) {
+template <bool ADD, typename T, typename I>
+static int wall_pass_as(vx_case *c, Cnt cn_tgt, hipStream_t st) {
     const int64_t n_tgt = cn_tgt.ub;  // bound: list sizes and the selection's grid
-    if (n_tgt <= 0 || c->P <= 0) return 0;
     // buffers grow on the main stream: a reallocation synchronises it, and
     // with it every earlier side-stream pass (joined into it)
     if (c->wlist.ensure((size_t)n_tgt, c->stream) || c->dcount.ensure(16, c->stream) ||
         (!ADD && c->wstage.ensure((size_t)(2 * n_tgt), c->stream)))
         return 1;
-    const int32_t npts = (int32_t)std::clamp<int64_t>(c->prm.n_of_points, 0, 1 << 24);
+    const I npts = (I)c->prm.n_of_points;
     const InWallBox pred{c->x.p, c->y.p, c->wall_box};
     if (ADD && n_tgt <= kScanMax) {
         const dim3 grid((unsigned)std::min<int64_t>(1024, (n_tgt + 3) / 4));
-        if (c->prm.precision == VX_PREC_MIXED)
-            hipLaunchKernelGGL(k_wall_scan<float>, grid, dim3(256), 0, st, pred, cn_tgt, c->d.p, c->pan, c->prm.nu, npts,
-                               c->u.p, c->v.p);
-        else
-            hipLaunchKernelGGL(k_wall_scan<double>, grid, dim3(256), 0, st, pred, cn_tgt, c->d.p, c->pan, c->prm.nu, npts,
-                               c->u.p, c->v.p);
+        hipLaunchKernelGGL((k_wall_scan<T, I>), grid, dim3(256), 0, st, pred, cn_tgt, c->d.p, c->pan, c->prm.nu, npts,
+                           c->u.p, c->v.p);
         VX_CHECK(hipGetLastError());
         return 0;
     }
@@ -254,14 +255,19 @@ static int wall_pass(vx_case *c, Cnt cn_tgt, hipStream_t st) {
     if (c->wtmp.ensure((size_t)prim::tiles_of(n_tgt) + 1, c->stream)) return 1;
     VX_CHECK(prim::select_flags(prim::pred_flag(pred, cn_tgt), n_tgt, prim::WriteIndex{c->wlist.p}, c->wtmp.p, cnt,
                                 st));
-    if (c->prm.precision == VX_PREC_MIXED)
-        hipLaunchKernelGGL((k_diffusion_wall<float, ADD>), dim3(1024), dim3(256), 0, st, c->x.p, c->y.p, c->d.p,
-                           c->wlist.p, cnt, c->pan, c->prm.nu, npts, c->wstage.p, c->u.p, c->v.p);
-    else
-        hipLaunchKernelGGL((k_diffusion_wall<double, ADD>), dim3(1024), dim3(256), 0, st, c->x.p, c->y.p, c->d.p,
-                           c->wlist.p, cnt, c->pan, c->prm.nu, npts, c->wstage.p, c->u.p, c->v.p);
+    hipLaunchKernelGGL((k_diffusion_wall<T, ADD, I>), dim3(1024), dim3(256), 0, st, c->x.p, c->y.p, c->d.p, c->wlist.p,
+                       cnt, c->pan, c->prm.nu, npts, c->wstage.p, c->u.p, c->v.p);
     VX_CHECK(hipGetLastError());
     return 0;
+}
+
+template <bool ADD>
+static int wall_pass(vx_case *c, Cnt cn_tgt, hipStream_t st) {
+    if (cn_tgt.ub <= 0 || c->P <= 0) return 0;
+    const bool shorts = c->prm.n_of_points <= kShortPoints;
+    if (c->prm.precision == VX_PREC_MIXED)
+        return shorts ? wall_pass_as<ADD, float, int32_t>(c, cn_tgt, st) : wall_pass_as<ADD, float, int64_t>(c, cn_tgt, st);
+    return shorts ? wall_pass_as<ADD, double, int32_t>(c, cn_tgt, st) : wall_pass_as<ADD, double, int64_t>(c, cn_tgt, st);
 }
 
 int launch_wall_side(vx_case *c, int64_t n_tgt, hipStream_t st) {
