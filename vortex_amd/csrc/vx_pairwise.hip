@@ -565,7 +565,8 @@ __global__ __launch_bounds__(1024) void k_biot_savart_ordered(const double *__re
                     r2[q] = fma(dx, dx, dy * dy);
                     const double a = fmax(r2[q], eps2);
                     double w = div_pos_exact(g, a);
-                    if (__builtin_expect(plain || __any(!(a < 1e300) || !(fabs(g) < 1e300)), 0)) {
+                    // (an infinite a or g leaves NaN)
+                    if (__builtin_expect(plain || __any(!(fabs(w) < INFINITY)), 0)) {
                         asm volatile("; rare: kept out of the main path");
                         w = g / a;
                     }
@@ -639,9 +640,10 @@ __global__ __launch_bounds__(1024) void k_biot_savart_ordered(const double *__re
 // The diffusion's three chains: x and y terms (w dx) e, (w dy) e with w = g /
 // r on lanes of their own, and I1's g e beside both.  A pair within the
 // threshold, or past the end, has e = 0.  A circulation that is no finite
-// number is staged as kNoNumber, which leaves such pairs' products zero; its own
-// value then comes with e.
-constexpr double kNoNumber = 0x1p-1074;
+// number is staged as kNoNumber, which leaves such pairs' products zero, and
+// far away, where every pair takes the plain expressions: they read its own
+// place and value, and the value comes with e.
+constexpr double kNoNumber = 0x1p-1074, kNoPlace = 1e300;
 
 template <int TG, int Q>
 __global__ __launch_bounds__(1024) void k_diffusion_ordered(const double *__restrict__ sx,
@@ -663,8 +665,7 @@ __global__ __launch_bounds__(1024) void k_diffusion_ordered(const double *__rest
     const bool stager = threadIdx.x < TILE;
     auto source = [&](int32_t j) {
         double3 q = ord_src(sx, sy, sg, j, n_src);
-        if (!(fabs(q.z) < INFINITY)) q.z = kNoNumber;
-        return q;
+        return fabs(q.z) < INFINITY ? q : double3{kNoPlace, q.y, kNoNumber};
     };
     if (stager && tiles) src.put(0, threadIdx.x, source(threadIdx.x));
     __syncthreads();
@@ -678,16 +679,18 @@ __global__ __launch_bounds__(1024) void k_diffusion_ordered(const double *__rest
 #pragma unroll
                 for (int q = 0; q < Q; ++q) {
                     const int jj = (q * kOrdWaves + wv) * SL + slot;
-                    const double dx = ax - src.c[b0][0][jj], dy = ay - src.c[b0][1][jj], g = src.c[b0][2][jj];
-                    const double r2 = fma(dx, dx, dy * dy);
+                    double dx = ax - src.c[b0][0][jj], dy = ay - src.c[b0][1][jj];
+                    const double g = src.c[b0][2][jj], r2 = fma(dx, dx, dy * dy);
                     double w, dist = sqrt_pos_exact(r2, g, w), own = 1.0;
-                    const bool rare = __any(r2 > 1e300 || g == kNoNumber);
+                    const bool rare = __any(r2 > 1e300);
                     if (__builtin_expect(rare, 0)) {
                         asm volatile("; rare: kept out of the main path");
-                        const double gj = g == kNoNumber ? sg[min(k * TILE + jj, n_src - 1)] : g;
-                        own = fabs(gj) < INFINITY ? 1.0 : gj;
-                        dist = sqrt(r2);
-                        w = gj / dist;
+                        const double3 q = ord_src(sx, sy, sg, k * TILE + jj, n_src);
+                        dx = ax - q.x;
+                        dy = ay - q.y;
+                        own = fabs(q.z) < INFINITY ? 1.0 : q.z;
+                        dist = sqrt(fma(dx, dx, dy * dy));
+                        w = q.z / dist;
                     }
                     const bool on = dist > thr && k * TILE + jj < n_src;
                     double e = exp(-dist * kd);
