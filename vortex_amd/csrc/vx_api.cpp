@@ -740,33 +740,31 @@ int vx_case_autotune(vx_case *c, double vinf_x, double vinf_y, vx_tuning *out) {
         best.ms_default = tdef;
         best.ms_best = tbest;
     } else {
-        // each direct kernel for each number of targets per thread
-        const int tpts[4] = {1, 2, 4, 8};
-        const int def = direct_tpt_default(c->prm.precision == VX_PREC_MIXED, s);
+        // each direct kernel for each number of targets per thread; where the
+        // kernels do not use it, once, and the setting stays
+        const bool uses = direct_uses_tpt(c->prm.precision == VX_PREC_MIXED, s);
+        const int def = direct_tpt_default();
         double bdef = 0.0, bbest = 1e300, ddef = 0.0, dbest = 1e300;
-        for (int q = 0; q < 4; ++q) {
-            c->tune.tpt_bs = tpts[q];
-            double t = 0.0;
-            if (time_ms(c, kReps, [&] { return launch_biot_savart(c, s, s, vinf_x, vinf_y); }, &t)) return 1;
-            ++best.trials;
-            if (tpts[q] == def) bdef = t;
-            if (t < bbest) {
-                bbest = t;
-                best.tpt_bs = tpts[q];
+        auto tune = [&](int32_t &field, int32_t &choice, auto run, double *tdef, double *tbest) {
+            const int32_t tpts[4] = {uses ? 1 : field, 2, 4, 8};
+            for (int k = 0; k < (uses ? 4 : 1); ++k) {
+                const int32_t q = tpts[k];
+                double t = 0.0;
+                field = q;
+                if (time_ms(c, kReps, run, &t)) return 1;
+                ++best.trials;
+                if (q == def || !uses) *tdef = t;
+                if (t < *tbest) {
+                    *tbest = t;
+                    choice = q;
+                }
             }
-        }
-        c->tune.tpt_bs = best.tpt_bs;
-        for (int q = 0; q < 4; ++q) {
-            c->tune.tpt_diff = tpts[q];
-            double t = 0.0;
-            if (time_ms(c, kReps, [&] { return launch_diffusion(c, s, s); }, &t)) return 1;
-            ++best.trials;
-            if (tpts[q] == def) ddef = t;
-            if (t < dbest) {
-                dbest = t;
-                best.tpt_diff = tpts[q];
-            }
-        }
+            field = choice;
+            return 0;
+        };
+        if (tune(c->tune.tpt_bs, best.tpt_bs, [&] { return launch_biot_savart(c, s, s, vinf_x, vinf_y); }, &bdef, &bbest) ||
+            tune(c->tune.tpt_diff, best.tpt_diff, [&] { return launch_diffusion(c, s, s); }, &ddef, &dbest))
+            return 1;
         best.ms_default = bdef + ddef;
         best.ms_best = bbest + dbest;
     }

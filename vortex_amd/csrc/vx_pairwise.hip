@@ -1553,11 +1553,12 @@ int launch_biot_savart(vx_case *c, int64_t n_tgt, int64_t n_src, double vinf_x, 
 // operands, so more targets per thread save no loads: 60001 vortices take
 // 1.02, 1.11, 1.44 and 1.53 ms (Biot-Savart, FP32) with 1, 2, 4 and 8, and
 // 2.42, 2.34, 2.52 and 3.00 ms in FP64.
-int direct_tpt_default(bool, int64_t) { return 1; }
+int direct_tpt_default() { return 1; }
+bool direct_uses_tpt(bool f32, int64_t n_src) { return f32 || n_src > kOrdered; }
 
-static int tpt_of(int want, bool f32, int64_t n_tgt) {
+static int tpt_of(int want) {
     if (want == 1 || want == 2 || want == 4 || want == 8) return want;
-    return direct_tpt_default(f32, n_tgt);
+    return direct_tpt_default();
 }
 
 // FP64: the ordered kernels up to kOrdered sources, the split ones above.  A
@@ -1597,7 +1598,7 @@ int launch_biot_savart(vx_case *c, Cnt n_tgt, Cnt n_src, double vinf_x, double v
     if (mixed(c)) {
         if (c->partial.ensure(direct_partials<float>(n_tgt, n_src, 6), c->stream) || launch_pack_f32(c, n_src))
             return 1;
-        bs_dispatch<float>(c, tpt_of(c->tune.tpt_bs, true, n_tgt.ub), c->xf.p, c->yf.p, c->gf.p, n_src, n_tgt,
+        bs_dispatch<float>(c, tpt_of(c->tune.tpt_bs), c->xf.p, c->yf.p, c->gf.p, n_src, n_tgt,
                            (float)eps2);
         hipLaunchKernelGGL(k_bs_sum<float>, gsum, dim3(256), 0, c->stream, c->partial.p, n_src, n_tgt, vinf_x, vinf_y,
                            c->u.p, c->v.p, c->d.p);
@@ -1614,7 +1615,7 @@ int launch_biot_savart(vx_case *c, Cnt n_tgt, Cnt n_src, double vinf_x, double v
         }
         if (takes_split(n_src)) {
             if (c->partial.ensure(direct_partials<double>(n_tgt, n_src, 6), c->stream)) return 1;
-            bs_dispatch<double>(c, tpt_of(c->tune.tpt_bs, false, n_tgt.ub), c->x.p, c->y.p, c->g.p, n_src, n_tgt,
+            bs_dispatch<double>(c, tpt_of(c->tune.tpt_bs), c->x.p, c->y.p, c->g.p, n_src, n_tgt,
                                 eps2);
             hipLaunchKernelGGL(k_bs_sum<double>, gsum, dim3(256), 0, c->stream, c->partial.p, n_src, n_tgt, vinf_x,
                                vinf_y, c->u.p, c->v.p, c->d.p);
@@ -1654,7 +1655,7 @@ int launch_diffusion(vx_case *c, Cnt n_tgt, Cnt n_src, bool packed) {
         if (c->partial.ensure(direct_partials<float>(n_tgt, n_src, 3), c->stream) ||
             (!packed && launch_pack_f32(c, n_src)))
             return 1;
-        diff_dispatch<float>(c, tpt_of(c->tune.tpt_diff, true, n_tgt.ub), c->xf.p, c->yf.p, c->gf.p, n_src, n_tgt,
+        diff_dispatch<float>(c, tpt_of(c->tune.tpt_diff), c->xf.p, c->yf.p, c->gf.p, n_src, n_tgt,
                              (float)(thr * thr));
         hipLaunchKernelGGL(k_diff_sum<float>, gsum, dim3(256), 0, c->stream, c->partial.p, n_src, n_tgt, c->d.p,
                            c->prm.nu, c->u.p, c->v.p);
@@ -1671,7 +1672,7 @@ int launch_diffusion(vx_case *c, Cnt n_tgt, Cnt n_src, bool packed) {
         }
         if (takes_split(n_src)) {
             if (c->partial.ensure(direct_partials<double>(n_tgt, n_src, 3), c->stream)) return 1;
-            diff_dispatch<double>(c, tpt_of(c->tune.tpt_diff, false, n_tgt.ub), c->x.p, c->y.p, c->g.p, n_src, n_tgt,
+            diff_dispatch<double>(c, tpt_of(c->tune.tpt_diff), c->x.p, c->y.p, c->g.p, n_src, n_tgt,
                                   thr);
             hipLaunchKernelGGL(k_diff_sum<double>, gsum, dim3(256), 0, c->stream, c->partial.p, n_src, n_tgt, c->d.p,
                                c->prm.nu, c->u.p, c->v.p);
