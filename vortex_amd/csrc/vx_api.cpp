@@ -824,7 +824,7 @@ static void step_key(vx_case *c, double vinf_x, double vinf_y, std::vector<uint6
     uint64_t w[2];
     memcpy(w, &vinf_x, 8);
     memcpy(w + 1, &vinf_y, 8);
-    k.insert(k.end(), {(uint64_t)c->n_ub, (uint64_t)step_tail_fits(c, c->n_ub), w[0], w[1], (uint64_t)c->prb_m,
+    k.insert(k.end(), {(uint64_t)c->n_ub, (uint64_t)step_tail_fits(c, c->n_ub), (uint64_t)direct_narrow(c), w[0], w[1], (uint64_t)c->prb_m,
                        (uint64_t)c->have_inverse, (uint64_t)c->tune.tpt_bs, (uint64_t)c->tune.tpt_diff,
                        (uint64_t)c->tune.col_share_min, (uint64_t)c->gr_cap});
     for (const void *p : std::initializer_list<const void *>{

@@ -355,6 +355,7 @@ int launch_live_box(vx_case *c);                       // box of g != 0 in [0, *
 // Collapse error flag in dcount[3].
 int launch_setka(vx_case *c, int kind, int64_t n_ub, bool prepare, bool after_pass = false);
 // default targets per thread of the direct kernels for n_tgt targets (vx_pairwise.hip)
+bool direct_narrow(const vx_case *c);                  // form of the ordered sums of a step on device counts
 int direct_tpt_default();                              // targets per thread
 bool direct_uses_tpt(bool f32, int64_t n_src);         // else the ordered sums, which have none
 // With reset, the collapse work arrays are left prepared for the next pass.

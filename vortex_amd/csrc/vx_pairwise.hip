@@ -1569,10 +1569,11 @@ static bool takes_split(Cnt n_src) { return n_src.ub > kOrdered; }
 // 16 targets per ordered work-group while that makes no more than one for each
 // CU, else 32: at 4000 vortices 40 and 52 us (Biot-Savart, diffusion) against
 // 47 and 82 with 32, at 6000 (two rounds of work-groups) 114 and 151 against
-// 73 and 126.  A device count goes by the host's last count; the results do
-// not depend on the choice.
+// 73 and 126.  A device count goes by the host's last count (a captured step is
+// kept for one of the two); the results do not depend on the choice.
 constexpr int64_t kOrdNarrow = 4096;
 static bool ord_narrow(const vx_case *c, Cnt n_tgt) { return (n_tgt.dev ? c->n : n_tgt.ub) <= kOrdNarrow; }
+bool direct_narrow(const vx_case *c) { return !mixed(c) && c->n <= kOrdNarrow; }
 
 template <typename T, int TPT>
 static void bs_launch(vx_case *c, const T *sx, const T *sy, const T *sg, Cnt n_src, Cnt n_tgt, T eps2) {
