@@ -3,10 +3,12 @@
 // velocities.  Each is templated on the arithmetic type:
 //   double  -- the reference formulas in FP64 (VX_PREC_F64);
 //   float   -- FP32 pair arithmetic, FP32 partial sums over one 256-source
-//              LDS tile, FP64 accumulation of the tile sums (VX_PREC_MIXED).
-// Sources are staged through LDS in 256-wide tiles (one wave64-aligned load
-// per thread, broadcast reads in the inner loop); each thread owns TPT
-// targets spaced one block apart so that target loads and stores coalesce.
+//              tile, FP64 accumulation of the tile sums (VX_PREC_MIXED).
+// The direct kernels read their sources as scalar operands and are cut over
+// targets (TPT a thread, spaced one block apart so that loads and stores
+// coalesce) and sources; FP64 sums over few sources are added in source order by
+// a wave of their own, from terms in LDS.  The probes and the right-hand side
+// stage their sources through LDS.
 #include <algorithm>
 #include <cfloat>
 #include <cmath>
@@ -64,7 +66,7 @@ constexpr int kTile = 256;
 //
 // 60001 vortices, FP32: Biot-Savart 2.66 -> 1.02 ms, diffusion 2.66 -> 1.29 ms
 // against one work-group per kTile targets over all sources; 20011 in FP64:
-// 1.76 -> 0.30 and 3.43 -> 0.47 ms.  With kDirectWork = 1024, 2048 and 8192
+// 1.76 -> 0.34 and 3.43 -> 0.69 ms.  With kDirectWork = 1024, 2048 and 8192
 // the first pair takes 1.30 and 1.59, 1.09 and 1.40, 1.01 and 1.27 ms; the
 // partials grow with it (48 B per target and run), so 4096.
 //
@@ -499,7 +501,7 @@ __global__ __launch_bounds__(256) void k_diff_sum(const double *__restrict__ par
 // ones alone 15; the reads of the next batch stand between the adds (all
 // before them: 3 % more).  2500 vortices: Biot-Savart 243 -> 25 us, diffusion
 // 475 -> 33 us against one lane per target over all sources.  Above kOrdered the split
-// sums are faster: at 17000 0.26 and 0.40 ms against 0.62 and 1.05 ms.
+// sums are faster: at 17000 0.27 and 0.54 ms against 0.64 and 1.12 ms.
 constexpr int kOrdWaves = 15;
 constexpr int kAhead = 6;  // pairs of terms per batch: the LDS latency of one is covered by the adds of another
 
@@ -1552,7 +1554,7 @@ int launch_biot_savart(vx_case *c, int64_t n_tgt, int64_t n_src, double vinf_x, 
 // same order, so the results do not depend on it.  Sources come as scalar
 // operands, so more targets per thread save no loads: 60001 vortices take
 // 1.02, 1.11, 1.44 and 1.53 ms (Biot-Savart, FP32) with 1, 2, 4 and 8, and
-// 2.42, 2.34, 2.52 and 3.00 ms in FP64.
+// 2.57, 2.58, 2.71 and 3.13 ms in FP64 (its diffusion 5.65, 5.73, 6.16, 7.21).
 int direct_tpt_default() { return 1; }
 bool direct_uses_tpt(bool f32, int64_t n_src) { return f32 || n_src > kOrdered; }
 

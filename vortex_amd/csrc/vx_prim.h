@@ -204,9 +204,9 @@ __global__ __launch_bounds__(kT) void k_flag_apply(F f, int64_t n, const int32_t
 }
 
 // Count, scan and apply in one launch of one work-group: a small selection is
-// all launch and latency (at 2785 of 8192 items, the hit candidates 23 -> 6.1 us,
-// the near sources 19 -> 5.4 us, the wall targets 16 -> 5.1 us; in a batch of
-// some 20000 each, 20 to 22 us -> 10 to 12).  The flags of a thread's items are
+// all launch and latency (at 2785 of 8192 items, the birth's near sources 19 ->
+// 5.4 us, the velocity stage's wall targets 16 -> 5.1 us; in a batch of some
+// 20000 each, 20 to 22 us -> 10 to 12).  The flags of a thread's items are
 // kept in a mask between the count and the writer, which sees each item once,
 // as above; its 32 bits set the limit.
 constexpr int64_t kOneMax = 32768;

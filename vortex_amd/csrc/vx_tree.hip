@@ -1417,9 +1417,9 @@ constexpr int kFarQ = 512;     // FP32: far nodes queued per wave before any M2L
 
 // S waves per bucket.  FP64 takes four up to kBsSplit buckets, each with every
 // fourth far node and near leaf: one each are three waves a SIMD at 131103
-// vortices, and the longest chain sets the time (0.54 -> 0.42 ms; 500000: 1.53
-// -> 1.46).  Each walks the tree by itself, which costs more than the balance
-// gives where there are waves enough (2^20: 2.89 -> 3.11).  FP32's far nodes
+// vortices, and the longest chain sets the time (0.61 -> 0.45 ms; 500000: 1.70
+// -> 1.59 to 1.66).  Each walks the tree by itself, which costs more than the
+// balance gives where there are waves enough (2^20: 3.05 -> 3.47).  FP32's far nodes
 // are translated 16 at a time, which wants them together: its first wave takes
 // them all, the near leaves are dealt over the four (66000 vortices: 142 ->
 // 120 us, 131103: 228 -> 177, 262177: 305 -> 290, 524288 the same, 2^20: 868
@@ -1994,11 +1994,15 @@ struct DiffPair<double> {
 // more per pair than a group's wave, though, and a sparse wake has many wide
 // targets side by side, which share their group's sources.  So FP64, whose
 // groups have four waves, draws the line at 10 % (66000, 90000 and 131103
-// vortices of a 10 x 4 wake: speed stage 2.52, 3.12 and 3.40 ms with 5 %, which
-// listed half of the targets and more; 1.23, 1.62 and 1.94 with 10 %, 1.25,
-// 1.58 and 1.94 with 20 %), FP32 at 5 %.  At most t.fcap targets are listed
+// vortices of a 10 x 4 wake: speed stage 1.62, 2.09 and 2.54 ms with 5 %, which
+// lists half of the targets and more; 1.33, 1.73 and 1.96 with 10 %, 1.28,
+// 1.70 and 1.98 with 20 %), FP32 at 5 %.  At most t.fcap targets are listed
 // (the most of kFarCap, one in 16 included vortices and a quarter more than
-// the last diffusion found); further ones stay in their group's wave.
+// the last diffusion found); further ones stay in their group's wave.  A case's
+// first diffusion knows no earlier count: where most targets are wide, all but
+// those many stay in their groups' waves then (mixed, 100000 vortices, 78993 of
+// them listed later: first speed stage 2.6 ms, the second, which also grows the
+// buffers, 1.4, then 0.9).
 constexpr int64_t kFarCap = 4096;
 template <typename T>
 constexpr double far_part() {
@@ -2024,11 +2028,10 @@ __device__ __forceinline__ int64_t far_count(const unsigned long long *cnt, int6
 // largest radius of its lanes reaches it and, lane by lane, when some lane's
 // own radius reaches it.  A lane whose radius exceeds far_radius() is listed for
 // k_diff_far instead and does not widen the wave's radius.  A group of at
-// most 32 targets gives each several lanes (LaneSplit).  In FP64 a group has
+// most 32 targets gives each several lanes (LaneSplit).  A group has
 // four waves, each with every fourth of the listed leaves: one each are two
-// waves a SIMD at 131103 vortices, and the longest chain sets the time (with the wider
-// groups of far_part, 1.46 -> 1.03 ms; the FP64 pair terms of vx_math.h
-// before that, 1.66 -> 1.06 ms).  cnt[0] +=
+// waves a SIMD at 131103 vortices, and the longest chain sets the time (1.46 -> 1.03 ms
+// when it was taken, with a shorter pair term; 1.21 now).  cnt[0] +=
 // evaluated pairs, cnt[2] the list length.
 constexpr int kDiffWaves = 4;  // per target group
 
@@ -2425,8 +2428,8 @@ __global__ __launch_bounds__(256) void k_chunk_box(TreeDev t, int64_t nchunk, do
 // within each target's radius, appended as (target, chunk) pairs, a chunk's
 // targets together (their waves then read the same buckets), with one atomic
 // for all of them.  One atomic and one chain of loads per target took 870 us
-// for the 78993 listed of 100000 vortices in mixed precision, more than their
-// sums (290); now 23.
+// for the 78993 listed of 100000 vortices in mixed precision (from a case's
+// second diffusion on, see far_part), more than their sums (290); now 23.
 __global__ __launch_bounds__(256) void k_far_pairs(TreeDev t, const int32_t *__restrict__ list,
                                                    const unsigned long long *__restrict__ cnt, int64_t nchunk,
                                                    const double4 *__restrict__ cbox, double cut,
