@@ -6,6 +6,8 @@
 
 #include <hip/hip_runtime.h>
 
+#include <cstdint>
+
 namespace vx {
 
 // g / a for a normal a > 0, correctly rounded as `/` gives it: the start's
@@ -69,14 +71,15 @@ __device__ __forceinline__ void keep4x4(double &m0, double &m1, double &m2, doub
 }
 
 // Neither NaN nor an infinity nor above 2^500, so that squares of differences
-// stay in range: the sizes (high words without sign) of several values are
-// compared at once by their maximum.  Integer operations only: on wave-uniform
-// values they run on the scalar unit.
-constexpr int kOrdinary = 0x5f300000;
-__device__ __forceinline__ int size_of(double v) { return __double2hiint(v) & 0x7fffffff; }
-__device__ __forceinline__ int size_of(float) { return 0; }  // FP32 takes every value through one path
+// stay in range.  odd_bit's top bit is set for any other value; the bits of several
+// values are or-ed.  Integer operations only: on wave-uniform values they run on
+// the scalar unit (a maximum of several would go to the vector unit's max3).
+__device__ __forceinline__ uint32_t odd_bit(double v) {
+    return ((uint32_t)__double2hiint(v) & 0x7fffffffu) + (0x80000000u - 0x5f300000u);
+}
+__device__ __forceinline__ uint32_t odd_bit(float) { return 0; }  // FP32 takes every value through one path
 template <typename T>
-__device__ __forceinline__ bool ordinary(T v) { return size_of(v) < kOrdinary; }
+__device__ __forceinline__ bool ordinary(T v) { return (int32_t)odd_bit(v) >= 0; }
 
 // A softening eps^2 that div_pos_exact divides by.
 __device__ __forceinline__ bool ordinary_eps2(double v) { return v > 0x1p-1000 && v < 0x1p1000; }

@@ -66,7 +66,7 @@ constexpr int kTile = 256;
 //
 // 60001 vortices, FP32: Biot-Savart 2.66 -> 1.02 ms, diffusion 2.66 -> 1.29 ms
 // against one work-group per kTile targets over all sources; 20011 in FP64:
-// 1.76 -> 0.34 and 3.43 -> 0.69 ms.  With kDirectWork = 1024, 2048 and 8192
+// 1.76 -> 0.32 and 3.43 -> 0.64 ms.  With kDirectWork = 1024, 2048 and 8192
 // the first pair takes 1.30 and 1.59, 1.09 and 1.40, 1.01 and 1.27 ms; the
 // partials grow with it (48 B per target and run), so 4096.
 //
@@ -204,15 +204,15 @@ __global__ __launch_bounds__(kTile) void k_biot_savart(const T *__restrict__ sx,
         int32_t j = base;
         for (; j + 4 <= end; j += 4) {
             T x[4], y[4], g[4];
-            int size = 0;
+            uint32_t odd = 0;
 #pragma unroll
             for (int q = 0; q < 4; ++q) {
                 x[q] = sx[j + q];
                 y[q] = sy[j + q];
                 g[q] = sg[j + q];
-                size = max(size, max(size_of(x[q]), max(size_of(y[q]), size_of(g[q]))));
+                odd |= odd_bit(x[q]) | odd_bit(y[q]) | odd_bit(g[q]);
             }
-            if (__builtin_expect(!tame || size >= kOrdinary, 0)) break;
+            if (__builtin_expect(!tame || (int32_t)odd < 0, 0)) break;
 #pragma unroll
             for (int k = 0; k < TPT; ++k) {
                 T r2[4];
@@ -362,26 +362,26 @@ __global__ __launch_bounds__(kTile) void k_diffusion(const T *__restrict__ sx, c
         int32_t j = lo;
         for (; j + 4 <= hi; j += 4) {
             double x[4], y[4], g[4];
-            int size = 0;
+            uint32_t odd = 0;
 #pragma unroll
             for (int q = 0; q < 4; ++q) {
                 x[q] = sx[j + q];
                 y[q] = sy[j + q];
                 g[q] = sg[j + q];
-                size = max(size, max(size_of(x[q]), max(size_of(y[q]), size_of(g[q]))));
+                odd |= odd_bit(x[q]) | odd_bit(y[q]) | odd_bit(g[q]);
             }
-            const bool plain = !tame || size >= kOrdinary;
+            const bool plain = !tame || (int32_t)odd < 0;
 #pragma unroll
             for (int k = 0; k < TPT; ++k) {
                 double r2[4];
-                bool near = plain;
+                uint64_t near = 0;
 #pragma unroll
                 for (int q = 0; q < 4; ++q) {
                     const double dx = ax[k] - x[q], dy = ay[k] - y[q];
                     r2[q] = fma(dx, dx, dy * dy);
-                    near = near || !(r2[q] > gap2);
+                    near |= __ballot(!(r2[q] > gap2));
                 }
-                if (__builtin_expect(__any(near), 0)) {
+                if (__builtin_expect(plain || near != 0, 0)) {
 #pragma unroll 1
                     for (int q = 0; q < 4; ++q)
                         diff_pair_plain(ax[k] - sx[j + q], ay[k] - sy[j + q], sg[j + q], kd[k], thr, sum[k]);
@@ -501,7 +501,7 @@ __global__ __launch_bounds__(256) void k_diff_sum(const double *__restrict__ par
 // ones alone 15; the reads of the next batch stand between the adds (all
 // before them: 3 % more).  2500 vortices: Biot-Savart 243 -> 25 us, diffusion
 // 475 -> 33 us against one lane per target over all sources.  Above kOrdered the split
-// sums are faster: at 17000 0.27 and 0.54 ms against 0.64 and 1.12 ms.
+// sums are faster: at 17000 0.25 and 0.50 ms against 0.64 and 1.12 ms.
 constexpr int kOrdWaves = 15;
 constexpr int kAhead = 6;  // pairs of terms per batch: the LDS latency of one is covered by the adds of another
 
@@ -1554,7 +1554,7 @@ int launch_biot_savart(vx_case *c, int64_t n_tgt, int64_t n_src, double vinf_x, 
 // same order, so the results do not depend on it.  Sources come as scalar
 // operands, so more targets per thread save no loads: 60001 vortices take
 // 1.02, 1.11, 1.44 and 1.53 ms (Biot-Savart, FP32) with 1, 2, 4 and 8, and
-// 2.57, 2.58, 2.71 and 3.13 ms in FP64 (its diffusion 5.65, 5.73, 6.16, 7.21).
+// 2.39, 2.45, 2.63 and 3.08 ms in FP64 (its diffusion 5.1, 5.4, 5.9, 7.0).
 int direct_tpt_default() { return 1; }
 bool direct_uses_tpt(bool f32, int64_t n_src) { return f32 || n_src > kOrdered; }
 
