@@ -274,8 +274,8 @@ int vx_collapse(vx_case *c, int kind, const int32_t *COL);
  * vx_case_autotune times every choice on the case's current state (the
  * direct kernels one by one below tree_min_n, the whole velocity stage
  * above it; FP64 direct sums that do not use the targets per thread are timed
- * once and leave the setting as it is), keeps the fastest and reports the default's and the chosen
- * configuration's time in milliseconds.  It overwrites u, v and d only. */
+ * once and leave the setting as it is), keeps the fastest and reports the
+ * default's and the chosen configuration's time in milliseconds.  It overwrites u, v and d only. */
 typedef struct vx_tuning {
     int32_t tpt_bs, tpt_diff;
     int32_t leaf_off;

@@ -762,8 +762,10 @@ int vx_case_autotune(vx_case *c, double vinf_x, double vinf_y, vx_tuning *out) {
             field = choice;
             return 0;
         };
-        if (tune(c->tune.tpt_bs, best.tpt_bs, [&] { return launch_biot_savart(c, s, s, vinf_x, vinf_y); }, &bdef, &bbest) ||
-            tune(c->tune.tpt_diff, best.tpt_diff, [&] { return launch_diffusion(c, s, s); }, &ddef, &dbest))
+        auto bs = [&] { return launch_biot_savart(c, s, s, vinf_x, vinf_y); };
+        auto diff = [&] { return launch_diffusion(c, s, s); };
+        if (tune(c->tune.tpt_bs, best.tpt_bs, bs, &bdef, &bbest) ||
+            tune(c->tune.tpt_diff, best.tpt_diff, diff, &ddef, &dbest))
             return 1;
         best.ms_default = bdef + ddef;
         best.ms_best = bbest + dbest;
@@ -824,8 +826,9 @@ static void step_key(vx_case *c, double vinf_x, double vinf_y, std::vector<uint6
     uint64_t w[2];
     memcpy(w, &vinf_x, 8);
     memcpy(w + 1, &vinf_y, 8);
-    k.insert(k.end(), {(uint64_t)c->n_ub, (uint64_t)step_tail_fits(c, c->n_ub), (uint64_t)direct_narrow(c), w[0], w[1], (uint64_t)c->prb_m,
-                       (uint64_t)c->have_inverse, (uint64_t)c->tune.tpt_bs, (uint64_t)c->tune.tpt_diff,
+    k.insert(k.end(), {(uint64_t)c->n_ub, (uint64_t)step_tail_fits(c, c->n_ub), (uint64_t)direct_narrow(c), w[0],
+                       w[1], (uint64_t)c->prb_m, (uint64_t)c->have_inverse, (uint64_t)c->tune.tpt_bs,
+                       (uint64_t)c->tune.tpt_diff,
                        (uint64_t)c->tune.col_share_min, (uint64_t)c->gr_cap});
     for (const void *p : std::initializer_list<const void *>{
              c->x.p,     c->y.p,     c->g.p,      c->u.p,      c->v.p,        c->d.p,      c->xf.p,    c->yf.p,
